@@ -1,5 +1,6 @@
 #include "context.h"
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -88,7 +89,7 @@ HostStaging::~HostStaging() {
 bool HostStaging::Init() {
   if (pinned_) return true;
   void* p = nullptr;
-  if (hipHostMalloc(&p, kChunks * kChunkBytes, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&p, kChunks * kChunkBytes + kDoneBytes, hipHostMallocCoherent) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
@@ -100,6 +101,7 @@ bool HostStaging::Init() {
     }
   }
   pinned_ = static_cast<char*>(p);
+  std::memset(pinned_ + kChunks * kChunkBytes, 0, kDoneBytes);
   return true;
 }
 
@@ -110,8 +112,15 @@ bool HostStaging::WaitFree(int c) {
   return true;
 }
 
+bool HostStaging::FlushPending(hipStream_t stream) {
+  const hipError_t status = LaunchUpload(stream, pending_);
+  pending_.count = 0;
+  return status == hipSuccess;
+}
+
 bool HostStaging::RetireCurrent(hipStream_t stream) {
   if (fill_ == 0) return true;
+  if (!Flush(stream)) return false;
   if (hipEventRecord(done_[current_], stream) != hipSuccess) return false;
   busy_[current_] = true;
   current_ = (current_ + 1) % kChunks;
@@ -134,7 +143,8 @@ bool IsPinnedHost(const void* p) {
 
 bool HostStaging::ToDevice(void* dst_dev, const void* src_host, std::size_t bytes, hipStream_t stream) {
   if (bytes == 0) return true;
-  if (IsPinnedHost(src_host))
+  const bool by_kernel = bytes <= kByKernel;
+  if (!by_kernel && IsPinnedHost(src_host))
     return hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream) == hipSuccess;
   if (!Init()) return false;
   const char* src = static_cast<const char*>(src_host);
@@ -151,7 +161,13 @@ bool HostStaging::ToDevice(void* dst_dev, const void* src_host, std::size_t byte
     const std::size_t n = bytes < kChunkBytes - at ? bytes : kChunkBytes - at;
     char* piece = pinned_ + std::size_t(current_) * kChunkBytes + at;
     std::memcpy(piece, src, n);
-    if (hipMemcpyAsync(dst, piece, n, hipMemcpyHostToDevice, stream) != hipSuccess) return false;
+    if (by_kernel) {  // (one piece: it fits a chunk)
+      if (pending_.count == UploadPieces::kMost && !FlushPending(stream)) return false;
+      pending_.from[pending_.count] = piece;
+      pending_.to[pending_.count] = dst;
+      pending_.bytes[pending_.count] = static_cast<uint32_t>(n);
+      ++pending_.count;
+    } else if (hipMemcpyAsync(dst, piece, n, hipMemcpyHostToDevice, stream) != hipSuccess) return false;
     fill_ = at + n;
     src += n;
     dst += n;
@@ -161,9 +177,49 @@ bool HostStaging::ToDevice(void* dst_dev, const void* src_host, std::size_t byte
   return true;
 }
 
+bool HostStaging::SmallToHost2D(char* dst, const void* src_dev, std::size_t pitch, std::size_t inner_bytes,
+                                std::size_t outer, hipStream_t stream, bool* drained) {
+  const std::size_t total = pitch * (outer - 1) + inner_bytes;
+  // The image goes behind what the current chunk already holds, if it fits.
+  std::size_t at = (fill_ + 255) & ~std::size_t(255);
+  if (at + total + 16 > kChunkBytes) {
+    if (!RetireCurrent(stream)) return false;
+    at = 0;
+  }
+  if (at == 0 && !WaitFree(current_)) return false;
+  char* const image = pinned_ + std::size_t(current_) * kChunkBytes + at;
+  uint32_t* const done = reinterpret_cast<uint32_t*>(pinned_ + kChunks * kChunkBytes);
+  const uint32_t value = ++downloads_;
+  if (LaunchDownload(stream, src_dev, image, total, done, value) != hipSuccess) return false;
+  const int words = DownloadBlocks(total);
+  // The words are looked at for some milliseconds, as long as any product of
+  // this size takes; beyond that (other work in front of it on the stream) the
+  // runtime does the waiting. Either way the copy has ended below.
+  using Clock = std::chrono::steady_clock;
+  const auto give_up = Clock::now() + std::chrono::milliseconds(10);
+  int seen = 0;
+  for (int looks = 1; seen < words; ++looks) {
+    while (seen < words && __atomic_load_n(done + seen, __ATOMIC_ACQUIRE) == value) ++seen;
+    if (seen < words && (looks & 255) == 0 && Clock::now() > give_up) break;
+  }
+  if (seen < words && hipStreamSynchronize(stream) != hipSuccess) return false;
+  *drained = true;
+  if (pitch == inner_bytes || outer == 1) {
+    std::memcpy(dst, image, total);
+  } else {
+    for (std::size_t run = 0; run < outer; ++run) std::memcpy(dst + run * pitch, image + run * pitch, inner_bytes);
+  }
+  return true;
+}
+
 bool HostStaging::ToHost2D(void* dst_host, const void* src_dev, std::size_t pitch, std::size_t inner_bytes,
-                           std::size_t outer, hipStream_t stream) {
+                           std::size_t outer, hipStream_t stream, bool* drained) {
+  *drained = false;
   if (inner_bytes == 0 || outer == 0) return true;
+  if (pitch * (outer - 1) + inner_bytes <= kByKernel) {
+    if (!Init()) return false;
+    return SmallToHost2D(static_cast<char*>(dst_host), src_dev, pitch, inner_bytes, outer, stream, drained);
+  }
   if (IsPinnedHost(dst_host)) {
     // Stream-ordered; complete once the caller has synchronised the stream.
     if (pitch == inner_bytes || outer == 1)
@@ -225,6 +281,7 @@ bool HostStaging::ToHost2D(void* dst_host, const void* src_dev, std::size_t pitc
 void HostStaging::Reset() {
   for (int c = 0; c < kChunks; ++c) busy_[c] = false;
   fill_ = 0;
+  pending_.count = 0;
 }
 
 }  // namespace ruyamd

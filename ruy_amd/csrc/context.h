@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "kernels/host_copy.h"
 #include "prepacked_cache.h"
 
 namespace ruyamd {
@@ -62,28 +63,53 @@ class Workspace {
 // pinned chunks: the CPU copies into (out of) a chunk while the copy engine
 // works on the previous ones, and every transfer the engine sees is a true
 // asynchronous pinned copy. Small operands share a chunk. Host memory that is
-// already page-locked skips the chunks and is copied directly. Used only by calls
+// already page-locked skips the chunks and is copied directly. Small transfers
+// (kByKernel bytes) do not use the copy engine at all: what a call uploads is
+// collected in a chunk and moved by one kernel when the first kernel that may
+// read it is about to be launched (Flush), and a small destination comes back
+// by a kernel whose completion the host sees in host memory
+// (kernels/host_copy.hip). Used only by calls
 // that were handed host pointers; such a call ends with a stream
-// synchronisation, after which Reset() makes all chunks available again.
+// synchronisation or a download seen to be complete, after which Reset()
+// makes all chunks available again.
 class HostStaging {
  public:
   ~HostStaging();
-  // dst_dev[0, bytes) = src_host[0, bytes), ordered on `stream`.
+  // dst_dev[0, bytes) = src_host[0, bytes), ordered on `stream` once Flush has
+  // been called. dst_dev is 16-byte aligned and has room for a whole number of
+  // 16-byte granules.
   bool ToDevice(void* dst_dev, const void* src_host, std::size_t bytes, hipStream_t stream);
   // Copies `outer` runs of `inner_bytes`, `pitch` bytes apart in both images,
   // from device to host after everything already enqueued on `stream`; the
   // bytes between the runs of the host image are not written. The host image
   // is complete when this returns (pageable destination) or once the stream
-  // has been synchronised (page-locked destination, copied directly).
+  // has been synchronised (page-locked destination, copied directly). *drained
+  // is set if everything enqueued on `stream` so far is known to have finished.
+  // src_dev as dst_dev in ToDevice.
   bool ToHost2D(void* dst_host, const void* src_dev, std::size_t pitch, std::size_t inner_bytes,
-                std::size_t outer, hipStream_t stream);
-  // Call after the stream has been synchronised.
+                std::size_t outer, hipStream_t stream, bool* drained);
+  // Forgets uploads that a failed call has left behind.
+  void DropPending() { pending_.count = 0; }
+  // Enqueues the uploads collected so far: before any kernel that may read them.
+  bool Flush(hipStream_t stream) { return pending_.count == 0 || FlushPending(stream); }
+  // Call after the stream has been synchronised (or seen drained).
   void Reset();
 
  private:
   static constexpr std::size_t kChunkBytes = std::size_t(4) << 20;
   static constexpr int kChunks = 4;
+  // Up to here a kernel moves a transfer faster than the copy engine does,
+  // counting what it costs the streams to hand over to that engine and back
+  // (int8, cached weights, whole calls by the copy engine -> by kernels: 200 KB
+  // each way 73 -> 40 us, 1 MiB each way 141 -> 118 us; 2 MiB and more gain from
+  // the engine's higher rate and from the CPU filling the next chunk meanwhile).
+  static constexpr std::size_t kByKernel = std::size_t(1) << 20;
+  // Behind the chunks: one word per workgroup of a download.
+  static constexpr std::size_t kDoneBytes = kByKernel / kHostCopyBlockBytes * sizeof(uint32_t);
   bool Init();
+  bool FlushPending(hipStream_t stream);
+  bool SmallToHost2D(char* dst, const void* src_dev, std::size_t pitch, std::size_t inner_bytes, std::size_t outer,
+                     hipStream_t stream, bool* drained);
   // Makes chunk c reusable: waits for the transfer that last used it.
   bool WaitFree(int c);
   bool RetireCurrent(hipStream_t stream);
@@ -91,7 +117,9 @@ class HostStaging {
   hipEvent_t done_[kChunks] = {};
   bool busy_[kChunks] = {};
   int current_ = 0;            // chunk being filled by ToDevice
-  std::size_t fill_ = 0;       // bytes of it already handed to the copy engine
+  std::size_t fill_ = 0;       // bytes of it already handed to the copy engine or collected in pending_
+  UploadPieces pending_;       // pieces of the current chunk that no launch has moved yet
+  uint32_t downloads_ = 0;     // the value the last download's workgroups left in their words
 };
 
 }  // namespace ruyamd
@@ -143,6 +171,14 @@ struct ruyamd_ctx {
   bool kernel_timing = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> timing_pending;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> timing_pool;
+  // The stream for a kernel that may read the call's operands: whatever has
+  // been collected for upload is enqueued first (upload_failed if that fails;
+  // the call then reports it).
+  hipStream_t LaunchStream() {
+    if (!staging.Flush(stream)) upload_failed = true;
+    return stream;
+  }
+  bool upload_failed = false;
   // Brackets for the dispatcher: Begin returns false if timing is off.
   bool TimingBegin();
   void TimingEnd();

@@ -289,6 +289,7 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
   ctx->ws->Reset();
 
   bool staged = false, ok = true;
+  ctx->staging.DropPending();
   const int channels = p->channel_dimension == RUYAMD_CHANNEL_ROW ? dst->rows : dst->cols;
   // The two source matrices are staged lazily by the dispatcher (a cache hit
   // needs no copy); the small per-channel vectors are staged now.
@@ -313,7 +314,12 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
   if (!rhs_dev) call.rhs_host_bytes = StorageElements(*rhs) * DtypeSize(rhs->dtype);
 
   std::string err;
-  const int rc = RunMul(ctx, &call, &err);
+  ctx->upload_failed = false;
+  int rc = RunMul(ctx, &call, &err);
+  if (rc == RUYAMD_OK && ctx->upload_failed) {
+    err = "staging host operands to the device failed";
+    rc = RUYAMD_E_HIP;
+  }
   if (rc != RUYAMD_OK) {
     if (no_alloc && ctx->ws->exhausted()) {
       char msg[192];
@@ -330,16 +336,17 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
   capture_scope.Recorded();
   staged = staged || call.staged_any;
 
+  bool drained = false;  // everything enqueued so far is known to have finished
   if (!dst_on_device) {
     const std::size_t inner = dst->order == RUYAMD_ORDER_COL_MAJOR ? dst->rows : dst->cols;
     const std::size_t outer = dst->order == RUYAMD_ORDER_COL_MAJOR ? dst->cols : dst->rows;
     const std::size_t pitch = std::size_t(dst->stride) * dst_elt;
-    if (!ctx->staging.ToHost2D(dst->data, dst_d, pitch, inner * dst_elt, outer, ctx->stream))
+    if (!ctx->staging.ToHost2D(dst->data, dst_d, pitch, inner * dst_elt, outer, ctx->stream, &drained))
       return Fail(ctx, RUYAMD_E_HIP, std::string("copying the destination back to the host failed: ") +
                                          hipGetErrorString(hipGetLastError()));
     staged = true;
   }
-  if ((ctx->synchronous || staged) && !ctx->capturing) {
+  if ((ctx->synchronous || staged) && !ctx->capturing && !drained) {
     if (hipStreamSynchronize(ctx->stream) != hipSuccess)
       return Fail(ctx, RUYAMD_E_HIP, std::string("kernel execution failed: ") + hipGetErrorString(hipGetLastError()));
   }
@@ -466,6 +473,8 @@ extern "C" int ruyamd_apply_multiplier(ruyamd_ctx* ctx, const int32_t* x, const 
   if (!x || !m || !e || !out) return Fail(ctx, RUYAMD_E_INVALID, "null argument");
   if (hipSetDevice(ctx->device) != hipSuccess) return Fail(ctx, RUYAMD_E_HIP, "hipSetDevice failed");
   ctx->workspace.Reset();
+  ctx->upload_failed = false;
+  ctx->staging.DropPending();
   bool staged = false, ok = true;
   const std::size_t bytes = std::size_t(n) * 4;
   const int32_t* xd = static_cast<const int32_t*>(StageIn(ctx, x, IsDevicePointer(x), bytes, &staged, &ok));
@@ -475,11 +484,14 @@ extern "C" int ruyamd_apply_multiplier(ruyamd_ctx* ctx, const int32_t* x, const 
   const bool out_dev = IsDevicePointer(out);
   int32_t* od = out_dev ? out : static_cast<int32_t*>(ctx->workspace.Alloc(bytes));
   if (!od) return Fail(ctx, RUYAMD_E_HIP, "device allocation failed");
-  if (LaunchApplyMultiplier(ctx->stream, xd, md, ed, od, n) != hipSuccess)
+  if (LaunchApplyMultiplier(ctx->LaunchStream(), xd, md, ed, od, n) != hipSuccess)
     return Fail(ctx, RUYAMD_E_HIP, "launch failed");
-  if (!out_dev && !ctx->staging.ToHost2D(out, od, bytes, bytes, 1, ctx->stream))
+  bool drained = false;
+  if (!out_dev && !ctx->staging.ToHost2D(out, od, bytes, bytes, 1, ctx->stream, &drained))
     return Fail(ctx, RUYAMD_E_HIP, "copy back failed");
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return Fail(ctx, RUYAMD_E_HIP, "kernel execution failed");
+  if (ctx->upload_failed) return Fail(ctx, RUYAMD_E_HIP, "staging failed");
+  if (!drained && hipStreamSynchronize(ctx->stream) != hipSuccess)
+    return Fail(ctx, RUYAMD_E_HIP, "kernel execution failed");
   ctx->staging.Reset();
   return RUYAMD_OK;
 }

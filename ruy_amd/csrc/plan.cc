@@ -61,7 +61,7 @@ int MaterializeSums(ruyamd_ctx* ctx, Operand8* op, int32_t K, std::string* err) 
     *err = "workspace allocation failed";
     return RUYAMD_E_HIP;
   }
-  if (LaunchSumsI8(ctx->stream, op->data, op->ld, op->count, K, sums, op->flip) != hipSuccess) {
+  if (LaunchSumsI8(ctx->LaunchStream(), op->data, op->ld, op->count, K, sums, op->flip) != hipSuccess) {
     *err = "sums kernel launch failed";
     return RUYAMD_E_HIP;
   }
@@ -108,10 +108,10 @@ bool WorthPairing(const PendingPack8& p) {
 int LaunchPendingPacks8(ruyamd_ctx* ctx, PendingPack8* a, PendingPack8* b, std::string* err) {
   hipError_t status = hipSuccess;
   if (a->pending && b->pending && WorthPairing(*a) && WorthPairing(*b)) {
-    status = LaunchPackI8Pair(ctx->stream, a->src, a->dst, a->ld, a->sums, b->src, b->dst, b->ld, b->sums);
+    status = LaunchPackI8Pair(ctx->LaunchStream(), a->src, a->dst, a->ld, a->sums, b->src, b->dst, b->ld, b->sums);
   } else {
-    if (a->pending) status = LaunchPackI8(ctx->stream, a->src, a->dst, a->ld, a->sums);
-    if (status == hipSuccess && b->pending) status = LaunchPackI8(ctx->stream, b->src, b->dst, b->ld, b->sums);
+    if (a->pending) status = LaunchPackI8(ctx->LaunchStream(), a->src, a->dst, a->ld, a->sums);
+    if (status == hipSuccess && b->pending) status = LaunchPackI8(ctx->LaunchStream(), b->src, b->dst, b->ld, b->sums);
   }
   a->pending = b->pending = false;
   if (status != hipSuccess) {
@@ -189,7 +189,7 @@ int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point
         return rc;
       }
       src = view();
-      if (LaunchPackI8(ctx->stream, src, static_cast<int8_t*>(pm.data), ld, pm.sums) != hipSuccess) {
+      if (LaunchPackI8(ctx->LaunchStream(), src, static_cast<int8_t*>(pm.data), ld, pm.sums) != hipSuccess) {
         ctx->cache->Erase(src_key, pm);
         *err = "pack kernel launch failed";
         return RUYAMD_E_HIP;
@@ -231,7 +231,7 @@ int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point
     defer->ld = ld;
     defer->sums = sums;
     defer->bytes = packed_bytes;
-  } else if (LaunchPackI8(ctx->stream, src, packed, ld, sums) != hipSuccess) {
+  } else if (LaunchPackI8(ctx->LaunchStream(), src, packed, ld, sums) != hipSuccess) {
     *err = "pack kernel launch failed";
     return RUYAMD_E_HIP;
   }
@@ -389,7 +389,7 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     }
     g.dst = call->dst;
     const bool timed = ctx->TimingBegin();
-    const hipError_t launched = LaunchGemvI8(ctx->stream, g);
+    const hipError_t launched = LaunchGemvI8(ctx->LaunchStream(), g);
     if (timed) ctx->TimingEnd();
     if (launched != hipSuccess) {
       *err = "int8 skinny kernel launch failed";
@@ -444,7 +444,7 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   if (sides & 1) args.ep.lhs_sums = nullptr;  // the kernel does not look there
   if (sides & 2) args.ep.rhs_sums = nullptr;
   const bool timed = ctx->TimingBegin();
-  const hipError_t launched = LaunchGemmI8(ctx->stream, args, ctx->multiprocessor_count);
+  const hipError_t launched = LaunchGemmI8(ctx->LaunchStream(), args, ctx->multiprocessor_count);
   if (timed) ctx->TimingEnd();
   if (launched != hipSuccess) {
     *err = "int8 MFMA kernel launch failed";
@@ -481,10 +481,10 @@ struct PendingPackF32 {
 int LaunchPendingPacksF32(ruyamd_ctx* ctx, PendingPackF32* a, PendingPackF32* b, std::string* err) {
   hipError_t status = hipSuccess;
   if (a->pending && b->pending && a->bytes <= kPairedPackLimit && b->bytes <= kPairedPackLimit) {
-    status = LaunchPackF32Pair(ctx->stream, a->src, a->dst, a->ld, b->src, b->dst, b->ld);
+    status = LaunchPackF32Pair(ctx->LaunchStream(), a->src, a->dst, a->ld, b->src, b->dst, b->ld);
   } else {
-    if (a->pending) status = LaunchPackF32(ctx->stream, a->src, a->dst, a->ld);
-    if (status == hipSuccess && b->pending) status = LaunchPackF32(ctx->stream, b->src, b->dst, b->ld);
+    if (a->pending) status = LaunchPackF32(ctx->LaunchStream(), a->src, a->dst, a->ld);
+    if (status == hipSuccess && b->pending) status = LaunchPackF32(ctx->LaunchStream(), b->src, b->dst, b->ld);
   }
   a->pending = b->pending = false;
   if (status != hipSuccess) {
@@ -534,7 +534,7 @@ int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy
         return rc;
       }
       src = view();
-      if (LaunchPackF32(ctx->stream, src, static_cast<float*>(pm.data), ld) != hipSuccess) {
+      if (LaunchPackF32(ctx->LaunchStream(), src, static_cast<float*>(pm.data), ld) != hipSuccess) {
         ctx->cache->Erase(src_key, pm);
         *err = "pack kernel launch failed";
         return RUYAMD_E_HIP;
@@ -570,7 +570,7 @@ int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy
     defer->dst = packed;
     defer->ld = ld;
     defer->bytes = packed_bytes;
-  } else if (LaunchPackF32(ctx->stream, src, packed, ld) != hipSuccess) {
+  } else if (LaunchPackF32(ctx->LaunchStream(), src, packed, ld) != hipSuccess) {
     *err = "pack kernel launch failed";
     return RUYAMD_E_HIP;
   }
@@ -628,7 +628,7 @@ int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     g.ep = call->ep;
     g.dst = call->dst;
     const bool timed = ctx->TimingBegin();
-    const hipError_t launched = LaunchGemvF32(ctx->stream, g);
+    const hipError_t launched = LaunchGemvF32(ctx->LaunchStream(), g);
     if (timed) ctx->TimingEnd();
     if (launched != hipSuccess) {
       *err = "fp32 skinny kernel launch failed";
@@ -656,7 +656,7 @@ int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   args.n_logical = args.N;
   PlanDepthSplit(ctx, GemmKind::kF32, &args);
   const bool timed = ctx->TimingBegin();
-  const hipError_t launched = LaunchGemmF32(ctx->stream, args, ctx->multiprocessor_count);
+  const hipError_t launched = LaunchGemmF32(ctx->LaunchStream(), args, ctx->multiprocessor_count);
   if (timed) ctx->TimingEnd();
   if (launched != hipSuccess) {
     *err = "fp32 matrix-core kernel launch failed";
@@ -726,7 +726,7 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
         const DevMat& m = side16 == 0 ? call->lhs : call->rhs;
         const PackSource fresh = side16 == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
                                              : PackSource{m.data, m.cs, m.rs, m.cols, m.rows, m.dtype};
-        if (LaunchPackI16Split(ctx->stream, fresh, static_cast<int8_t*>(pm.data), ld) != hipSuccess) {
+        if (LaunchPackI16Split(ctx->LaunchStream(), fresh, static_cast<int8_t*>(pm.data), ld) != hipSuccess) {
           ctx->cache->Erase(key16, pm);
           *err = "int16 pack kernel launch failed";
           return RUYAMD_E_HIP;
@@ -782,7 +782,7 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
       PlanDepthSplit(ctx, GemmKind::kInt8Int16, &args);
       if (GemmI8I16CanUseRawInt16(args, ctx->multiprocessor_count)) {
         const bool timed = ctx->TimingBegin();
-        const hipError_t launched = LaunchGemmI8I16Raw(ctx->stream, args, ctx->multiprocessor_count);
+        const hipError_t launched = LaunchGemmI8I16Raw(ctx->LaunchStream(), args, ctx->multiprocessor_count);
         if (timed) ctx->TimingEnd();
         if (launched != hipSuccess) {
           *err = "int8 x int16 matrix-core kernel launch failed";
@@ -799,7 +799,7 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
       *err = "workspace allocation failed";
       return RUYAMD_E_HIP;
     }
-    if (LaunchPackI16Split(ctx->stream, fresh, planes, ld) != hipSuccess) {
+    if (LaunchPackI16Split(ctx->LaunchStream(), fresh, planes, ld) != hipSuccess) {
       *err = "int16 pack kernel launch failed";
       return RUYAMD_E_HIP;
     }
@@ -810,7 +810,7 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   if (int rc = decide_sums()) return rc;
   if (args.split_k == 1) PlanDepthSplit(ctx, GemmKind::kInt8Int16, &args);
   const bool timed = ctx->TimingBegin();
-  const hipError_t launched = LaunchGemmI8I16(ctx->stream, args, ctx->multiprocessor_count);
+  const hipError_t launched = LaunchGemmI8I16(ctx->LaunchStream(), args, ctx->multiprocessor_count);
   if (timed) ctx->TimingEnd();
   if (launched != hipSuccess) {
     *err = "int8 x int16 matrix-core kernel launch failed";
@@ -979,7 +979,7 @@ int CacheGenericOperand(ruyamd_ctx* ctx, MulCall* call, int side, std::string* e
       ctx->cache->Erase(key, pm);
       return rc;
     }
-    if (LaunchReorder(ctx->stream, m, copy) != hipSuccess) {
+    if (LaunchReorder(ctx->LaunchStream(), m, copy) != hipSuccess) {
       ctx->cache->Erase(key, pm);
       *err = "copy kernel launch failed";
       return RUYAMD_E_HIP;
@@ -995,7 +995,7 @@ int RunGeneric(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   if (int rc = CacheGenericOperand(ctx, call, 1, err)) return rc;
   if (int rc = EnsureOnDevice(ctx, call, 0, err)) return rc;
   if (int rc = EnsureOnDevice(ctx, call, 1, err)) return rc;
-  if (LaunchGeneric(ctx->stream, call->lhs, call->rhs, call->ep, call->dst, call->accum_dtype) != hipSuccess) {
+  if (LaunchGeneric(ctx->LaunchStream(), call->lhs, call->rhs, call->ep, call->dst, call->accum_dtype) != hipSuccess) {
     *err = "generic kernel launch failed";
     return RUYAMD_E_HIP;
   }
@@ -1030,7 +1030,7 @@ int RunTuned(ruyamd_ctx* ctx, MulCall* call, TunedPath path, std::string* err) {
       t.cs = dst_col_major ? 1 : t.rows;
       if (int rc = RunI8I16(ctx, &flipped, err)) return rc;
       call->staged_any = call->staged_any || flipped.staged_any;
-      if (LaunchReorder(ctx->stream, t, call->dst) != hipSuccess) {
+      if (LaunchReorder(ctx->LaunchStream(), t, call->dst) != hipSuccess) {
         *err = "reorder kernel launch failed";
         return RUYAMD_E_HIP;
       }

@@ -207,6 +207,26 @@ def test_large_host_pointer_operands_and_the_staging_advisory(device_ctx):
     compare(f, D.host_pointer_mul(device_ctx, f, dst_fill=0), O.oracle_mul(f, fill=0))
 
 
+@pytest.mark.parametrize("shape", [
+    (1, 16, 1),            # single bytes
+    (128, 40, 128),        # a destination of exactly one workgroup's 16 KiB
+    (113, 145, 145),       # ... and of one byte more
+    (1024, 1024, 1024),    # everything exactly at the limit of the kernel copies
+    (1025, 1023, 1025),    # a destination beyond it, operands on either side
+    (2049, 512, 511)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_host_pointer_transfers_by_kernels_and_by_the_copy_engine(device_ctx, shape, strided):
+    """Sizes at the edges of what the copy kernels move (a block's 16 KiB, the
+    limit of 1 MiB), repeated so that chunks and completion words are reused."""
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(shape[0])
+    for orders in (cases.RCC, (0, 1, 1)):
+        p = W.random_problem(rng, S.I8, S.I8, S.I32, S.I8, *shape, *orders, strided=strided, name="host %s" % (shape,))
+        want = expected(p, fill=0x5A)
+        for _ in range(3):
+            compare(p, D.host_pointer_mul(device_ctx, p, dst_fill=0x5A), want)
+
+
 def test_empty_and_degenerate_shapes(device_ctx):
     from ruy_amd import device_problem as D
     rng = np.random.default_rng(6)
