@@ -1,4 +1,4 @@
-// Launch interfaces of the int8 kernels and of the pack / sums kernels.
+// Launch interfaces of the matrix-core and skinny kernels and of the sums kernel.
 #ifndef RUY_AMD_CSRC_KERNELS_GEMM_I8_H_
 #define RUY_AMD_CSRC_KERNELS_GEMM_I8_H_
 
@@ -254,45 +254,6 @@ hipError_t LaunchGemvF32(hipStream_t stream, const GemvI8Args& args);
 // Its 2..16-vector case: the matrix-core streaming kernel of the int8 path on
 // fp32 matrix instructions.
 hipError_t LaunchGemvF32Mma(hipStream_t stream, const GemvI8Args& args);
-
-// A matrix seen as `count` depth-vectors of length K: vector c, depth k is
-// data[c * stride_c + k * stride_k] (elements of `dtype`, uint8 or int8).
-struct PackSource {
-  const void* data = nullptr;
-  int64_t stride_c = 0;
-  int64_t stride_k = 0;
-  int32_t count = 0;
-  int32_t K = 0;
-  int32_t dtype = 0;
-};
-
-// The device form of the reference's Pack (ruy/pack.h:105-132 with the
-// uint8 -> int8 conversion of ruy/pack_common.h:36-58): writes vector c as int8
-// at dst + c*ld (depth-contiguous, zero-filled from K up to ld) and, when
-// `sums` is non-null, sums[c] = sum over the K real depth positions of the
-// packed values.
-hipError_t LaunchPackI8(hipStream_t stream, const PackSource& src, int8_t* dst, int32_t ld,
-                        int32_t* sums);
-
-// int16 operand for the int8 matrix cores: each value v is split into
-// hi = v >> 8 (signed) and lo = (v & 0xff) - 128, both int8, so that
-// v = 256*hi + lo + 128. For every group of 32 vectors the 32 hi vectors are
-// written first, then the 32 lo vectors: vector c of plane p lands at
-// dst + ((c/32)*64 + p*32 + c%32) * ld. Vectors past `count` inside the last
-// group and depth past K are zero. The destination holds
-// ceil(count/32)*64 vectors.
-hipError_t LaunchPackI16Split(hipStream_t stream, const PackSource& src, int8_t* dst, int32_t ld);
-
-// fp32 counterpart: vector c as floats at dst + c*ld (ld in elements, a
-// multiple of 4), zero-filled from K up to ld. `src.dtype` is fp32.
-hipError_t LaunchPackF32(hipStream_t stream, const PackSource& src, float* dst, int32_t ld);
-// Both operands of a small multiplication packed by one launch (same results
-// as two LaunchPackI8 / LaunchPackF32 calls).
-hipError_t LaunchPackI8Pair(hipStream_t stream, const PackSource& src_a, int8_t* dst_a, int32_t ld_a,
-                            int32_t* sums_a, const PackSource& src_b, int8_t* dst_b, int32_t ld_b,
-                            int32_t* sums_b);
-hipError_t LaunchPackF32Pair(hipStream_t stream, const PackSource& src_a, float* dst_a, int32_t ld_a,
-                             const PackSource& src_b, float* dst_b, int32_t ld_b);
 
 // dst(i, j) = src(i, j): same shape and element size, any two storage orders
 // (strides in elements).

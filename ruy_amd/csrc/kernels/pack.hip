@@ -11,6 +11,7 @@
 
 #include "../internal.h"
 #include "gemm_i8.h"
+#include "pack.h"
 
 namespace ruyamd {
 namespace {
@@ -18,9 +19,13 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t UnalignedU32 __attribute__((aligned(1)));
 
-constexpr int kTileC = 64;  // vectors per block
-constexpr int kTileK = 64;  // depth bytes per step
+typedef v4i v4i_unaligned __attribute__((aligned(1)));
+
+constexpr int kThreads = 256;
+constexpr int kTileC = 64;  // transposed 8-bit source: vectors per block
+constexpr int kTileK = 64;  // ... and depth bytes per step
 constexpr int kPitch = kTileK + 4;  // LDS row pitch in bytes (breaks bank alignment)
+constexpr int kTile32 = 32;  // transposed fp32 source: vectors per block and depth positions per step
 
 __device__ __forceinline__ int WaveSum(int v) {
 #pragma unroll
@@ -28,197 +33,115 @@ __device__ __forceinline__ int WaveSum(int v) {
   return v;
 }
 
-__global__ void ZeroI32Kernel(int32_t* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-// Block = 256 threads = one 64-vector x (k_span) slab, walked 64 depth bytes at
-// a time through LDS so that both the read (along the source's contiguous
-// dimension) and the write (along depth) are coalesced.
-// (`bx`, `by` of `ny`: which slab of vectors and which depth span.)
-__device__ __forceinline__ void PackI8Block(const PackSource& src, int8_t* dst, int32_t ld, int32_t* sums,
-                                            int k_span, int bx, int by, int ny, uint8_t* tile) {
-  const int tid = threadIdx.x;
-  const int c0 = bx * kTileC;
-  const int k_begin = by * k_span;
-  const int k_end = min(k_begin + k_span, ld);  // includes the zero-filled padding
-  const uint8_t* s = static_cast<const uint8_t*>(src.data);
-  const uint32_t flip = src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
-  const bool depth_contiguous = src.stride_k == 1;
-  // writer role: vector wc, 16-byte granule wg of the 64-byte step
-  const int wc = tid >> 2;
-  const int wg = tid & 3;
-  int32_t sum = 0;
-  for (int k0 = k_begin; k0 < k_end; k0 += kTileK) {
-    if (depth_contiguous) {
-      const int tx = tid & 63;  // depth
-      const int k = k0 + tx;
-#pragma unroll 4
-      for (int cc = tid >> 6; cc < kTileC; cc += 4) {
-        const int c = c0 + cc;
-        uint8_t v = 0;
-        if (c < src.count && k < src.K) v = s[c * src.stride_c + k];
-        tile[cc * kPitch + tx] = v;
-      }
-    } else {
-      const int tx = tid & 63;  // vector
-      const int c = c0 + tx;
-#pragma unroll 4
-      for (int kk = tid >> 6; kk < kTileK; kk += 4) {
-        const int k = k0 + kk;
-        uint8_t v = 0;
-        if (c < src.count && k < src.K) v = s[c * src.stride_c + k * src.stride_k];
-        tile[tx * kPitch + kk] = v;
-      }
-    }
-    __syncthreads();
-    const int c = c0 + wc;
-    const int k = k0 + wg * 16;
-    if (c < src.count && k < ld) {
-      const uint32_t* row = reinterpret_cast<const uint32_t*>(tile + wc * kPitch + wg * 16);
-      v4i out;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        // Padding bytes were stored as 0 and must stay 0: flip only real ones.
-        uint32_t w = row[d];
-        const int kd = k + 4 * d;
-        if (flip) {
-          uint32_t mask = kd + 4 <= src.K ? 0xffffffffu
-                          : kd >= src.K  ? 0u
-                                         : (0xffffffffu >> (8 * (kd + 4 - src.K)));
-          w ^= flip & mask;
-        }
-        out[d] = static_cast<int>(w);
-        sum = __builtin_amdgcn_sdot4(static_cast<int>(w), 0x01010101, sum, false);
-      }
-      *reinterpret_cast<v4i*>(dst + int64_t(c) * ld + k) = out;
-    }
-    __syncthreads();
-  }
-  if (sums) {
-    // the 4 granule-writers of a vector are adjacent lanes
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    const int c = c0 + wc;
-    if (wg == 0 && c < src.count) {
-      if (ny == 1)
-        sums[c] = sum;
-      else
-        atomicAdd(&sums[c], sum);
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void PackI8Kernel(PackSource src, int8_t* dst, int32_t ld,
-                                                   int32_t* sums, int k_span) {
-  __shared__ __attribute__((aligned(16))) uint8_t tile[kTileC * kPitch];
-  PackI8Block(src, dst, ld, sums, k_span, blockIdx.x, blockIdx.y, gridDim.y, tile);
-}
-
-
-// Depth-contiguous source (any alignment, any depth): one wave per vector (or
-// per part of a vector when there are few vectors) streams it 1024 bytes at a
-// time, 16 output bytes per lane. The source is read as aligned dwords - up
-// to five around the lane's 16 bytes - and brought into place with
-// v_alignbyte_b32, so no byte loads are needed for unaligned rows. A dword
-// may reach up to three bytes before or past the row, always inside an
-// aligned dword that also holds a byte of the row.
-__device__ __forceinline__ void PackI8RowsBlock(const PackSource& src, int8_t* dst, int32_t ld, int32_t* sums,
-                                                int k_span, int bx, int by, int ny) {
-  const int lane = threadIdx.x & 63;
-  const int c = bx * 4 + (threadIdx.x >> 6);
-  if (c >= src.count) return;
-  const uint8_t* row = static_cast<const uint8_t*>(src.data) + int64_t(c) * src.stride_c;
-  const uint32_t flip = src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
-  const int K = src.K;
-  const int k_begin = by * k_span;
-  const int k_end = min(k_begin + k_span, ld);
-  int8_t* out_row = dst + int64_t(c) * ld;
-  int32_t sum = 0;
-  for (int k = k_begin + lane * 16; k < k_end; k += 1024) {
-    v4i out = {0, 0, 0, 0};
-    if (k < K) {
-      const uintptr_t address = reinterpret_cast<uintptr_t>(row + k);
-      const int shift = static_cast<int>(address & 3);
-      const uint32_t* p = reinterpret_cast<const uint32_t*>(address - shift);
-      const int n = min(16, K - k);             // source bytes this lane needs
-      const int words = (shift + n + 3) >> 2;   // aligned dwords that hold them, 1..5
-      uint32_t d[5];
-#pragma unroll
-      for (int i = 0; i < 5; ++i) d[i] = i < words ? p[i] : 0u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        uint32_t w = __builtin_amdgcn_alignbyte(d[i + 1], d[i], shift);
-        const int kd = k + 4 * i;
-        // Bytes past the depth are padding and stay 0 (they are not flipped either).
-        const uint32_t mask = kd + 4 <= K ? 0xffffffffu : kd >= K ? 0u : (0xffffffffu >> (8 * (kd + 4 - K)));
-        w = (w & mask) ^ (flip & mask);
-        out[i] = static_cast<int>(w);
-        sum = __builtin_amdgcn_sdot4(static_cast<int>(w), 0x01010101, sum, false);
-      }
-    }
-    *reinterpret_cast<v4i*>(out_row + k) = out;
-  }
-  if (sums) {
-    const int32_t total = WaveSum(sum);
-    if (lane == 0) {
-      if (ny == 1)
-        sums[c] = total;
-      else
-        atomicAdd(&sums[c], total);
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void PackI8RowsKernel(PackSource src, int8_t* dst, int32_t ld,
-                                                       int32_t* sums, int k_span) {
-  PackI8RowsBlock(src, dst, ld, sums, k_span, blockIdx.x, blockIdx.y, gridDim.y);
-}
-
-// Both operands of a small multiplication in one launch (blockIdx.z says which
-// one): the second launch would cost more than the packing itself. Each side
-// is packed over its whole depth by the depth-contiguous scheme above or by
-// the generic one.
-struct PackPairI8 {
-  PackSource src[2];
-  int8_t* dst[2];
-  int32_t ld[2];
-  int32_t* sums[2];
+// How a launch packs one operand: depth-contiguous rows with 16 or 64 lanes to
+// a row, or a transposed source. Compile-time, so that a kernel holds nothing
+// but what it needs (these kernels run for a microsecond or two: fetching the
+// instructions of the other kinds, a division by a lane count and a shuffle
+// loop of unknown length cost them a third of that).
+enum PackKind { kNone, kRows16, kRows64, kTranspose8, kTranspose32, kPackKinds };
+struct PackPlan {
+  PackKind kind = kNone;
+  int32_t blocks_c = 0;        // workgroups along the vectors ...
+  int32_t parts = 1;           // ... and along the depth
+  int32_t k_span = 0;          // depth bytes (fp32: positions) of a part
 };
-__global__ __launch_bounds__(256) void PackI8PairKernel(PackPairI8 pair) {
-  __shared__ __attribute__((aligned(16))) uint8_t tile[kTileC * kPitch];
-  const int side = blockIdx.z;
-  const PackSource& src = pair.src[side];
-  if (src.stride_k == 1) {
-    if (static_cast<int>(blockIdx.x) * 4 >= src.count) return;
-    const int whole_depth = (pair.ld[side] + 1023) / 1024 * 1024;
-    PackI8RowsBlock(src, pair.dst[side], pair.ld[side], pair.sums[side], whole_depth, blockIdx.x, 0, 1);
-  } else {
-    if (static_cast<int>(blockIdx.x) * kTileC >= src.count) return;
-    const int whole_depth = (pair.ld[side] + kTileK - 1) / kTileK * kTileK;
-    PackI8Block(src, pair.dst[side], pair.ld[side], pair.sums[side], whole_depth, blockIdx.x, 0, 1, tile);
+
+// Low `n` bytes of a 32-bit word (n <= 0: none, n >= 4: all).
+__device__ __forceinline__ uint32_t LowBytes(int n) {
+  return n >= 4 ? 0xffffffffu : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
+}
+
+// The granule (16 bytes) at depth byte k of a row of `bytes` bytes, without
+// reading outside the row. Global memory takes any byte address (an odd one
+// costs no more than an aligned one, measured), so that is one load; a granule
+// that reaches past the row's end is taken from the 16 bytes that end there
+// and moved down to where it belongs afterwards, zeros following. Load and
+// rest are apart so that a lane's loads are all issued before the first is
+// waited for.
+__device__ __forceinline__ v4i LoadGranule(const uint8_t* row, int k, int bytes) {
+  if (bytes >= 16) return *reinterpret_cast<const v4i_unaligned*>(row + min(k, bytes - 16));  // (uniform)
+  v4i x = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 15; ++i)
+    if (i < bytes) x[i / 4] |= static_cast<int>(uint32_t(row[i]) << (8 * (i & 3)));
+  return x;
+}
+__device__ __forceinline__ v4i PlaceGranule(v4i x, int k, int bytes) {
+  if (bytes < 16) return k == 0 ? x : v4i{0, 0, 0, 0};
+  const int shift = k - min(k, bytes - 16);  // 0: a whole granule; 16 and more: nothing of the row
+  if (shift & 8) x = v4i{x[2], x[3], 0, 0};
+  if (shift & 4) x = v4i{x[1], x[2], x[3], 0};
+  const int s = shift & 3;
+  x[0] = static_cast<int>(__builtin_amdgcn_alignbyte(x[1], x[0], s));
+  x[1] = static_cast<int>(__builtin_amdgcn_alignbyte(x[2], x[1], s));
+  x[2] = static_cast<int>(__builtin_amdgcn_alignbyte(x[3], x[2], s));
+  x[3] = static_cast<int>(__builtin_amdgcn_alignbyte(0, x[3], s));
+  if (k >= bytes) x = v4i{0, 0, 0, 0};
+  return x;
+}
+
+// Depth-contiguous source of any alignment and depth (8-bit or fp32: bytes are
+// moved): kLanes lanes to a vector, four granules of a lane in flight.
+template <int kLanes>
+__device__ __forceinline__ void PackRows(const PackJob& job, int k_span, int bx, int by) {
+  constexpr int kStep = kLanes * 16;
+  const int lane = threadIdx.x % kLanes;
+  const int c = bx * (kThreads / kLanes) + static_cast<int>(threadIdx.x / kLanes);
+  const bool exists = c < job.src.count;
+  const int element = job.src.dtype == RUYAMD_DTYPE_F32 ? 4 : 1;
+  const int bytes = job.src.K * element;
+  const uint8_t* row =
+      static_cast<const uint8_t*>(job.src.data) + int64_t(min(c, job.src.count - 1)) * job.src.stride_c * element;
+  const uint32_t flip = job.src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
+  const int k_end = min(job.ld, (by + 1) * k_span);
+  const int end = min(k_end, bytes);
+  char* out = static_cast<char*>(job.dst) + int64_t(c) * job.ld;
+  constexpr int kInFlight = 4;
+  int sum = 0;
+  for (int base = by * k_span; base < k_end; base += kInFlight * kStep) {
+    v4i x[kInFlight];
+#pragma unroll
+    for (int i = 0; i < kInFlight; ++i)
+      if (i == 0 || base + i * kStep < end) x[i] = LoadGranule(row, base + i * kStep + lane * 16, bytes);  // (uniform)
+#pragma unroll
+    for (int i = 0; i < kInFlight; ++i) {
+      if (i > 0 && base + i * kStep >= end) break;
+      const int k = base + i * kStep + lane * 16;
+      x[i] = PlaceGranule(x[i], k, bytes);
+      if (flip) {  // (the padding stays zero)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) x[i][d] ^= static_cast<int>(flip & LowBytes(bytes - k - 4 * d));
+      }
+      if (exists && k < k_end) *reinterpret_cast<v4i*>(out + k) = x[i];
+      // (Granules at k_end and beyond: zero, or of a depth in parts, which has no sums.)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) sum = __builtin_amdgcn_sdot4(x[i][d], 0x01010101, sum, false);
+    }
+  }
+  if (job.sums) {
+#pragma unroll
+    for (int off = kLanes / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if (exists && lane == 0) job.sums[c] = sum;
   }
 }
 
-// Source contiguous along the vectors (the transposed case), base and pitch
-// of any alignment (global loads take any byte address on this target; with
-// an odd pitch the dword loads are merely slower than aligned ones, not the
-// byte loads they would otherwise have to be: a 2048 x 2048 operand of pitch
-// 2049 packs in 8 us instead of 40): a block moves a 64-vector x 64-depth tile
-// per step.
+// 8-bit source contiguous along the vectors (the transposed case), base and
+// pitch of any alignment (global loads take any byte address on this target;
+// with an odd pitch the dword loads are merely slower than aligned ones): a
+// block moves a 64-vector x 64-depth tile per step.
 // Each thread loads four dwords (4 vectors x 4 consecutive depth positions),
 // transposes the 4x4 bytes in registers with v_perm_b32 and writes four
 // dwords to the LDS tile, from which the block writes depth-contiguous
-// 16-byte pieces as in the generic kernel.
-__global__ __launch_bounds__(256) void PackI8TransposeKernel(PackSource src, int8_t* dst, int32_t ld,
-                                                            int32_t* sums, int k_span) {
-  __shared__ __attribute__((aligned(16))) uint8_t tile[kTileC * kPitch];
+// 16-byte pieces.
+__device__ __forceinline__ void PackTranspose8(const PackJob& job, int k_span, int bx, int by, uint8_t* tile) {
+  const PackSource& src = job.src;
   const int tid = threadIdx.x;
-  const int c0 = blockIdx.x * kTileC;
-  const int k_begin = blockIdx.y * k_span;
+  const int c0 = bx * kTileC;
+  const int ld = job.ld;
+  const int k_begin = by * k_span;
   const int k_end = min(k_begin + k_span, ld);
   const uint8_t* s = static_cast<const uint8_t*>(src.data);
+  int8_t* dst = static_cast<int8_t*>(job.dst);
   const uint32_t flip = src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
   const int cq = tid & 15;   // quad of vectors
   const int kq = tid >> 4;   // quad of depth positions
@@ -263,10 +186,7 @@ __global__ __launch_bounds__(256) void PackI8TransposeKernel(PackSource src, int
       v4i out;
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        uint32_t w = row[d];
-        const int kd = k + 4 * d;
-        const uint32_t mask = kd + 4 <= src.K ? 0xffffffffu : kd >= src.K ? 0u : (0xffffffffu >> (8 * (kd + 4 - src.K)));
-        w = (w & mask) ^ (flip & mask);
+        const uint32_t w = row[d] ^ (flip & LowBytes(src.K - k - 4 * d));
         out[d] = static_cast<int>(w);
         sum = __builtin_amdgcn_sdot4(static_cast<int>(w), 0x01010101, sum, false);
       }
@@ -274,17 +194,165 @@ __global__ __launch_bounds__(256) void PackI8TransposeKernel(PackSource src, int
     }
     __syncthreads();
   }
-  if (sums) {
+  if (job.sums) {
+    // The four granule writers of a vector are adjacent lanes.
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);
     const int c = c0 + wc;
-    if (wg == 0 && c < src.count) {
-      if (gridDim.y == 1)
-        sums[c] = sum;
-      else
-        atomicAdd(&sums[c], sum);
-    }
+    if (wg == 0 && c < src.count) job.sums[c] = sum;
   }
+}
+
+// The same for fp32: 32 vectors x 32 depth positions per step through LDS.
+// There are no sums and no conversion for floating point
+// (ruy/pack_common.h:100-133).
+__device__ __forceinline__ void PackTranspose32(const PackJob& job, int k_span, int bx, int by,
+                                                float (*tile)[kTile32 + 1]) {
+  const PackSource& src = job.src;
+  const int tx = threadIdx.x & 31;
+  const int ty = threadIdx.x >> 5;  // 0..7
+  const int c0 = bx * kTile32;
+  const int ld = job.ld / 4;
+  const float* s = static_cast<const float*>(src.data);
+  float* dst = static_cast<float*>(job.dst);
+  const int k_end = min(ld, (by + 1) * k_span);
+  for (int k0 = by * k_span; k0 < k_end; k0 += kTile32) {
+#pragma unroll
+    for (int t = ty; t < kTile32; t += 8) {
+      const int c = c0 + tx;
+      const int k = k0 + t;
+      float v = 0.f;
+      if (c < src.count && k < src.K) v = s[c + k * src.stride_k];
+      tile[tx][t] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = ty; t < kTile32; t += 8) {
+      const int c = c0 + t;
+      const int k = k0 + tx;
+      if (c < src.count && k < ld) dst[int64_t(c) * ld + k] = tile[t][tx];
+    }
+    __syncthreads();
+  }
+}
+
+// Both operands of a product in one launch: a second one would cost more than
+// the packing of all but the largest. Where the depth of a vector is dealt to
+// several workgroups nobody forms its sums here (adding the parts up took a
+// launch in front that cleared the words): the product does, as for operands
+// used in place. Calls with both packed, as up to four launches in front of the
+// product -> as one: 1000 x 1500 x 700 int8 with one side transposed 20.4 ->
+// 13.3 us, 64 x 147 x 12544 uint8 13.5 -> 9.8 us, 256 x 1968 x 645 uint8 20.9 ->
+// 13.8 us. The first `first` workgroups take the first operand.
+struct PackLaunch {
+  PackJob job[2];
+  int32_t blocks_c[2];
+  int32_t k_span[2];
+  int32_t first;  // workgroups of the first operand
+};
+template <int kKind>
+__device__ __forceinline__ void PackOperand(const PackJob& job, int k_span, int blocks_c, int block, void* tile) {
+  const int by = block < blocks_c ? 0 : block / blocks_c;
+  const int bx = block - by * blocks_c;
+  if constexpr (kKind == kRows16) PackRows<16>(job, k_span, bx, by);
+  if constexpr (kKind == kRows64) PackRows<64>(job, k_span, bx, by);
+  if constexpr (kKind == kTranspose8) PackTranspose8(job, k_span, bx, by, static_cast<uint8_t*>(tile));
+  if constexpr (kKind == kTranspose32)
+    PackTranspose32(job, k_span, bx, by, static_cast<float(*)[kTile32 + 1]>(tile));
+}
+constexpr int TileBytes(int kind) {
+  return kind == kTranspose8 ? kTileC * kPitch : kind == kTranspose32 ? kTile32 * (kTile32 + 1) * 4 : 16;
+}
+template <int kFirst, int kSecond>
+__global__ __launch_bounds__(kThreads) void PackKernel(PackLaunch launch) {
+  constexpr int kBytes = TileBytes(kFirst) > TileBytes(kSecond) ? TileBytes(kFirst) : TileBytes(kSecond);
+  __shared__ __attribute__((aligned(16))) char tile[kBytes];
+  const int block = blockIdx.x;
+  if (kSecond == kNone || block < launch.first)
+    PackOperand<kFirst>(launch.job[0], launch.k_span[0], launch.blocks_c[0], block, tile);
+  else
+    PackOperand<kSecond>(launch.job[1], launch.k_span[1], launch.blocks_c[1], block - launch.first, tile);
+}
+
+// The kernel for two kinds (operands of one product have one element size).
+using PackFunction = void (*)(PackLaunch);
+template <int kFirst>
+PackFunction KernelFor(PackKind second) {
+  constexpr int kTransposed = kFirst == kTranspose32 ? kTranspose32 : kTranspose8;
+  switch (second) {
+    case kNone:
+      return PackKernel<kFirst, kNone>;
+    case kRows16:
+      return PackKernel<kFirst, kRows16>;
+    case kRows64:
+      return PackKernel<kFirst, kRows64>;
+    case kTranspose32:
+      if constexpr (kFirst == kRows16 || kFirst == kRows64) return PackKernel<kFirst, kTranspose32>;
+      [[fallthrough]];
+    default:
+      return second == kTransposed ? PackKernel<kFirst, kTransposed> : nullptr;
+  }
+}
+PackFunction KernelFor(PackKind first, PackKind second) {
+  switch (first) {
+    case kRows16:
+      return KernelFor<kRows16>(second);
+    case kRows64:
+      return KernelFor<kRows64>(second);
+    case kTranspose8:
+      return KernelFor<kTranspose8>(second);
+    case kTranspose32:
+      return KernelFor<kTranspose32>(second);
+    default:
+      return nullptr;
+  }
+}
+
+// Parts of a depth of `steps` steps so that some `blocks_wanted` workgroups
+// are in flight, each with at least one step; returns the steps of a part.
+int StepsPerPart(int steps, int blocks_c, int blocks_wanted, int* parts) {
+  int wanted = std::min(steps, std::max(1, (blocks_wanted + blocks_c - 1) / blocks_c));
+  const int per_part = (steps + wanted - 1) / wanted;
+  *parts = (steps + per_part - 1) / per_part;
+  return per_part;
+}
+
+PackPlan PlanOf(const PackSource& src, int32_t ld) {
+  PackPlan plan;
+  if (src.stride_k == 1) {
+    // 16 lanes to a row of up to 1 KiB (what they have in flight at a time).
+    plan.kind = ld <= 1024 ? kRows16 : kRows64;
+    const int lanes = plan.kind == kRows16 ? 16 : 64;
+    const int rows_per_block = kThreads / lanes;
+    plan.blocks_c = (src.count + rows_per_block - 1) / rows_per_block;
+    // A vector of up to twice what its lanes have in flight is walked in one
+    // place (the sums come with it), and so is any when there are a thousand
+    // waves; otherwise the depth is dealt out, a granule a lane (1 KiB) at
+    // least. So it is for a handful of vectors (the narrow side of a skinny
+    // product: 10 x 7805 int8 4.3 us in 3 workgroups, 1.8 in 24).
+    const int step = lanes * 16;
+    const int steps = (ld + step - 1) / step;
+    int per_part = steps;
+    if ((steps > 8 && plan.blocks_c < 256) || plan.blocks_c < 16)
+      per_part = StepsPerPart(steps, plan.blocks_c, 512, &plan.parts);
+    plan.k_span = per_part * step;
+  } else if (src.dtype == RUYAMD_DTYPE_F32) {
+    plan.kind = kTranspose32;
+    plan.blocks_c = (src.count + kTile32 - 1) / kTile32;
+    plan.k_span = kTile32 * StepsPerPart((ld / 4 + kTile32 - 1) / kTile32, plan.blocks_c, 4096, &plan.parts);
+  } else {
+    plan.kind = kTranspose8;
+    plan.blocks_c = (src.count + kTileC - 1) / kTileC;
+    // A block's steps are a chain of load, transposition through LDS and store
+    // (about a microsecond each), so a block gets as few of them as some two
+    // thousand blocks allow (a 2048 x 2048 operand: 7.2 -> 3.6 us); one or two
+    // stay together, and the sums come with them.
+    const int steps = (ld + kTileK - 1) / kTileK;
+    int per_part = steps;
+    if (steps > 2) per_part = StepsPerPart(steps, plan.blocks_c, 2048, &plan.parts);
+    plan.k_span = per_part * kTileK;
+  }
+  return plan;
 }
 
 // One wave per vector, 16 bytes per lane per step.
@@ -314,58 +382,6 @@ __global__ __launch_bounds__(256) void SumsI8Kernel(const int8_t* data, int32_t 
   }
   const int32_t total = WaveSum(s0 + s1);
   if (lane == 0) sums[c] = total;
-}
-
-// fp32 re-layout: 32 vectors x 32 depth positions per step through LDS, so that
-// reads follow the source's contiguous dimension and writes follow depth.
-// There are no sums and no conversion for floating point
-// (ruy/pack_common.h:100-133).
-__device__ __forceinline__ void PackF32Block(const PackSource& src, float* dst, int32_t ld, int bx, int by,
-                                             int ny, float (*tile)[33]) {
-  const int tx = threadIdx.x & 31;
-  const int ty = threadIdx.x >> 5;  // 0..7
-  const int c0 = bx * 32;
-  const float* s = static_cast<const float*>(src.data);
-  const bool depth_contiguous = src.stride_k == 1;
-  for (int k0 = by * 32; k0 < ld; k0 += ny * 32) {
-#pragma unroll
-    for (int t = ty; t < 32; t += 8) {
-      // (c, k) read so that tx runs along the contiguous source dimension
-      const int c = c0 + (depth_contiguous ? t : tx);
-      const int k = k0 + (depth_contiguous ? tx : t);
-      float v = 0.f;
-      if (c < src.count && k < src.K) v = s[c * src.stride_c + k * src.stride_k];
-      if (depth_contiguous)
-        tile[t][tx] = v;
-      else
-        tile[tx][t] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = ty; t < 32; t += 8) {
-      const int c = c0 + t;
-      const int k = k0 + tx;
-      if (c < src.count && k < ld) dst[int64_t(c) * ld + k] = tile[t][tx];
-    }
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(256) void PackF32Kernel(PackSource src, float* dst, int32_t ld) {
-  __shared__ float tile[32][33];
-  PackF32Block(src, dst, ld, blockIdx.x, blockIdx.y, gridDim.y, tile);
-}
-
-struct PackPairF32 {
-  PackSource src[2];
-  float* dst[2];
-  int32_t ld[2];
-};
-__global__ __launch_bounds__(256) void PackF32PairKernel(PackPairF32 pair) {
-  __shared__ float tile[32][33];
-  const int side = blockIdx.z;
-  if (static_cast<int>(blockIdx.x) * 32 >= pair.src[side].count) return;
-  PackF32Block(pair.src[side], pair.dst[side], pair.ld[side], blockIdx.x, blockIdx.y, gridDim.y, tile);
 }
 
 // int16 -> two int8 planes. Block = 32 vectors (one group) x a depth span; the
@@ -522,97 +538,34 @@ hipError_t LaunchPackI16Split(hipStream_t stream, const PackSource& src, int8_t*
   return hipGetLastError();
 }
 
-hipError_t LaunchPackF32(hipStream_t stream, const PackSource& src, float* dst, int32_t ld) {
-  if (src.count == 0 || ld == 0) return hipSuccess;
-  const int blocks_c = (src.count + 31) / 32;
-  int blocks_k = (ld + 31) / 32;
-  if (blocks_k > 64) blocks_k = 64;
-  hipLaunchKernelGGL(PackF32Kernel, dim3(blocks_c, blocks_k), dim3(256), 0, stream, src, dst, ld);
+hipError_t LaunchPack(hipStream_t stream, const PackJob* jobs, int count) {
+  PackLaunch launch = {};
+  PackKind kinds[2] = {kNone, kNone};
+  int used = 0, blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    const PackJob& job = jobs[i];
+    if (job.src.count == 0 || job.ld == 0) continue;
+    const PackPlan plan = PlanOf(job.src, job.ld);
+    if (used == 2 || job.ld % 16 != 0 || (job.src.stride_k != 1 && job.src.stride_c != 1) ||
+        (job.sums && !PackFormsSums(job.src, job.ld)))
+      return hipErrorInvalidValue;
+    launch.job[used] = job;
+    launch.blocks_c[used] = plan.blocks_c;
+    launch.k_span[used] = plan.k_span;
+    if (used == 0) launch.first = plan.blocks_c * plan.parts;
+    kinds[used] = plan.kind;
+    blocks += plan.blocks_c * plan.parts;
+    ++used;
+  }
+  if (used == 0) return hipSuccess;
+  const PackFunction kernel = KernelFor(kinds[0], kinds[1]);
+  if (!kernel) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, stream, launch);
   return hipGetLastError();
 }
 
-hipError_t LaunchPackI8(hipStream_t stream, const PackSource& src, int8_t* dst, int32_t ld,
-                        int32_t* sums) {
-  if (src.count == 0 || ld == 0) return hipSuccess;
-  if (src.stride_k == 1) {
-    // Depth-contiguous source: one wave per vector; with few vectors the depth
-    // is split so that some two thousand waves are in flight.
-    const int steps = (ld + 1023) / 1024;
-    int k_split = 1;
-    if (src.count < 2048 && steps > 1) k_split = min((2048 + src.count - 1) / src.count, steps);
-    const int steps_per = (steps + k_split - 1) / k_split;
-    k_split = (steps + steps_per - 1) / steps_per;
-    if (sums && k_split > 1) {
-      hipLaunchKernelGGL(ZeroI32Kernel, dim3((src.count + 255) / 256), dim3(256), 0, stream, sums,
-                         src.count);
-    }
-    hipLaunchKernelGGL(PackI8RowsKernel, dim3((src.count + 3) / 4, k_split), dim3(256), 0, stream, src,
-                       dst, ld, sums, steps_per * 1024);
-    return hipGetLastError();
-  }
-  const int blocks_c = (src.count + kTileC - 1) / kTileC;
-  // Split the depth when there are too few vector slabs to fill the device: a
-  // block's steps are a chain of load, transposition through LDS and store
-  // (about a microsecond each), so a block gets as few of them as some two
-  // thousand blocks allow (a 2048 x 2048 operand: 7.2 -> 3.6 us).
-  int k_split = 1;
-  const int k_steps = (ld + kTileK - 1) / kTileK;
-  // (Not for one or two steps: the launch that clears the sums for the parts to add to would cost more.)
-  if (blocks_c < 2048 && k_steps > 2) k_split = min((2048 + blocks_c - 1) / blocks_c, k_steps);
-  const int steps_per = (k_steps + k_split - 1) / k_split;
-  const int k_span = steps_per * kTileK;
-  k_split = (k_steps + steps_per - 1) / steps_per;
-  if (sums && k_split > 1) {
-    hipLaunchKernelGGL(ZeroI32Kernel, dim3((src.count + 255) / 256), dim3(256), 0, stream, sums,
-                       src.count);
-  }
-  // The transposed case (vectors contiguous): dword loads; any other strides: bytes.
-  if (src.stride_c == 1) {
-    hipLaunchKernelGGL(PackI8TransposeKernel, dim3(blocks_c, k_split), dim3(256), 0, stream, src, dst, ld,
-                       sums, k_span);
-  } else {
-    hipLaunchKernelGGL(PackI8Kernel, dim3(blocks_c, k_split), dim3(256), 0, stream, src, dst, ld, sums,
-                       k_span);
-  }
-  return hipGetLastError();
-}
-
-hipError_t LaunchPackI8Pair(hipStream_t stream, const PackSource& src_a, int8_t* dst_a, int32_t ld_a,
-                            int32_t* sums_a, const PackSource& src_b, int8_t* dst_b, int32_t ld_b,
-                            int32_t* sums_b) {
-  PackPairI8 pair;
-  pair.src[0] = src_a;
-  pair.src[1] = src_b;
-  pair.dst[0] = dst_a;
-  pair.dst[1] = dst_b;
-  pair.ld[0] = ld_a;
-  pair.ld[1] = ld_b;
-  pair.sums[0] = sums_a;
-  pair.sums[1] = sums_b;
-  auto blocks_of = [](const PackSource& src) {
-    return src.stride_k == 1 ? (src.count + 3) / 4 : (src.count + kTileC - 1) / kTileC;
-  };
-  const int blocks = std::max(blocks_of(src_a), blocks_of(src_b));
-  if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(PackI8PairKernel, dim3(blocks, 1, 2), dim3(256), 0, stream, pair);
-  return hipGetLastError();
-}
-
-hipError_t LaunchPackF32Pair(hipStream_t stream, const PackSource& src_a, float* dst_a, int32_t ld_a,
-                             const PackSource& src_b, float* dst_b, int32_t ld_b) {
-  PackPairF32 pair;
-  pair.src[0] = src_a;
-  pair.src[1] = src_b;
-  pair.dst[0] = dst_a;
-  pair.dst[1] = dst_b;
-  pair.ld[0] = ld_a;
-  pair.ld[1] = ld_b;
-  const int blocks_c = (std::max(src_a.count, src_b.count) + 31) / 32;
-  if (blocks_c == 0) return hipSuccess;
-  int blocks_k = (std::max(ld_a, ld_b) + 31) / 32;
-  if (blocks_k > 16) blocks_k = 16;
-  hipLaunchKernelGGL(PackF32PairKernel, dim3(blocks_c, blocks_k, 2), dim3(256), 0, stream, pair);
-  return hipGetLastError();
+bool PackFormsSums(const PackSource& src, int32_t ld) {
+  return src.dtype != RUYAMD_DTYPE_F32 && (src.count == 0 || ld == 0 || PlanOf(src, ld).parts == 1);
 }
 
 hipError_t LaunchSumsI8(hipStream_t stream, const int8_t* data, int32_t ld, int32_t count, int32_t K,

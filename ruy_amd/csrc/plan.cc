@@ -5,6 +5,7 @@
 
 #include "kernels/fused_sums.h"
 #include "kernels/gemm_i8.h"
+#include "kernels/pack.h"
 #include "kernels/static_scratch.h"
 
 namespace ruyamd {
@@ -84,41 +85,32 @@ const char kCaptureCacheMiss[] =
     "the stream is capturing and an operand with a cache policy is not in the prepacked cache yet: "
     "run the same call once before the capture";
 
-// A pack into the workspace that has been set up but not launched yet: when
-// both sides of a small multiplication need one, a single launch does both.
-struct PendingPack8 {
+// A pack into the workspace that has been set up but not launched yet: one
+// launch does both sides of a product.
+struct PendingPack {
   bool pending = false;
-  PackSource src;
-  int8_t* dst = nullptr;
-  int32_t ld = 0;
-  int32_t* sums = nullptr;
-  uint64_t bytes = 0;
+  PackJob job;
 };
-// Packed operands up to this size are worth pairing (the launch saved costs
-// more than the paired kernel, in which a block walks the whole depth of its
-// vectors, loses on them): 256 KiB for a depth-contiguous source, 16 KiB for a
-// transposed one, which the paired kernel moves byte by byte (512^3 with both
-// operands transposed: 26.8 us paired, 11 us as two launches).
-constexpr uint64_t kPairedPackLimit = 256 * 1024;
-constexpr uint64_t kPairedTransposedPackLimit = 16 * 1024;
-bool WorthPairing(const PendingPack8& p) {
-  return p.bytes <= (p.src.stride_k == 1 ? kPairedPackLimit : kPairedTransposedPackLimit);
-}
 
-int LaunchPendingPacks8(ruyamd_ctx* ctx, PendingPack8* a, PendingPack8* b, std::string* err) {
-  hipError_t status = hipSuccess;
-  if (a->pending && b->pending && WorthPairing(*a) && WorthPairing(*b)) {
-    status = LaunchPackI8Pair(ctx->LaunchStream(), a->src, a->dst, a->ld, a->sums, b->src, b->dst, b->ld, b->sums);
-  } else {
-    if (a->pending) status = LaunchPackI8(ctx->LaunchStream(), a->src, a->dst, a->ld, a->sums);
-    if (status == hipSuccess && b->pending) status = LaunchPackI8(ctx->LaunchStream(), b->src, b->dst, b->ld, b->sums);
-  }
-  a->pending = b->pending = false;
-  if (status != hipSuccess) {
+int LaunchPendingPacks(ruyamd_ctx* ctx, const PendingPack& a, const PendingPack& b, std::string* err) {
+  PackJob jobs[2];
+  int count = 0;
+  for (const PendingPack* p : {&a, &b})
+    if (p->pending) jobs[count++] = p->job;
+  if (count && LaunchPack(ctx->LaunchStream(), jobs, count) != hipSuccess) {
     *err = "pack kernel launch failed";
     return RUYAMD_E_HIP;
   }
   return RUYAMD_OK;
+}
+
+// Packs one operand for the prepacked cache: here the sums are part of the
+// entry, wherever they are formed.
+hipError_t PackForCache8(ruyamd_ctx* ctx, const PackSource& src, int8_t* dst, int32_t ld, int32_t* sums) {
+  PackJob job{src, dst, ld, PackFormsSums(src, ld) ? sums : nullptr};
+  const hipError_t status = LaunchPack(ctx->LaunchStream(), &job, 1);
+  if (status != hipSuccess || job.sums) return status;
+  return LaunchSumsI8(ctx->LaunchStream(), dst, ld, src.count, ld, sums);
 }
 
 // In place: already int8 (or uint8 that the kernel flips on the way in, if the
@@ -134,14 +126,14 @@ bool UsableInPlace8(const PackSource& src, int u8_depth_step) {
          (src.stride_c % 16 == 0 || src.count == 1) && extent < (uint64_t(1) << 31);
 }
 
-// Prepares one side: from the cache, in place, or packed into the workspace
-// (with `defer`, that pack is only set up, for LaunchPendingPacks8).
+// Prepares one side: from the cache, in place, or to be packed into the
+// workspace (*pack is set up for LaunchPendingPacks).
 // `src` views the side as `count` depth vectors (LHS rows / RHS columns).
 // `u8_depth_step`: uint8 data may be used in place (the kernel flips the top
 // bit of every byte) if the depth is a multiple of this; 0 = never.
 int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point, bool need_sums,
                     int cache_policy, const void* src_key, int other_width, int u8_depth_step,
-                    Operand8* out, std::string* err, PendingPack8* defer = nullptr) {
+                    Operand8* out, PendingPack* pack, std::string* err) {
   // View of the side as `count` depth vectors; its data pointer is only valid
   // on the device after EnsureOnDevice.
   auto view = [&]() {
@@ -189,7 +181,7 @@ int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point
         return rc;
       }
       src = view();
-      if (LaunchPackI8(ctx->LaunchStream(), src, static_cast<int8_t*>(pm.data), ld, pm.sums) != hipSuccess) {
+      if (PackForCache8(ctx, src, static_cast<int8_t*>(pm.data), ld, pm.sums) != hipSuccess) {
         ctx->cache->Erase(src_key, pm);
         *err = "pack kernel launch failed";
         return RUYAMD_E_HIP;
@@ -218,26 +210,22 @@ int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point
     return RUYAMD_OK;
   }
 
+  const bool sums_with_pack = need_sums && PackFormsSums(src, ld);
   int8_t* packed = static_cast<int8_t*>(ctx->ws->Alloc(packed_bytes ? packed_bytes : 16));
-  int32_t* sums = need_sums ? static_cast<int32_t*>(ctx->ws->Alloc(std::size_t(src.count) * 4)) : nullptr;
-  if (!packed || (need_sums && !sums)) {
+  int32_t* sums = sums_with_pack ? static_cast<int32_t*>(ctx->ws->Alloc(std::size_t(src.count) * 4)) : nullptr;
+  if (!packed || (sums_with_pack && !sums)) {
     *err = "workspace allocation failed";
     return RUYAMD_E_HIP;
   }
-  if (defer) {
-    defer->pending = true;
-    defer->src = src;
-    defer->dst = packed;
-    defer->ld = ld;
-    defer->sums = sums;
-    defer->bytes = packed_bytes;
-  } else if (LaunchPackI8(ctx->LaunchStream(), src, packed, ld, sums) != hipSuccess) {
-    *err = "pack kernel launch failed";
-    return RUYAMD_E_HIP;
-  }
+  pack->pending = true;
+  pack->job = PackJob{src, packed, ld, sums};
   out->data = packed;
   out->ld = ld;
   out->sums = sums;
+  // (A depth walked by several workgroups: the sums are left to whoever reads
+  // the packed operand, as for one used in place.)
+  out->sums_pending = need_sums && !sums_with_pack;
+  out->count = src.count;
   out->bytes = static_cast<uint32_t>(packed_bytes);
   return RUYAMD_OK;
 }
@@ -343,14 +331,14 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   }
   // Row sums of one side are needed iff the other side's zero point is not 0
   // (ruy/kernel.h:219-232).
-  PendingPack8 pack_a, pack_b;
+  PendingPack pack_a, pack_b;
   if (int rc = PrepareOperand8(ctx, call, 0, lhs.zero_point, rzp != 0, call->lhs_cache_policy,
-                               call->lhs_src_key, N, u8_depth_step, &a, err, &pack_a))
+                               call->lhs_src_key, N, u8_depth_step, &a, &pack_a, err))
     return rc;
   if (int rc = PrepareOperand8(ctx, call, 1, rhs.zero_point, lzp != 0, call->rhs_cache_policy,
-                               call->rhs_src_key, M, u8_depth_step, &b, err, &pack_b))
+                               call->rhs_src_key, M, u8_depth_step, &b, &pack_b, err))
     return rc;
-  if (int rc = LaunchPendingPacks8(ctx, &pack_a, &pack_b, err)) return rc;
+  if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   const int32_t zp_product_depth =
       static_cast<int32_t>(static_cast<uint32_t>(lzp) * static_cast<uint32_t>(rzp) * static_cast<uint32_t>(K));
   if (skinny) {
@@ -470,33 +458,9 @@ struct OperandF32 {
   uint32_t bytes = 0;
 };
 
-struct PendingPackF32 {
-  bool pending = false;
-  PackSource src;
-  float* dst = nullptr;
-  int32_t ld = 0;
-  uint64_t bytes = 0;
-};
-
-int LaunchPendingPacksF32(ruyamd_ctx* ctx, PendingPackF32* a, PendingPackF32* b, std::string* err) {
-  hipError_t status = hipSuccess;
-  if (a->pending && b->pending && a->bytes <= kPairedPackLimit && b->bytes <= kPairedPackLimit) {
-    status = LaunchPackF32Pair(ctx->LaunchStream(), a->src, a->dst, a->ld, b->src, b->dst, b->ld);
-  } else {
-    if (a->pending) status = LaunchPackF32(ctx->LaunchStream(), a->src, a->dst, a->ld);
-    if (status == hipSuccess && b->pending) status = LaunchPackF32(ctx->LaunchStream(), b->src, b->dst, b->ld);
-  }
-  a->pending = b->pending = false;
-  if (status != hipSuccess) {
-    *err = "pack kernel launch failed";
-    return RUYAMD_E_HIP;
-  }
-  return RUYAMD_OK;
-}
-
 int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy,
-                      const void* src_key, int other_width, OperandF32* out, std::string* err,
-                      PendingPackF32* defer = nullptr) {
+                      const void* src_key, int other_width, OperandF32* out, PendingPack* pack,
+                      std::string* err) {
   auto view = [&]() {
     const DevMat& m = side == 0 ? call->lhs : call->rhs;
     return side == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
@@ -534,7 +498,8 @@ int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy
         return rc;
       }
       src = view();
-      if (LaunchPackF32(ctx->LaunchStream(), src, static_cast<float*>(pm.data), ld) != hipSuccess) {
+      const PackJob job{src, pm.data, ld * 4, nullptr};
+      if (LaunchPack(ctx->LaunchStream(), &job, 1) != hipSuccess) {
         ctx->cache->Erase(src_key, pm);
         *err = "pack kernel launch failed";
         return RUYAMD_E_HIP;
@@ -564,16 +529,8 @@ int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy
     *err = "workspace allocation failed";
     return RUYAMD_E_HIP;
   }
-  if (defer) {
-    defer->pending = true;
-    defer->src = src;
-    defer->dst = packed;
-    defer->ld = ld;
-    defer->bytes = packed_bytes;
-  } else if (LaunchPackF32(ctx->LaunchStream(), src, packed, ld) != hipSuccess) {
-    *err = "pack kernel launch failed";
-    return RUYAMD_E_HIP;
-  }
+  pack->pending = true;
+  pack->job = PackJob{src, packed, ld * 4, nullptr};
   out->data = packed;
   out->ld = ld;
   out->bytes = static_cast<uint32_t>(packed_bytes);
@@ -604,12 +561,12 @@ bool SetupDestination(const MulCall& call, GemmArgs* args) {
 int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   const int M = call->lhs.rows, K = call->lhs.cols, N = call->rhs.cols;
   OperandF32 a, b;
-  PendingPackF32 pack_a, pack_b;
-  if (int rc = PrepareOperandF32(ctx, call, 0, call->lhs_cache_policy, call->lhs_src_key, N, &a, err, &pack_a))
+  PendingPack pack_a, pack_b;
+  if (int rc = PrepareOperandF32(ctx, call, 0, call->lhs_cache_policy, call->lhs_src_key, N, &a, &pack_a, err))
     return rc;
-  if (int rc = PrepareOperandF32(ctx, call, 1, call->rhs_cache_policy, call->rhs_src_key, M, &b, err, &pack_b))
+  if (int rc = PrepareOperandF32(ctx, call, 1, call->rhs_cache_policy, call->rhs_src_key, M, &b, &pack_b, err))
     return rc;
-  if (int rc = LaunchPendingPacksF32(ctx, &pack_a, &pack_b, err)) return rc;
+  if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   if (N <= kSkinnyKernelWidth || M <= kSkinnyKernelWidth) {
     // Bandwidth-bound shapes: stream the wide side exactly once.
     GemvI8Args g;
@@ -678,11 +635,13 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   const int side8 = swap ? 1 : 0;
   const int side16 = 1 - side8;
   Operand8 a;
+  PendingPack pack_a;
   if (int rc = PrepareOperand8(ctx, call, side8, 0, /*need_sums=*/true,
                                side8 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy,
                                side8 == 0 ? call->lhs_src_key : call->rhs_src_key,
-                               side8 == 0 ? N : M, /*u8_depth_step=*/0, &a, err))
+                               side8 == 0 ? N : M, /*u8_depth_step=*/0, &a, &pack_a, err))
     return rc;
+  if (int rc = LaunchPendingPacks(ctx, pack_a, PendingPack(), err)) return rc;
   const DevMat& m16 = side16 == 0 ? call->lhs : call->rhs;  // shape only: its data may still be host memory
   const PackSource src = side16 == 0 ? PackSource{m16.data, m16.rs, m16.cs, m16.rows, m16.cols, m16.dtype}
                                      : PackSource{m16.data, m16.cs, m16.rs, m16.cols, m16.rows, m16.dtype};

@@ -207,6 +207,21 @@ def test_large_host_pointer_operands_and_the_staging_advisory(device_ctx):
     compare(f, D.host_pointer_mul(device_ctx, f, dst_fill=0), O.oracle_mul(f, fill=0))
 
 
+@pytest.mark.parametrize("depth", [1, 3, 15, 17, 33, 65, 145, 257, 1023, 1025, 1041, 4099, 9001])
+@pytest.mark.parametrize("tup", [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.U8, S.I32, S.I32), (S.F32, S.F32, S.F32, S.F32)])
+def test_packed_operands_at_the_edges_of_granules_and_parts(device_ctx, tup, depth):
+    """Depths either side of a 16-byte granule, of what a row's lanes hold and
+    of a depth dealt to several workgroups; counts that end inside a block; one
+    or both operands packed, by rows or transposed, in one launch."""
+    rng = np.random.default_rng(depth)
+    for rows, cols in [(65, 37), (19, 130)]:
+        for orders in [(1, 0, 0), (0, 0, 0), (1, 1, 1), (0, 1, 0)]:
+            p = W.random_problem(rng, *tup, rows, depth, cols, *orders, strided=bool(depth % 4 == 1),
+                                 name="pack %dx%dx%d %s" % (rows, depth, cols, orders))
+            got, want = run_both(device_ctx, p)
+            compare(p, got, want, exact_fp=False)
+
+
 @pytest.mark.parametrize("shape", [
     (1, 16, 1),            # single bytes
     (128, 40, 128),        # a destination of exactly one workgroup's 16 KiB
