@@ -38,11 +38,14 @@ struct GemmArgs {
   // column pitch may have any alignment the element type allows.
   DevMat dst;
   int32_t dst_elt = 1;
-  // Keeps the fields below where the kernels were compiled without scratch
-  // memory: with one word less here, the struct has a hole in front of its
+  // Not 0: the operands need none of the above but rows that are runs of
+  // k_valid >= 16 bytes, of any alignment and pitch (LaunchGemmI8Staged);
+  // k_bytes is then k_valid rounded up to 16, and uint8 data (a_flip, b_flip)
+  // may have any depth.
+  // (With one word less here, the struct has a hole in front of its
   // last pointers and the compiler copies that part of the kernel arguments
-  // through scratch in some kernels.
-  int32_t unused_padding = 0;
+  // through scratch in some kernels.)
+  int32_t k_valid = 0;
   // int8 kernel, small problems only (GemmI8CanFuseSums): when fuse_sums is
   // set the kernel forms the depth sums of a's rows and b's columns itself
   // and subtracts fused_a_factor * rowsum(i) + fused_b_factor * colsum(j)
@@ -164,6 +167,15 @@ int GemmI8RowSumsProducers(const GemmArgs& args, int num_cus);
 bool GemmI8CanFormColumnSums(const GemmArgs& args, int num_cus, bool rows_in_launch);
 int GemmI8ColumnSumsOffset(const GemmArgs& args);
 hipError_t LaunchGemmI8(hipStream_t stream, const GemmArgs& args, int num_cus);
+// The smallest tile with operands that cannot be used in place as they are
+// (k_valid): rows of any alignment and length are read through registers
+// instead of being packed first. Whether that beats packing in front of the
+// best tile for a product of this `depth` (`in_place`: beats the best tile on
+// operands that need no packing). The launch forms pending sums itself
+// (fuse_sums) and has no depth split.
+constexpr int kGemmI8StagedDepth = 1024;  // what its ring holds
+bool GemmI8StagedIsBetter(const GemmArgs& args, int num_cus, int depth, bool in_place);
+hipError_t LaunchGemmI8Staged(hipStream_t stream, const GemmArgs& args);
 // `count` <= kGemmBatchMax products of the shape and parameters of `args`, each
 // on its own buffers, in one launch. Only for arguments that run on the
 // smallest tile (GemmI8CanFuseSums), without sums arrays (zero points 0, or the

@@ -1,0 +1,58 @@
+// The int8 GEMM on operands of any alignment and depth, read through registers
+// instead of being packed first (mfma_gemm.h, kStaged).
+#include <hip/hip_runtime.h>
+
+#include "int8_traits.h"
+#include "mfma_gemm.h"
+
+namespace ruyamd {
+
+// Where all workgroups run at once - two to a CU with the ring of four stages,
+// one with that of eight - the product is little more than its launch, one
+// round trip to memory and its write-back, and a pack launch in front costs two
+// thirds of that again: 1024 x 333 x 1024 9.4 us packed, 6.6 staged; 1024 x
+// 1023 x 1024 11.9 and 9.9 (8.4 at a depth of 1020, whose rows start at whole
+// dwords), 4236 x 106 x 256 10.0 and 5.9, 64 x 147 x 12544 uint8 9.5 and 6.0.
+// In rounds it loses to larger tiles on packed operands: 2048 x 251 x 2048
+// (1024 tiles of 64x64) 11.1 packed and 11.7 staged, 1500 x 1000 x 1500 (576)
+// 17.1 and 21.8.
+// Operands that can be used in place gain less, since nothing is packed. Up to
+// 384 bytes of depth the direct loads are as good (256^3 4.8, staged 5.0), from
+// 900 on the schedule that deals the depth to the waves; in between, and where
+// two workgroups a CU take a grid that would otherwise go to a larger tile, it
+// wins: 512^3 6.1 -> 5.7, 1024 x 640 x 1024 uint8 6.9 -> 6.0, 4096 x 256 x 512
+// 6.9 -> 5.6, 2048 x 128 x 1024 6.0 -> 4.8.
+bool GemmI8StagedIsBetter(const GemmArgs& args, int num_cus, int depth, bool in_place) {
+  if (depth < 16 || depth > kGemmI8StagedDepth) return false;
+  if (args.forced_tile_rows && (in_place || args.forced_tile_rows != 64 || args.forced_tile_cols != 64)) return false;
+  const int tiles = mfma_gemm::TileCount(args, 64, 64);
+  if (tiles > num_cus * (depth <= 512 ? 2 : 1)) return false;
+  return !in_place || tiles > num_cus || (depth > 384 && depth <= 896);
+}
+
+namespace {
+
+template <int kStages, int kForm>
+hipError_t LaunchForm(hipStream_t stream, const GemmArgs& args) {
+  return args.fuse_sums
+             ? mfma_gemm::Launch<Int8Traits, 1, 1, 128, kStages, true, false, false, false, false, kForm>(stream, args)
+             : mfma_gemm::Launch<Int8Traits, 1, 1, 128, kStages, false, false, false, false, false, kForm>(stream, args);
+}
+
+}  // namespace
+
+hipError_t LaunchGemmI8Staged(hipStream_t stream, const GemmArgs& args) {
+  if (args.k_valid < 16 || args.k_valid > kGemmI8StagedDepth || args.k_bytes != (args.k_valid + 15) / 16 * 16 ||
+      args.row_sums || args.split_k != 1)
+    return hipErrorInvalidValue;
+  const bool dwords = ((reinterpret_cast<uintptr_t>(args.a) | reinterpret_cast<uintptr_t>(args.b) |
+                        static_cast<uint32_t>(args.lda) | static_cast<uint32_t>(args.ldb)) & 3) == 0;
+  if (args.k_valid <= 512) {
+    return dwords ? LaunchForm<4, mfma_gemm::kStagedDwords>(stream, args)
+                  : LaunchForm<4, mfma_gemm::kStagedBytes>(stream, args);
+  }
+  return dwords ? LaunchForm<8, mfma_gemm::kStagedDwords>(stream, args)
+                : LaunchForm<8, mfma_gemm::kStagedBytes>(stream, args);
+}
+
+}  // namespace ruyamd

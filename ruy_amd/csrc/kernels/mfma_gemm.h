@@ -55,6 +55,7 @@
 #include "depth_split.h"
 #include "fused_sums.h"
 #include "gemm_i8.h"
+#include "granule.h"
 #include "paired_schedule.h"
 
 namespace ruyamd {
@@ -254,9 +255,24 @@ RUYAMD_HOST_DEVICE inline int LeadShareLanesPerRow(int rows_in_share, int k_byte
 // workgroups of its first round, a share each; the 128x128, 128x64 and 64x128
 // tiles, and the 64x64 tile on its depth-per-wave schedule, have either
 // operand's done that second way (args.row_sums_sides).
+//
+// kStaged (64x64 tile of the int8 kernel, depths that the ring holds as a
+// whole): operand rows of any alignment and length (GemmArgs::k_valid). A
+// direct-to-LDS load takes 16 aligned bytes, so such rows used to be packed by
+// a launch in front, which costs more than the product wherever both are
+// small. Here the loads go through registers on their way to the ring, all of
+// them issued before the first is awaited. 1: rows that start at multiples of
+// 4 bytes, where a 16-byte load costs what an aligned one does. 2: any byte
+// address. There a 16-byte load takes a CU's address unit four times as long
+// (64 cycles), so it is taken as the aligned dwords that hold the 16 bytes -
+// four in one load, the fifth in another - and shifted into place.
+enum StagedForm { kNotStaged = 0, kStagedDwords = 1, kStagedBytes = 2 };
 template <typename Traits, int WM, int WN, int BK, int STAGES, bool kFusedSums = false, bool kFlip = false,
-          bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false>
+          bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false, int kStaged = kNotStaged>
 __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
+  static_assert(!kStaged || (WM == 1 && WN == 1 && BK == 128 && Traits::kBlock == 32 && !kFlip && !kRowSums &&
+                             !kDepthWaves && !Traits::kSplitB),
+                "staged loading exists for the 64x64 tile");
   static_assert(!kRowSums || !kFusedSums, "one way of forming the sums at a time");
   // kRowSums on the tiles of 32x32 blocks whose waves share every step: the
   // rows of an operand are dealt out over the workgroups of the grid's first
@@ -452,7 +468,9 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   // part (the descriptors below start there as well), and walks them from
   // step 0.
   const int part_begin = kSplitLarge ? first_step_of_part * kBK : 0;  // bytes
-  const int K = kSplitLarge ? min(args.k_bytes - part_begin, steps_of_part * kBK) : args.k_bytes;  // depth in bytes
+  const int K = kStaged       ? args.k_valid
+                : kSplitLarge ? min(args.k_bytes - part_begin, steps_of_part * kBK)
+                              : args.k_bytes;  // depth in bytes
   const v4i a_rsrc = MakeRsrc(static_cast<const char*>(args.a) + part_begin, args.a_bytes - uint32_t(part_begin));
   const v4i b_rsrc = MakeRsrc(static_cast<const char*>(args.b) + part_begin, args.b_bytes - uint32_t(part_begin));
   uint32_t a_goff[C::kALoads];
@@ -1309,20 +1327,95 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     };
     using Even = std::integral_constant<int, 0>;
     using Odd = std::integral_constant<int, 1>;
-    if (C::kKSteps % 2 == 0 && k_tiles <= C::kStages) {
+    if (C::kKSteps % 2 == 0 && (kStaged || k_tiles <= C::kStages)) {
       // A depth that fits the ring as a whole (256 bytes on the 64x64 tile's
       // four stages, say): only the steps that exist are fetched, everything is
       // awaited once, and the loop carries neither loads nor waits nor
       // barriers. (The general form below fetches kStages steps past the end
       // of every depth, as zeros, to keep its load counts fixed: nothing for a
       // long depth, a third of the kernel's loads for this one.)
+      if constexpr (kStaged) {
+        // (The launcher sends nothing deeper here.)
+        // Load n of a stage: rows of a, then rows of b; the first byte of the
+        // lane's row, and where in a stage its granules go.
+        constexpr int kLoads = C::kLoadsPerStage;
+        const char* row_of[kLoads];
+        int k_of[kLoads], at[kLoads];
+        StaticFor<kLoads>([&](auto n) {
+          constexpr bool kIsA = n < C::kALoads;
+          constexpr int i = kIsA ? n : n - C::kALoads;
+          const int chunk = wave * (kIsA ? C::kALoads : C::kBLoads) + i;
+          const int r = chunk * C::kRowsPerLoad + lane / C::kGranulesPerRow;
+          // (Rows past the end read the last one; nothing of them is stored.)
+          row_of[n] = kIsA ? static_cast<const char*>(args.a) + MulLo(min(m0 + r, args.M - 1), args.lda)
+                           : static_cast<const char*>(args.b) + MulLo(min(n0 + r, args.N - 1), args.ldb);
+          k_of[n] = kIsA ? a_k[i] : b_k[i];
+          at[n] = (kIsA ? 0 : C::kBM * kBK) + chunk * 1024 + lane * kGranule;
+        });
+        v4i held[C::kStages][kLoads];
+        int fifth[C::kStages][kLoads];
+        typedef v4i v4i_dwords __attribute__((aligned(4)));
+        // A granule that reaches past the end of its row: the 16 bytes that
+        // end there (placed below), so that nothing is read outside the row
+        // but the rest of an aligned dword that holds a byte of it.
+        auto address_of = [&](int stage, int n) { return row_of[n] + min(stage * kBK + k_of[n], K - kGranule); };
+        StaticFor<C::kStages>([&](auto s) {
+          if (s < k_tiles) {
+            StaticFor<kLoads>([&](auto n) {
+              const char* from = address_of(s, n);
+              if constexpr (kStaged == kStagedDwords) {
+                held[s][n] = *reinterpret_cast<const v4i_unaligned*>(from);
+              } else {
+                const int shift = static_cast<int>(reinterpret_cast<uintptr_t>(from) & 3);
+                held[s][n] = *reinterpret_cast<const v4i_dwords*>(from - shift);
+                fifth[s][n] = *reinterpret_cast<const int*>(from - shift + (shift ? 16 : 12));
+              }
+            });
+          }
+        });
+        load_edge_params();
+        StaticFor<C::kStages>([&](auto s) {
+          if (s < k_tiles) {
+            StaticFor<kLoads>([&](auto n) {
+              v4i x = held[s][n];
+              if constexpr (kStaged == kStagedBytes) {
+                const uint32_t shift = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(address_of(s, n)) & 3);
 #pragma unroll
-      for (int s = 0; s < C::kStages; ++s)
-        if (s < k_tiles) issue(s);
-      if constexpr (kLeadSums) add_up_rows_of_share();
-      WaitVmcnt<0>();
-      __syncthreads();
-      load_edge_params();
+                for (int d = 0; d < 4; ++d)
+                  x[d] = static_cast<int>(__builtin_amdgcn_alignbyte(d < 3 ? held[s][n][d + 1] : fifth[s][n], x[d], shift));
+              }
+              x ^= static_cast<int>(n < C::kALoads ? args.a_flip : args.b_flip);
+              *reinterpret_cast<v4i*>(lds + s * C::kStageBytes + at[n]) = x;
+            });
+          }
+        });
+        // The last stage of a depth that is no whole number of stages: this
+        // wave's granules once more, those at the end moved into place and the
+        // padding zero whatever was read for it. (Reads and writes of a wave
+        // in LDS are performed in order.)
+        if (K % kBK != 0) {
+          const int last = (k_tiles - 1) * kBK;
+          char* const stage = lds + (k_tiles - 1) * C::kStageBytes;
+          StaticFor<kLoads>([&](auto n) {
+            const uint32_t flip = n < C::kALoads ? args.a_flip : args.b_flip;
+            const int k = last + k_of[n];
+            v4i x = *reinterpret_cast<const v4i*>(stage + at[n]);
+            x = granule::PlaceGranule(x ^ static_cast<int>(flip), k, K);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) x[d] ^= static_cast<int>(flip & granule::LowBytes(K - k - 4 * d));
+            *reinterpret_cast<v4i*>(stage + at[n]) = x;
+          });
+        }
+        __syncthreads();
+      } else {
+#pragma unroll
+        for (int s = 0; s < C::kStages; ++s)
+          if (s < k_tiles) issue(s);
+        if constexpr (kLeadSums) add_up_rows_of_share();
+        WaitVmcnt<0>();
+        __syncthreads();
+        load_edge_params();
+      }
       read_frags(0, 0, f[0]);
       for (int kt = 0; kt < k_tiles; ++kt) ring_step(kt, std::false_type(), Even(), std::false_type());
     } else {
@@ -2074,9 +2167,9 @@ constexpr int WavesPerSimdWanted() {
   return (!kDepthWaves && STAGES == 2 && WM * WN == 2) ? 3 : 1;
 }
 template <typename Traits, int WM, int WN, int BK, int STAGES, bool kFusedSums = false, bool kFlip = false,
-          bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false>
+          bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false, int kStaged = kNotStaged>
 __global__ __launch_bounds__(256, (WavesPerSimdWanted<WM, WN, STAGES, kDepthWaves>())) void MfmaGemmKernel(GemmArgs args) {
-  MfmaGemmBody<Traits, WM, WN, BK, STAGES, kFusedSums, kFlip, kDepthWaves, kRowSums, kSplitLarge>(args);
+  MfmaGemmBody<Traits, WM, WN, BK, STAGES, kFusedSums, kFlip, kDepthWaves, kRowSums, kSplitLarge, kStaged>(args);
 }
 
 // Several products of one shape in one launch: grid.z counts the products,
@@ -2115,7 +2208,7 @@ hipError_t LaunchBatch(hipStream_t stream, const GemmArgs& args, const GemmBatch
 }
 
 template <typename Traits, int WM, int WN, int BK, int STAGES, bool kFusedSums = false, bool kFlip = false,
-          bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false>
+          bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false, int kStaged = kNotStaged>
 hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
   using C = Cfg<WM, WN, BK, STAGES, Traits::kSplitB, Traits::kBlock>;
   const int tiles_m = (args.M + C::kBM - 1) / C::kBM;
@@ -2124,7 +2217,8 @@ hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
   const int grid = ((total + 7) / 8) * 8;
   // The depth-per-wave schedule: two ring slots of 16 KiB for each of four waves.
   const size_t lds_bytes = kDepthWaves ? size_t(4 * 2 * 128 * BK) : size_t(C::kLdsBytes);
-  auto kernel = MfmaGemmKernel<Traits, WM, WN, BK, STAGES, kFusedSums, kFlip, kDepthWaves, kRowSums, kSplitLarge>;
+  auto kernel = MfmaGemmKernel<Traits, WM, WN, BK, STAGES, kFusedSums, kFlip, kDepthWaves, kRowSums, kSplitLarge, kStaged>;
+  if ((kStaged != kNotStaged) != (args.k_valid != 0)) return hipErrorInvalidValue;
   if (kRowSums != (args.row_sums != nullptr)) return hipErrorInvalidValue;
   if (kRowSums && (!args.row_sums_to_zero || tiles_m * C::kBM > fused_sums::kMaxRows ||
                    args.row_sums_zero_rows > fused_sums::kMaxRows))

@@ -53,6 +53,10 @@ struct Operand8 {
   int32_t count = 0;
   // kFlipU8 if `data` is the caller's uint8 storage used in place.
   uint32_t flip = 0;
+  // Neither cached nor usable in place: `src` is to be packed (PackOperand8) or
+  // read as it is by a kernel that can (AsStaged).
+  bool unpacked = false;
+  PackSource src;
 };
 
 int MaterializeSums(ruyamd_ctx* ctx, Operand8* op, int32_t K, std::string* err) {
@@ -126,14 +130,13 @@ bool UsableInPlace8(const PackSource& src, int u8_depth_step) {
          (src.stride_c % 16 == 0 || src.count == 1) && extent < (uint64_t(1) << 31);
 }
 
-// Prepares one side: from the cache, in place, or to be packed into the
-// workspace (*pack is set up for LaunchPendingPacks).
+// Prepares one side: from the cache, in place, or left unpacked.
 // `src` views the side as `count` depth vectors (LHS rows / RHS columns).
 // `u8_depth_step`: uint8 data may be used in place (the kernel flips the top
 // bit of every byte) if the depth is a multiple of this; 0 = never.
 int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point, bool need_sums,
                     int cache_policy, const void* src_key, int other_width, int u8_depth_step,
-                    Operand8* out, PendingPack* pack, std::string* err) {
+                    Operand8* out, std::string* err) {
   // View of the side as `count` depth vectors; its data pointer is only valid
   // on the device after EnsureOnDevice.
   auto view = [&]() {
@@ -210,24 +213,52 @@ int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point
     return RUYAMD_OK;
   }
 
-  const bool sums_with_pack = need_sums && PackFormsSums(src, ld);
-  int8_t* packed = static_cast<int8_t*>(ctx->ws->Alloc(packed_bytes ? packed_bytes : 16));
-  int32_t* sums = sums_with_pack ? static_cast<int32_t*>(ctx->ws->Alloc(std::size_t(src.count) * 4)) : nullptr;
+  out->unpacked = true;
+  out->src = src;
+  out->ld = ld;
+  out->bytes = static_cast<uint32_t>(packed_bytes);
+  out->count = src.count;
+  out->sums_pending = need_sums;
+  return RUYAMD_OK;
+}
+
+// Room in the workspace for an operand that PrepareOperand8 left unpacked; the
+// pack itself is set up for LaunchPendingPacks. Nothing to do for any other.
+int PackOperand8(ruyamd_ctx* ctx, Operand8* op, PendingPack* pack, std::string* err) {
+  if (!op->unpacked) return RUYAMD_OK;
+  const bool sums_with_pack = op->sums_pending && PackFormsSums(op->src, op->ld);
+  int8_t* packed = static_cast<int8_t*>(ctx->ws->Alloc(op->bytes ? op->bytes : 16));
+  int32_t* sums = sums_with_pack ? static_cast<int32_t*>(ctx->ws->Alloc(std::size_t(op->count) * 4)) : nullptr;
   if (!packed || (sums_with_pack && !sums)) {
     *err = "workspace allocation failed";
     return RUYAMD_E_HIP;
   }
   pack->pending = true;
-  pack->job = PackJob{src, packed, ld, sums};
-  out->data = packed;
-  out->ld = ld;
-  out->sums = sums;
+  pack->job = PackJob{op->src, packed, op->ld, sums};
+  op->unpacked = false;
+  op->data = packed;
+  op->sums = sums;
   // (A depth walked by several workgroups: the sums are left to whoever reads
   // the packed operand, as for one used in place.)
-  out->sums_pending = need_sums && !sums_with_pack;
-  out->count = src.count;
-  out->bytes = static_cast<uint32_t>(packed_bytes);
+  if (sums_with_pack) op->sums_pending = false;
   return RUYAMD_OK;
+}
+
+// The operand as the staged form of the int8 kernel reads it: rows of any
+// alignment and length. False if it cannot (a transposed source, a depth
+// below 16, an extent its 32-bit offsets do not reach).
+bool AsStaged(const Operand8& op, int32_t K, Operand8* out) {
+  *out = op;
+  if (!op.unpacked) return K >= 16;
+  const PackSource& src = op.src;
+  const uint64_t extent = src.count > 0 ? uint64_t(src.count - 1) * uint64_t(src.stride_c) + K : 0;
+  if (src.stride_k != 1 || K < 16 || extent >= (uint64_t(1) << 31)) return false;
+  out->unpacked = false;
+  out->data = static_cast<const int8_t*>(src.data);
+  out->ld = src.count == 1 ? K : static_cast<int32_t>(src.stride_c);
+  out->bytes = static_cast<uint32_t>(extent);
+  out->flip = src.dtype == RUYAMD_DTYPE_U8 ? kFlipU8 : 0;
+  return true;
 }
 
 // How often a workgroup of the 256x256 tile's depth split looks for the other
@@ -271,8 +302,10 @@ void PlanDepthSplit(ruyamd_ctx* ctx, GemmKind kind, GemmArgs* args) {
 // args->fuse_sums is set: the kernel forms them itself (one launch instead of
 // two or three) and the zero point that multiplies a side's sums moves from
 // the write-back to the fused factor.
+// `staged`: for the staged form of that tile, which forms them wherever they
+// are pending.
 bool SetupInt8Gemm(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp,
-                   int32_t rzp, GemmArgs* out) {
+                   int32_t rzp, bool staged, GemmArgs* out) {
   GemmArgs& args = *out;
   args.forced_tile_rows = ctx->forced_tile_rows;
   args.forced_depth_parts = ctx->forced_depth_parts;
@@ -299,7 +332,8 @@ bool SetupInt8Gemm(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, cons
   args.ep.rhs_zero_point = swap ? lzp : rzp;
   args.sums_wanted = (x.sums_pending ? 1 : 0) | (y.sums_pending ? 2 : 0) |
                      (ctx->row_sums_in_launch && !ctx->capturing && !ctx->no_alloc ? 4 : 0);
-  if ((a.sums_pending || b.sums_pending) && GemmI8CanFuseSums(args, ctx->multiprocessor_count)) {
+  if (staged) args.sums_wanted &= 3;
+  if ((a.sums_pending || b.sums_pending) && (staged || GemmI8CanFuseSums(args, ctx->multiprocessor_count))) {
     args.fuse_sums = 1;
     if (x.sums_pending) {
       args.fused_a_factor = args.ep.rhs_zero_point;
@@ -311,6 +345,32 @@ bool SetupInt8Gemm(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, cons
     }
   }
   return swap;
+}
+
+// The product on the staged form of the smallest tile, where the planner finds
+// that better (*done): it reads operands that cannot be used in place as they
+// are, without a pack launch in front, and forms pending sums itself.
+int RunInt8Staged(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
+                  bool* done, std::string* err) {
+  const int K = call.lhs.cols;
+  Operand8 sa, sb;
+  if (!AsStaged(a, K, &sa) || !AsStaged(b, K, &sb)) return RUYAMD_OK;
+  GemmArgs args;
+  const bool swap = SetupInt8Gemm(ctx, call, sa, sb, lzp, rzp, /*staged=*/true, &args);
+  if (!GemmI8StagedIsBetter(args, ctx->multiprocessor_count, K, !a.unpacked && !b.unpacked)) return RUYAMD_OK;
+  args.k_valid = K;
+  args.ep.lhs_sums = (swap ? sb : sa).sums;
+  args.ep.rhs_sums = (swap ? sa : sb).sums;
+  const bool timed = ctx->TimingBegin();
+  const hipError_t launched = LaunchGemmI8Staged(ctx->LaunchStream(), args);
+  if (timed) ctx->TimingEnd();
+  if (launched != hipSuccess) {
+    *err = "int8 MFMA kernel launch failed";
+    return RUYAMD_E_HIP;
+  }
+  ctx->last_kernel = RUYAMD_KERNEL_I8_MFMA;
+  *done = true;
+  return RUYAMD_OK;
 }
 
 int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
@@ -331,13 +391,20 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   }
   // Row sums of one side are needed iff the other side's zero point is not 0
   // (ruy/kernel.h:219-232).
-  PendingPack pack_a, pack_b;
   if (int rc = PrepareOperand8(ctx, call, 0, lhs.zero_point, rzp != 0, call->lhs_cache_policy,
-                               call->lhs_src_key, N, u8_depth_step, &a, &pack_a, err))
+                               call->lhs_src_key, N, u8_depth_step, &a, err))
     return rc;
   if (int rc = PrepareOperand8(ctx, call, 1, rhs.zero_point, lzp != 0, call->rhs_cache_policy,
-                               call->rhs_src_key, M, u8_depth_step, &b, &pack_b, err))
+                               call->rhs_src_key, M, u8_depth_step, &b, err))
     return rc;
+  if (!skinny) {
+    bool done = false;
+    if (int rc = RunInt8Staged(ctx, *call, a, b, lzp, rzp, &done, err)) return rc;
+    if (done) return RUYAMD_OK;
+  }
+  PendingPack pack_a, pack_b;
+  if (int rc = PackOperand8(ctx, &a, &pack_a, err)) return rc;
+  if (int rc = PackOperand8(ctx, &b, &pack_b, err)) return rc;
   if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   const int32_t zp_product_depth =
       static_cast<int32_t>(static_cast<uint32_t>(lzp) * static_cast<uint32_t>(rzp) * static_cast<uint32_t>(K));
@@ -387,7 +454,7 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     return RUYAMD_OK;
   }
   GemmArgs args;
-  const bool swap = SetupInt8Gemm(ctx, *call, a, b, lzp, rzp, &args);
+  const bool swap = SetupInt8Gemm(ctx, *call, a, b, lzp, rzp, /*staged=*/false, &args);
   // The largest tile can form the sums of the rows of its `a` operand in
   // passing (kernels/fused_sums.h): one launch instead of a sums kernel and
   // the product. Not for a call that is being recorded (a replayed launch
@@ -635,12 +702,13 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   const int side8 = swap ? 1 : 0;
   const int side16 = 1 - side8;
   Operand8 a;
-  PendingPack pack_a;
   if (int rc = PrepareOperand8(ctx, call, side8, 0, /*need_sums=*/true,
                                side8 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy,
                                side8 == 0 ? call->lhs_src_key : call->rhs_src_key,
-                               side8 == 0 ? N : M, /*u8_depth_step=*/0, &a, &pack_a, err))
+                               side8 == 0 ? N : M, /*u8_depth_step=*/0, &a, err))
     return rc;
+  PendingPack pack_a;
+  if (int rc = PackOperand8(ctx, &a, &pack_a, err)) return rc;
   if (int rc = LaunchPendingPacks(ctx, pack_a, PendingPack(), err)) return rc;
   const DevMat& m16 = side16 == 0 ? call->lhs : call->rhs;  // shape only: its data may still be host memory
   const PackSource src = side16 == 0 ? PackSource{m16.data, m16.rs, m16.cs, m16.rows, m16.cols, m16.dtype}
@@ -821,7 +889,7 @@ int RunMulBatch(ruyamd_ctx* ctx, const MulCall& first, const BatchBuffers* items
   const Operand8 a = in_place(lhs, M, lhs.rs, rzp != 0);
   const Operand8 b = in_place(rhs, N, rhs.cs, lzp != 0);
   GemmArgs args;
-  const bool swap = SetupInt8Gemm(ctx, first, a, b, lzp, rzp, &args);
+  const bool swap = SetupInt8Gemm(ctx, first, a, b, lzp, rzp, /*staged=*/false, &args);
   if ((a.sums_pending || b.sums_pending) && !args.fuse_sums) return RUYAMD_OK;
   const bool timed = ctx->TimingBegin();
   hipError_t launched = hipSuccess;

@@ -222,6 +222,33 @@ def test_packed_operands_at_the_edges_of_granules_and_parts(device_ctx, tup, dep
             compare(p, got, want, exact_fp=False)
 
 
+@pytest.mark.parametrize("depth", [16, 17, 31, 127, 128, 130, 383, 400, 511, 512, 513, 896, 1000, 1023, 1024, 1025])
+@pytest.mark.parametrize("tup", [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I16), (S.I8, S.U8, S.I32, S.I32)])
+def test_small_products_read_through_registers(device_ctx, tup, depth):
+    """The 64x64 tile on rows of any length and alignment: depths either side of
+    its ring of four and of eight stages and of a granule, counts either side of
+    a tile, rows that start at whole dwords and at odd bytes, a packed operand
+    from the cache beside a raw one."""
+    rng = np.random.default_rng(depth)
+    for rows, cols, pad, cached in [(64, 64, False, False), (65, 129, True, False), (17, 63, False, True)]:
+        p = W.random_problem(rng, *tup, rows, depth, cols, 1, 0, depth % 2, strided=pad,
+                             name="staged %dx%dx%d" % (rows, depth, cols))
+        p.lhs.cache_policy = S.CACHE_ALWAYS if cached else S.CACHE_NEVER
+        for misalign in (0, 1):
+            from ruy_amd import device_problem as D
+            compare(p, D.device_mul(device_ctx, p, misalign=misalign), expected(p))
+        device_ctx.clear_prepacked_cache()
+
+
+def test_small_products_on_two_workgroups_a_cu(device_ctx):
+    """Grids of more tiles than CUs, on operands used in place and on raw ones."""
+    rng = np.random.default_rng(12)
+    for shape in [(2048, 128, 1024), (4096, 250, 500), (2048, 512, 1024)]:
+        p = W.random_problem(rng, S.I8, S.I8, S.I32, S.I8, *shape, 1, 0, 0, name="two a CU %s" % (shape,))
+        got, want = run_both(device_ctx, p)
+        compare(p, got, want)
+
+
 @pytest.mark.parametrize("shape", [
     (1, 16, 1),            # single bytes
     (128, 40, 128),        # a destination of exactly one workgroup's 16 KiB
