@@ -78,6 +78,13 @@ for _name, (_res, _args) in PROTOTYPES.items():
     _fn.argtypes = _args
 
 
+try:
+    from . import _native as native  # api.mul's call path (csrc/python/native.cc)
+except ImportError as e:
+    raise ImportError("ruy_amd/_native.so is missing or does not fit this interpreter: build it with "
+                      "`python -m ruy_amd.build`") from e
+
+
 def check(rc, ctx=None):
     if rc != 0:
         msg = lib.ruyamd_ctx_last_error(ctx).decode() if ctx else ""

@@ -14,7 +14,7 @@ call goes to libruy_amd.so, and importing it without that library raises.
 import ctypes as C
 
 from . import _structs as S
-from ._capi import lib, check
+from ._capi import lib, check, native
 
 
 class Order:
@@ -241,11 +241,13 @@ class Context:
         if rc != 0 or not h:
             raise RuyAmdError(rc, "ruyamd_ctx_create failed (no usable gfx950 device?)")
         self._h = h
+        self._address = h.value
 
     def close(self):
         if getattr(self, "_h", None):
             lib.ruyamd_ctx_destroy(self._h)
             self._h = None
+            self._address = 0
 
     def __del__(self):
         try:
@@ -376,8 +378,17 @@ def mul_batch(items, context):
 
 def mul(lhs, rhs, mul_params, context, dst):
     """ruy::Mul (ruy/ruy.h:96-102)."""
+    rc = native.mul(lhs, rhs, mul_params, context._address, dst)
+    if rc is not None:
+        if rc:
+            context._check(rc)
+        return
+    # Objects the native path leaves to this one (subclasses, values that need converting), and mistakes.
     if mul_params.dst_dtype != dst.dtype:
         raise ValueError("MulParams DstScalar does not match the destination matrix")
     l, r, d = lhs.to_struct(), rhs.to_struct(), dst.to_struct()
     p = mul_params.to_struct()
     context._check(lib.ruyamd_mul(context._h, C.byref(l), C.byref(r), C.byref(p), C.byref(d)))
+
+
+native.bind(C.cast(lib.ruyamd_mul, C.c_void_p).value, Matrix, Layout, MulParams)

@@ -1,4 +1,5 @@
-"""Builds ruy_amd/libruy_amd.so for gfx950 with hipcc.
+"""Builds ruy_amd/libruy_amd.so for gfx950 with hipcc, and the Python mirror's
+native call path ruy_amd/_native.so with g++.
 
     python -m ruy_amd.build [--force]
 
@@ -11,12 +12,14 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "_obj")
 LIB = os.path.join(HERE, "libruy_amd.so")
+NATIVE = os.path.join(HERE, "_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-I" + os.path.join(ROOT, "include"),
@@ -65,9 +68,22 @@ def build(force=False, verbose=True):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed: %s\n%s%s" % (" ".join(cmd), r.stdout, r.stderr))
+    build_native()
     if verbose:
         print("built", LIB)
     return LIB
+
+
+def build_native():
+    """The extension module behind api.mul (csrc/python/native.cc); it calls the
+    library through an address it is given, so it links against nothing."""
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "python", "native.cc"), "-o", NATIVE]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("build failed: %s\n%s%s" % (" ".join(cmd), r.stdout, r.stderr))
+    return NATIVE
 
 
 def build_cpp_tests(verbose=True):

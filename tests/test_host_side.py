@@ -223,3 +223,64 @@ def test_tile_choice_of_the_timing_model():
     with pytest.raises(ValueError):
         api.tile_for(0, 64, 64, 64, compute_units=0)
 
+
+
+def test_the_native_call_path_gathers_what_to_struct_does():
+    """api.mul's native path (csrc/python/native.cc) hands ruyamd_mul the same
+    structs as the Python conversion, and leaves what it does not handle to it."""
+    import ctypes as C
+    import numpy as np
+    import torch
+    from ruy_amd import _structs as S
+    from ruy_amd import api
+    from ruy_amd._capi import lib, native
+    seen = []
+    proto = C.CFUNCTYPE(C.c_int, C.c_void_p, C.POINTER(S.Mat), C.POINTER(S.Mat), C.POINTER(S.MulParamsStruct),
+                        C.POINTER(S.Mat))
+
+    def fields(struct):  # (without the padding behind the last one)
+        return bytes(struct)[:type(struct).reserved.offset + 1]
+
+    def capture(ctx, lhs, rhs, params, dst):
+        seen.append((ctx,) + tuple(fields(x.contents) for x in (lhs, rhs, params, dst)))
+        return 7
+
+    callback = proto(capture)
+    kinds = (api.Matrix, api.Layout, api.MulParams)
+    native.bind(C.cast(callback, C.c_void_p).value, *kinds)
+    try:
+        buffers = [np.zeros(64, np.int8), torch.zeros(64, dtype=torch.int8), 1 << 40, None]
+        for i, data in enumerate(buffers):
+            lhs = api.Matrix(S.I8, data, api.Layout(3 + i, 5, 2 ** 31 - 1 - i, 1), -7 - i, 3)
+            rhs = api.Matrix(S.U8, buffers[i - 1], api.Layout(5, 4, 5, 0), 255, 0)
+            dst = api.Matrix(S.I16, buffers[1], api.Layout(3 + i, 4, 9, 0), 2 ** 32 + 3)
+            params = api.MulParams(S.I32, S.I16)
+            params.set_bias(data)
+            params.set_clamp_min(-5)
+            params.set_clamp_max(np.float64(77.5))
+            params.set_channel_dimension(i % 2)
+            params.set_perchannel_buffers_capacity_rounding(8)
+            if i % 2:
+                params.set_multiplier_fixedpoint(-(2 ** 31) + i)
+                params.set_multiplier_exponent(-9)
+            else:
+                params.set_multiplier_fixedpoint_perchannel(buffers[0])
+                params.set_multiplier_exponent_perchannel(buffers[1])
+            assert native.mul(lhs, rhs, params, 1234, dst) == 7
+            want = tuple(fields(x.to_struct()) for x in (lhs, rhs, params, dst))
+            assert seen.pop() == (1234,) + want
+        # Left to the Python path: other types, values that need converting, mismatched types.
+        class Other(api.Matrix):
+            pass
+        assert native.mul(Other(S.I8), rhs, params, 1, dst) is None
+        lhs.zero_point = 2.0
+        assert native.mul(lhs, rhs, params, 1, dst) is None
+        lhs.zero_point = 2
+        lhs.data = object()
+        assert native.mul(lhs, rhs, params, 1, dst) is None
+        lhs.data = None
+        dst.dtype = S.I8
+        assert native.mul(lhs, rhs, params, 1, dst) is None
+        assert not seen
+    finally:
+        native.bind(C.cast(lib.ruyamd_mul, C.c_void_p).value, *kinds)
