@@ -222,20 +222,20 @@ __device__ __forceinline__ v4i RsrcWords(const void* p, uint32_t bytes) {
 }
 
 // ---------------------------------------------------------------------------
-// Matrix-core variant for 2..16 narrow vectors. One wave per workgroup owns 16
-// wide vectors and walks the whole depth 512 bytes at a time through a ring
-// of LDS stages that only it uses (no barriers): a stage holds the 16 x 512
-// wide bytes and the 8 x 512 (or 16 x 512) narrow bytes of one depth step,
-// both brought in by direct-to-LDS loads in which every instruction fetches
-// whole 512-byte runs. The products are formed by v_mfma_i32_16x16x64_i8 with
+// Matrix-core variant for 2..16 narrow vectors. A workgroup owns 16 wide
+// vectors, and each of its waves walks a share of the depth 256 or 512 bytes at
+// a time (MmaShapeFor) through a ring of LDS stages that only it uses (no
+// barriers): a stage holds that many bytes of the 16 wide and the 8 (or 16)
+// narrow vectors, both brought in by direct-to-LDS loads in which every
+// instruction fetches whole runs of a vector. The products are formed by v_mfma_i32_16x16x64_i8 with
 // the wide vectors as matrix rows and the narrow vectors as columns (when
 // only 8 are staged, columns 8..15 read a 16-byte slot of zeros), which also
 // does the summation over the depth that the dot-product kernel above spends
-// most of its vector instructions on: per depth step the wave issues 12 (16)
+// most of its vector instructions on: per 512 bytes the wave issues 12 (16)
 // loads, 16 LDS reads and 8 matrix instructions and otherwise waits for HBM.
 //
-// LDS layout of a stage: vector v (0..15 wide, 16.. narrow) at v*512; the
-// 16-byte chunk c of the vector's 512-byte run sits in slot c ^ (v & 7), so
+// LDS layout of a stage: vector v (0..15 wide, 16.. narrow) at v*kStep; the
+// 16-byte chunk c of the vector's run sits in slot c ^ (v & 7), so
 // that the 16 lanes of a matrix-operand read (16 vectors, one chunk index)
 // fall into different bank groups.
 // ---------------------------------------------------------------------------
@@ -285,7 +285,7 @@ struct F32Elements {
   }
 };
 
-// kStep: depth bytes per ring stage (256, 512 or 1024). kSplit: waves per
+// kStep: depth bytes per ring stage (256 or 512, MmaShapeFor below). kSplit: waves per
 // workgroup; wave w walks the w-th part of the depth and the partial result
 // blocks are added through LDS at the end. kNarrow: narrow vectors staged, 8
 // or 16 (with 16 every column of the matrix instruction is a real one).
@@ -477,20 +477,64 @@ hipError_t LaunchMma(hipStream_t stream, const GemvI8Args& args) {
   return hipGetLastError();
 }
 
-template <int kSplit, int kNarrow>
-hipError_t LaunchMmaFlip(hipStream_t stream, const GemvI8Args& args, bool flip) {
-  return flip ? LaunchMma<Int8Elements, 2, 512, kSplit, kNarrow, true>(stream, args)
-              : LaunchMma<Int8Elements, 2, 512, kSplit, kNarrow, false>(stream, args);
+template <typename Elements, int kStep, int kSplit, int kNarrow>
+hipError_t LaunchMmaFlip(hipStream_t stream, const GemvI8Args& args) {
+  if constexpr (Elements::kInteger) {
+    if (args.wide_flip != 0 || args.narrow_flip != 0)
+      return LaunchMma<Elements, 2, kStep, kSplit, kNarrow, true>(stream, args);
+  }
+  return LaunchMma<Elements, 2, kStep, kSplit, kNarrow, false>(stream, args);
 }
 
-// Depth split: with few groups of 16 wide vectors the depth is divided over
-// the waves of a workgroup to get enough loads in flight.
-int MmaDepthSplit(const GemvI8Args& args) {
+// Depth bytes per stage and depth split. What bounds these launches is the
+// bytes the waves of a CU keep in flight, and how evenly the groups of 16 wide
+// vectors fall on the CUs. Figures: us a call, weights fetched from memory or
+// its cache on every call, int8 4096 x 4096 x 4 unless another size is given.
+//
+// Stages of 256 bytes take a wave's ring to 12 KiB (8 narrow vectors; 16 KiB
+// with 16), so that a CU holds three (two) workgroups of four waves where
+// 512-byte stages leave room for one, and a grid that is no multiple of the
+// CUs has no second round: fp32 5000 x 2048 x 2 13.3 -> 10.1, 10000 x 4096 x 8
+// 35.1 -> 30.0, 4096 x 4096 x 4 13.1 -> 12.0; int8 16384 x 8192 x 4 28.4 ->
+// 22.0, 8192 x 4096 x 4 10.6 -> 8.3. Deeper rings of them lose (fp32 4096 x
+// 4096 x 4 12.4 with three stages, 13.1 with four): they cost the third
+// workgroup.
+// Vectors of 32 KiB and more want the longer runs: fp32 3000 x 16384 x 3 34.2
+// in 512-byte stages, 39.0 in 256-byte ones, 16384 x 8192 x 16 78.2 and 80.9.
+// Except where half the CUs or fewer have a group: there eight waves share the
+// depth of each (of four steps and more a wave, or their ring never fills):
+// fp32 512 x 16384 x 7 30.9 -> 23.0, 2048 x 8192 x 4 17.9 -> 14.0, int8 512 x
+// 16384 x 7 9.1 -> 6.9.
+// Four waves to a group up to four groups to a CU (one wave: fp32 8192 x 4096 x
+// 4 36.4, two: 25.1, four: 22.6), one beyond (int8 16384 x 512 x 4 4.7, four:
+// 6.5). With 16 narrow vectors a CU holds ten waves, and two to a group do
+// better from two groups to a CU on (int8 9000 x 4096 x 10 9.3, four: 11.0).
+struct MmaShape {
+  int step, split;
+};
+MmaShape MmaShapeFor(const GemvI8Args& args) {
   const int groups = (args.rows + kMmaRows - 1) / kMmaRows;
-  const int steps = (args.K + 511) / 512;
-  if (groups >= 1024 || steps < 4) return 1;
-  if (groups >= 512) return steps >= 16 ? 2 : 1;
-  return steps < 8 ? 2 : 4;
+  const int steps = (args.K + 255) / 256;
+  if (groups <= 128 && steps >= 32) return {256, 8};
+  if (args.K >= 32768) return {512, groups >= 1024 ? 1 : groups >= 512 ? 2 : 4};
+  if (groups >= 1024 || steps < 2) return {256, 1};
+  return {256, groups >= 512 && args.narrow_count > 8 ? 2 : 4};
+}
+
+template <typename Elements, int kNarrow>
+hipError_t LaunchMmaShaped(hipStream_t stream, const GemvI8Args& args) {
+  const MmaShape shape = MmaShapeFor(args);
+  if (shape.step == 512) {
+    if (shape.split == 1) return LaunchMmaFlip<Elements, 512, 1, kNarrow>(stream, args);
+    if (shape.split == 2) return LaunchMmaFlip<Elements, 512, 2, kNarrow>(stream, args);
+    return LaunchMmaFlip<Elements, 512, 4, kNarrow>(stream, args);
+  }
+  if (shape.split == 1) return LaunchMmaFlip<Elements, 256, 1, kNarrow>(stream, args);
+  if constexpr (kNarrow == 16) {
+    if (shape.split == 2) return LaunchMmaFlip<Elements, 256, 2, kNarrow>(stream, args);
+  }
+  if (shape.split == 4) return LaunchMmaFlip<Elements, 256, 4, kNarrow>(stream, args);
+  return LaunchMmaFlip<Elements, 256, 8, kNarrow>(stream, args);
 }
 
 }  // namespace
@@ -520,15 +564,8 @@ hipError_t LaunchGemvI8(hipStream_t stream, const GemvI8Args& caller_args) {
       Launch<1, 2, false>(stream, args);
     return hipGetLastError();
   }
-  const int split = MmaDepthSplit(args);
-  if (args.narrow_count <= 8) {
-    if (split == 1) return LaunchMmaFlip<1, 8>(stream, args, flip);
-    if (split == 2) return LaunchMmaFlip<2, 8>(stream, args, flip);
-    return LaunchMmaFlip<4, 8>(stream, args, flip);
-  }
-  if (split == 1) return LaunchMmaFlip<1, 16>(stream, args, flip);
-  if (split == 2) return LaunchMmaFlip<2, 16>(stream, args, flip);
-  return LaunchMmaFlip<4, 16>(stream, args, flip);
+  return args.narrow_count <= 8 ? LaunchMmaShaped<Int8Elements, 8>(stream, args)
+                                : LaunchMmaShaped<Int8Elements, 16>(stream, args);
 }
 
 // fp32 with 2..16 narrow vectors: the same streaming kernel on
@@ -540,15 +577,8 @@ hipError_t LaunchGemvF32Mma(hipStream_t stream, const GemvI8Args& caller_args) {
   if (args.narrow_count > 16 || args.K % 16 != 0 || args.ld_wide % 16 != 0 || args.ld_narrow % 16 != 0 ||
       (reinterpret_cast<uintptr_t>(args.wide) | reinterpret_cast<uintptr_t>(args.narrow)) % 16 != 0)
     return hipErrorInvalidValue;
-  const int split = MmaDepthSplit(args);
-  if (args.narrow_count <= 8) {
-    if (split == 1) return LaunchMma<F32Elements, 2, 512, 1, 8, false>(stream, args);
-    if (split == 2) return LaunchMma<F32Elements, 2, 512, 2, 8, false>(stream, args);
-    return LaunchMma<F32Elements, 2, 512, 4, 8, false>(stream, args);
-  }
-  if (split == 1) return LaunchMma<F32Elements, 2, 512, 1, 16, false>(stream, args);
-  if (split == 2) return LaunchMma<F32Elements, 2, 512, 2, 16, false>(stream, args);
-  return LaunchMma<F32Elements, 2, 512, 4, 16, false>(stream, args);
+  return args.narrow_count <= 8 ? LaunchMmaShaped<F32Elements, 8>(stream, args)
+                                : LaunchMmaShaped<F32Elements, 16>(stream, args);
 }
 
 }  // namespace ruyamd

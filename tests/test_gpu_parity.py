@@ -751,6 +751,27 @@ def test_skinny_nine_to_sixteen_vectors(device_ctx, tup):
             assert device_ctx.last_kernel_name() == ("f32_gemv" if tup[0] == S.F32 else "i8_gemv")
 
 
+@pytest.mark.parametrize("tup", [(S.I8, S.I8, S.I32, S.I32), (S.U8, S.U8, S.I32, S.U8), (S.F32, S.F32, S.F32, S.F32)],
+                         ids=cases.tuple_name)
+@pytest.mark.parametrize("narrow", [2, 8, 9, 16])
+def test_skinny_stage_sizes_and_depth_splits(device_ctx, tup, narrow):
+    """Both sides of every line between the forms of the streaming kernel: one
+    and two 256-byte steps, 32 of them (eight waves to a group of 16 rows) and
+    one less, 128 groups and one more, 32 KiB vectors and a little less, 512 and
+    1024 groups; depths of whole 512 bytes (uint8 in place), of a ragged last
+    step and with waves left without one."""
+    rng = np.random.default_rng(77)
+    size = 4 if tup[0] == S.F32 else 1
+    for rows, depth_bytes in [(40, 256), (40, 512), (40, 7936), (40, 7952), (2048, 8192), (2049, 8192), (2064, 32768),
+                              (2064, 32752), (40, 33024), (8176, 1024), (8177, 1040), (16368, 512), (16369, 528)]:
+        p = W.random_problem(rng, *tup, rows, depth_bytes // size, narrow, *cases.RCC, strided=False,
+                             name="%s %dx%dx%d" % (cases.tuple_name(tup), rows, depth_bytes // size, narrow))
+        announce(p.name)
+        got, want = run_both(device_ctx, p)
+        compare(p, got, want)
+        assert device_ctx.last_kernel_name() == ("f32_gemv" if tup[0] == S.F32 else "i8_gemv")
+
+
 def test_caller_stream_asynchronous_calls_and_kernel_timing(device_ctx):
     """Device-side controls without a counterpart in the reference: launching on
     a caller-owned stream, returning before completion, per-kernel timing."""
