@@ -488,8 +488,8 @@ hipError_t LaunchMmaFlip(hipStream_t stream, const GemvI8Args& args) {
 
 // Depth bytes per stage and depth split. What bounds these launches is the
 // bytes the waves of a CU keep in flight, and how evenly the groups of 16 wide
-// vectors fall on the CUs. Figures: us a call, weights fetched from memory or
-// its cache on every call, int8 4096 x 4096 x 4 unless another size is given.
+// vectors fall on the CUs. Figures: us a call, sizes M x K x N, three sets of
+// operands in turn.
 //
 // Stages of 256 bytes take a wave's ring to 12 KiB (8 narrow vectors; 16 KiB
 // with 16), so that a CU holds three (two) workgroups of four waves where
