@@ -43,8 +43,10 @@ __global__ __launch_bounds__(kThreads) void UploadKernel(UploadPieces pieces) {
 __global__ __launch_bounds__(kThreads) void DownloadKernel(const void* from, void* to, uint32_t bytes, uint32_t* done,
                                                            uint32_t value) {
   CopyBlock(from, to, bytes);
-  // One release per workgroup, behind the barrier that orders the other
-  // waves' stores in front of it.
+  // Every wave writes back and awaits its own stores before the barrier: the
+  // barrier itself waits for no store, and the release behind it only for those
+  // of the one wave that stores the word.
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(done + blockIdx.x, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }

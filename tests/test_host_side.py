@@ -99,6 +99,31 @@ def test_ring_schedule_of_the_largest_tile_model():
     assert out.count("altered (") >= 12
 
 
+def test_every_wave_of_a_download_awaits_its_stores(tmp_path):
+    """The word that tells the host a workgroup's part of a download is there is
+    stored by one wave (kernels/host_copy.hip). A workgroup barrier by itself
+    waits for no store on this target, so each wave has to write back and await
+    its own in front of it: looked up in the assembly, between the last store of
+    the copy and the barrier."""
+    from ruy_amd import build
+    asm = str(tmp_path / "host_copy.s")
+    subprocess.check_call([build.HIPCC] + build.COMMON + build.DEVICE + [
+        "--offload-device-only", "-S", os.path.join(build.CSRC, "kernels", "host_copy.hip"), "-o", asm])
+    lines = [l.split(";")[0].strip() for l in open(asm)]
+    start = next(i for i, l in enumerate(lines) if "DownloadKernel" in l and l.endswith(":"))
+    body = lines[start:lines.index("s_endpgm", start)]
+    barrier = body.index("s_barrier")
+    last_store = max(i for i, l in enumerate(body[:barrier]) if l.startswith("global_store_dwordx4"))
+    between = body[last_store + 1:barrier]
+    write_back = [i for i, l in enumerate(between) if re.match(r"buffer_wbl2\s+sc0 sc1", l)]
+    awaited = [i for i, l in enumerate(between) if l.startswith("s_waitcnt") and "vmcnt(0)" in l]
+    assert write_back and awaited and awaited[-1] > write_back[-1], between
+    # ... and every wave gets there: the copy's own bounds tests have ended.
+    assert any(l.startswith("s_or_b64 exec, exec") for l in between[:write_back[-1]]), between
+    flag = [i for i, l in enumerate(body) if re.match(r"global_store_dword\s", l)]
+    assert len(flag) == 1 and flag[0] > barrier, flag
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
