@@ -108,6 +108,16 @@ int LaunchPendingPacks(ruyamd_ctx* ctx, const PendingPack& a, const PendingPack&
   return RUYAMD_OK;
 }
 
+// EnsureOnDevice for an operand from which a new entry of the prepacked cache
+// is about to be packed: its upload is enqueued here, so that an entry whose
+// source never arrived can be taken out again.
+int EnsureUploaded(ruyamd_ctx* ctx, MulCall* call, int side, std::string* err) {
+  if (int rc = EnsureOnDevice(ctx, call, side, err)) return rc;
+  if (ctx->staging.Flush(ctx->stream)) return RUYAMD_OK;
+  *err = "staging a host operand to the device failed";
+  return RUYAMD_E_HIP;
+}
+
 // Packs one operand for the prepacked cache: here the sums are part of the
 // entry, wherever they are formed.
 hipError_t PackForCache8(ruyamd_ctx* ctx, const PackSource& src, int8_t* dst, int32_t ld, int32_t* sums) {
@@ -179,7 +189,7 @@ int PrepareOperand8(ruyamd_ctx* ctx, MulCall* call, int side, int32_t zero_point
     if (action == PrepackedCache::Action::kInsertedNewEntry) {
       // The entry exists from here on; if it cannot be filled it must not stay,
       // or the next call would hit buffers that were never packed.
-      if (int rc = EnsureOnDevice(ctx, call, side, err)) {
+      if (int rc = EnsureUploaded(ctx, call, side, err)) {
         ctx->cache->Erase(src_key, pm);
         return rc;
       }
@@ -560,7 +570,7 @@ int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy
       return RUYAMD_E_HIP;
     }
     if (action == PrepackedCache::Action::kInsertedNewEntry) {
-      if (int rc = EnsureOnDevice(ctx, call, side, err)) {
+      if (int rc = EnsureUploaded(ctx, call, side, err)) {
         ctx->cache->Erase(src_key, pm);
         return rc;
       }
@@ -746,7 +756,7 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
         return RUYAMD_E_HIP;
       }
       if (action == PrepackedCache::Action::kInsertedNewEntry) {
-        if (int rc = EnsureOnDevice(ctx, call, side16, err)) {
+        if (int rc = EnsureUploaded(ctx, call, side16, err)) {
           ctx->cache->Erase(key16, pm);
           return rc;
         }
@@ -1002,7 +1012,7 @@ int CacheGenericOperand(ruyamd_ctx* ctx, MulCall* call, int side, std::string* e
   copy.rs = side == 0 ? depth : 1;
   copy.cs = side == 0 ? 1 : depth;
   if (action == PrepackedCache::Action::kInsertedNewEntry) {
-    if (int rc = EnsureOnDevice(ctx, call, side, err)) {
+    if (int rc = EnsureUploaded(ctx, call, side, err)) {
       ctx->cache->Erase(key, pm);
       return rc;
     }

@@ -1,0 +1,377 @@
+// The library's host side run against a model of the HIP runtime: this program
+// defines the runtime's functions itself (they take precedence over those of
+// libamdhip64), with "device" memory in host memory and one stream whose work
+// is performed only when something waits for it. Kernels are not executed, but
+// for the two that copy between host and device; every launch is logged by
+// name. That shows in which order a call enqueues its work, what it does when a
+// launch fails, and what it asks for while its stream records a graph, none of
+// which a GPU is needed (or, for the failures, wanted) for.
+//
+//   runtime_model_test failed_upload
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "kernels/host_copy.h"
+#include "ruy_amd/c_api.h"
+
+static int g_failures = 0;
+#define EXPECT(cond, ...)                                                              \
+  do {                                                                                 \
+    if (!(cond)) {                                                                     \
+      std::fprintf(stderr, "%s:%d: EXPECT failed: %s: ", __FILE__, __LINE__, #cond);   \
+      std::fprintf(stderr, __VA_ARGS__);                                               \
+      std::fprintf(stderr, "\n");                                                      \
+      ++g_failures;                                                                    \
+    }                                                                                  \
+  } while (0)
+
+namespace {
+
+// Everything the model knows. (A function-local object: the library registers
+// its kernels before this program's own static objects are constructed.)
+struct Runtime {
+  std::map<const void*, std::string> kernels;
+  std::map<const char*, std::size_t> device, pinned;  // base -> size
+  std::vector<std::function<void()>> queue;           // enqueued, not performed yet
+  std::vector<std::string> log;                       // kernel names and "event"
+  std::vector<std::vector<char>> uploads;             // what each upload that was performed brought
+  std::string fail_kernel;                            // fail the fail_at-th launch of a kernel so named
+  int fail_at = 0;
+  hipError_t last_error = hipSuccess;
+  bool capturing = false;
+  int capture_violations = 0;
+  dim3 grid, block;
+  std::size_t shared = 0;
+  hipStream_t stream = nullptr;
+};
+Runtime& R() {
+  static Runtime* r = new Runtime;
+  return *r;
+}
+
+void Drain() {
+  std::vector<std::function<void()>> work;
+  work.swap(R().queue);
+  for (auto& f : work) f();
+}
+
+// What a stream that records a graph cannot take.
+void NotWhileCapturing() {
+  if (R().capturing) ++R().capture_violations;
+}
+
+const char* In(const std::map<const char*, std::size_t>& ranges, const void* p) {
+  auto it = ranges.upper_bound(static_cast<const char*>(p));
+  if (it == ranges.begin()) return nullptr;
+  --it;
+  return static_cast<const char*>(p) < it->first + it->second ? it->first : nullptr;
+}
+
+void Upload(void* to, const void* from, std::size_t bytes, std::size_t moved) {
+  std::memcpy(to, from, moved);
+  const char* c = static_cast<const char*>(from);
+  R().uploads.emplace_back(c, c + bytes);
+}
+
+}  // namespace
+
+extern "C" {
+
+void** __hipRegisterFatBinary(const void*) {
+  static void* module = nullptr;
+  return &module;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+  R().kernels[host] = name;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, std::size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, std::size_t shared, hipStream_t stream) {
+  R().grid = grid;
+  R().block = block;
+  R().shared = shared;
+  R().stream = stream;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, std::size_t* shared, hipStream_t* stream) {
+  *grid = R().grid;
+  *block = R().block;
+  *shared = R().shared;
+  *stream = R().stream;
+  return hipSuccess;
+}
+
+hipError_t hipLaunchKernel(const void* function, dim3, dim3, void** args, std::size_t, hipStream_t) {
+  const std::string& name = R().kernels[function];
+  if (!R().fail_kernel.empty() && name.find(R().fail_kernel) != std::string::npos && --R().fail_at == 0) {
+    R().last_error = hipErrorLaunchOutOfResources;
+    return R().last_error;
+  }
+  R().log.push_back(name);
+  if (name.find("UploadKernel") != std::string::npos) {
+    const ruyamd::UploadPieces pieces = *static_cast<const ruyamd::UploadPieces*>(args[0]);
+    R().queue.push_back([pieces] {
+      for (int i = 0; i < pieces.count; ++i) {
+        EXPECT(reinterpret_cast<std::uintptr_t>(pieces.from[i]) % 16 == 0, "piece %d", i);
+        Upload(pieces.to[i], pieces.from[i], pieces.bytes[i], (pieces.bytes[i] + 15) / 16 * 16);
+      }
+    });
+  }
+  if (name.find("DownloadKernel") != std::string::npos) {
+    const void* from = *static_cast<const void**>(args[0]);
+    void* to = *static_cast<void**>(args[1]);
+    const uint32_t bytes = *static_cast<uint32_t*>(args[2]);
+    uint32_t* done = *static_cast<uint32_t**>(args[3]);
+    const uint32_t value = *static_cast<uint32_t*>(args[4]);
+    R().queue.push_back([=] {
+      std::memcpy(to, from, (bytes + 15) / 16 * 16);
+      for (int b = 0; b < ruyamd::DownloadBlocks(bytes); ++b) done[b] = value;
+    });
+    Drain();  // (a GPU gets there by itself)
+  }
+  return hipSuccess;
+}
+
+static hipError_t Take(std::map<const char*, std::size_t>* ranges, void** p, std::size_t bytes) {
+  *p = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096 + 4096);
+  std::memset(*p, 0xCD, bytes);
+  (*ranges)[static_cast<char*>(*p)] = bytes;
+  NotWhileCapturing();
+  return hipSuccess;
+}
+static hipError_t Give(std::map<const char*, std::size_t>* ranges, void* p) {
+  Drain();
+  if (p) ranges->erase(static_cast<char*>(p));
+  std::free(p);
+  NotWhileCapturing();
+  return hipSuccess;
+}
+hipError_t hipMalloc(void** p, std::size_t bytes) { return Take(&R().device, p, bytes); }
+hipError_t hipFree(void* p) { return Give(&R().device, p); }
+hipError_t hipHostMalloc(void** p, std::size_t bytes, unsigned) { return Take(&R().pinned, p, bytes); }
+hipError_t hipHostFree(void* p) { return Give(&R().pinned, p); }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  std::memset(a, 0, sizeof(*a));
+  const bool device = In(R().device, p), host = In(R().pinned, p);
+  if (!device && !host) return R().last_error = hipErrorInvalidValue;
+  a->type = device ? hipMemoryTypeDevice : hipMemoryTypeHost;
+  a->devicePointer = const_cast<void*>(p);
+  if (host) a->hostPointer = const_cast<void*>(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* to, const void* from, std::size_t bytes, hipMemcpyKind kind, hipStream_t) {
+  NotWhileCapturing();
+  R().queue.push_back([=] {
+    if (kind == hipMemcpyHostToDevice)
+      Upload(to, from, bytes, bytes);
+    else
+      std::memcpy(to, from, bytes);
+  });
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* to, const void* from, std::size_t bytes, hipMemcpyKind) {
+  Drain();
+  std::memcpy(to, from, bytes);
+  return hipSuccess;
+}
+hipError_t hipMemcpy2DAsync(void* to, std::size_t to_pitch, const void* from, std::size_t from_pitch, std::size_t width,
+                            std::size_t height, hipMemcpyKind, hipStream_t) {
+  NotWhileCapturing();
+  R().queue.push_back([=] {
+    for (std::size_t i = 0; i < height; ++i)
+      std::memcpy(static_cast<char*>(to) + i * to_pitch, static_cast<const char*>(from) + i * from_pitch, width);
+  });
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* p, int value, std::size_t bytes, hipStream_t) {
+  NotWhileCapturing();
+  R().queue.push_back([=] { std::memset(p, value, bytes); });
+  return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t* e) {
+  *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) {
+  std::free(e);
+  return hipSuccess;
+}
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 1;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) {
+  R().log.push_back("event");
+  NotWhileCapturing();
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t) {
+  Drain();
+  NotWhileCapturing();
+  return hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipGetDeviceCount(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+  std::memset(p, 0, sizeof(*p));
+  std::strcpy(p->gcnArchName, "gfx950:sramecc+:xnack-");
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "an error of the runtime model"; }
+hipError_t hipGetLastError() {
+  const hipError_t e = R().last_error;
+  R().last_error = hipSuccess;
+  return e;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) {
+  static void* area = nullptr;
+  if (!area) (void)Take(&R().device, &area, std::size_t(64) << 20);
+  *p = area;
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = reinterpret_cast<hipStream_t>(std::malloc(1));
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) {
+  std::free(s);
+  return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+  *s = R().capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+  Drain();
+  NotWhileCapturing();
+  return hipSuccess;
+}
+
+}  // extern "C"
+
+namespace {
+
+int SizeOf(int dtype) {
+  switch (dtype) {
+    case RUYAMD_DTYPE_U8:
+    case RUYAMD_DTYPE_I8:
+      return 1;
+    case RUYAMD_DTYPE_I16:
+      return 2;
+    case RUYAMD_DTYPE_F64:
+      return 8;
+    default:
+      return 4;
+  }
+}
+
+ruyamd_mat Mat(int dtype, void* data, int rows, int cols, int order, int zero_point = 0,
+               int cache = RUYAMD_CACHE_NEVER) {
+  ruyamd_mat m = {};
+  m.data = data;
+  m.rows = rows;
+  m.cols = cols;
+  m.stride = order == RUYAMD_ORDER_COL_MAJOR ? rows : cols;
+  m.zero_point = zero_point;
+  m.order = static_cast<uint8_t>(order);
+  m.dtype = static_cast<uint8_t>(dtype);
+  m.cache_policy = static_cast<uint8_t>(cache);
+  return m;
+}
+
+ruyamd_mul_params Params(int dst) {
+  ruyamd_mul_params p = {};
+  const bool fp = dst == RUYAMD_DTYPE_F32 || dst == RUYAMD_DTYPE_F64;
+  p.accum_dtype = static_cast<uint8_t>(fp ? dst : RUYAMD_DTYPE_I32);
+  p.clamp_min = fp ? -1e30 : -128;
+  p.clamp_max = fp ? 1e30 : 127;
+  p.multiplier_fixedpoint = fp ? 0 : 1 << 30;
+  p.multiplier_exponent = fp ? 0 : -9;
+  return p;
+}
+
+struct Context {
+  ruyamd_ctx* ctx = nullptr;
+  Context() {
+    if (ruyamd_ctx_create(&ctx) != RUYAMD_OK) std::abort();
+    R().log.clear();
+    R().uploads.clear();
+    R().capture_violations = 0;
+  }
+  ~Context() { ruyamd_ctx_destroy(ctx); }
+};
+
+int Count(const char* name) {
+  return static_cast<int>(std::count_if(R().log.begin(), R().log.end(),
+                                        [&](const std::string& s) { return s.find(name) != std::string::npos; }));
+}
+
+struct Types {
+  const char* name;
+  int lhs, rhs, dst;
+};
+const Types kTypes[] = {{"int8", RUYAMD_DTYPE_I8, RUYAMD_DTYPE_I8, RUYAMD_DTYPE_I8},
+                        {"fp32", RUYAMD_DTYPE_F32, RUYAMD_DTYPE_F32, RUYAMD_DTYPE_F32},
+                        {"int8 x int16", RUYAMD_DTYPE_I8, RUYAMD_DTYPE_I16, RUYAMD_DTYPE_I16},
+                        {"generic", RUYAMD_DTYPE_F64, RUYAMD_DTYPE_F64, RUYAMD_DTYPE_F64}};
+
+// A cached operand whose upload could not be launched leaves no entry: the next
+// call uploads and packs it.
+void FailedUpload() {
+  const int M = 96, K = 160, N = 64;
+  for (const Types& t : kTypes) {
+    for (int fail_at = 1; fail_at <= 2; ++fail_at) {
+      Context c;
+      std::vector<char> lhs(M * K * 8, 1), rhs(K * N * 8, 2), dst(M * N * 8);
+      const ruyamd_mat l = Mat(t.lhs, lhs.data(), M, K, RUYAMD_ORDER_ROW_MAJOR, 0, RUYAMD_CACHE_ALWAYS);
+      const ruyamd_mat r = Mat(t.rhs, rhs.data(), K, N, RUYAMD_ORDER_COL_MAJOR, 0, RUYAMD_CACHE_ALWAYS);
+      const ruyamd_mat d = Mat(t.dst, dst.data(), M, N, RUYAMD_ORDER_COL_MAJOR);
+      const ruyamd_mul_params p = Params(t.dst);
+      R().fail_kernel = "UploadKernel";
+      R().fail_at = fail_at;
+      EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) != RUYAMD_OK, "%s, upload %d", t.name, fail_at);
+      R().fail_kernel.clear();
+      // The operands go up one after the other: those before the failure are cached.
+      EXPECT(ruyamd_ctx_cache_matrix_count(c.ctx) == fail_at - 1, "%s, upload %d: %d entries", t.name, fail_at,
+             ruyamd_ctx_cache_matrix_count(c.ctx));
+      R().uploads.clear();
+      EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", t.name);
+      EXPECT(static_cast<int>(R().uploads.size()) == 3 - fail_at, "%s, upload %d: %d operands uploaded by the next call",
+             t.name, fail_at, static_cast<int>(R().uploads.size()));
+      EXPECT(ruyamd_ctx_cache_matrix_count(c.ctx) == 2, "%s", t.name);
+    }
+  }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string which = argc > 1 ? argv[1] : "";
+  if (which == "failed_upload") FailedUpload();
+  else return 2;
+  if (g_failures) {
+    std::printf("%d failures\n", g_failures);
+    return 1;
+  }
+  std::printf("%s: all passed\n", which.c_str());
+  return 0;
+}

@@ -124,6 +124,31 @@ def test_every_wave_of_a_download_awaits_its_stores(tmp_path):
     assert len(flag) == 1 and flag[0] > barrier, flag
 
 
+@pytest.fixture(scope="module")
+def runtime_model(tmp_path_factory):
+    """tests/cpp/runtime_model_test.cc: the library on a model of the HIP runtime."""
+    from ruy_amd import build
+    exe = str(tmp_path_factory.mktemp("runtime_model") / "runtime_model_test")
+    here = os.path.join(ROOT, "ruy_amd")
+    rocm = os.path.dirname(os.path.dirname(build.HIPCC))
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-rdynamic", "-D__HIP_PLATFORM_AMD__",
+                           "-I" + os.path.join(rocm, "include"), "-I" + os.path.join(ROOT, "include"),
+                           "-I" + build.CSRC, os.path.join(ROOT, "tests", "cpp", "runtime_model_test.cc"),
+                           "-L" + here, "-lruy_amd", "-Wl,-rpath," + here,
+                           "-Wl,-rpath-link," + os.path.join(rocm, "lib"), "-o", exe])
+
+    def run(what):
+        result = subprocess.run([exe, what], capture_output=True, text=True)
+        assert result.returncode == 0 and "all passed" in result.stdout, result.stdout + result.stderr
+    return run
+
+
+def test_a_failed_upload_leaves_no_cache_entry(runtime_model):
+    """Whichever of a call's uploads cannot be launched, no entry packed from
+    memory that was never written stays in the prepacked cache (every type)."""
+    runtime_model("failed_upload")
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
