@@ -128,24 +128,43 @@ bool HostStaging::RetireCurrent(hipStream_t stream) {
   return true;
 }
 
-namespace {
-// Page-locked host memory (hipHostMalloc, torch's pinned tensors): the copy
-// engine reaches it directly, no staging needed.
-bool IsPinnedHost(const void* p) {
+Memory MemoryOf(const void* p) {
   hipPointerAttribute_t attr;
   if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
-    (void)hipGetLastError();  // ordinary pageable memory
-    return false;
+    (void)hipGetLastError();  // memory the runtime does not know
+    return Memory::kPageable;
   }
-  return attr.type == hipMemoryTypeHost;
+  switch (attr.type) {
+    case hipMemoryTypeDevice:
+    case hipMemoryTypeManaged:
+    case hipMemoryTypeArray:
+      return Memory::kDevice;
+    case hipMemoryTypeHost:
+      return attr.devicePointer == p ? Memory::kPageLockedMapped : Memory::kPageLocked;
+    default:
+      return Memory::kPageable;
+  }
 }
-}  // namespace
 
-bool HostStaging::ToDevice(void* dst_dev, const void* src_host, std::size_t bytes, hipStream_t stream) {
+bool HostStaging::Collect(void* to, const void* from, std::size_t bytes, hipStream_t stream) {
+  if (pending_.count == UploadPieces::kMost && !FlushPending(stream)) return false;
+  pending_.from[pending_.count] = from;
+  pending_.to[pending_.count] = to;
+  pending_.bytes[pending_.count] = static_cast<uint32_t>(bytes);
+  ++pending_.count;
+  return true;
+}
+
+bool HostStaging::ToDevice(void* dst_dev, const void* src_host, std::size_t bytes, Memory source, hipStream_t stream) {
   if (bytes == 0) return true;
   const bool by_kernel = bytes <= kByKernel;
-  if (!by_kernel && IsPinnedHost(src_host))
+  if (source != Memory::kPageable) {
+    // (The kernel reads whole 16-byte granules: from an aligned address those
+    // that hold a byte of the source, so nothing beyond its page.)
+    if (by_kernel && source == Memory::kPageLockedMapped && (reinterpret_cast<uintptr_t>(src_host) & 15) == 0)
+      return Collect(dst_dev, src_host, bytes, stream);
     return hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream) == hipSuccess;
+  }
   if (!Init()) return false;
   const char* src = static_cast<const char*>(src_host);
   char* dst = static_cast<char*>(dst_dev);
@@ -162,11 +181,7 @@ bool HostStaging::ToDevice(void* dst_dev, const void* src_host, std::size_t byte
     char* piece = pinned_ + std::size_t(current_) * kChunkBytes + at;
     std::memcpy(piece, src, n);
     if (by_kernel) {  // (one piece: it fits a chunk)
-      if (pending_.count == UploadPieces::kMost && !FlushPending(stream)) return false;
-      pending_.from[pending_.count] = piece;
-      pending_.to[pending_.count] = dst;
-      pending_.bytes[pending_.count] = static_cast<uint32_t>(n);
-      ++pending_.count;
+      if (!Collect(dst, piece, n, stream)) return false;
     } else if (hipMemcpyAsync(dst, piece, n, hipMemcpyHostToDevice, stream) != hipSuccess) return false;
     fill_ = at + n;
     src += n;
@@ -213,14 +228,14 @@ bool HostStaging::SmallToHost2D(char* dst, const void* src_dev, std::size_t pitc
 }
 
 bool HostStaging::ToHost2D(void* dst_host, const void* src_dev, std::size_t pitch, std::size_t inner_bytes,
-                           std::size_t outer, hipStream_t stream, bool* drained) {
+                           std::size_t outer, Memory destination, hipStream_t stream, bool* drained) {
   *drained = false;
   if (inner_bytes == 0 || outer == 0) return true;
   if (pitch * (outer - 1) + inner_bytes <= kByKernel) {
     if (!Init()) return false;
     return SmallToHost2D(static_cast<char*>(dst_host), src_dev, pitch, inner_bytes, outer, stream, drained);
   }
-  if (IsPinnedHost(dst_host)) {
+  if (destination != Memory::kPageable) {
     // Stream-ordered; complete once the caller has synchronised the stream.
     if (pitch == inner_bytes || outer == 1)
       return hipMemcpyAsync(dst_host, src_dev, pitch * (outer - 1) + inner_bytes, hipMemcpyDeviceToHost,

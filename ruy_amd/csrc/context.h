@@ -59,16 +59,28 @@ class Workspace {
   bool exhausted_ = false;
 };
 
+// What the runtime knows about a buffer of a call.
+enum class Memory {
+  kDevice,            // (managed memory too)
+  kPageable,          // ordinary host memory
+  kPageLocked,        // hipHostMalloc, torch's pinned tensors
+  kPageLockedMapped,  // the same, at the same address for kernels
+};
+Memory MemoryOf(const void* p);
+
 // Moves pageable host memory to and from the device through a small ring of
 // pinned chunks: the CPU copies into (out of) a chunk while the copy engine
 // works on the previous ones, and every transfer the engine sees is a true
-// asynchronous pinned copy. Small operands share a chunk. Host memory that is
-// already page-locked skips the chunks and is copied directly. Small transfers
-// (kByKernel bytes) do not use the copy engine at all: what a call uploads is
-// collected in a chunk and moved by one kernel when the first kernel that may
-// read it is about to be launched (Flush), and a small destination comes back
-// by a kernel whose completion the host sees in host memory
-// (kernels/host_copy.hip). Used only by calls
+// asynchronous pinned copy. Small operands share a chunk. A source that is
+// already page-locked skips the chunks: it is read where it lies, in stream
+// order, so that a call may follow the work that fills it on the same stream;
+// a large page-locked destination is written by the copy engine directly.
+// Small transfers (kByKernel bytes) do not use the copy engine at all: what a
+// call uploads is collected - in a chunk, or where it lies if that is 16-byte
+// aligned page-locked memory - and moved by one kernel when the first kernel
+// that may read it is about to be launched (Flush), and a small destination
+// comes back through a chunk by a kernel whose completion the host sees in host
+// memory (kernels/host_copy.hip). Used only by calls
 // that were handed host pointers; such a call ends with a stream
 // synchronisation or a download seen to be complete, after which Reset()
 // makes all chunks available again.
@@ -77,17 +89,18 @@ class HostStaging {
   ~HostStaging();
   // dst_dev[0, bytes) = src_host[0, bytes), ordered on `stream` once Flush has
   // been called. dst_dev is 16-byte aligned and has room for a whole number of
-  // 16-byte granules.
-  bool ToDevice(void* dst_dev, const void* src_host, std::size_t bytes, hipStream_t stream);
+  // 16-byte granules. A pageable source is read before this returns, a
+  // page-locked one (`source`) when the stream gets there.
+  bool ToDevice(void* dst_dev, const void* src_host, std::size_t bytes, Memory source, hipStream_t stream);
   // Copies `outer` runs of `inner_bytes`, `pitch` bytes apart in both images,
   // from device to host after everything already enqueued on `stream`; the
   // bytes between the runs of the host image are not written. The host image
-  // is complete when this returns (pageable destination) or once the stream
-  // has been synchronised (page-locked destination, copied directly). *drained
-  // is set if everything enqueued on `stream` so far is known to have finished.
-  // src_dev as dst_dev in ToDevice.
+  // is complete when this returns (pageable or small destination) or once the
+  // stream has been synchronised (large page-locked `destination`, copied
+  // directly). *drained is set if everything enqueued on `stream` so far is
+  // known to have finished. src_dev as dst_dev in ToDevice.
   bool ToHost2D(void* dst_host, const void* src_dev, std::size_t pitch, std::size_t inner_bytes,
-                std::size_t outer, hipStream_t stream, bool* drained);
+                std::size_t outer, Memory destination, hipStream_t stream, bool* drained);
   // Forgets uploads that a failed call has left behind.
   void DropPending() { pending_.count = 0; }
   // Enqueues the uploads collected so far: before any kernel that may read them.
@@ -107,6 +120,7 @@ class HostStaging {
   // Behind the chunks: one word per workgroup of a download.
   static constexpr std::size_t kDoneBytes = kByKernel / kHostCopyBlockBytes * sizeof(uint32_t);
   bool Init();
+  bool Collect(void* to, const void* from, std::size_t bytes, hipStream_t stream);
   bool FlushPending(hipStream_t stream);
   bool SmallToHost2D(char* dst, const void* src_dev, std::size_t pitch, std::size_t inner_bytes, std::size_t outer,
                      hipStream_t stream, bool* drained);
@@ -118,7 +132,7 @@ class HostStaging {
   bool busy_[kChunks] = {};
   int current_ = 0;            // chunk being filled by ToDevice
   std::size_t fill_ = 0;       // bytes of it already handed to the copy engine or collected in pending_
-  UploadPieces pending_;       // pieces of the current chunk that no launch has moved yet
+  UploadPieces pending_;       // pieces (of the current chunk or page-locked sources) that no launch has moved yet
   uint32_t downloads_ = 0;     // the value the last download's workgroups left in their words
 };
 

@@ -93,15 +93,10 @@ int Validate(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs,
   return RUYAMD_OK;
 }
 
-bool IsDevicePointer(const void* p) {
-  hipPointerAttribute_t attr;
-  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
-    (void)hipGetLastError();  // unregistered host memory
-    return false;
-  }
-  return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged ||
-         attr.type == hipMemoryTypeArray;
-}
+bool IsDevicePointer(const void* p) { return MemoryOf(p) == Memory::kDevice; }
+
+// Null pointers need nothing done to them either.
+Memory MemoryOfOptional(const void* p) { return p ? MemoryOf(p) : Memory::kDevice; }
 
 int64_t StorageElements(const ruyamd_mat& m) {
   const int64_t inner = m.order == RUYAMD_ORDER_COL_MAJOR ? m.rows : m.cols;
@@ -110,12 +105,11 @@ int64_t StorageElements(const ruyamd_mat& m) {
   return (outer - 1) * m.stride + inner;
 }
 
-// Makes `bytes` of host memory readable on the device (`on_device`: it already is).
-const void* StageIn(ruyamd_ctx* ctx, const void* p, bool on_device, std::size_t bytes, bool* staged_any,
-                    bool* ok) {
-  if (!p || bytes == 0 || on_device) return p;
+// Makes `bytes` of memory readable on the device.
+const void* StageIn(ruyamd_ctx* ctx, const void* p, Memory where, std::size_t bytes, bool* staged_any, bool* ok) {
+  if (!p || bytes == 0 || where == Memory::kDevice) return p;
   void* d = ctx->ws->Alloc(bytes);
-  if (!d || !ctx->staging.ToDevice(d, p, bytes, ctx->stream)) {
+  if (!d || !ctx->staging.ToDevice(d, p, bytes, where, ctx->stream)) {
     *ok = false;
     return nullptr;
   }
@@ -271,13 +265,16 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
   CaptureScope capture_scope(ctx);
 
   // Every buffer of the call is classified once.
-  const bool lhs_dev = !lhs->data || IsDevicePointer(lhs->data);
-  const bool rhs_dev = !rhs->data || IsDevicePointer(rhs->data);
-  const bool dst_on_device = IsDevicePointer(dst->data);
-  const bool bias_dev = !p->bias || IsDevicePointer(p->bias);
-  const bool mf_dev = !p->multiplier_fixedpoint_perchannel || IsDevicePointer(p->multiplier_fixedpoint_perchannel);
-  const bool me_dev = !p->multiplier_exponent_perchannel || IsDevicePointer(p->multiplier_exponent_perchannel);
-  if ((ctx->capturing || no_alloc) && !(lhs_dev && rhs_dev && dst_on_device && bias_dev && mf_dev && me_dev))
+  const Memory lhs_mem = MemoryOfOptional(lhs->data);
+  const Memory rhs_mem = MemoryOfOptional(rhs->data);
+  const Memory dst_mem = MemoryOf(dst->data);
+  const Memory bias_mem = MemoryOfOptional(p->bias);
+  const Memory mf_mem = MemoryOfOptional(p->multiplier_fixedpoint_perchannel);
+  const Memory me_mem = MemoryOfOptional(p->multiplier_exponent_perchannel);
+  const bool dst_on_device = dst_mem == Memory::kDevice;
+  bool all_on_device = true;
+  for (Memory m : {lhs_mem, rhs_mem, dst_mem, bias_mem, mf_mem, me_mem}) all_on_device = all_on_device && m == Memory::kDevice;
+  if ((ctx->capturing || no_alloc) && !all_on_device)
     return Fail(ctx, RUYAMD_E_UNSUPPORTED,
                 no_alloc ? "ruyamd_mul_no_alloc: every buffer must be device memory (staging host memory allocates)"
                          : "the stream is capturing: every buffer must be device memory");
@@ -293,9 +290,9 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
   const int channels = p->channel_dimension == RUYAMD_CHANNEL_ROW ? dst->rows : dst->cols;
   // The two source matrices are staged lazily by the dispatcher (a cache hit
   // needs no copy); the small per-channel vectors are staged now.
-  const void* bias_d = StageIn(ctx, p->bias, bias_dev, std::size_t(channels) * DtypeSize(p->accum_dtype), &staged, &ok);
-  const void* mf_d = StageIn(ctx, p->multiplier_fixedpoint_perchannel, mf_dev, std::size_t(channels) * 4, &staged, &ok);
-  const void* me_d = StageIn(ctx, p->multiplier_exponent_perchannel, me_dev, std::size_t(channels) * 4, &staged, &ok);
+  const void* bias_d = StageIn(ctx, p->bias, bias_mem, std::size_t(channels) * DtypeSize(p->accum_dtype), &staged, &ok);
+  const void* mf_d = StageIn(ctx, p->multiplier_fixedpoint_perchannel, mf_mem, std::size_t(channels) * 4, &staged, &ok);
+  const void* me_d = StageIn(ctx, p->multiplier_exponent_perchannel, me_mem, std::size_t(channels) * 4, &staged, &ok);
   if (!ok) return Fail(ctx, RUYAMD_E_HIP, "staging host operands to the device failed");
 
   // Destination: device memory is written in place; host memory gets a device
@@ -310,8 +307,10 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
 
   MulCall call;
   FillCall(*lhs, *rhs, *p, *dst, bias_d, mf_d, me_d, dst_d, &call);
-  if (!lhs_dev) call.lhs_host_bytes = StorageElements(*lhs) * DtypeSize(lhs->dtype);
-  if (!rhs_dev) call.rhs_host_bytes = StorageElements(*rhs) * DtypeSize(rhs->dtype);
+  call.lhs_memory = lhs_mem;
+  call.rhs_memory = rhs_mem;
+  if (lhs_mem != Memory::kDevice) call.lhs_host_bytes = StorageElements(*lhs) * DtypeSize(lhs->dtype);
+  if (rhs_mem != Memory::kDevice) call.rhs_host_bytes = StorageElements(*rhs) * DtypeSize(rhs->dtype);
 
   std::string err;
   ctx->upload_failed = false;
@@ -341,7 +340,7 @@ int MulImpl(ruyamd_ctx* ctx, const ruyamd_mat* lhs, const ruyamd_mat* rhs, const
     const std::size_t inner = dst->order == RUYAMD_ORDER_COL_MAJOR ? dst->rows : dst->cols;
     const std::size_t outer = dst->order == RUYAMD_ORDER_COL_MAJOR ? dst->cols : dst->rows;
     const std::size_t pitch = std::size_t(dst->stride) * dst_elt;
-    if (!ctx->staging.ToHost2D(dst->data, dst_d, pitch, inner * dst_elt, outer, ctx->stream, &drained))
+    if (!ctx->staging.ToHost2D(dst->data, dst_d, pitch, inner * dst_elt, outer, dst_mem, ctx->stream, &drained))
       return Fail(ctx, RUYAMD_E_HIP, std::string("copying the destination back to the host failed: ") +
                                          hipGetErrorString(hipGetLastError()));
     staged = true;
@@ -477,17 +476,18 @@ extern "C" int ruyamd_apply_multiplier(ruyamd_ctx* ctx, const int32_t* x, const 
   ctx->staging.DropPending();
   bool staged = false, ok = true;
   const std::size_t bytes = std::size_t(n) * 4;
-  const int32_t* xd = static_cast<const int32_t*>(StageIn(ctx, x, IsDevicePointer(x), bytes, &staged, &ok));
-  const int32_t* md = static_cast<const int32_t*>(StageIn(ctx, m, IsDevicePointer(m), bytes, &staged, &ok));
-  const int32_t* ed = static_cast<const int32_t*>(StageIn(ctx, e, IsDevicePointer(e), bytes, &staged, &ok));
+  const int32_t* xd = static_cast<const int32_t*>(StageIn(ctx, x, MemoryOf(x), bytes, &staged, &ok));
+  const int32_t* md = static_cast<const int32_t*>(StageIn(ctx, m, MemoryOf(m), bytes, &staged, &ok));
+  const int32_t* ed = static_cast<const int32_t*>(StageIn(ctx, e, MemoryOf(e), bytes, &staged, &ok));
   if (!ok) return Fail(ctx, RUYAMD_E_HIP, "staging failed");
-  const bool out_dev = IsDevicePointer(out);
+  const Memory out_mem = MemoryOf(out);
+  const bool out_dev = out_mem == Memory::kDevice;
   int32_t* od = out_dev ? out : static_cast<int32_t*>(ctx->workspace.Alloc(bytes));
   if (!od) return Fail(ctx, RUYAMD_E_HIP, "device allocation failed");
   if (LaunchApplyMultiplier(ctx->LaunchStream(), xd, md, ed, od, n) != hipSuccess)
     return Fail(ctx, RUYAMD_E_HIP, "launch failed");
   bool drained = false;
-  if (!out_dev && !ctx->staging.ToHost2D(out, od, bytes, bytes, 1, ctx->stream, &drained))
+  if (!out_dev && !ctx->staging.ToHost2D(out, od, bytes, bytes, 1, out_mem, ctx->stream, &drained))
     return Fail(ctx, RUYAMD_E_HIP, "copy back failed");
   if (ctx->upload_failed) return Fail(ctx, RUYAMD_E_HIP, "staging failed");
   if (!drained && hipStreamSynchronize(ctx->stream) != hipSuccess)

@@ -932,7 +932,7 @@ int EnsureOnDevice(ruyamd_ctx* ctx, MulCall* call, int side, std::string* err) {
   std::size_t& bytes = side == 0 ? call->lhs_host_bytes : call->rhs_host_bytes;
   if (bytes == 0) return RUYAMD_OK;
   void* d = ctx->ws->Alloc(bytes);
-  if (!d || !ctx->staging.ToDevice(d, m.data, bytes, ctx->stream)) {
+  if (!d || !ctx->staging.ToDevice(d, m.data, bytes, side == 0 ? call->lhs_memory : call->rhs_memory, ctx->stream)) {
     *err = "staging a host operand to the device failed";
     return RUYAMD_E_HIP;
   }

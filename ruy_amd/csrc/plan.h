@@ -25,6 +25,7 @@ struct MulCall {
   // pointer; EnsureOnDevice replaces it with a device copy.
   std::size_t lhs_host_bytes = 0;
   std::size_t rhs_host_bytes = 0;
+  Memory lhs_memory = Memory::kDevice, rhs_memory = Memory::kDevice;  // what kind of memory that is
   bool staged_any = false;
 };
 

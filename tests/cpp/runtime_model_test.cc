@@ -7,8 +7,9 @@
 // launch fails, and what it asks for while its stream records a graph, none of
 // which a GPU is needed (or, for the failures, wanted) for.
 //
-//   runtime_model_test failed_upload
+//   runtime_model_test failed_upload | page_locked_sources
 #include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <cstdint>
@@ -362,11 +363,69 @@ void FailedUpload() {
   }
 }
 
+// Page-locked memory whose last bytes are those in front of a page that cannot
+// be touched: `bytes` bytes that start `from_end` bytes before it.
+struct PageLocked {
+  char* base;
+  char* data;
+  std::size_t room;
+  PageLocked(std::size_t bytes, std::size_t from_end) {
+    room = (std::max(bytes, from_end) + 4095) / 4096 * 4096;
+    base = static_cast<char*>(mmap(nullptr, room + 4096, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0));
+    if (base == MAP_FAILED || mprotect(base + room, 4096, PROT_NONE) != 0) std::abort();
+    data = base + room - from_end;
+    R().pinned[base] = room;
+  }
+  ~PageLocked() {
+    R().pinned.erase(base);
+    munmap(base, room + 4096);
+  }
+};
+
+// A page-locked operand is read in stream order: what work enqueued in front of
+// the call writes to it is what the call multiplies by. At any address and
+// size, and nothing outside the 16 aligned bytes that hold a byte of it.
+void PageLockedSources() {
+  const int M = 70, N = 40;
+  for (int K : {33, 48, 128, 20000}) {       // (the last: 1.4 MB and 0.8 MB, either side of the kernel copies' limit)
+    for (int misalign : {0, 1, 4}) {
+      Context c;
+      const std::size_t sizes[4] = {std::size_t(M) * K, std::size_t(K) * N, std::size_t(M) * 4, std::size_t(M) * 4};
+      std::vector<PageLocked*> operands;
+      for (std::size_t size : sizes) {
+        // As close to the end as the alignment allows.
+        operands.push_back(new PageLocked(size, size + (16 - (size + misalign) % 16) % 16));
+      }
+      for (int i = 0; i < 4; ++i) std::memset(operands[i]->data, 0x11, sizes[i]);
+      std::vector<char> mf(M * 4, 0x22), dst(M * N);  // (a pageable one among them)
+      const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, operands[0]->data, M, K, RUYAMD_ORDER_ROW_MAJOR);
+      const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, operands[1]->data, K, N, RUYAMD_ORDER_COL_MAJOR, 3);
+      const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, dst.data(), M, N, RUYAMD_ORDER_COL_MAJOR);
+      ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+      p.bias = operands[2]->data;
+      p.multiplier_fixedpoint_perchannel = reinterpret_cast<const int32_t*>(mf.data());
+      p.multiplier_exponent_perchannel = reinterpret_cast<const int32_t*>(operands[3]->data);
+      R().queue.push_back([&] {  // work on the call's stream, in front of it
+        for (int i = 0; i < 4; ++i) std::memset(operands[i]->data, 0x40 + i, sizes[i]);
+      });
+      EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+      for (int i = 0; i < 4; ++i) {
+        const std::vector<char> want(sizes[i], static_cast<char>(0x40 + i));
+        EXPECT(std::count(R().uploads.begin(), R().uploads.end(), want) == 1, "depth %d, %d bytes off: operand %d", K,
+               misalign, i);
+      }
+      EXPECT(std::count(R().uploads.begin(), R().uploads.end(), mf) == 1, "pageable operand");
+      for (PageLocked* o : operands) delete o;
+    }
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "failed_upload") FailedUpload();
+  else if (which == "page_locked_sources") PageLockedSources();
   else return 2;
   if (g_failures) {
     std::printf("%d failures\n", g_failures);

@@ -269,6 +269,46 @@ def test_host_pointer_transfers_by_kernels_and_by_the_copy_engine(device_ctx, sh
             compare(p, D.host_pointer_mul(device_ctx, p, dst_fill=0x5A), want)
 
 
+@pytest.mark.parametrize("depth", [45, 1024, 9000])
+@pytest.mark.parametrize("offset", [0, 1, 16])
+def test_page_locked_operands_are_read_in_stream_order(depth, offset):
+    """A page-locked buffer that work on the context's stream fills right before
+    the call: the product is of what that work wrote, whether the operand goes up
+    by kernel (16-byte aligned, up to 1 MiB) or by the copy engine."""
+    import ctypes as C
+    import torch
+    from ruy_amd import api
+    rng = np.random.default_rng(depth)
+    p = W.random_problem(rng, S.I8, S.I8, S.I32, S.I8, 200, depth, 130, *cases.RCC, name="page-locked")
+    ctx = api.Context()
+    try:
+        stream = torch.cuda.Stream()
+        ctx.set_stream(stream.cuda_stream)
+        busy = torch.rand(4096, 4096, device="cuda")
+
+        def filled_late(array):
+            fresh = torch.from_numpy(array).cuda()
+            host = torch.zeros(array.size + offset, dtype=fresh.dtype).pin_memory()[offset:]
+            return fresh, host
+
+        buffers = [filled_late(a) for a in (p.lhs.storage, p.rhs.storage, p.bias) if a is not None]
+        out = torch.full((p.dst.n_storage + offset,), 0x5A, dtype=torch.int8).pin_memory()[offset:]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            for _ in range(20):  # some milliseconds
+                busy = busy @ busy
+            for fresh, host in buffers:
+                host.copy_(fresh, non_blocking=True)
+        addresses = [host.data_ptr() for _, host in buffers]
+        l, r, d = p.lhs.struct(addresses[0]), p.rhs.struct(addresses[1]), p.dst.struct(out.data_ptr())
+        ps = p.params_struct(addresses[2]) if p.bias is not None else p.params_struct()
+        ctx._check(api.lib.ruyamd_mul(ctx._h, C.byref(l), C.byref(r), C.byref(ps), C.byref(d)))
+        compare(p, out.numpy(), expected(p))
+    finally:
+        torch.cuda.synchronize()
+        ctx.close()
+
+
 def test_empty_and_degenerate_shapes(device_ctx):
     from ruy_amd import device_problem as D
     rng = np.random.default_rng(6)

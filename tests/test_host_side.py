@@ -149,6 +149,11 @@ def test_a_failed_upload_leaves_no_cache_entry(runtime_model):
     runtime_model("failed_upload")
 
 
+def test_page_locked_sources_are_read_in_stream_order(runtime_model):
+    """... at any alignment and size, and without a byte beyond their page."""
+    runtime_model("page_locked_sources")
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
