@@ -505,10 +505,17 @@ hipError_t LaunchMmaFlip(hipStream_t stream, const GemvI8Args& args) {
 // depth of each (of four steps and more a wave, or their ring never fills):
 // fp32 512 x 16384 x 7 30.9 -> 23.0, 2048 x 8192 x 4 17.9 -> 14.0, int8 512 x
 // 16384 x 7 9.1 -> 6.9.
-// Four waves to a group up to four groups to a CU (one wave: fp32 8192 x 4096 x
-// 4 36.4, two: 25.1, four: 22.6), one beyond (int8 16384 x 512 x 4 4.7, four:
-// 6.5). With 16 narrow vectors a CU holds ten waves, and two to a group do
-// better from two groups to a CU on (int8 9000 x 4096 x 10 9.3, four: 11.0).
+// Four waves to a group while all groups run at once, which three to a CU do
+// with up to 8 narrow vectors (768 groups; fp32 8192 x 4096 x 4 22.6, two waves:
+// 25.1, one: 36.4; 12288 x 1024 x 2 9.9, one: 10.6). From there to four groups to a CU
+// one wave, unless the vectors are beyond 8 KiB, where it has too little in
+// flight: int8 12416 x 512 x 8 5.3 with four waves, 3.9 with one, 16368 x 4096 x
+// 8 13.6 and 12.2, 12416 x 8192 x 2 22.8 and 20.1, fp32 16368 x 128 x 8 4.7 and
+// 3.3, 16368 x 2048 x 2 28.0 and 23.6; but fp32 12416 x 3072 x 2 29.2 and 31.6,
+// 12416 x 4096 x 2 38.6 and 40.5. (int8 16368 x 3072 x 2 10.8 with one, 10.3
+// with two.) One wave beyond four groups to a CU (int8 16384 x 512 x 4 4.7,
+// four: 6.5). With 16 narrow vectors a CU holds ten waves, and two to a group
+// do better from two groups to a CU on (int8 9000 x 4096 x 10 9.3, four: 11.0).
 struct MmaShape {
   int step, split;
 };
@@ -518,6 +525,7 @@ MmaShape MmaShapeFor(const GemvI8Args& args) {
   if (groups <= 128 && steps >= 32) return {256, 8};
   if (args.K >= 32768) return {512, groups >= 1024 ? 1 : groups >= 512 ? 2 : 4};
   if (groups >= 1024 || steps < 2) return {256, 1};
+  if (groups > 768 && args.narrow_count <= 8 && args.K <= 8192) return {256, 1};
   return {256, groups >= 512 && args.narrow_count > 8 ? 2 : 4};
 }
 

@@ -4,10 +4,11 @@
 // is performed only when something waits for it. Kernels are not executed, but
 // for the two that copy between host and device; every launch is logged by
 // name. That shows in which order a call enqueues its work, what it does when a
-// launch fails, and what it asks for while its stream records a graph, none of
-// which a GPU is needed (or, for the failures, wanted) for.
+// launch fails, what it asks for while its stream records a graph and which
+// kernel it runs on, none of which a GPU is needed (or, for the failures,
+// wanted) for.
 //
-//   runtime_model_test failed_upload | page_locked_sources
+//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -420,12 +421,60 @@ void PageLockedSources() {
   }
 }
 
+// A product of device operands that no kernel here ever reads.
+struct DeviceCall {
+  void* lhs;
+  void* rhs;
+  void* dst;
+  DeviceCall(std::size_t lhs_bytes, std::size_t rhs_bytes, std::size_t dst_bytes) {
+    (void)hipMalloc(&lhs, lhs_bytes);
+    (void)hipMalloc(&rhs, rhs_bytes);
+    (void)hipMalloc(&dst, dst_bytes);
+  }
+  ~DeviceCall() {
+    (void)hipFree(lhs);
+    (void)hipFree(rhs);
+    (void)hipFree(dst);
+  }
+};
+
+// The streaming kernel's waves to a group of 16 rows: four only where all
+// groups run at once (three workgroups to a CU), or one would have too little
+// in flight.
+void SkinnyShapes() {
+  struct {
+    int rows, depth_bytes, narrow;
+    const char* shape;  // stages, bytes of one, waves, narrow vectors staged
+  } const cases[] = {
+      {768 * 16, 1024, 8, "Li2ELi256ELi4ELi8E"},     {768 * 16 + 1, 1024, 8, "Li2ELi256ELi1ELi8E"},
+      {900 * 16, 512, 2, "Li2ELi256ELi1ELi8E"},      {1023 * 16, 4096, 4, "Li2ELi256ELi1ELi8E"},
+      {1023 * 16, 8192, 8, "Li2ELi256ELi1ELi8E"},    {1023 * 16, 8208, 8, "Li2ELi256ELi4ELi8E"},
+      {1023 * 16 + 1, 8208, 8, "Li2ELi256ELi1ELi8E"}, {900 * 16, 1024, 9, "Li2ELi256ELi2ELi16E"},
+  };
+  for (const auto& c : cases) {
+    for (const Types& t : {kTypes[0], kTypes[1]}) {
+      Context ctx;
+      const int depth = c.depth_bytes / SizeOf(t.lhs);
+      DeviceCall call(std::size_t(c.rows) * c.depth_bytes, std::size_t(c.narrow) * c.depth_bytes,
+                      std::size_t(c.rows) * c.narrow * SizeOf(t.dst));
+      const ruyamd_mat l = Mat(t.lhs, call.lhs, c.rows, depth, RUYAMD_ORDER_ROW_MAJOR);
+      const ruyamd_mat r = Mat(t.rhs, call.rhs, depth, c.narrow, RUYAMD_ORDER_COL_MAJOR);
+      const ruyamd_mat d = Mat(t.dst, call.dst, c.rows, c.narrow, RUYAMD_ORDER_COL_MAJOR);
+      const ruyamd_mul_params p = Params(t.dst);
+      EXPECT(ruyamd_mul(ctx.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(ctx.ctx));
+      EXPECT(R().log.size() == 1 && Count("GemvMmaKernel") == 1 && Count(c.shape) == 1, "%s %d x %d bytes x %d: %s", t.name,
+             c.rows, c.depth_bytes, c.narrow, R().log.empty() ? "nothing" : R().log.back().c_str());
+    }
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "failed_upload") FailedUpload();
   else if (which == "page_locked_sources") PageLockedSources();
+  else if (which == "skinny_shapes") SkinnyShapes();
   else return 2;
   if (g_failures) {
     std::printf("%d failures\n", g_failures);

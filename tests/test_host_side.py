@@ -154,6 +154,10 @@ def test_page_locked_sources_are_read_in_stream_order(runtime_model):
     runtime_model("page_locked_sources")
 
 
+def test_waves_to_a_group_of_the_streaming_kernel(runtime_model):
+    runtime_model("skinny_shapes")
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
