@@ -312,7 +312,7 @@ bool ruyamd_ctx::TimingBegin() {
   } else {
     if (hipEventCreate(&ev.first) != hipSuccess || hipEventCreate(&ev.second) != hipSuccess) return false;
   }
-  (void)hipEventRecord(ev.first, stream);
+  (void)hipEventRecord(ev.first, LaunchStream());  // (behind the uploads, which are not the kernel's)
   timing_pending.push_back(ev);
   return true;
 }

@@ -8,7 +8,7 @@
 // kernel it runs on, none of which a GPU is needed (or, for the failures,
 // wanted) for.
 //
-//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes
+//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -421,6 +421,29 @@ void PageLockedSources() {
   }
 }
 
+// Kernel timing of a call on host memory brackets the product, not the upload.
+void Timing() {
+  const int M = 96, K = 160;
+  for (const Types& t : kTypes) {
+    if (t.dst == RUYAMD_DTYPE_F64) continue;  // (the generic kernel is not timed)
+    for (int N : {64, 4}) {
+      Context c;
+      (void)ruyamd_ctx_set_kernel_timing(c.ctx, 1);
+      std::vector<char> lhs(M * K * 8, 1), rhs(K * N * 8, 2), dst(M * N * 8), bias(M * 4, 3);
+      const ruyamd_mat l = Mat(t.lhs, lhs.data(), M, K, RUYAMD_ORDER_ROW_MAJOR);
+      const ruyamd_mat r = Mat(t.rhs, rhs.data(), K, N, RUYAMD_ORDER_COL_MAJOR);
+      const ruyamd_mat d = Mat(t.dst, dst.data(), M, N, RUYAMD_ORDER_COL_MAJOR);
+      ruyamd_mul_params p = Params(t.dst);
+      p.bias = bias.data();
+      EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+      const auto begin = std::find(R().log.begin(), R().log.end(), "event");
+      const auto end = std::find(begin == R().log.end() ? begin : begin + 1, R().log.end(), "event");
+      EXPECT(end - begin == 2, "%s x %d: %d launches inside the bracket", t.name, N, static_cast<int>(end - begin) - 1);
+      EXPECT(Count("UploadKernel") == 1, "%s", t.name);
+    }
+  }
+}
+
 // A product of device operands that no kernel here ever reads.
 struct DeviceCall {
   void* lhs;
@@ -475,6 +498,7 @@ int main(int argc, char** argv) {
   if (which == "failed_upload") FailedUpload();
   else if (which == "page_locked_sources") PageLockedSources();
   else if (which == "skinny_shapes") SkinnyShapes();
+  else if (which == "timing") Timing();
   else return 2;
   if (g_failures) {
     std::printf("%d failures\n", g_failures);

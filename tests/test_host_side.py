@@ -158,6 +158,10 @@ def test_waves_to_a_group_of_the_streaming_kernel(runtime_model):
     runtime_model("skinny_shapes")
 
 
+def test_kernel_timing_leaves_the_upload_out(runtime_model):
+    runtime_model("timing")
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
