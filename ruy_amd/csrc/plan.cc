@@ -50,6 +50,7 @@ struct Operand8 {
   // An operand used in place whose sums are needed but have not been computed:
   // the dispatcher either lets the kernel form them or calls MaterializeSums.
   bool sums_pending = false;
+  int32_t* sums_room = nullptr;  // for MaterializeSums (ReserveSums)
   int32_t count = 0;
   // kFlipU8 if `data` is the caller's uint8 storage used in place.
   uint32_t flip = 0;
@@ -59,9 +60,28 @@ struct Operand8 {
   PackSource src;
 };
 
+// Room for the sums of an operand that nobody has formed yet, taken before
+// anything of the call is launched. A call that is being recorded, or may not
+// allocate, forms them in a launch of their own where an ordinary one leaves
+// them to the product; the ordinary call takes the room all the same (if it can
+// be had: it does not depend on it), so that a recorded one finds it there.
+int ReserveSums(ruyamd_ctx* ctx, Operand8* op, bool formed_by_product, std::string* err) {
+  if (!op->sums_pending) return RUYAMD_OK;
+  const std::size_t bytes = std::size_t(op->count) * 4;
+  if (!ctx->capturing && !ctx->no_alloc) {
+    op->sums_room = static_cast<int32_t*>(ctx->ws->AllocOptional(bytes));
+    return RUYAMD_OK;
+  }
+  if (formed_by_product) return RUYAMD_OK;
+  op->sums_room = static_cast<int32_t*>(ctx->ws->Alloc(bytes));
+  if (op->sums_room) return RUYAMD_OK;
+  *err = "workspace allocation failed";
+  return RUYAMD_E_HIP;
+}
+
 int MaterializeSums(ruyamd_ctx* ctx, Operand8* op, int32_t K, std::string* err) {
   if (!op->sums_pending) return RUYAMD_OK;
-  int32_t* sums = static_cast<int32_t*>(ctx->ws->Alloc(std::size_t(op->count) * 4));
+  int32_t* sums = op->sums_room ? op->sums_room : static_cast<int32_t*>(ctx->ws->Alloc(std::size_t(op->count) * 4));
   if (!sums) {
     *err = "workspace allocation failed";
     return RUYAMD_E_HIP;
@@ -415,10 +435,10 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   PendingPack pack_a, pack_b;
   if (int rc = PackOperand8(ctx, &a, &pack_a, err)) return rc;
   if (int rc = PackOperand8(ctx, &b, &pack_b, err)) return rc;
-  if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   const int32_t zp_product_depth =
       static_cast<int32_t>(static_cast<uint32_t>(lzp) * static_cast<uint32_t>(rzp) * static_cast<uint32_t>(K));
   if (skinny) {
+    if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
     // Bandwidth-bound shapes: stream the wide side exactly once. Sums that are
     // still pending (operands used in place) are formed by the kernel itself.
     GemvI8Args g;
@@ -465,6 +485,9 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   }
   GemmArgs args;
   const bool swap = SetupInt8Gemm(ctx, *call, a, b, lzp, rzp, /*staged=*/false, &args);
+  if (int rc = ReserveSums(ctx, &a, args.fuse_sums != 0, err)) return rc;
+  if (int rc = ReserveSums(ctx, &b, args.fuse_sums != 0, err)) return rc;
+  if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   // The largest tile can form the sums of the rows of its `a` operand in
   // passing (kernels/fused_sums.h): one launch instead of a sums kernel and
   // the product. Not for a call that is being recorded (a replayed launch

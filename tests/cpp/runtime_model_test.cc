@@ -8,7 +8,7 @@
 // kernel it runs on, none of which a GPU is needed (or, for the failures,
 // wanted) for.
 //
-//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing
+//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing | capture
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -491,6 +491,55 @@ void SkinnyShapes() {
   }
 }
 
+// A call can be recorded once it has run: what it then needs of scratch memory
+// is there, although a recorded call forms some sums in a launch of their own.
+// One that is refused, on a context that has run nothing, records nothing.
+void Capture() {
+  struct {
+    int M, K, N, lhs_order, rhs_order, lhs_zero, rhs_zero;
+  } const cases[] = {
+      {2048, 2048, 2048, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_COL_MAJOR, 0, 3},   // packed, its sums with the product
+      {2048, 2048, 2048, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 3, 3},
+      {2048, 2048, 2048, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, -5, 3},
+      {2048, 2048, 2048, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 3, 3},   // in place
+      {3000, 4096, 2500, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 0, 3},
+      {4096, 1024, 4096, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 0, 3},
+      {1000, 1500, 700, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_COL_MAJOR, 4, -3},
+      {1000, 4099, 700, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 4, -3},
+      {1100, 1100, 1100, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 4, -3},
+      {1104, 1104, 1104, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 4, -3},
+      {300, 16384, 260, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 4, -3},   // a depth in parts
+      {64, 8192, 100, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 4, -3},
+      {4096, 5000, 7, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 4, -3},     // skinny
+      {77, 131, 45, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 4, -3},
+  };
+  for (const auto& k : cases) {
+    for (const Types& t : kTypes) {
+      if (t.dst == RUYAMD_DTYPE_F64) continue;
+      const bool zero_points = t.rhs == RUYAMD_DTYPE_I8;
+      DeviceCall call(std::size_t(k.M) * k.K * SizeOf(t.lhs), std::size_t(k.K) * k.N * SizeOf(t.rhs),
+                      std::size_t(k.M) * k.N * SizeOf(t.dst));
+      const ruyamd_mat l = Mat(t.lhs, call.lhs, k.M, k.K, k.lhs_order, zero_points ? k.lhs_zero : 0);
+      const ruyamd_mat r = Mat(t.rhs, call.rhs, k.K, k.N, k.rhs_order, zero_points ? k.rhs_zero : 0);
+      const ruyamd_mat d = Mat(t.dst, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
+      const ruyamd_mul_params p = Params(t.dst);
+      for (int warm = 0; warm <= 1; ++warm) {
+        Context c;
+        if (warm) EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+        R().log.clear();
+        R().capturing = true;
+        const int rc = ruyamd_mul(c.ctx, &l, &r, &p, &d);
+        R().capturing = false;
+        EXPECT(R().capture_violations == 0, "%s %d x %d x %d", t.name, k.M, k.K, k.N);
+        EXPECT(rc == RUYAMD_OK || !warm, "%s %d x %d x %d (orders %d %d): %s", t.name, k.M, k.K, k.N, k.lhs_order,
+               k.rhs_order, ruyamd_ctx_last_error(c.ctx));
+        EXPECT(rc == RUYAMD_OK || R().log.empty(), "%s %d x %d x %d: refused%s with %d launches recorded", t.name, k.M, k.K,
+               k.N, warm ? "" : " cold", static_cast<int>(R().log.size()));
+      }
+    }
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -499,6 +548,7 @@ int main(int argc, char** argv) {
   else if (which == "page_locked_sources") PageLockedSources();
   else if (which == "skinny_shapes") SkinnyShapes();
   else if (which == "timing") Timing();
+  else if (which == "capture") Capture();
   else return 2;
   if (g_failures) {
     std::printf("%d failures\n", g_failures);

@@ -138,6 +138,52 @@ def test_captured_calls_replay_correctly():
         ctx.close()
 
 
+@pytest.mark.parametrize("size,lhs_order,rhs_order", [(1100, S.ORDER_COL_MAJOR, S.ORDER_ROW_MAJOR),   # both packed
+                                                      (1104, S.ORDER_ROW_MAJOR, S.ORDER_COL_MAJOR)])  # in place
+def test_large_operands_with_sums_are_recorded_after_one_call(size, lhs_order, rhs_order):
+    """A recorded call forms the sums in a launch of their own where the call
+    before it left them to the product: there has to be room for them."""
+    import torch
+    from ruy_amd import device_problem as D
+    from ruy_amd import api
+    from test_gpu_parity import expected
+
+    rng = np.random.default_rng(size)
+    p = W.random_problem(rng, S.I8, S.I8, S.I32, S.I8, size, size, size, lhs_order, rhs_order, S.ORDER_COL_MAJOR,
+                         name="recorded %d" % size)
+    p.lhs.zero_point, p.rhs.zero_point = 4, -3
+    ctx = api.Context()
+    try:
+        stream = torch.cuda.Stream()
+        ctx.set_stream(stream.cuda_stream)
+        ctx.set_synchronous(False)
+        dp = D.DeviceProblem(p, dst_fill=0)
+        with torch.cuda.stream(stream):
+            dp.run(ctx)
+        torch.cuda.synchronize()
+        _check(p, dp.dst_t.cpu().numpy(), expected(p, fill=0))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            dp.run(ctx)
+        for _ in range(3):
+            _refill_rhs(p, dp, rng)
+            dp.dst_all.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+            torch.cuda.synchronize()
+            want = expected(p, fill=0)
+            _check(p, dp.dst_t.cpu().numpy(), want)
+            with torch.cuda.stream(stream):  # ... and an eager call between the replays
+                dp.dst_all.zero_()
+                dp.run(ctx)
+            torch.cuda.synchronize()
+            _check(p, dp.dst_t.cpu().numpy(), want)
+        del graph
+    finally:
+        ctx.close()
+
+
 def test_captured_cache_entries_survive_ejection():
     """A cache entry that a recorded call reads stays put when newer entries
     overflow the budget; the replay after that still gives the right answer."""

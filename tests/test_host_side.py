@@ -162,6 +162,11 @@ def test_kernel_timing_leaves_the_upload_out(runtime_model):
     runtime_model("timing")
 
 
+def test_one_ordinary_call_is_enough_for_a_capture(runtime_model):
+    """... whatever forms the sums then, and a refused call records nothing."""
+    runtime_model("capture")
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
