@@ -742,7 +742,6 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     return rc;
   PendingPack pack_a;
   if (int rc = PackOperand8(ctx, &a, &pack_a, err)) return rc;
-  if (int rc = LaunchPendingPacks(ctx, pack_a, PendingPack(), err)) return rc;
   const DevMat& m16 = side16 == 0 ? call->lhs : call->rhs;  // shape only: its data may still be host memory
   const PackSource src = side16 == 0 ? PackSource{m16.data, m16.rs, m16.cs, m16.rows, m16.cols, m16.dtype}
                                      : PackSource{m16.data, m16.cs, m16.rs, m16.cols, m16.rows, m16.dtype};
@@ -807,26 +806,23 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   args.ep.lhs_zero_point = 0;
   args.ep.rhs_zero_point = -128;  // the low plane stores (v & 0xff) - 128
   args.ep.zp_product_depth = 0;
-  bool fuse_decided = false;
-  auto decide_sums = [&]() -> int {
-    if (fuse_decided) return RUYAMD_OK;
-    fuse_decided = true;
-    if (a.sums_pending && GemmI8I16CanFuseSums(args, ctx->multiprocessor_count)) {
-      // Small problem, int8 side used in place: the kernel forms its row sums.
-      args.fuse_sums = 1;
-      args.fused_a_factor = args.ep.rhs_zero_point;
-      args.ep.rhs_zero_point = 0;
-    } else if (int rc = MaterializeSums(ctx, &a, K, err)) {
-      return rc;
-    }
-    args.ep.lhs_sums = a.sums;
-    return RUYAMD_OK;
-  };
-  if (!planes) {
+  // Memory first, launches afterwards, so that a call refused for want of it
+  // has recorded nothing.
+  if (a.sums_pending && GemmI8I16CanFuseSums(args, ctx->multiprocessor_count)) {
+    // Small problem, sums of the int8 side not there yet: the kernel forms them.
+    args.fuse_sums = 1;
+    args.fused_a_factor = args.ep.rhs_zero_point;
+    args.ep.rhs_zero_point = 0;
+  }
+  if (int rc = ReserveSums(ctx, &a, args.fuse_sums != 0, err)) return rc;
+  bool raw = false;
+  PackSource fresh;
+  const bool planes_cached = planes != nullptr;
+  if (!planes_cached) {
     if (int rc = EnsureOnDevice(ctx, call, side16, err)) return rc;
     const DevMat& m = side16 == 0 ? call->lhs : call->rhs;
-    const PackSource fresh = side16 == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
-                                         : PackSource{m.data, m.cs, m.rs, m.cols, m.rows, m.dtype};
+    fresh = side16 == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
+                        : PackSource{m.data, m.cs, m.rs, m.cols, m.rows, m.dtype};
     // The int16 operand where it lies, split into planes inside the kernel: no
     // pack launch. Needs the layout of an in-place operand and a launch on the
     // smallest tile with at least two depth steps per part.
@@ -838,36 +834,42 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
       args.b = fresh.data;
       args.b_bytes = static_cast<uint32_t>(extent16);
       args.ldb = fresh.count == 1 ? RoundUp(K, 16) * 2 : static_cast<int32_t>(fresh.stride_c * 2);
-      if (int rc = decide_sums()) return rc;
       PlanDepthSplit(ctx, GemmKind::kInt8Int16, &args);
-      if (GemmI8I16CanUseRawInt16(args, ctx->multiprocessor_count)) {
-        const bool timed = ctx->TimingBegin();
-        const hipError_t launched = LaunchGemmI8I16Raw(ctx->LaunchStream(), args, ctx->multiprocessor_count);
-        if (timed) ctx->TimingEnd();
-        if (launched != hipSuccess) {
-          *err = "int8 x int16 matrix-core kernel launch failed";
-          return RUYAMD_E_HIP;
-        }
-        ctx->last_kernel = RUYAMD_KERNEL_I8I16_MFMA;
-        return RUYAMD_OK;
+      raw = GemmI8I16CanUseRawInt16(args, ctx->multiprocessor_count);
+      // (If not that launch after all, a depth split planned here stays valid:
+      // it depends on the shape only.)
+    }
+    if (!raw) {
+      planes = static_cast<int8_t*>(ctx->ws->Alloc(packed_bytes));
+      if (!planes) {
+        *err = "workspace allocation failed";
+        return RUYAMD_E_HIP;
       }
-      // Not that launch after all: the planes are packed as usual. (A depth
-      // split planned above stays valid: it depends on the shape only.)
     }
-    planes = static_cast<int8_t*>(ctx->ws->Alloc(packed_bytes));
-    if (!planes) {
-      *err = "workspace allocation failed";
+  }
+  if (int rc = LaunchPendingPacks(ctx, pack_a, PendingPack(), err)) return rc;
+  if (!args.fuse_sums) {
+    if (int rc = MaterializeSums(ctx, &a, K, err)) return rc;
+  }
+  args.ep.lhs_sums = a.sums;
+  if (raw) {
+    const bool timed = ctx->TimingBegin();
+    const hipError_t launched = LaunchGemmI8I16Raw(ctx->LaunchStream(), args, ctx->multiprocessor_count);
+    if (timed) ctx->TimingEnd();
+    if (launched != hipSuccess) {
+      *err = "int8 x int16 matrix-core kernel launch failed";
       return RUYAMD_E_HIP;
     }
-    if (LaunchPackI16Split(ctx->LaunchStream(), fresh, planes, ld) != hipSuccess) {
-      *err = "int16 pack kernel launch failed";
-      return RUYAMD_E_HIP;
-    }
+    ctx->last_kernel = RUYAMD_KERNEL_I8I16_MFMA;
+    return RUYAMD_OK;
+  }
+  if (!planes_cached && LaunchPackI16Split(ctx->LaunchStream(), fresh, planes, ld) != hipSuccess) {
+    *err = "int16 pack kernel launch failed";
+    return RUYAMD_E_HIP;
   }
   args.b = planes;
   args.b_bytes = static_cast<uint32_t>(packed_bytes);
   args.ldb = ld;
-  if (int rc = decide_sums()) return rc;
   if (args.split_k == 1) PlanDepthSplit(ctx, GemmKind::kInt8Int16, &args);
   const bool timed = ctx->TimingBegin();
   const hipError_t launched = LaunchGemmI8I16(ctx->LaunchStream(), args, ctx->multiprocessor_count);

@@ -493,7 +493,8 @@ void SkinnyShapes() {
 
 // A call can be recorded once it has run: what it then needs of scratch memory
 // is there, although a recorded call forms some sums in a launch of their own.
-// One that is refused, on a context that has run nothing, records nothing.
+// One that is refused, on a context that has run nothing or a smaller call,
+// records nothing.
 void Capture() {
   struct {
     int M, K, N, lhs_order, rhs_order, lhs_zero, rhs_zero;
@@ -523,18 +524,25 @@ void Capture() {
       const ruyamd_mat r = Mat(t.rhs, call.rhs, k.K, k.N, k.rhs_order, zero_points ? k.rhs_zero : 0);
       const ruyamd_mat d = Mat(t.dst, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
       const ruyamd_mul_params p = Params(t.dst);
-      for (int warm = 0; warm <= 1; ++warm) {
+      for (const std::string before : {"nothing", "a smaller call", "the same call"}) {
         Context c;
-        if (warm) EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+        ruyamd_mat sl = l, sr = r, sd = d;
+        if (before == "a smaller call") {
+          sl.rows = sd.rows = std::min(k.M, 40);
+          sr.cols = sd.cols = std::min(k.N, 40);
+          sl.cols = sr.rows = std::min(k.K, 77);
+        }
+        if (before != "nothing")
+          EXPECT(ruyamd_mul(c.ctx, &sl, &sr, &p, &sd) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
         R().log.clear();
         R().capturing = true;
         const int rc = ruyamd_mul(c.ctx, &l, &r, &p, &d);
         R().capturing = false;
         EXPECT(R().capture_violations == 0, "%s %d x %d x %d", t.name, k.M, k.K, k.N);
-        EXPECT(rc == RUYAMD_OK || !warm, "%s %d x %d x %d (orders %d %d): %s", t.name, k.M, k.K, k.N, k.lhs_order,
+        EXPECT(rc == RUYAMD_OK || before != "the same call", "%s %d x %d x %d (orders %d %d): %s", t.name, k.M, k.K, k.N, k.lhs_order,
                k.rhs_order, ruyamd_ctx_last_error(c.ctx));
-        EXPECT(rc == RUYAMD_OK || R().log.empty(), "%s %d x %d x %d: refused%s with %d launches recorded", t.name, k.M, k.K,
-               k.N, warm ? "" : " cold", static_cast<int>(R().log.size()));
+        EXPECT(rc == RUYAMD_OK || R().log.empty(), "%s %d x %d x %d (orders %d %d) after %s: refused with %d launches recorded",
+               t.name, k.M, k.K, k.N, k.lhs_order, k.rhs_order, before.c_str(), static_cast<int>(R().log.size()));
       }
     }
   }
