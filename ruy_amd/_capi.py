@@ -5,6 +5,7 @@ this module raises ImportError naming the build command.
 """
 import ctypes as C
 import os
+import warnings
 
 from . import _structs as S
 
@@ -80,9 +81,12 @@ for _name, (_res, _args) in PROTOTYPES.items():
 
 try:
     from . import _native as native  # api.mul's call path (csrc/python/native.cc)
-except ImportError as e:
-    raise ImportError("ruy_amd/_native.so is missing or does not fit this interpreter: build it with "
-                      "`python -m ruy_amd.build`") from e
+except ImportError:
+    # Not built for this interpreter: api.mul gathers the fields in Python, which
+    # makes the same calls and costs some 2 us of each.
+    native = None
+    warnings.warn("ruy_amd/_native has not been built for this interpreter, ruy_amd.api.mul takes longer to start "
+                  "a call without it: `python -m ruy_amd.build` builds it", RuntimeWarning)
 
 
 def check(rc, ctx=None):

@@ -378,7 +378,7 @@ def mul_batch(items, context):
 
 def mul(lhs, rhs, mul_params, context, dst):
     """ruy::Mul (ruy/ruy.h:96-102)."""
-    rc = native.mul(lhs, rhs, mul_params, context._address, dst)
+    rc = native.mul(lhs, rhs, mul_params, context._address, dst) if native else None
     if rc is not None:
         if rc:
             context._check(rc)
@@ -391,4 +391,5 @@ def mul(lhs, rhs, mul_params, context, dst):
     context._check(lib.ruyamd_mul(context._h, C.byref(l), C.byref(r), C.byref(p), C.byref(d)))
 
 
-native.bind(C.cast(lib.ruyamd_mul, C.c_void_p).value, Matrix, Layout, MulParams)
+if native:
+    native.bind(C.cast(lib.ruyamd_mul, C.c_void_p).value, Matrix, Layout, MulParams)

@@ -1,5 +1,5 @@
 """Builds ruy_amd/libruy_amd.so for gfx950 with hipcc, and the Python mirror's
-native call path ruy_amd/_native.so with g++.
+native call path ruy_amd/_native.*.so with g++.
 
     python -m ruy_amd.build [--force]
 
@@ -19,7 +19,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "_obj")
 LIB = os.path.join(HERE, "libruy_amd.so")
-NATIVE = os.path.join(HERE, "_native.so")
+# (Named after the interpreter it is built for: no other one picks it up.)
+NATIVE = os.path.join(HERE, "_native" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-I" + os.path.join(ROOT, "include"),
@@ -68,18 +69,26 @@ def build(force=False, verbose=True):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed: %s\n%s%s" % (" ".join(cmd), r.stdout, r.stderr))
-    build_native()
+    build_native(force)
     if verbose:
         print("built", LIB)
     return LIB
 
 
-def build_native():
+def build_native(force=False):
     """The extension module behind api.mul (csrc/python/native.cc); it calls the
-    library through an address it is given, so it links against nothing."""
+    library through an address it is given, so it links against nothing. Without
+    this interpreter's headers there is none (None), and api.mul does without."""
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        sys.stderr.write("no Python.h in %s: the native call path of api.mul is not built\n" % include)
+        return None
+    src = os.path.join(CSRC, "python", "native.cc")
+    newest = max(os.path.getmtime(f) for f in (src, os.path.join(ROOT, "include", "ruy_amd", "c_api.h")))
+    if not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) > newest:
+        return NATIVE
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
-           "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"],
-           os.path.join(CSRC, "python", "native.cc"), "-o", NATIVE]
+           "-I" + os.path.join(ROOT, "include"), "-I" + include, src, "-o", NATIVE]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("build failed: %s\n%s%s" % (" ".join(cmd), r.stdout, r.stderr))

@@ -7,6 +7,7 @@ import os
 import re
 import shutil
 import subprocess
+import sys
 
 import pytest
 
@@ -352,3 +353,47 @@ def test_the_native_call_path_gathers_what_to_struct_does():
         assert not seen
     finally:
         native.bind(C.cast(lib.ruyamd_mul, C.c_void_p).value, *kinds)
+
+
+def test_the_package_works_without_its_native_call_path():
+    """Another interpreter than the one it was built for, or one without its
+    headers: the mirror's own conversion makes the same calls."""
+    code = """if 1:
+        import sys, warnings
+        sys.modules["ruy_amd._native"] = None  # importing it raises ImportError
+        with warnings.catch_warnings(record=True) as caught:
+            warnings.simplefilter("always")
+            from ruy_amd import _structs as S, api
+        assert any("_native" in str(w.message) for w in caught), caught
+        calls = []
+        class Lib:
+            def ruyamd_mul(self, ctx, l, r, p, d):
+                calls.append((l._obj.rows, r._obj.cols, p._obj.clamp_max, d._obj.stride))
+                return 0
+        class Context:
+            _h, _address = None, 0
+            def _check(self, rc):
+                assert rc == 0
+        api.lib = Lib()
+        make = lambda rows, cols: api.Matrix(S.I8, 4096, api.make_simple_layout(rows, cols, api.Order.kColMajor))
+        api.mul(make(3, 5), make(5, 7), api.MulParams(S.I32, S.I8), Context(), make(3, 7))
+        assert calls == [(3, 7, 127.0, 3)], calls
+    """
+    subprocess.check_call([sys.executable, "-c", code], cwd=ROOT)
+
+
+def test_the_native_call_path_is_built_where_it_can_be_and_when_it_has_to(tmp_path, monkeypatch):
+    from ruy_amd import build
+    monkeypatch.setattr(build, "NATIVE", str(tmp_path / "_native.so"))
+    paths = build.sysconfig.get_paths()
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: dict(paths, include=str(tmp_path)))
+    assert build.build_native() is None and not os.path.exists(build.NATIVE)  # no Python.h there
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: paths)
+    if not os.path.exists(os.path.join(paths["include"], "Python.h")):
+        pytest.skip("this interpreter has no headers")
+    assert build.build_native() == build.NATIVE
+    built = os.stat(build.NATIVE).st_mtime_ns
+    build.build_native()
+    assert os.stat(build.NATIVE).st_mtime_ns == built  # up to date: left alone
+    build.build_native(force=True)
+    assert os.stat(build.NATIVE).st_mtime_ns > built
