@@ -8,7 +8,8 @@
 // kernel it runs on, none of which a GPU is needed (or, for the failures,
 // wanted) for.
 //
-//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing | capture
+//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing | capture |
+//       staged_rule
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -548,6 +549,39 @@ void Capture() {
   }
 }
 
+bool Staged(const std::string& kernel) {
+  return kernel.find("MfmaGemmKernel") != std::string::npos &&
+         (kernel.find("Lb0ELi1EEEv") != std::string::npos || kernel.find("Lb0ELi2EEEv") != std::string::npos);
+}
+
+// Which products of operands usable in place the staged form of the smallest
+// tile takes: whole stages of depth only, since the end of a row costs it more
+// than a direct load does (and short depths whose sums it forms).
+void StagedRule() {
+  struct {
+    int M, K, N, rhs_zero;
+    bool staged;
+  } const cases[] = {
+      {2048, 128, 1024, 0, true},  {2048, 384, 1024, 0, true},  {2048, 320, 1024, 0, false}, {2048, 320, 1024, 3, false},
+      {2048, 144, 1024, 0, false}, {2048, 144, 1024, 3, true},  {2048, 240, 1024, 3, true},  {2048, 256, 1024, 3, true},
+      {2048, 272, 1024, 3, false}, {2048, 496, 1024, 3, false}, {2048, 512, 1024, 3, true},  {2048, 528, 1024, 3, false},
+      {1024, 384, 1024, 0, false}, {1024, 400, 1024, 0, false}, {1024, 512, 1024, 0, true},  {1024, 624, 1024, 3, false},
+      {1024, 640, 1024, 0, true},  {1024, 784, 1024, 0, false}, {1024, 896, 1024, 3, true},  {1024, 1024, 1024, 0, false},
+      {1024, 144, 1024, 3, false}, {2112, 128, 1024, 0, false},
+  };
+  for (const auto& k : cases) {
+    Context c;
+    DeviceCall call(std::size_t(k.M) * k.K, std::size_t(k.K) * k.N, std::size_t(k.M) * k.N);
+    const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, k.M, k.K, RUYAMD_ORDER_ROW_MAJOR);
+    const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, call.rhs, k.K, k.N, RUYAMD_ORDER_COL_MAJOR, k.rhs_zero);
+    const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
+    const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+    EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+    EXPECT(Staged(R().log.back()) == k.staged, "%d x %d x %d, zero point %d: %s", k.M, k.K, k.N, k.rhs_zero,
+           R().log.back().c_str());
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -557,6 +591,7 @@ int main(int argc, char** argv) {
   else if (which == "skinny_shapes") SkinnyShapes();
   else if (which == "timing") Timing();
   else if (which == "capture") Capture();
+  else if (which == "staged_rule") StagedRule();
   else return 2;
   if (g_failures) {
     std::printf("%d failures\n", g_failures);

@@ -168,6 +168,10 @@ def test_one_ordinary_call_is_enough_for_a_capture(runtime_model):
     runtime_model("capture")
 
 
+def test_products_the_staged_form_of_the_smallest_tile_takes(runtime_model):
+    runtime_model("staged_rule")
+
+
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
                     reason="reference tree not present")
 @pytest.mark.parametrize("std", ["c++14", "c++17"])
