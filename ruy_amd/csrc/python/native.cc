@@ -35,18 +35,33 @@ RUYAMD_NAMES(RUYAMD_DECLARE)
 // What a step of the conversion came to.
 enum Outcome { kDone, kNotHandled, kError };
 
-// A field of an instance, borrowed; null if it is not in the dictionary.
-PyObject* Field(PyObject* dict, PyObject* name) { return PyDict_GetItemWithError(dict, name); }
+// A reference of our own. Asking a buffer for its address or a value for its
+// float may run any code, also code that takes that object out of the instance
+// it was found in, or the instance's dictionary away.
+class Ref {
+ public:
+  explicit Ref(PyObject* borrowed) : p_(borrowed) { Py_XINCREF(p_); }
+  ~Ref() { Py_XDECREF(p_); }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+  operator PyObject*() const { return p_; }
 
-PyObject* DictOf(PyObject* object) {
+ private:
+  PyObject* p_;
+};
+
+// A field of an instance; null if it is not in the dictionary (or there is none).
+Ref Field(PyObject* dict, PyObject* name) { return Ref(dict ? PyDict_GetItemWithError(dict, name) : nullptr); }
+
+Ref DictOf(PyObject* object) {
   PyObject** p = _PyObject_GetDictPtr(object);
-  return p ? *p : nullptr;
+  return Ref(p ? *p : nullptr);
 }
 
 // Only Python integers are taken here (as ctypes does, bits beyond the field's
 // are dropped); anything else is left to the Python code.
 bool Integer(PyObject* dict, PyObject* name, uint64_t* out) {
-  PyObject* v = dict ? Field(dict, name) : nullptr;
+  const Ref v = Field(dict, name);
   if (!v || !PyLong_Check(v)) return false;
   *out = PyLong_AsUnsignedLongLongMask(v);
   return true;
@@ -86,11 +101,11 @@ Outcome Address(PyObject* buffer, void** out) {
 
 Outcome Matrix(PyObject* object, ruyamd_mat* m) {
   if (Py_TYPE(object) != matrix_type) return kNotHandled;
-  PyObject* dict = DictOf(object);
-  PyObject* layout = dict ? Field(dict, name_layout) : nullptr;
-  PyObject* data = dict ? Field(dict, name_data) : nullptr;
+  const Ref dict = DictOf(object);
+  const Ref layout = Field(dict, name_layout);
+  const Ref data = Field(dict, name_data);
   if (!layout || !data || Py_TYPE(layout) != layout_type) return kNotHandled;
-  PyObject* shape = DictOf(layout);
+  const Ref shape = DictOf(layout);
   uint64_t rows, cols, stride, order, zero_point, dtype, policy;
   if (!Integer(shape, name_rows, &rows) || !Integer(shape, name_cols, &cols) ||
       !Integer(shape, name_stride, &stride) || !Integer(shape, name_order, &order) ||
@@ -110,8 +125,8 @@ Outcome Matrix(PyObject* object, ruyamd_mat* m) {
 
 Outcome Params(PyObject* object, ruyamd_mul_params* p, uint64_t* dst_dtype) {
   if (Py_TYPE(object) != params_type) return kNotHandled;
-  PyObject* dict = DictOf(object);
-  PyObject* perchannel = dict ? Field(dict, name__perchannel) : nullptr;
+  const Ref dict = DictOf(object);
+  const Ref perchannel = Field(dict, name__perchannel);
   uint64_t accum, channel, rounding;
   if (!perchannel || !PyBool_Check(perchannel) || !Integer(dict, name_accum_dtype, &accum) ||
       !Integer(dict, name_dst_dtype, dst_dtype) || !Integer(dict, name_channel_dimension, &channel) ||
@@ -121,20 +136,20 @@ Outcome Params(PyObject* object, ruyamd_mul_params* p, uint64_t* dst_dtype) {
   p->accum_dtype = static_cast<uint8_t>(accum);
   p->channel_dimension = static_cast<uint8_t>(channel);
   p->perchannel_buffers_capacity_rounding_log2 = static_cast<uint8_t>(rounding);
-  PyObject* clamp_min = Field(dict, name_clamp_min);
-  PyObject* clamp_max = Field(dict, name_clamp_max);
+  const Ref clamp_min = Field(dict, name_clamp_min);
+  const Ref clamp_max = Field(dict, name_clamp_max);
   if (!clamp_min || !clamp_max) return kNotHandled;
   p->clamp_min = PyFloat_AsDouble(clamp_min);
   p->clamp_max = PyFloat_AsDouble(clamp_max);
   if (PyErr_Occurred()) return kError;
-  PyObject* bias = Field(dict, name_bias);
+  const Ref bias = Field(dict, name_bias);
   if (!bias) return kNotHandled;
   void* address = nullptr;
   if (Outcome o = Address(bias, &address)) return o;
   p->bias = address;
   if (perchannel == Py_True) {
-    PyObject* mf = Field(dict, name__mf_pc);
-    PyObject* me = Field(dict, name__me_pc);
+    const Ref mf = Field(dict, name__mf_pc);
+    const Ref me = Field(dict, name__me_pc);
     if (!mf || !me) return kNotHandled;
     if (Outcome o = Address(mf, &address)) return o;
     p->multiplier_fixedpoint_perchannel = static_cast<const int32_t*>(address);

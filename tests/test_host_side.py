@@ -359,6 +359,46 @@ def test_the_native_call_path_gathers_what_to_struct_does():
         native.bind(C.cast(lib.ruyamd_mul, C.c_void_p).value, *kinds)
 
 
+def test_the_native_call_path_holds_what_it_asks():
+    """A buffer that takes itself out of its matrix when asked for its address,
+    and a bound that takes the other one away: both are still there when they are
+    asked the next thing."""
+    from ruy_amd import _structs as S
+    from ruy_amd import api
+    from ruy_amd._capi import native
+    events = []
+
+    class Tracked:
+        def __init__(self, name):
+            self.name = name
+
+        def __del__(self):
+            events.append(self.name + " gone")
+
+    class Buffer(Tracked):
+        def data_ptr(self):
+            rhs.data = None
+            raise AttributeError("data_ptr")
+
+        @property
+        def ctypes(self):
+            events.append("buffer asked")
+            raise AttributeError("ctypes")
+
+    class Bound(Tracked):
+        def __float__(self):
+            events.append(self.name + " asked")
+            params.clamp_max = 1.0
+            return 0.0
+
+    layout = api.Layout(4, 4, 4, 0)
+    lhs, rhs, dst = api.Matrix(S.I8, 0, layout), api.Matrix(S.I8, Buffer("buffer"), layout), api.Matrix(S.I8, 0, layout)
+    params = api.MulParams(S.I32, S.I8)
+    params.clamp_min, params.clamp_max = Bound("lower"), Bound("upper")
+    assert native.mul(lhs, rhs, params, 0, dst) is None
+    assert events == ["lower asked", "upper asked", "upper gone", "buffer asked", "buffer gone"]
+
+
 def test_the_package_works_without_its_native_call_path():
     """Another interpreter than the one it was built for, or one without its
     headers: the mirror's own conversion makes the same calls."""
