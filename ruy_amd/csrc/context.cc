@@ -41,7 +41,13 @@ void* Workspace::Alloc(std::size_t bytes) {
     exhausted_ = true;
     return nullptr;
   }
-  std::size_t size = need < (std::size_t(1) << 20) ? (std::size_t(1) << 20) : need;
+  // A large block has room for what follows a large operand, above all the sums
+  // of one operand or the other: the first call on a context takes one block
+  // then, and the second has none to merge (2048^3 int8, one operand packed, both
+  // sums left to the product: first call 343 us, second 355 with a second block
+  // for the sums; 56 and 33 with room in the first).
+  constexpr std::size_t kLeast = std::size_t(1) << 20, kBehind = std::size_t(256) << 10;
+  std::size_t size = need + kBehind < kLeast ? kLeast : need + kBehind;
   void* p = nullptr;
   if (hipMalloc(&p, size) != hipSuccess) {
     (void)hipGetLastError();

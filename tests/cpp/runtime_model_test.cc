@@ -9,7 +9,7 @@
 // wanted) for.
 //
 //   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing | capture |
-//       staged_rule
+//       scratch_blocks | staged_rule
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -52,6 +52,7 @@ struct Runtime {
   hipError_t last_error = hipSuccess;
   bool capturing = false;
   int capture_violations = 0;
+  int allocations = 0;                                // of device memory
   dim3 grid, block;
   std::size_t shared = 0;
   hipStream_t stream = nullptr;
@@ -158,7 +159,10 @@ static hipError_t Give(std::map<const char*, std::size_t>* ranges, void* p) {
   NotWhileCapturing();
   return hipSuccess;
 }
-hipError_t hipMalloc(void** p, std::size_t bytes) { return Take(&R().device, p, bytes); }
+hipError_t hipMalloc(void** p, std::size_t bytes) {
+  ++R().allocations;
+  return Take(&R().device, p, bytes);
+}
 hipError_t hipFree(void* p) { return Give(&R().device, p); }
 hipError_t hipHostMalloc(void** p, std::size_t bytes, unsigned) { return Take(&R().pinned, p, bytes); }
 hipError_t hipHostFree(void* p) { return Give(&R().pinned, p); }
@@ -549,6 +553,33 @@ void Capture() {
   }
 }
 
+// A packed operand and the sums of both are in one block of scratch memory: a
+// first call takes one block, and the next has no blocks to merge.
+void ScratchBlocks() {
+  struct {
+    int M, K, N, lhs_zero, rhs_zero;
+  } const cases[] = {
+      {2048, 2048, 2048, 0, 3},  // its sums formed by the product
+      {2048, 2048, 2048, 4, 3},  // ... and those of the other operand, which is used in place
+      {8192, 128, 1024, 0, 3},   // by the pack
+      {2048, 2048, 2048, 0, 0},  // none
+  };
+  for (const auto& k : cases) {
+    DeviceCall call(std::size_t(k.M) * k.K, std::size_t(k.K) * k.N, std::size_t(k.M) * k.N);
+    const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, k.M, k.K, RUYAMD_ORDER_COL_MAJOR, k.lhs_zero);
+    const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, call.rhs, k.K, k.N, RUYAMD_ORDER_COL_MAJOR, k.rhs_zero);
+    const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
+    const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+    Context c;
+    for (int want : {1, 0}) {
+      R().allocations = 0;
+      EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+      EXPECT(R().allocations == want, "%d x %d x %d, zero points %d %d: %d allocations, expected %d", k.M, k.K,
+             k.N, k.lhs_zero, k.rhs_zero, R().allocations, want);
+    }
+  }
+}
+
 bool Staged(const std::string& kernel) {
   return kernel.find("MfmaGemmKernel") != std::string::npos &&
          (kernel.find("Lb0ELi1EEEv") != std::string::npos || kernel.find("Lb0ELi2EEEv") != std::string::npos);
@@ -591,6 +622,7 @@ int main(int argc, char** argv) {
   else if (which == "skinny_shapes") SkinnyShapes();
   else if (which == "timing") Timing();
   else if (which == "capture") Capture();
+  else if (which == "scratch_blocks") ScratchBlocks();
   else if (which == "staged_rule") StagedRule();
   else return 2;
   if (g_failures) {

@@ -168,6 +168,10 @@ def test_one_ordinary_call_is_enough_for_a_capture(runtime_model):
     runtime_model("capture")
 
 
+def test_a_packed_operand_and_the_sums_share_a_block_of_scratch_memory(runtime_model):
+    runtime_model("scratch_blocks")
+
+
 def test_products_the_staged_form_of_the_smallest_tile_takes(runtime_model):
     runtime_model("staged_rule")
 
