@@ -237,13 +237,15 @@ bool HostStaging::ToHost2D(void* dst_host, const void* src_dev, std::size_t pitc
                            std::size_t outer, Memory destination, hipStream_t stream, bool* drained) {
   *drained = false;
   if (inner_bytes == 0 || outer == 0) return true;
-  if (pitch * (outer - 1) + inner_bytes <= kByKernel) {
+  const bool pageable = destination == Memory::kPageable;
+  const bool one_run = pitch == inner_bytes || outer == 1;
+  if (pitch * (outer - 1) + inner_bytes <= (pageable ? kByKernel : one_run ? kThroughChunk : kRunsThroughChunk)) {
     if (!Init()) return false;
     return SmallToHost2D(static_cast<char*>(dst_host), src_dev, pitch, inner_bytes, outer, stream, drained);
   }
-  if (destination != Memory::kPageable) {
+  if (!pageable) {
     // Stream-ordered; complete once the caller has synchronised the stream.
-    if (pitch == inner_bytes || outer == 1)
+    if (one_run)
       return hipMemcpyAsync(dst_host, src_dev, pitch * (outer - 1) + inner_bytes, hipMemcpyDeviceToHost,
                             stream) == hipSuccess;
     return hipMemcpy2DAsync(dst_host, pitch, src_dev, pitch, inner_bytes, outer, hipMemcpyDeviceToHost,

@@ -96,8 +96,8 @@ class HostStaging {
   // from device to host after everything already enqueued on `stream`; the
   // bytes between the runs of the host image are not written. The host image
   // is complete when this returns (pageable or small destination) or once the
-  // stream has been synchronised (large page-locked `destination`, copied
-  // directly). *drained is set if everything enqueued on `stream` so far is
+  // stream has been synchronised (page-locked `destination` above kThroughChunk,
+  // written directly). *drained is set if everything enqueued on `stream` so far is
   // known to have finished. src_dev as dst_dev in ToDevice.
   bool ToHost2D(void* dst_host, const void* src_dev, std::size_t pitch, std::size_t inner_bytes,
                 std::size_t outer, Memory destination, hipStream_t stream, bool* drained);
@@ -117,6 +117,14 @@ class HostStaging {
   // each way 73 -> 40 us, 1 MiB each way 141 -> 118 us; 2 MiB and more gain from
   // the engine's higher rate and from the CPU filling the next chunk meanwhile).
   static constexpr std::size_t kByKernel = std::size_t(1) << 20;
+  // A page-locked destination the engine writes directly, where the kernel's way
+  // ends with the CPU's copy out of a chunk, which costs more when it is one of
+  // many runs (whole calls, destination by the engine -> by the kernel: 64 KiB 33
+  // to 37 -> 24 us, 196 KiB 40 to 44 -> 35, 384 KiB 41 to 45 -> 41, 640 KiB 46 to
+  // 50 -> 53, 1000 KiB 82 to 86 -> 105; in runs 64 KiB 32 to 34 -> 25, 196 KiB 37
+  // to 41 -> 42, 512 KiB 44 to 47 -> 65).
+  static constexpr std::size_t kThroughChunk = std::size_t(384) << 10;
+  static constexpr std::size_t kRunsThroughChunk = std::size_t(128) << 10;
   // Behind the chunks: one word per workgroup of a download.
   static constexpr std::size_t kDoneBytes = kByKernel / kHostCopyBlockBytes * sizeof(uint32_t);
   bool Init();

@@ -8,8 +8,8 @@
 // kernel it runs on, none of which a GPU is needed (or, for the failures,
 // wanted) for.
 //
-//   runtime_model_test failed_upload | page_locked_sources | skinny_shapes | timing | capture |
-//       scratch_blocks | staged_rule
+//   runtime_model_test failed_upload | page_locked_sources | page_locked_destinations | skinny_shapes |
+//       timing | capture | scratch_blocks | staged_rule
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -426,6 +426,41 @@ void PageLockedSources() {
   }
 }
 
+// A page-locked destination comes back by a kernel and the CPU only while that
+// is the shorter way, in one run or in many; either way all of it is there when
+// the call returns, and nothing between its runs.
+void PageLockedDestinations() {
+  struct {
+    int rows, cols, pad;
+    bool locked, by_kernel;
+  } const cases[] = {
+      {1024, 384, 0, true, true},  {1024, 385, 0, true, false},  {1024, 128, 32, true, true},
+      {1024, 129, 32, true, false}, {1024, 1024, 0, false, true}, {1024, 1024, 32, false, true},
+      {1024, 1025, 0, false, false}, {3000, 1, 64, true, true},
+  };
+  for (const auto& k : cases) {
+    Context c;
+    const int K = 33, rows = k.rows - k.pad;
+    std::vector<char> lhs(k.rows * K, 1), rhs(K * k.cols, 2), pageable(std::size_t(k.rows) * k.cols);
+    PageLocked locked(pageable.size(), pageable.size());
+    char* dst = k.locked ? locked.data : pageable.data();
+    std::memset(dst, 0x5A, pageable.size());
+    const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, lhs.data(), rows, K, RUYAMD_ORDER_ROW_MAJOR);
+    const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, rhs.data(), K, k.cols, RUYAMD_ORDER_COL_MAJOR);
+    ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, dst, rows, k.cols, RUYAMD_ORDER_COL_MAJOR);
+    d.stride = k.rows;
+    const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+    EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+    EXPECT(Count("DownloadKernel") == k.by_kernel, "%d x %d, %d between the runs", rows, k.cols, k.pad);
+    // (No kernel has written the device's image of it: it is as memory is allocated here.)
+    int wrong = 0;
+    for (int j = 0; j < k.cols; ++j)
+      for (int i = 0; i < k.rows; ++i)
+        wrong += dst[std::size_t(j) * k.rows + i] != (i < rows ? static_cast<char>(0xCD) : 0x5A);
+    EXPECT(wrong == 0, "%d x %d, %d between the runs: %d bytes", rows, k.cols, k.pad, wrong);
+  }
+}
+
 // Kernel timing of a call on host memory brackets the product, not the upload.
 void Timing() {
   const int M = 96, K = 160;
@@ -619,6 +654,7 @@ int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "failed_upload") FailedUpload();
   else if (which == "page_locked_sources") PageLockedSources();
+  else if (which == "page_locked_destinations") PageLockedDestinations();
   else if (which == "skinny_shapes") SkinnyShapes();
   else if (which == "timing") Timing();
   else if (which == "capture") Capture();

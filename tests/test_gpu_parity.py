@@ -191,7 +191,7 @@ def test_large_host_pointer_operands_and_the_staging_advisory(device_ctx):
     assert not device_ctx.performance_advisory(S.ADVISORY_STAGED_THROUGH_HOST)
     for _ in range(3):                                          # repeated host calls reuse the chunks
         compare(small, D.host_pointer_mul(device_ctx, small, dst_fill=0x5A), want)
-    # page-locked host memory is copied directly, without the staging chunks
+    # large page-locked operands are copied directly, without the staging chunks
     import ctypes as C
     import torch
     from ruy_amd import api
@@ -267,6 +267,32 @@ def test_host_pointer_transfers_by_kernels_and_by_the_copy_engine(device_ctx, sh
         want = expected(p, fill=0x5A)
         for _ in range(3):
             compare(p, D.host_pointer_mul(device_ctx, p, dst_fill=0x5A), want)
+
+
+@pytest.mark.parametrize("shape", [(1024, 70, 384), (1024, 70, 385), (1024, 70, 100), (1021, 70, 130), (65, 70, 33)])
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_page_locked_destinations(device_ctx, shape, strided, offset):
+    """Either side of the sizes from which the copy engine writes a page-locked
+    destination itself, in one run and in many, at any address; repeated, and with
+    the other way in between."""
+    import ctypes as C
+    import torch
+    from ruy_amd import api
+    rng = np.random.default_rng(shape[2])
+    p = W.random_problem(rng, S.I8, S.I8, S.I32, S.I8, *shape, *cases.RCC, strided=strided, name="to %s" % (shape,))
+    want = expected(p, fill=0x5A)
+    out = torch.empty(p.dst.n_storage + offset + 16, dtype=torch.int8).pin_memory()
+    for _ in range(3):
+        out.fill_(0x5A)
+        l, r, d = p.lhs.struct(), p.rhs.struct(), p.dst.struct(out.data_ptr() + offset)
+        ps = p.params_struct()
+        device_ctx._check(api.lib.ruyamd_mul(device_ctx._h, C.byref(l), C.byref(r), C.byref(ps), C.byref(d)))
+        got = out.numpy()
+        compare(p, got[offset:offset + p.dst.n_storage], want)
+        assert (got[:offset] == 0x5A).all() and (got[offset + p.dst.n_storage:] == 0x5A).all()
+        from ruy_amd import device_problem as D
+        compare(p, D.host_pointer_mul(device_ctx, p, dst_fill=0x5A), want)
 
 
 @pytest.mark.parametrize("depth", [45, 1024, 9000])

@@ -155,6 +155,10 @@ def test_page_locked_sources_are_read_in_stream_order(runtime_model):
     runtime_model("page_locked_sources")
 
 
+def test_page_locked_destinations_come_back_the_shorter_way(runtime_model):
+    runtime_model("page_locked_destinations")
+
+
 def test_waves_to_a_group_of_the_streaming_kernel(runtime_model):
     runtime_model("skinny_shapes")
 
