@@ -100,19 +100,37 @@ def test_ring_schedule_of_the_largest_tile_model():
     assert out.count("altered (") >= 12
 
 
+def kernel_assembly(tmp_path, source):
+    """The instructions of the first kernel of a source file whose name holds a text."""
+    from ruy_amd import build
+    asm = str(tmp_path / "kernels.s")
+    subprocess.check_call([build.HIPCC] + build.COMMON + build.DEVICE + [
+        "--offload-device-only", "-S", os.path.join(build.CSRC, "kernels", source), "-o", asm])
+    lines = [l.split(";")[0].strip() for l in open(asm)]
+
+    def body(name):
+        start = next(i for i, l in enumerate(lines) if name in l and l.endswith(":"))
+        return lines[start:next(i for i in range(start, len(lines)) if lines[i].startswith(".Lfunc_end"))]
+    return body
+
+
+def test_a_lane_of_a_row_pack_has_four_loads_in_flight(tmp_path):
+    """Rows of 16 and of 64 lanes: none of a lane's four loads is awaited before
+    the last of them is issued."""
+    body = kernel_assembly(tmp_path, "pack.hip")
+    for kernel in ("PackKernelILi1ELi0E", "PackKernelILi2ELi0E"):
+        steps = "".join("L" if l.startswith("global_load_dwordx4") else
+                        "w" if l.startswith("s_waitcnt") and "vmcnt" in l else "" for l in body(kernel))
+        assert "LLLL" in steps and steps.count("L") == 4, (kernel, steps)
+
+
 def test_every_wave_of_a_download_awaits_its_stores(tmp_path):
     """The word that tells the host a workgroup's part of a download is there is
     stored by one wave (kernels/host_copy.hip). A workgroup barrier by itself
     waits for no store on this target, so each wave has to write back and await
     its own in front of it: looked up in the assembly, between the last store of
     the copy and the barrier."""
-    from ruy_amd import build
-    asm = str(tmp_path / "host_copy.s")
-    subprocess.check_call([build.HIPCC] + build.COMMON + build.DEVICE + [
-        "--offload-device-only", "-S", os.path.join(build.CSRC, "kernels", "host_copy.hip"), "-o", asm])
-    lines = [l.split(";")[0].strip() for l in open(asm)]
-    start = next(i for i, l in enumerate(lines) if "DownloadKernel" in l and l.endswith(":"))
-    body = lines[start:lines.index("s_endpgm", start)]
+    body = kernel_assembly(tmp_path, "host_copy.hip")("DownloadKernel")
     barrier = body.index("s_barrier")
     last_store = max(i for i, l in enumerate(body[:barrier]) if l.startswith("global_store_dwordx4"))
     between = body[last_store + 1:barrier]
