@@ -20,8 +20,11 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int kThreads = 256;
 constexpr int kPerThread = int(kHostCopyBlockBytes) / 16 / kThreads;
 
-// 16 KiB per workgroup, four 16-byte accesses in flight per thread: bound by
-// PCIe and its latency, not by the number of workgroups.
+// 16 KiB per workgroup, four 16-byte accesses per thread, one after the other
+// (each load stands behind a bounds test of its own and is awaited there): bound
+// by PCIe and its latency. With the four in flight together 64 KiB up take 4.1 us
+// instead of 6.7 and 196 KiB 6.7 instead of 8.2, but 1 MiB 26 instead of 22, and a
+// whole call that moves 1 MiB up and 0.5 MiB down 83 instead of 78.
 __device__ __forceinline__ void CopyBlock(const void* from, void* to, uint32_t bytes) {
   const int granules = static_cast<int>((bytes + 15) / 16);
   const int first = int(blockIdx.x) * kThreads * kPerThread + int(threadIdx.x);
