@@ -41,13 +41,7 @@ void* Workspace::Alloc(std::size_t bytes) {
     exhausted_ = true;
     return nullptr;
   }
-  // A large block has room for what follows a large operand, above all the sums
-  // of one operand or the other: the first call on a context takes one block
-  // then, and the second has none to merge (2048^3 int8, one operand packed, both
-  // sums left to the product: first call 343 us, second 355 with a second block
-  // for the sums; 56 and 33 with room in the first).
-  constexpr std::size_t kLeast = std::size_t(1) << 20, kBehind = std::size_t(256) << 10;
-  std::size_t size = need + kBehind < kLeast ? kLeast : need + kBehind;
+  std::size_t size = need < (std::size_t(1) << 20) ? (std::size_t(1) << 20) : need;
   void* p = nullptr;
   if (hipMalloc(&p, size) != hipSuccess) {
     (void)hipGetLastError();
@@ -376,20 +370,22 @@ int ruyamd_ctx_create(ruyamd_ctx** out) {
     return RUYAMD_E_HIP;
   }
   ctx->stream = ctx->own_stream;
-  // One zeroed allocation: the two sets of words of the row sums formed
-  // inside a launch, then the depth split's counters.
+  // One allocation: the words of sums formed by a launch of their own, and,
+  // zeroed, the two sets of words of the row sums formed inside a launch, then
+  // the depth split's counters.
   const std::size_t split_words = std::size_t(ruyamd::GemmDepthSplitCounters());
   const std::size_t set_words = std::size_t(ruyamd::fused_sums::kMaxRows);
   const std::size_t counter_bytes = 2 * set_words * sizeof(long long) + split_words * sizeof(uint32_t);
-  void* const zeroed = DeviceAlloc(counter_bytes);
-  if (zeroed) {
-    ctx->row_sums_sets[0] = static_cast<long long*>(zeroed);
+  ctx->sums_words = static_cast<int32_t*>(DeviceAlloc(2 * set_words * sizeof(int32_t) + counter_bytes));
+  if (ctx->sums_words) {
+    ctx->row_sums_sets[0] = reinterpret_cast<long long*>(ctx->sums_words + 2 * set_words);
     ctx->row_sums_sets[1] = ctx->row_sums_sets[0] + set_words;
     ctx->split_counters = reinterpret_cast<uint32_t*>(ctx->row_sums_sets[1] + set_words);
   }
-  if (!zeroed || hipMemsetAsync(zeroed, 0, counter_bytes, ctx->own_stream) != hipSuccess ||
+  if (!ctx->sums_words ||
+      hipMemsetAsync(ctx->row_sums_sets[0], 0, counter_bytes, ctx->own_stream) != hipSuccess ||
       hipStreamSynchronize(ctx->own_stream) != hipSuccess) {
-    DeviceFree(zeroed);
+    DeviceFree(ctx->sums_words);
     (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
     return RUYAMD_E_HIP;
@@ -399,7 +395,7 @@ int ruyamd_ctx_create(ruyamd_ctx** out) {
   void* static_scratch = nullptr;
   if (ruyamd::StaticScratchOfCurrentDevice(&static_scratch) != hipSuccess) {
     (void)hipGetLastError();
-    DeviceFree(ctx->row_sums_sets[0]);
+    DeviceFree(ctx->sums_words);
     (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
     return RUYAMD_E_HIP;
@@ -417,7 +413,7 @@ void ruyamd_ctx_destroy(ruyamd_ctx* ctx) {
   if (!ctx) return;
   (void)hipStreamSynchronize(ctx->stream);
   ctx->cache.reset();
-  DeviceFree(ctx->row_sums_sets[0]);  // (the depth split's counters lie behind the two sets)
+  DeviceFree(ctx->sums_words);  // (the row sums' sets and the depth split's counters lie behind them)
   for (auto* v : {&ctx->timing_pending, &ctx->timing_pool})
     for (auto& ev : *v) {
       (void)hipEventDestroy(ev.first);

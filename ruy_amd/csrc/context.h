@@ -178,6 +178,11 @@ struct ruyamd_ctx {
   uint32_t* split_counters = nullptr;
   // The same in this GPU's static scratch area, for calls that may not allocate.
   uint32_t* static_split_counters = nullptr;
+  // Room for sums formed by a launch of their own, of one operand and of the
+  // other (fused_sums::kMaxRows each; more come from the workspace): there from
+  // the start, since a call that is being recorded needs it where an ordinary
+  // one does not.
+  int32_t* sums_words = nullptr;
   // Row sums formed inside the launch of the largest int8 tile
   // (kernels/fused_sums.h): two sets of 64-bit words, one per row, all zero
   // when a launch starts. A launch uses set `row_sums_next` and clears what

@@ -60,19 +60,29 @@ struct Operand8 {
   PackSource src;
 };
 
-// Room for the sums of an operand that nobody has formed yet, taken before
-// anything of the call is launched. A call that is being recorded, or may not
-// allocate, forms them in a launch of their own where an ordinary one leaves
-// them to the product; the ordinary call takes the room all the same (if it can
-// be had: it does not depend on it), so that a recorded one finds it there.
-int ReserveSums(ruyamd_ctx* ctx, Operand8* op, bool formed_by_product, std::string* err) {
-  if (!op->sums_pending) return RUYAMD_OK;
+// Room for the sums of an operand (`side` 0 or 1) that nobody has formed yet,
+// taken before anything of the call is launched. A call that is being recorded
+// forms them in a launch of their own where an ordinary one shares them out over
+// the product's workgroups, so what room they need must not depend on that: the
+// context has it, for up to kMaxRows vectors. For more, the ordinary call takes
+// it from the workspace as well (if it can be had: it does not depend on it), so
+// that a recorded one finds it there. Not where each workgroup forms what it
+// multiplies by itself (formed_by_product: an ordinary call that does so is the
+// same launch when recorded, since sums that must not be shared out only make
+// the other tiles dearer). Taken by every ordinary call from the workspace, the
+// room cost it a block of its own (2048^3, one operand packed, both sums left to
+// the product: first call 56 -> 343 us, second 33 -> 355).
+int ReserveSums(ruyamd_ctx* ctx, Operand8* op, int side, bool formed_by_product, std::string* err) {
+  if (!op->sums_pending || formed_by_product) return RUYAMD_OK;
+  if (op->count <= fused_sums::kMaxRows && !ctx->no_alloc) {
+    op->sums_room = ctx->sums_words + side * fused_sums::kMaxRows;
+    return RUYAMD_OK;
+  }
   const std::size_t bytes = std::size_t(op->count) * 4;
   if (!ctx->capturing && !ctx->no_alloc) {
     op->sums_room = static_cast<int32_t*>(ctx->ws->AllocOptional(bytes));
     return RUYAMD_OK;
   }
-  if (formed_by_product) return RUYAMD_OK;
   op->sums_room = static_cast<int32_t*>(ctx->ws->Alloc(bytes));
   if (op->sums_room) return RUYAMD_OK;
   *err = "workspace allocation failed";
@@ -485,8 +495,8 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   }
   GemmArgs args;
   const bool swap = SetupInt8Gemm(ctx, *call, a, b, lzp, rzp, /*staged=*/false, &args);
-  if (int rc = ReserveSums(ctx, &a, args.fuse_sums != 0, err)) return rc;
-  if (int rc = ReserveSums(ctx, &b, args.fuse_sums != 0, err)) return rc;
+  if (int rc = ReserveSums(ctx, &a, 0, args.fuse_sums != 0, err)) return rc;
+  if (int rc = ReserveSums(ctx, &b, 1, args.fuse_sums != 0, err)) return rc;
   if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   // The largest tile can form the sums of the rows of its `a` operand in
   // passing (kernels/fused_sums.h): one launch instead of a sums kernel and
@@ -814,7 +824,7 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     args.fused_a_factor = args.ep.rhs_zero_point;
     args.ep.rhs_zero_point = 0;
   }
-  if (int rc = ReserveSums(ctx, &a, args.fuse_sums != 0, err)) return rc;
+  if (int rc = ReserveSums(ctx, &a, 0, args.fuse_sums != 0, err)) return rc;
   bool raw = false;
   PackSource fresh;
   const bool planes_cached = planes != nullptr;

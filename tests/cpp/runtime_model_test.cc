@@ -553,6 +553,8 @@ void Capture() {
       {64, 8192, 100, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 4, -3},
       {4096, 5000, 7, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 4, -3},     // skinny
       {77, 131, 45, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_ROW_MAJOR, 4, -3},
+      {100000, 512, 256, RUYAMD_ORDER_COL_MAJOR, RUYAMD_ORDER_COL_MAJOR, 0, 3},   // more rows than a context has room for
+      {100000, 512, 256, RUYAMD_ORDER_ROW_MAJOR, RUYAMD_ORDER_COL_MAJOR, 0, 3},
   };
   for (const auto& k : cases) {
     for (const Types& t : kTypes) {
@@ -588,25 +590,28 @@ void Capture() {
   }
 }
 
-// A packed operand and the sums of both are in one block of scratch memory: a
-// first call takes one block, and the next has no blocks to merge.
+// Sums left to the product cost a call no scratch memory, although a recorded
+// call forms some of them in a launch of their own: a first call takes a block
+// for an operand that is packed and the sums the pack forms, nothing more.
 void ScratchBlocks() {
   struct {
-    int M, K, N, lhs_zero, rhs_zero;
+    int M, K, N, lhs_order, lhs_zero, rhs_zero, blocks;
   } const cases[] = {
-      {2048, 2048, 2048, 0, 3},  // its sums formed by the product
-      {2048, 2048, 2048, 4, 3},  // ... and those of the other operand, which is used in place
-      {8192, 128, 1024, 0, 3},   // by the pack
-      {2048, 2048, 2048, 0, 0},  // none
+      {2048, 2048, 2048, RUYAMD_ORDER_COL_MAJOR, 0, 3, 1},  // its sums formed by the product
+      {2048, 2048, 2048, RUYAMD_ORDER_COL_MAJOR, 4, 3, 1},  // ... and those of the other operand, used in place
+      {1024, 128, 8192, RUYAMD_ORDER_COL_MAJOR, 0, 3, 1},   // by the pack
+      {2048, 2048, 2048, RUYAMD_ORDER_COL_MAJOR, 0, 0, 1},  // none
+      {2048, 2048, 2048, RUYAMD_ORDER_ROW_MAJOR, 0, 3, 0},  // in place, its sums shared out (not so when recorded)
+      {256, 256, 256, RUYAMD_ORDER_ROW_MAJOR, 0, 3, 0},     // in place, formed by each workgroup by itself
   };
   for (const auto& k : cases) {
     DeviceCall call(std::size_t(k.M) * k.K, std::size_t(k.K) * k.N, std::size_t(k.M) * k.N);
-    const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, k.M, k.K, RUYAMD_ORDER_COL_MAJOR, k.lhs_zero);
+    const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, k.M, k.K, k.lhs_order, k.lhs_zero);
     const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, call.rhs, k.K, k.N, RUYAMD_ORDER_COL_MAJOR, k.rhs_zero);
     const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
     const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
     Context c;
-    for (int want : {1, 0}) {
+    for (int want : {k.blocks, 0}) {
       R().allocations = 0;
       EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
       EXPECT(R().allocations == want, "%d x %d x %d, zero points %d %d: %d allocations, expected %d", k.M, k.K,

@@ -190,7 +190,7 @@ def test_one_ordinary_call_is_enough_for_a_capture(runtime_model):
     runtime_model("capture")
 
 
-def test_a_packed_operand_and_the_sums_share_a_block_of_scratch_memory(runtime_model):
+def test_sums_left_to_the_product_take_no_scratch_memory(runtime_model):
     runtime_model("scratch_blocks")
 
 
