@@ -501,6 +501,10 @@ hipError_t LaunchMmaFlip(hipStream_t stream, const GemvI8Args& args) {
 // workgroup.
 // Vectors of 32 KiB and more want the longer runs: fp32 3000 x 16384 x 3 34.2
 // in 512-byte stages, 39.0 in 256-byte ones, 16384 x 8192 x 16 78.2 and 80.9.
+// int8 has them there too: better below 512 groups (3000 x 32768 x 2 17.9 and
+// 20.1, 2500 x 65536 x 2 30.3 and 34.9), which is not so from there on (8192 x
+// 32768 x 8 44.1 and 42.2, 14000 x 65536 x 8 164.7 and 147.8, 20000 x 32768 x 16
+// 140.5 and 109.5).
 // Except where half the CUs or fewer have a group: there eight waves share the
 // depth of each (of four steps and more a wave, or their ring never fills):
 // fp32 512 x 16384 x 7 30.9 -> 23.0, 2048 x 8192 x 4 17.9 -> 14.0, int8 512 x
