@@ -626,19 +626,21 @@ bool Staged(const std::string& kernel) {
 }
 
 // Which products of operands usable in place the staged form of the smallest
-// tile takes: whole stages of depth only, since the end of a row costs it more
-// than a direct load does (and short depths whose sums it forms).
+// tile takes: with one workgroup a CU whole stages of depth only, since the end of
+// a row costs it more than a direct load does; with two also those whose sums it
+// forms, or whose columns end in many rows that are stored one by one.
 void StagedRule() {
   struct {
     int M, K, N, rhs_zero;
     bool staged;
   } const cases[] = {
-      {2048, 128, 1024, 0, true},  {2048, 384, 1024, 0, true},  {2048, 320, 1024, 0, false}, {2048, 320, 1024, 3, false},
+      {2048, 128, 1024, 0, true},  {2048, 384, 1024, 0, true},  {2048, 320, 1024, 0, false}, {2048, 320, 1024, 3, true},
       {2048, 144, 1024, 0, false}, {2048, 144, 1024, 3, true},  {2048, 240, 1024, 3, true},  {2048, 256, 1024, 3, true},
-      {2048, 272, 1024, 3, false}, {2048, 496, 1024, 3, false}, {2048, 512, 1024, 3, true},  {2048, 528, 1024, 3, false},
+      {2048, 272, 1024, 3, true},  {2048, 496, 1024, 3, true},  {2048, 512, 1024, 3, true},  {2048, 528, 1024, 3, false},
+      {2039, 320, 1024, 0, false}, {2040, 320, 1024, 0, true},  {2047, 144, 1024, 0, true},  {2040, 528, 1024, 0, false},
       {1024, 384, 1024, 0, false}, {1024, 400, 1024, 0, false}, {1024, 512, 1024, 0, true},  {1024, 624, 1024, 3, false},
       {1024, 640, 1024, 0, true},  {1024, 784, 1024, 0, false}, {1024, 896, 1024, 3, true},  {1024, 1024, 1024, 0, false},
-      {1024, 144, 1024, 3, false}, {2112, 128, 1024, 0, false},
+      {1024, 144, 1024, 3, false}, {1016, 496, 1024, 0, false}, {2112, 128, 1024, 0, false},
   };
   for (const auto& k : cases) {
     Context c;
