@@ -221,7 +221,7 @@ __device__ __forceinline__ void PackTranspose32(const PackJob& job, int k_span, 
 // launch in front that cleared the words): the product does, as for operands
 // used in place. Calls with both packed, as up to four launches in front of the
 // product -> as one: 1000 x 1500 x 700 int8 with one side transposed 20.4 ->
-// 13.3 us, 64 x 147 x 12544 uint8 13.5 -> 9.8 us, 256 x 1968 x 645 uint8 20.9 ->
+// 13.0 us, 64 x 147 x 12544 uint8 13.5 -> 9.8 us, 256 x 1968 x 645 uint8 20.9 ->
 // 13.8 us. The first `first` workgroups take the first operand.
 struct PackLaunch {
   PackJob job[2];
