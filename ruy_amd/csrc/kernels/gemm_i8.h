@@ -176,6 +176,26 @@ hipError_t LaunchGemmI8(hipStream_t stream, const GemmArgs& args, int num_cus);
 constexpr int kGemmI8StagedDepth = 1024;  // what its ring holds
 bool GemmI8StagedIsBetter(const GemmArgs& args, int num_cus, int depth, bool in_place);
 hipError_t LaunchGemmI8Staged(hipStream_t stream, const GemmArgs& args);
+// 32x32 tiles with operands of any layout and alignment, read where they lie
+// (small_gemm.h): how each operand lies, and how the depth is dealt out.
+enum SmallGemmSource { kSmallRows, kSmallRowsBytes, kSmallAcross, kSmallAcrossBytes };
+struct SmallGemmPlan {
+  int waves = 0;   // of a workgroup; 0: not for the small tiles
+  int step = 128;  // bytes of depth
+  int source_a = kSmallRows, source_b = kSmallRows;
+};
+// Uses of GemmArgs: k_valid is the depth in bytes (at least 16), lda and ldb the
+// bytes from one vector to the next, or across the vectors from one depth
+// position to the next; both operands have at least 16 vectors, whose extent is
+// below 2 GiB; no depth split; pending sums are formed by the launch
+// (fused_a_factor, fused_b_factor).
+// The plan for a product (args as above) that is better on these tiles than on
+// the others, with `packed_bytes` of operands packed in front of those; waves =
+// 0 for any other. `plan` comes with the sources.
+SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes);
+SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes);
+hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan);
+hipError_t LaunchSmallGemmF32(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan);
 // `count` <= kGemmBatchMax products of the shape and parameters of `args`, each
 // on its own buffers, in one launch. Only for arguments that run on the
 // smallest tile (GemmI8CanFuseSums), without sums arrays (zero points 0, or the

@@ -1,0 +1,504 @@
+// Matrix-core GEMM for products whose run time is that of a launch, a trip to
+// memory and a write-back: 32x32 tiles, so that few destination values still
+// keep every CU busy, and operands of any layout and alignment read where they
+// lie, so that no pack launch stands in front.
+//
+// One workgroup per tile. The depth is dealt to its waves in steps of S bytes:
+// wave w takes steps w, w + kWaves, ..., computes the whole tile for them and
+// never waits for another wave until the partial tiles are added through LDS.
+// The loads of a step go through registers (in flight while the steps before
+// are multiplied) into a slot of LDS that is the wave's own, where an operand
+// lies depth-contiguous with its 16-byte granules XOR-swizzled by the row
+// number, and from there to the matrix instructions. On the way:
+//   kSmallRows         rows of depth-contiguous values that start at multiples
+//                      of 4 bytes: one 16-byte load a granule;
+//   kSmallRowsBytes    ... at any byte: the aligned dwords that hold the
+//                      granule, four in one load and the fifth in another,
+//                      shifted into place (a 16-byte load at an odd address
+//                      takes a CU's address unit four times as long);
+//   kSmallAcross       values contiguous along the vectors (the transposed
+//                      storage order): a lane loads 16 bytes of vectors at
+//                      each of four depth positions and transposes them in its
+//                      registers;
+//   kSmallAcrossBytes  ... at any byte.
+// uint8 data becomes int8 there (the top bit flipped) and what lies past the
+// end of the depth zero. Pending depth sums (zero points) come from the
+// fragments, a v_dot4 per dword, and are added through LDS like the tiles.
+#ifndef RUY_AMD_CSRC_KERNELS_SMALL_GEMM_H_
+#define RUY_AMD_CSRC_KERNELS_SMALL_GEMM_H_
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "../epilogue.h"
+#include "gemm_i8.h"
+#include "granule.h"
+
+namespace ruyamd {
+namespace small_gemm {
+
+using granule::LowBytes;
+using granule::PlaceGranule;
+using granule::v4i;
+typedef v4i v4i_dwords __attribute__((aligned(4)));
+
+constexpr int kTile = 32;  // rows and columns
+
+RUYAMD_HOST_DEVICE constexpr bool IsAcross(int source) {
+  return source == kSmallAcross || source == kSmallAcrossBytes;
+}
+RUYAMD_HOST_DEVICE constexpr bool IsAnyByte(int source) {
+  return source == kSmallRowsBytes || source == kSmallAcrossBytes;
+}
+
+// Granule g of vector r of a slot whose vectors are S bytes: 16 consecutive
+// vectors at one granule index lie in 16 different groups of four banks.
+template <int S>
+__device__ __forceinline__ int SlotOffset(int r, int g) {
+  static_assert(S == 64 || S == 128, "");
+  return r * S + ((g ^ (S == 64 ? (r >> 2) & 3 : (r >> 1) & 7)) << 4);
+}
+
+// The kTile vectors of one operand that a tile needs, from vector `first` on.
+template <int S, int kSource, int kElement>
+struct Side {
+  static constexpr bool kAcross = IsAcross(kSource);
+  static constexpr bool kAnyByte = IsAnyByte(kSource);
+  static constexpr int kGranules = S / 16;
+  // Across the vectors: a piece is 16 bytes of vectors (16 or 4 of them) at
+  // four depth positions (4 or 16 bytes of depth).
+  static constexpr int kVectors = 16 / kElement;
+  static constexpr int kPieceDepth = 4 * kElement;
+  static constexpr int kGroups = kTile / kVectors;
+  // What a step's work comes to a lane: granules, or pieces.
+  static constexpr int kAll = kAcross ? kGroups * (S / kPieceDepth) : kTile * kGranules;
+  static constexpr int kUnits = (kAll + 63) / 64;
+  static constexpr int kLoads = kAcross ? 4 : 1;  // of a unit
+
+  const char* data;
+  int pitch, count, first, bytes;
+  uint32_t flip;
+  int lane;
+  uint32_t offset[kUnits];  // of the unit's vector (first vector)
+
+  struct Held {
+    v4i x[kUnits][kLoads];
+    int fifth[kUnits][kAnyByte ? kLoads : 1];
+  };
+
+  __device__ __forceinline__ bool Exists(int u) const { return kAll % 64 == 0 || u * 64 + lane < kAll; }
+  // Vector (first vector) of unit u, counted inside the tile, and its first
+  // byte of depth, counted inside a step.
+  __device__ __forceinline__ int VectorOf(int u) const {
+    const int p = u * 64 + lane;
+    return kAcross ? p % kGroups * kVectors : p / kGranules;
+  }
+  __device__ __forceinline__ int DepthOf(int u) const {
+    const int p = u * 64 + lane;
+    return kAcross ? p / kGroups * kPieceDepth : p % kGranules * 16;
+  }
+  __device__ __forceinline__ void Start(const void* d, int pitch_, int count_, int first_, int bytes_, uint32_t flip_,
+                                        int lane_) {
+    data = static_cast<const char*>(d);
+    pitch = pitch_;
+    count = count_;
+    first = first_;
+    bytes = bytes_;
+    flip = flip_;
+    lane = lane_;
+    // Vectors past the end read the last one; nothing of them is stored.
+    // (Across them: the 16 bytes that end with the last one, moved into place
+    // in Store.)
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u)
+      offset[u] = kAcross ? uint32_t(min(first + VectorOf(u), count - kVectors) * kElement)
+                          : uint32_t(min(first + VectorOf(u), count - 1)) * uint32_t(pitch);
+  }
+
+  // Where load j of unit u of a step reads.
+  __device__ __forceinline__ const char* From(int step, int u, int j) const {
+    const int k = step * S + DepthOf(u);
+    // A granule that reaches past the end of its vector: the 16 bytes that end
+    // there, moved down in Store.
+    if constexpr (!kAcross) return data + (offset[u] + uint32_t(min(k, bytes - 16)));
+    // Depth positions past the end read the last one and become zero in Store.
+    return data + (uint32_t(min(k / kElement + j, bytes / kElement - 1)) * uint32_t(pitch) + offset[u]);
+  }
+  // kAnyByte: whether the fifth dword of a lane's 16 bytes is loaded. Of a row it
+  // mostly is the first one of the next lane's, whose 16 bytes follow in memory:
+  // not at the end of a run of lanes, nor in the step that the depth ends in,
+  // whose last granule is read from elsewhere than its place. (512 tiles of 4097
+  // bytes of depth: 16.9 us with every lane's loaded, 15.3 so. Across the vectors
+  // a run is two lanes: 256 tiles 11.9 us, 15.1 so.)
+  __device__ __forceinline__ bool LoadsFifth(int step, int u) const {
+    return kAcross || (step + 1) * S > bytes || DepthOf(u) == S - 16;
+  }
+  __device__ __forceinline__ void Load(int step, Held& h) const {
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      if (!Exists(u)) continue;
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        const char* from = From(step, u, j);
+        if constexpr (!kAnyByte) {
+          h.x[u][j] = *reinterpret_cast<const v4i_dwords*>(from);
+        } else {
+          const int shift = static_cast<int>(reinterpret_cast<uintptr_t>(from) & 3);
+          h.x[u][j] = *reinterpret_cast<const v4i_dwords*>(from - shift);
+        }
+      }
+      if constexpr (kAnyByte) {
+        if (LoadsFifth(step, u)) {
+#pragma unroll
+          for (int j = 0; j < kLoads; ++j) {
+            const char* from = From(step, u, j);
+            const int shift = static_cast<int>(reinterpret_cast<uintptr_t>(from) & 3);
+            h.fifth[u][j] = *reinterpret_cast<const int*>(from - shift + (shift ? 16 : 12));
+          }
+        }
+      }
+    }
+  }
+
+  // Puts what Load has fetched of `step` into the slot.
+  __device__ __forceinline__ void Store(int step, const Held& h, char* slot) const {
+    const bool partial = (step + 1) * S > bytes;  // (wave-uniform)
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      if (!Exists(u)) continue;
+      const int k = step * S + DepthOf(u);
+      v4i x[kLoads];
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        x[j] = h.x[u][j];
+        if constexpr (kAnyByte) {
+          const uint32_t shift = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(From(step, u, j)) & 3);
+          int fifth = h.fifth[u][j];
+          if constexpr (!kAcross) {
+            // (row_shl:1: from the next lane of the 16.)
+            const int next = __builtin_amdgcn_update_dpp(0, h.x[u][j][0], 0x101, 0xf, 0xf, false);
+            if (!LoadsFifth(step, u)) fifth = next;
+          }
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            x[j][d] = static_cast<int>(__builtin_amdgcn_alignbyte(d < 3 ? h.x[u][j][d + 1] : fifth, h.x[u][j][d], shift));
+        }
+        if constexpr (kAcross) {
+          if (first + kTile > count) x[j] = PlaceGranule(x[j], (first + VectorOf(u)) * kElement, count * kElement);
+        }
+        if constexpr (kElement == 1) x[j] ^= static_cast<int>(flip);
+      }
+      const int vector = VectorOf(u);
+      if constexpr (!kAcross) {
+        if (partial) {
+          // (The flip of the padding is taken back by the mask.)
+          if constexpr (kElement == 1) x[0] ^= static_cast<int>(flip);
+          x[0] = PlaceGranule(x[0], k, bytes);
+#pragma unroll
+          for (int d = 0; d < 4; ++d) x[0][d] ^= static_cast<int>(flip & LowBytes(bytes - k - 4 * d));
+        }
+        *reinterpret_cast<v4i*>(slot + SlotOffset<S>(vector, DepthOf(u) / 16)) = x[0];
+      } else if constexpr (kElement == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v4i y = {x[0][i], x[1][i], x[2][i], x[3][i]};
+          if (partial) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) y[d] = k + 4 * d < bytes ? y[d] : 0;
+          }
+          *reinterpret_cast<v4i*>(slot + SlotOffset<S>(vector + i, DepthOf(u) / 16)) = y;
+        }
+      } else {
+        const uint32_t valid = partial ? LowBytes(bytes - k) : 0xffffffffu;
+#pragma unroll
+        for (int quad = 0; quad < 4; ++quad) {
+          // 4 x 4 bytes: t[i] = four depth positions of vector 4 * quad + i.
+          const uint32_t x0 = __builtin_amdgcn_perm(x[1][quad], x[0][quad], 0x05010400u);
+          const uint32_t x1 = __builtin_amdgcn_perm(x[1][quad], x[0][quad], 0x07030602u);
+          const uint32_t y0 = __builtin_amdgcn_perm(x[3][quad], x[2][quad], 0x05010400u);
+          const uint32_t y1 = __builtin_amdgcn_perm(x[3][quad], x[2][quad], 0x07030602u);
+          const uint32_t t[4] = {__builtin_amdgcn_perm(y0, x0, 0x05040100u), __builtin_amdgcn_perm(y0, x0, 0x07060302u),
+                                 __builtin_amdgcn_perm(y1, x1, 0x05040100u), __builtin_amdgcn_perm(y1, x1, 0x07060302u)};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<uint32_t*>(slot + SlotOffset<S>(vector + 4 * quad + i, DepthOf(u) / 16) + DepthOf(u) % 16) =
+                t[i] & valid;
+        }
+      }
+    }
+  }
+};
+
+// LDS of a workgroup: the waves' slots, and later in the same memory their
+// partial tiles (16 bytes - four consecutive rows of a column - at a time, in
+// runs of 32 columns padded by one so that a column's pieces lie in different
+// banks); behind that the partial sums of the tile's vectors and the
+// write-back parameters of its rows and columns.
+template <int S, int kWaves>
+struct Memory {
+  static constexpr int kVectors = 2 * kTile;
+  static constexpr int kSlot = kVectors * S;
+  static constexpr int kPart = 8 * 33;  // granules of a wave's partial tile
+  static constexpr int kSums = std::max(kWaves * kSlot, kWaves * kPart * 16);
+  static constexpr int kParams = kSums + kWaves * kVectors * 4;
+  static constexpr int kBytes = kParams + 3 * kVectors * 4;
+};
+
+template <typename T, int S, int kWaves, int kSourceA, int kSourceB>
+__global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void SmallGemmKernel(GemmArgs args) {
+  using Mem = Memory<S, kWaves>;
+  constexpr int kSubSteps = S / 32;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+
+  // The tile: every XCD (workgroups go to them round-robin) gets a contiguous
+  // run of the tiles, in bands of four tile rows, so that those it holds share
+  // operand panels in its L2.
+  const int tiles_m = (args.M + kTile - 1) / kTile;
+  const int tiles_n = (args.N + kTile - 1) / kTile;
+  const int total = tiles_m * tiles_n;
+  const int per_xcd = (total + 7) / 8;
+  const int t = int(blockIdx.x % 8) * per_xcd + int(blockIdx.x / 8);
+  if (t >= total) return;
+  constexpr int kGroupM = 4;
+  const int band = t / (kGroupM * tiles_n);
+  const int band_rows = min(kGroupM, tiles_m - band * kGroupM);
+  const int in_band = t - band * kGroupM * tiles_n;
+  const int m0 = (band * kGroupM + in_band % band_rows) * kTile;
+  const int n0 = in_band / band_rows * kTile;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int K = args.k_valid;  // depth in bytes
+  const int steps = (K + S - 1) / S;
+  const int my_steps = steps > wave ? (steps - wave + kWaves - 1) / kWaves : 0;
+
+  using SideA = Side<S, kSourceA, T::kElement>;
+  using SideB = Side<S, kSourceB, T::kElement>;
+  SideA a;
+  SideB b;
+  a.Start(args.a, args.lda, args.M, m0, K, args.a_flip, lane);
+  b.Start(args.b, args.ldb, args.N, n0, K, args.b_flip, lane);
+  // Steps whose loads are in flight (16 waves: 128 registers a lane).
+  constexpr int kAhead = kWaves > 8 ? 1 : 2;
+  typename SideA::Held held_a[kAhead];
+  typename SideB::Held held_b[kAhead];
+  auto load = [&](int i, auto at) {
+    a.Load(wave + kWaves * i, held_a[decltype(at)::value]);
+    b.Load(wave + kWaves * i, held_b[decltype(at)::value]);
+  };
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, kAhead - 1>;
+  if (my_steps > 0) load(0, First());
+  if (kAhead > 1 && my_steps > 1) load(1, Second());
+
+  // What the write-back needs of the tile's rows and columns: fetched here,
+  // a vector a thread, and used after the last step.
+  typename T::Params params;
+  const bool is_row = tid < kTile;
+  if (tid < Mem::kVectors)
+    T::LoadParams(args.ep, is_row, is_row ? min(m0 + tid, args.M - 1) : min(n0 + tid - kTile, args.N - 1), params);
+
+  // (fp32: several accumulators in turn, so that the chains of additions are no
+  // longer than where a depth is split over workgroups: four of eight waves, two
+  // where there are more waves or the registers decide how many workgroups a CU
+  // holds. Against 64 bits, 256 x 2048 x 256: split 2.1e-7, here 1.6e-7.)
+  constexpr int kChains = T::kElement == 1 ? 1 : kWaves == 8 ? 4 : 2;
+  typename T::Acc acc[kChains];
+#pragma unroll
+  for (int c = 0; c < kChains; ++c)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[c][v] = 0;
+  int sum_a = 0, sum_b = 0;
+  const bool sums_of_a = T::kElement == 1 && args.fused_a_factor != 0;
+  const bool sums_of_b = T::kElement == 1 && args.fused_b_factor != 0;
+
+  char* const slot = lds + wave * Mem::kSlot;
+  auto step_of = [&](int i, auto at) {
+    const int step = wave + kWaves * i;
+    a.Store(step, held_a[decltype(at)::value], slot);
+    b.Store(step, held_b[decltype(at)::value], slot + kTile * S);
+    if (i + kAhead < my_steps) load(i + kAhead, at);
+    // (Written and read by this wave only, whose LDS operations are performed
+    // in order.)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    v4i fa[kSubSteps], fb[kSubSteps];
+#pragma unroll
+    for (int ks = 0; ks < kSubSteps; ++ks) {
+      const int offset = SlotOffset<S>(lane & 31, ks * 2 + lane / 32);
+      fa[ks] = *reinterpret_cast<const v4i*>(slot + offset);
+      fb[ks] = *reinterpret_cast<const v4i*>(slot + kTile * S + offset);
+    }
+#pragma unroll
+    for (int ks = 0; ks < kSubSteps; ++ks) T::Mma(fa[ks], fb[ks], acc, ks);
+    if (sums_of_a) {
+#pragma unroll
+      for (int ks = 0; ks < kSubSteps; ++ks)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) sum_a = __builtin_amdgcn_sdot4(fa[ks][d], 0x01010101, sum_a, false);
+    }
+    if (sums_of_b) {
+#pragma unroll
+      for (int ks = 0; ks < kSubSteps; ++ks)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) sum_b = __builtin_amdgcn_sdot4(fb[ks][d], 0x01010101, sum_b, false);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  if constexpr (kAhead == 1) {
+    for (int i = 0; i < my_steps; ++i) step_of(i, First());
+  } else {
+    int i = 0;
+    for (; i + 1 < my_steps; i += 2) {
+      step_of(i, First());
+      step_of(i + 1, Second());
+    }
+    if (i < my_steps) step_of(i, First());
+  }
+
+  // ---- the partial tiles, added through LDS ----
+  __syncthreads();  // every wave is done with its slot
+  v4i* const parts = reinterpret_cast<v4i*>(lds);
+  int* const sums = reinterpret_cast<int*>(lds + Mem::kSums);
+  int* const area = reinterpret_cast<int*>(lds + Mem::kParams);
+  if (my_steps > 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v4i w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        typename T::Value sum = acc[0][4 * q + e];
+        if constexpr (kChains == 2) sum += acc[1][4 * q + e];
+        if constexpr (kChains == 4) sum = (sum + acc[1][4 * q + e]) + (acc[2][4 * q + e] + acc[3][4 * q + e]);
+        w[e] = T::Bits(sum);
+      }
+      // Rows 8 q + 4 (lane / 32) .. + 3 of column lane % 32.
+      parts[wave * Mem::kPart + (2 * q + lane / 32) * 33 + (lane & 31)] = w;
+    }
+    // Lanes l and l + 32 hold the two halves of a vector's sum.
+    auto put = [&](int value, int vector) {
+      const auto halves = __builtin_amdgcn_permlane32_swap(value, value, false, false);
+      if (lane < 32) sums[wave * Mem::kVectors + vector + lane] = halves[0] + halves[1];
+    };
+    if (sums_of_a) put(sum_a, 0);
+    if (sums_of_b) put(sum_b, kTile);
+  }
+  if (tid < Mem::kVectors) T::StageParams(args.ep, is_row, params, area + tid, Mem::kVectors);
+  __syncthreads();
+
+  // A thread finishes four consecutive rows of a column.
+  if (tid >= kTile * kTile / 4) return;
+  const int row = tid % 8 * 4, col = tid / 8;
+  const int active = min(steps, kWaves);
+  typename T::Value value[4] = {0, 0, 0, 0};
+  uint32_t of_column = 0, of_row[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < active) {
+      const v4i x = parts[w * Mem::kPart + row / 4 * 33 + col];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) value[e] += T::FromBits(x[e]);
+      if (sums_of_a) {
+        const v4i s = *reinterpret_cast<const v4i*>(sums + w * Mem::kVectors + row);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) of_row[e] += static_cast<uint32_t>(s[e]);
+      }
+      if (sums_of_b) of_column += static_cast<uint32_t>(sums[w * Mem::kVectors + kTile + col]);
+    }
+  }
+  if constexpr (T::kElement == 1) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      value[e] = static_cast<int>(static_cast<uint32_t>(value[e]) - static_cast<uint32_t>(args.fused_a_factor) * of_row[e] -
+                                  static_cast<uint32_t>(args.fused_b_factor) * of_column);
+  }
+  int vals[4];
+  T::Finish(value, area, Mem::kVectors, row, kTile + col, args.ep, vals);
+  const int i0 = m0 + row, j = n0 + col;
+  if (j >= args.N || i0 >= args.M) return;
+  char* const out = static_cast<char*>(args.dst.data) + (int64_t(j) * args.dst.cs + i0) * args.dst_elt;
+  // (Stores of any width take any address.)
+  if (i0 + 4 <= args.M) {
+    if (args.dst_elt == 1) {
+      const uint32_t w = uint32_t(vals[0] & 0xff) | uint32_t(vals[1] & 0xff) << 8 | uint32_t(vals[2] & 0xff) << 16 |
+                         uint32_t(vals[3]) << 24;
+      __builtin_memcpy(out, &w, sizeof(w));
+    } else if (args.dst_elt == 2) {
+      const uint32_t w[2] = {uint32_t(vals[0] & 0xffff) | uint32_t(vals[1]) << 16,
+                             uint32_t(vals[2] & 0xffff) | uint32_t(vals[3]) << 16};
+      __builtin_memcpy(out, w, sizeof(w));
+    } else {
+      __builtin_memcpy(out, vals, sizeof(vals));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      if (i0 + e < args.M) {
+        if (args.dst_elt == 1)
+          reinterpret_cast<int8_t*>(out)[e] = static_cast<int8_t>(vals[e]);
+        else if (args.dst_elt == 2)
+          reinterpret_cast<int16_t*>(out)[e] = static_cast<int16_t>(vals[e]);
+        else
+          reinterpret_cast<int32_t*>(out)[e] = vals[e];
+      }
+    }
+  }
+}
+
+template <typename T, int S, int kWaves, int kSourceA, int kSourceB>
+hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
+  using Mem = Memory<S, kWaves>;
+  // (Rows: a granule must fit; across: 16 bytes of vectors.)
+  if (args.k_valid < 16 || args.M < 16 || args.N < 16 || args.split_k != 1 || args.row_sums) return hipErrorInvalidValue;
+  const int64_t total = int64_t((args.M + kTile - 1) / kTile) * ((args.N + kTile - 1) / kTile);
+  if (total > (1 << 24)) return hipErrorInvalidValue;
+  const int grid = static_cast<int>((total + 7) / 8 * 8);
+  auto kernel = SmallGemmKernel<T, S, kWaves, kSourceA, kSourceB>;
+  if (Mem::kBytes > 48 * 1024) {
+    // Once per process; static initialisation is safe against concurrent callers.
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, Mem::kBytes);
+    if (attr != hipSuccess) return attr;
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kWaves), Mem::kBytes, stream, args);
+  return hipGetLastError();
+}
+
+// The instantiation for a plan. Operands at any byte: both sides' byte forms
+// (which read aligned ones as well).
+template <typename T, int S, int kWaves>
+hipError_t LaunchSources(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
+  const bool across_a = IsAcross(plan.source_a), across_b = IsAcross(plan.source_b);
+  const bool bytes = IsAnyByte(plan.source_a) || IsAnyByte(plan.source_b);
+  if constexpr (T::kElement == 1) {
+    if (bytes) {
+      if (across_a && across_b) return Launch<T, S, kWaves, kSmallAcrossBytes, kSmallAcrossBytes>(stream, args);
+      if (across_a) return Launch<T, S, kWaves, kSmallAcrossBytes, kSmallRowsBytes>(stream, args);
+      if (across_b) return Launch<T, S, kWaves, kSmallRowsBytes, kSmallAcrossBytes>(stream, args);
+      return Launch<T, S, kWaves, kSmallRowsBytes, kSmallRowsBytes>(stream, args);
+    }
+  }
+  if (bytes) return hipErrorInvalidValue;
+  if (across_a && across_b) return Launch<T, S, kWaves, kSmallAcross, kSmallAcross>(stream, args);
+  if (across_a) return Launch<T, S, kWaves, kSmallAcross, kSmallRows>(stream, args);
+  if (across_b) return Launch<T, S, kWaves, kSmallRows, kSmallAcross>(stream, args);
+  return Launch<T, S, kWaves, kSmallRows, kSmallRows>(stream, args);
+}
+template <typename T>
+hipError_t LaunchPlan(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
+  if (plan.step == 64 && plan.waves == 4) return LaunchSources<T, 64, 4>(stream, args, plan);
+  if (plan.step == 64 && plan.waves == 8) return LaunchSources<T, 64, 8>(stream, args, plan);
+  if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 128, 4>(stream, args, plan);
+  if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 128, 8>(stream, args, plan);
+  if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 128, 16>(stream, args, plan);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace small_gemm
+}  // namespace ruyamd
+
+#endif  // RUY_AMD_CSRC_KERNELS_SMALL_GEMM_H_

@@ -1,0 +1,93 @@
+// The GEMM on 32x32 tiles (small_gemm.h) for fp32.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "mfma_gemm.h"
+#include "small_gemm.h"
+
+namespace ruyamd {
+namespace {
+
+using granule::v4i;
+
+struct F32Small {
+  using Acc = mfma_gemm::v16f;
+  using Value = float;
+  static constexpr int kElement = 4;
+  // A granule holds four consecutive depth values of a vector.
+  template <int kChains>
+  static __device__ __forceinline__ void Mma(const v4i& a, const v4i& b, Acc (&acc)[kChains], int sub_step) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      Acc& to = acc[kChains == 4 ? sub_step % 2 * 2 + e % 2 : sub_step % kChains];
+      to = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(a[e]), __int_as_float(b[e]), to, 0, 0, 0);
+    }
+  }
+  static __device__ __forceinline__ int Bits(float x) { return __float_as_int(x); }
+  static __device__ __forceinline__ float FromBits(int x) { return __int_as_float(x); }
+
+  struct Params {
+    float bias;
+  };
+  static __device__ __forceinline__ void LoadParams(const Epilogue& ep, bool is_row, int index, Params& p) {
+    p.bias = is_row != (ep.channel_is_col != 0) && ep.bias ? static_cast<const float*>(ep.bias)[index] : 0.f;
+  }
+  static __device__ __forceinline__ void StageParams(const Epilogue&, bool, const Params& p, int* at, int) {
+    at[0] = __float_as_int(p.bias);
+  }
+  static __device__ __forceinline__ void Finish(const float (&total)[4], const int* area, int, int row, int col,
+                                                const Epilogue& ep, int (&vals)[4]) {
+    const float column_bias = __int_as_float(area[col]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = total[e];
+      if (ep.bias) v = v + (ep.channel_is_col ? column_bias : __int_as_float(area[row + e]));
+      v = ep.clamp_max_f < v ? ep.clamp_max_f : v;
+      v = v < ep.clamp_min_f ? ep.clamp_min_f : v;
+      vals[e] = __float_as_int(v);
+    }
+  }
+};
+
+}  // namespace
+
+// The time of these tiles by a fit to 16 to 1536 of them and depths of 16 to 2048
+// (within 10 % mostly): 3.9 us, 0.33 us for every tile a CU has beyond the first,
+// and 1.25 us to a KiB of depth and tile (their matrix instructions at two thirds
+// of their rate), 1.3 where an operand is transposed on the way. Held against
+// the other tiles' timing model and a pack in front of them: us, other route ->
+// this, 512^3 12.8 -> 6.0; 512 tiles in place x 512 13.2 -> 8.6, x 2048 23.9 -> 23.5;
+// 1024 x 256 10.7 -> 8.9, x 1024 22.1 -> 23.1; 256 tiles with one side transposed x
+// 1024 19.7 -> 9.2, both 21.8 -> 9.4; 1536 x 1024 43.4 -> 36.6, both 47.6 -> 39.5.
+SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
+  const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
+  const int K = args.k_valid;
+  const bool across = small_gemm::IsAcross(plan.source_a) || small_gemm::IsAcross(plan.source_b);
+  plan.waves = 0;
+  if (K < 16 || tiles > 6 * num_cus) return plan;
+  const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
+  const double here = 3.9 + 0.33 * (a_cu - 1) + (across ? 1.3 : 1.25) * a_cu * K / 1024.0;
+  const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kF32);
+  double other = 1e30;
+  for (int i = 0; i < model.count; ++i)
+    other = std::min(other, mfma_gemm::ModelledMicroseconds(args, num_cus, model, model.tiles[i]));
+  if (packed_bytes) other += 2.3 + 0.5e-6 * static_cast<double>(packed_bytes);
+  if (here >= other) return plan;
+  plan.waves = 4;
+  plan.step = 64;
+  if (a_cu == 1) {
+    plan.waves = K > 256 ? 8 : 4;
+    if (across && K >= 1024) plan.step = 128;
+    if (across && K >= 4096) plan.waves = 16;
+  } else if (across ? K >= 512 || a_cu == 2 : K >= 4096 && a_cu > 2) {
+    plan.step = 128;
+  }
+  return plan;
+}
+
+hipError_t LaunchSmallGemmF32(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
+  return small_gemm::LaunchPlan<F32Small>(stream, args, plan);
+}
+
+}  // namespace ruyamd

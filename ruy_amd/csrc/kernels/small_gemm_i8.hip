@@ -1,0 +1,134 @@
+// The GEMM on 32x32 tiles (small_gemm.h) for 8-bit operands.
+#include <hip/hip_runtime.h>
+
+#include "int8_traits.h"
+#include "small_gemm.h"
+
+namespace ruyamd {
+namespace {
+
+struct Int8Small {
+  using Acc = mfma_gemm::v16i;
+  using Value = int;
+  static constexpr int kElement = 1;
+  static __device__ __forceinline__ void Mma(const v4i& a, const v4i& b, Acc (&acc)[1], int) {
+    acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc[0], 0, 0, 0);
+  }
+  static __device__ __forceinline__ int Bits(int x) { return x; }
+  static __device__ __forceinline__ int FromBits(int x) { return x; }
+
+  // Of one row or column: bias, the other side's zero point's share if its sums
+  // are at hand, multiplier and exponent if the channels run that way.
+  struct Params {
+    int32_t bias, sum, m, e;
+  };
+  static __device__ __forceinline__ void LoadParams(const Epilogue& ep, bool is_row, int index, Params& p) {
+    const bool channel = is_row != (ep.channel_is_col != 0);
+    const int32_t* sums = is_row ? ep.lhs_sums : ep.rhs_sums;
+    p.bias = channel && ep.bias ? static_cast<const int32_t*>(ep.bias)[index] : 0;
+    p.sum = (is_row ? ep.rhs_zero_point : ep.lhs_zero_point) && sums ? sums[index] : 0;
+    p.m = channel && ep.mult_fixedpoint ? ep.mult_fixedpoint[index] : ep.mult_fixedpoint_scalar;
+    p.e = channel && ep.mult_fixedpoint ? ep.mult_exponent[index] : ep.mult_exponent_scalar;
+  }
+  static __device__ __forceinline__ void StageParams(const Epilogue& ep, bool is_row, const Params& p, int* at, int stride) {
+    const uint32_t zero_point = static_cast<uint32_t>(is_row ? ep.rhs_zero_point : ep.lhs_zero_point);
+    at[0] = static_cast<int32_t>(static_cast<uint32_t>(p.bias) - zero_point * static_cast<uint32_t>(p.sum) +
+                                 (is_row ? static_cast<uint32_t>(ep.zp_product_depth) : 0u));
+    at[stride] = p.m;
+    at[2 * stride] = p.e;
+  }
+  static __device__ __forceinline__ void Finish(const int (&total)[4], const int* area, int stride, int row, int col,
+                                                const Epilogue& ep, int (&vals)[4]) {
+    const int column_add = area[col];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      vals[e] = static_cast<int>(static_cast<uint32_t>(total[e]) + static_cast<uint32_t>(area[row + e]) +
+                                 static_cast<uint32_t>(column_add));
+    if (ep.requantize && !ep.mult_fixedpoint && ep.mult_exponent_scalar <= -2) {
+      const int high_shift = -1 - ep.mult_exponent_scalar;  // (31 - e) - 32
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vals[e] = RequantHigh(vals[e], ep.mult_fixedpoint_scalar, high_shift);
+    } else if (ep.requantize) {
+      if (ep.channel_is_col) {
+        const int m = area[stride + col], exponent = area[2 * stride + col];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vals[e] = MultiplyByQuantizedMultiplier(vals[e], m, exponent);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          vals[e] = MultiplyByQuantizedMultiplier(vals[e], area[stride + row + e], area[2 * stride + row + e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      vals[e] = Median3(static_cast<int32_t>(static_cast<uint32_t>(vals[e]) + static_cast<uint32_t>(ep.dst_zero_point)),
+                        ep.clamp_min_i, ep.clamp_max_i);
+  }
+};
+
+}  // namespace
+
+// What the tiles of 32x32 win on is the time that does not depend on the work:
+// no pack launch (2.5 us and more), a quarter of the loads, of the adding up and
+// of the write-back of a 64x64 tile to a workgroup. What they lose is reuse: they
+// read an operand byte twice as often. So the lines run along tiles to a CU, with
+// a limit on the depth from where the two sides met on a grid of depths (64 to
+// 8192) and of 16 to 1536 tiles (us, other route -> this):
+//   used in place: 256 tiles x 512 5.2 -> 3.9, x 1024 6.8 -> 4.4, x 8192 11.8 -> 10.1;
+//     512 x 2048 8.0 -> 6.8, x 4096 10.3 -> 9.5, x 8192 14.3 -> 16.1; 768 x 1024
+//     6.9 -> 6.1, x 2048 7.9 -> 8.2; 1024 x 512 5.5 -> 5.5.
+//   packed by rows otherwise: 256 x 257 6.1 -> 4.5, x 2049 12.9 -> 7.8, x 8193 23.1 ->
+//     15.3; 512 x 1025 10.3 -> 7.5, x 4097 18.2 -> 15.3; 768 x 1025 10.7 -> 9.1, x
+//     4097 20.5 -> 19.6; 1024 x 65 5.0 -> 4.9, x 513 7.7 -> 8.0.
+//   one side transposed, at whole dwords: 256 x 512 8.2 -> 4.4, x 8192 19.0 -> 15.2; 512 x
+//     4096 16.4 -> 15.3; 768 x 1024 10.0 -> 9.4; 1024 x 512 8.5 -> 7.6, x 1024 10.1 ->
+//     11.4; 1536 x 256 9.0 -> 7.7, x 512 10.1 -> 10.5.
+//   ... and at odd bytes: 256 x 8192 22.5 -> 21.5; 512 x 2048 13.4 -> 12.4, x 4096
+//     19.3 -> 20.8; 768 x 512 8.9 -> 8.1, x 1024 11.4 -> 11.5; 1024 x 128 7.4 -> 7.1.
+// More waves to a workgroup, or longer steps, where the grid leaves CUs room for
+// them: 256 tiles in place x 1024 4.8 with four waves, 4.4 with eight, packed x 8193
+// 20.3 with eight, 15.3 with sixteen.
+SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
+  const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
+  const int K = args.k_valid;
+  const bool across = small_gemm::IsAcross(plan.source_a) || small_gemm::IsAcross(plan.source_b);
+  const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b);
+  const int a_cu = tiles <= num_cus ? 1 : tiles <= 2 * num_cus ? 2 : 4 * tiles <= 13 * num_cus ? 3 : tiles <= 4 * num_cus ? 4 : 6;
+  int deepest = 0;
+  if (tiles > 6 * num_cus || K < 16) {
+    deepest = 0;
+  } else if (across) {
+    deepest = a_cu == 1 ? 8192 : a_cu == 2 ? (bytes ? 2048 : 4096) : a_cu == 3 ? (bytes ? 512 : 1024)
+              : a_cu == 4 ? (bytes ? 128 : 512) : 256;
+  } else if (packed_bytes) {
+    deepest = a_cu == 1 ? 8192 : a_cu <= 3 ? 4100 : a_cu == 4 ? 128 : 0;
+  } else {
+    deepest = a_cu == 1 ? 8192 : a_cu == 2 ? 4096 : a_cu == 3 ? 1024 : 0;
+  }
+  plan.waves = 0;
+  if (K > deepest) return plan;
+  plan.waves = 4;
+  plan.step = 64;
+  if (a_cu == 1) {
+    plan.waves = K > 256 ? 8 : 4;
+    if (across || !bytes) plan.step = K >= 512 ? 128 : 64;
+    if (across ? K >= 4096 : bytes && K >= 2048) {
+      plan.waves = 16;
+      plan.step = 128;
+    }
+  } else if (across) {
+    if (a_cu == 2) plan.step = 128;
+  } else if (bytes) {
+    if (a_cu == 2 && K > 128) plan.waves = 8;
+    if (a_cu == 3 && K >= 2048) plan.step = 128;
+  } else if (K >= 2048) {
+    plan.step = 128;
+  }
+  return plan;
+}
+
+hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
+  return small_gemm::LaunchPlan<Int8Small>(stream, args, plan);
+}
+
+}  // namespace ruyamd

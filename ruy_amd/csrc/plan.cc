@@ -387,6 +387,86 @@ bool SetupInt8Gemm(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, cons
   return swap;
 }
 
+// How an operand lies for the small tiles (small_gemm.h), and its pitch there:
+// false if they cannot read it where it is (an extent that 32-bit offsets do not
+// reach).
+bool SmallSourceOf(const PackSource& src, SmallGemmSource* source, int32_t* pitch, uint32_t* bytes) {
+  const bool rows = src.stride_k == 1;
+  if (!rows && src.stride_c != 1) return false;
+  const int element = DtypeSize(src.dtype);
+  const int64_t stride = (rows ? src.stride_c : src.stride_k) * element;
+  const uint64_t extent =
+      uint64_t((rows ? src.count : src.K) - 1) * uint64_t(stride) + uint64_t(rows ? src.K : src.count) * element;
+  if (extent >= (uint64_t(1) << 31)) return false;
+  const bool dwords = ((reinterpret_cast<uintptr_t>(src.data) | static_cast<uint64_t>(stride)) & 3) == 0;
+  *source = rows ? (dwords ? kSmallRows : kSmallRowsBytes) : (dwords ? kSmallAcross : kSmallAcrossBytes);
+  *pitch = static_cast<int32_t>(stride);
+  *bytes = static_cast<uint32_t>(extent);
+  return true;
+}
+
+// An int8 operand on the small tiles.
+bool AsSmall(const Operand8& op, Operand8* out, SmallGemmSource* source) {
+  *out = op;
+  *source = kSmallRows;
+  if (!op.unpacked) return true;
+  if (!SmallSourceOf(op.src, source, &out->ld, &out->bytes)) return false;
+  out->unpacked = false;
+  out->data = static_cast<const int8_t*>(op.src.data);
+  out->flip = op.src.dtype == RUYAMD_DTYPE_U8 ? kFlipU8 : 0;
+  return true;
+}
+
+// The small tiles need no packed copy of an operand. A call that is recorded or
+// may not allocate is refused all the same where there is no room for one, so
+// that it does not depend on the tiles whether it is; and so that one that has
+// run can be recorded, an ordinary call takes the room (if it can be had).
+bool HasRoomToPack(ruyamd_ctx* ctx, bool unpacked, uint32_t bytes, int32_t sums) {
+  if (!unpacked) return true;
+  bool room = true;
+  for (const std::size_t size : {std::size_t(bytes ? bytes : 16), std::size_t(sums) * 4}) {
+    if (!size) continue;
+    room = (ctx->capturing || ctx->no_alloc ? ctx->ws->Alloc(size) : ctx->ws->AllocOptional(size)) && room;
+  }
+  return room || !(ctx->capturing || ctx->no_alloc);
+}
+
+// The product on the small tiles, where the planner finds that better (*done).
+int RunInt8Small(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
+                 bool* done, std::string* err) {
+  const int K = call.lhs.cols;
+  Operand8 sa, sb;
+  SmallGemmSource source_a, source_b;
+  if (ctx->forced_tile_rows || K < 16 || !AsSmall(a, &sa, &source_a) || !AsSmall(b, &sb, &source_b)) return RUYAMD_OK;
+  GemmArgs args;
+  const bool swap = SetupInt8Gemm(ctx, call, sa, sb, lzp, rzp, /*staged=*/true, &args);
+  args.k_valid = K;
+  SmallGemmPlan plan;
+  plan.source_a = swap ? source_b : source_a;
+  plan.source_b = swap ? source_a : source_b;
+  plan = PlanSmallGemmI8(args, ctx->multiprocessor_count, plan, uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes);
+  if (plan.waves == 0) return RUYAMD_OK;
+  for (const Operand8* op : {&a, &b}) {
+    const bool sums = op->unpacked && op->sums_pending && PackFormsSums(op->src, op->ld);
+    if (!HasRoomToPack(ctx, op->unpacked, op->bytes, sums ? op->count : 0)) {
+      *err = "workspace allocation failed";
+      return RUYAMD_E_HIP;
+    }
+  }
+  args.ep.lhs_sums = (swap ? sb : sa).sums;
+  args.ep.rhs_sums = (swap ? sa : sb).sums;
+  const bool timed = ctx->TimingBegin();
+  const hipError_t launched = LaunchSmallGemmI8(ctx->LaunchStream(), args, plan);
+  if (timed) ctx->TimingEnd();
+  if (launched != hipSuccess) {
+    *err = "int8 MFMA kernel launch failed";
+    return RUYAMD_E_HIP;
+  }
+  ctx->last_kernel = RUYAMD_KERNEL_I8_MFMA;
+  *done = true;
+  return RUYAMD_OK;
+}
+
 // The product on the staged form of the smallest tile, where the planner finds
 // that better (*done): it reads operands that cannot be used in place as they
 // are, without a pack launch in front, and forms pending sums itself.
@@ -439,6 +519,8 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     return rc;
   if (!skinny) {
     bool done = false;
+    if (int rc = RunInt8Small(ctx, *call, a, b, lzp, rzp, &done, err)) return rc;
+    if (done) return RUYAMD_OK;
     if (int rc = RunInt8Staged(ctx, *call, a, b, lzp, rzp, &done, err)) return rc;
     if (done) return RUYAMD_OK;
   }
@@ -566,11 +648,14 @@ struct OperandF32 {
   const float* data = nullptr;
   int32_t ld = 0;  // elements
   uint32_t bytes = 0;
+  // Neither cached nor usable in place: `src` is to be packed (PackOperandF32) or
+  // read as it is by a kernel that can.
+  bool unpacked = false;
+  PackSource src;
 };
 
 int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy,
-                      const void* src_key, int other_width, OperandF32* out, PendingPack* pack,
-                      std::string* err) {
+                      const void* src_key, int other_width, OperandF32* out, std::string* err) {
   auto view = [&]() {
     const DevMat& m = side == 0 ? call->lhs : call->rhs;
     return side == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
@@ -634,16 +719,26 @@ int PrepareOperandF32(ruyamd_ctx* ctx, MulCall* call, int side, int cache_policy
     out->bytes = static_cast<uint32_t>(extent);
     return RUYAMD_OK;
   }
-  float* packed = static_cast<float*>(ctx->ws->Alloc(packed_bytes ? packed_bytes : 16));
+  out->unpacked = true;
+  out->src = src;
+  out->ld = ld;
+  out->bytes = static_cast<uint32_t>(packed_bytes);
+  return RUYAMD_OK;
+}
+
+// Room in the workspace for an operand that PrepareOperandF32 left unpacked, as
+// PackOperand8.
+int PackOperandF32(ruyamd_ctx* ctx, OperandF32* op, PendingPack* pack, std::string* err) {
+  if (!op->unpacked) return RUYAMD_OK;
+  float* packed = static_cast<float*>(ctx->ws->Alloc(op->bytes ? op->bytes : 16));
   if (!packed) {
     *err = "workspace allocation failed";
     return RUYAMD_E_HIP;
   }
   pack->pending = true;
-  pack->job = PackJob{src, packed, ld * 4, nullptr};
-  out->data = packed;
-  out->ld = ld;
-  out->bytes = static_cast<uint32_t>(packed_bytes);
+  pack->job = PackJob{op->src, packed, op->ld * 4, nullptr};
+  op->unpacked = false;
+  op->data = packed;
   return RUYAMD_OK;
 }
 
@@ -668,14 +763,78 @@ bool SetupDestination(const MulCall& call, GemmArgs* args) {
   return swap;
 }
 
+// An fp32 product on the small tiles, where the planner finds that better (*done).
+int RunF32Small(ruyamd_ctx* ctx, const MulCall& call, const OperandF32& a, const OperandF32& b, bool* done,
+                std::string* err) {
+  const int M = call.lhs.rows, K = call.lhs.cols, N = call.rhs.cols;
+  if (ctx->forced_tile_rows || K < 4) return RUYAMD_OK;
+  struct Small {
+    const void* data;
+    SmallGemmSource source;
+    int32_t pitch;
+    uint32_t bytes;
+  } sides[2];
+  for (int i = 0; i < 2; ++i) {
+    const OperandF32& op = i == 0 ? a : b;
+    Small& s = sides[i];
+    s = {op.data, kSmallRows, op.ld * 4, op.bytes};
+    if (!op.unpacked) continue;
+    s.data = op.src.data;
+    if (!SmallSourceOf(op.src, &s.source, &s.pitch, &s.bytes) || s.source == kSmallRowsBytes ||
+        s.source == kSmallAcrossBytes)
+      return RUYAMD_OK;
+  }
+  GemmArgs args;
+  const bool swap = SetupDestination(call, &args);
+  const Small& x = sides[swap ? 1 : 0];
+  const Small& y = sides[swap ? 0 : 1];
+  args.a = x.data;
+  args.b = y.data;
+  args.a_bytes = x.bytes;
+  args.b_bytes = y.bytes;
+  args.lda = x.pitch;
+  args.ldb = y.pitch;
+  args.M = swap ? N : M;
+  args.N = swap ? M : N;
+  args.n_logical = args.N;
+  args.k_bytes = RoundUp(K, 4) * 4;
+  args.k_valid = K * 4;
+  SmallGemmPlan plan;
+  plan.source_a = x.source;
+  plan.source_b = y.source;
+  plan = PlanSmallGemmF32(args, ctx->multiprocessor_count, plan, uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes);
+  if (plan.waves == 0) return RUYAMD_OK;
+  for (const OperandF32* op : {&a, &b}) {
+    if (!HasRoomToPack(ctx, op->unpacked, op->bytes, 0)) {
+      *err = "workspace allocation failed";
+      return RUYAMD_E_HIP;
+    }
+  }
+  const bool timed = ctx->TimingBegin();
+  const hipError_t launched = LaunchSmallGemmF32(ctx->LaunchStream(), args, plan);
+  if (timed) ctx->TimingEnd();
+  if (launched != hipSuccess) {
+    *err = "fp32 matrix-core kernel launch failed";
+    return RUYAMD_E_HIP;
+  }
+  ctx->last_kernel = RUYAMD_KERNEL_F32_MFMA;
+  *done = true;
+  return RUYAMD_OK;
+}
+
 int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   const int M = call->lhs.rows, K = call->lhs.cols, N = call->rhs.cols;
   OperandF32 a, b;
+  if (int rc = PrepareOperandF32(ctx, call, 0, call->lhs_cache_policy, call->lhs_src_key, N, &a, err)) return rc;
+  if (int rc = PrepareOperandF32(ctx, call, 1, call->rhs_cache_policy, call->rhs_src_key, M, &b, err)) return rc;
+  if (N > kSkinnyKernelWidth && M > kSkinnyKernelWidth) {
+    bool done = false;
+    if (int rc = RunF32Small(ctx, *call, a, b, &done, err)) return rc;
+    if (done) return RUYAMD_OK;
+  }
   PendingPack pack_a, pack_b;
-  if (int rc = PrepareOperandF32(ctx, call, 0, call->lhs_cache_policy, call->lhs_src_key, N, &a, &pack_a, err))
-    return rc;
-  if (int rc = PrepareOperandF32(ctx, call, 1, call->rhs_cache_policy, call->rhs_src_key, M, &b, &pack_b, err))
-    return rc;
+  if (int rc = PackOperandF32(ctx, &a, &pack_a, err)) return rc;
+  if (int rc = PackOperandF32(ctx, &b, &pack_b, err)) return rc;
   if (int rc = LaunchPendingPacks(ctx, pack_a, pack_b, err)) return rc;
   if (N <= kSkinnyKernelWidth || M <= kSkinnyKernelWidth) {
     // Bandwidth-bound shapes: stream the wide side exactly once.

@@ -249,6 +249,27 @@ def test_small_products_on_two_workgroups_a_cu(device_ctx):
         compare(p, got, want)
 
 
+@pytest.mark.parametrize("tup", [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I16), (S.I8, S.U8, S.I32, S.I32),
+                                 (S.F32, S.F32, S.F32, S.F32)], ids=cases.tuple_name)
+@pytest.mark.parametrize("depth", [4, 16, 17, 31, 63, 64, 65, 127, 128, 131, 255, 257, 511, 513, 1029, 2049, 4095])
+def test_products_on_tiles_of_32(device_ctx, tup, depth):
+    """Operands read where they lie, in every storage order: depths either side of
+    a granule, of a step of either length and of what each number of waves takes;
+    counts either side of a tile and of 16 bytes of vectors; pitches of whole
+    dwords and of odd bytes; one operand from the cache."""
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(depth)
+    shapes = [(17, 33), (64, 31), (97, 100)] + ([(520, 517)] if depth < 600 else [])
+    for n, (rows, cols) in enumerate(shapes):
+        for orders in [(1, 0, 0), (0, 0, 1), (1, 1, 0), (0, 1, 1)]:
+            p = W.random_problem(rng, *tup, rows, depth, cols, *orders, strided=(depth + n) % 3 == 0,
+                                 name="tiles of 32 %dx%dx%d %s" % (rows, depth, cols, orders))
+            p.lhs.cache_policy = S.CACHE_ALWAYS if (depth + n) % 4 == 0 else S.CACHE_NEVER
+            for misalign in (0, 4 if tup[0] == S.F32 else 1):
+                compare(p, D.device_mul(device_ctx, p, misalign=misalign), expected(p), exact_fp=False)
+                device_ctx.clear_prepacked_cache()
+
+
 @pytest.mark.parametrize("shape", [
     (1, 16, 1),            # single bytes
     (128, 40, 128),        # a destination of exactly one workgroup's 16 KiB
