@@ -25,6 +25,7 @@ struct F32Traits {
   }
   static __device__ __forceinline__ void DrainMma() {}
   static constexpr int kBlock = 32;
+  static constexpr bool kAnyDepth = true;
   static constexpr bool kRawB = false;
   static constexpr bool kPaired = false;
   using LargeTile = F32Traits;

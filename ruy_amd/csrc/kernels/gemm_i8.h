@@ -39,7 +39,8 @@ struct GemmArgs {
   DevMat dst;
   int32_t dst_elt = 1;
   // Not 0: the operands need none of the above but rows that are runs of
-  // k_valid >= 16 bytes, of any alignment and pitch (LaunchGemmI8Staged);
+  // k_valid >= 16 bytes, of any alignment and pitch (LaunchGemmI8Staged) or of
+  // whole dwords at multiples of 4 bytes (LaunchGemmF32);
   // k_bytes is then k_valid rounded up to 16, and uint8 data (a_flip, b_flip)
   // may have any depth.
   // (With one word less here, the struct has a hole in front of its

@@ -162,9 +162,11 @@ struct Side {
     }
   }
 
-  // Puts what Load has fetched of `step` into the slot.
+  // Puts what Load has fetched of `step` into the slot. kInside: the step lies
+  // inside the depth.
+  template <bool kInside>
   __device__ __forceinline__ void Store(int step, const Held& h, char* slot) const {
-    const bool partial = (step + 1) * S > bytes;  // (wave-uniform)
+    const bool partial = !kInside && (step + 1) * S > bytes;  // (wave-uniform)
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) {
       if (!Exists(u)) continue;
@@ -179,7 +181,7 @@ struct Side {
           if constexpr (!kAcross) {
             // (row_shl:1: from the next lane of the 16.)
             const int next = __builtin_amdgcn_update_dpp(0, h.x[u][j][0], 0x101, 0xf, 0xf, false);
-            if (!LoadsFifth(step, u)) fifth = next;
+            if (!(partial || DepthOf(u) == S - 16)) fifth = next;
           }
 #pragma unroll
           for (int d = 0; d < 4; ++d)
@@ -316,11 +318,15 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
   const bool sums_of_b = T::kElement == 1 && args.fused_b_factor != 0;
 
   char* const slot = lds + wave * Mem::kSlot;
-  auto step_of = [&](int i, auto at) {
+  // `steady`: a step that lies inside the depth and whose place step i + kAhead
+  // takes. (Without conditions, or the wait for a step's loads is one for all
+  // that may be in flight.)
+  auto step_of = [&](int i, auto at, auto steady) {
+    constexpr bool kSteady = decltype(steady)::value;
     const int step = wave + kWaves * i;
-    a.Store(step, held_a[decltype(at)::value], slot);
-    b.Store(step, held_b[decltype(at)::value], slot + kTile * S);
-    if (i + kAhead < my_steps) load(i + kAhead, at);
+    a.template Store<kSteady>(step, held_a[decltype(at)::value], slot);
+    b.template Store<kSteady>(step, held_b[decltype(at)::value], slot + kTile * S);
+    if (kSteady || i + kAhead < my_steps) load(i + kAhead, at);
     // (Written and read by this wave only, whose LDS operations are performed
     // in order.)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -333,6 +339,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
       fa[ks] = *reinterpret_cast<const v4i*>(slot + offset);
       fb[ks] = *reinterpret_cast<const v4i*>(slot + kTile * S + offset);
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < kSubSteps; ++ks) T::Mma(fa[ks], fb[ks], acc, ks);
     if (sums_of_a) {
@@ -349,15 +356,22 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
     }
     __builtin_amdgcn_wave_barrier();
   };
+  int i = 0;
+  using Steady = std::true_type;
+  using Last = std::false_type;
   if constexpr (kAhead == 1) {
-    for (int i = 0; i < my_steps; ++i) step_of(i, First());
+    for (; i + 1 < my_steps; ++i) step_of(i, First(), Steady());
+    if (i < my_steps) step_of(i, First(), Last());
   } else {
-    int i = 0;
-    for (; i + 1 < my_steps; i += 2) {
-      step_of(i, First());
-      step_of(i + 1, Second());
+    for (; i + 3 < my_steps; i += 2) {
+      step_of(i, First(), Steady());
+      step_of(i + 1, Second(), Steady());
     }
-    if (i < my_steps) step_of(i, First());
+    for (; i + 1 < my_steps; i += 2) {
+      step_of(i, First(), Last());
+      step_of(i + 1, Second(), Last());
+    }
+    if (i < my_steps) step_of(i, First(), Last());
   }
 
   // ---- the partial tiles, added through LDS ----

@@ -52,22 +52,27 @@ struct F32Small {
 
 }  // namespace
 
-// The time of these tiles by a fit to 16 to 1536 of them and depths of 16 to 2048
+// The time of these tiles by a fit to 16 to 2112 of them and depths of 16 to 2048
 // (within 10 % mostly): 3.9 us, 0.33 us for every tile a CU has beyond the first,
-// and 1.25 us to a KiB of depth and tile (their matrix instructions at two thirds
-// of their rate), 1.3 where an operand is transposed on the way. Held against
-// the other tiles' timing model and a pack in front of them: us, other route ->
-// this, 512^3 12.8 -> 6.0; 512 tiles in place x 512 13.2 -> 8.6, x 2048 23.9 -> 23.5;
-// 1024 x 256 10.7 -> 8.9, x 1024 22.1 -> 23.1; 256 tiles with one side transposed x
-// 1024 19.7 -> 9.2, both 21.8 -> 9.4; 1536 x 1024 43.4 -> 36.6, both 47.6 -> 39.5.
+// and 1.22 us to a KiB of depth and tile (their matrix instructions alone take 1.03
+// at the clock they leave the card), 1.4 where rows do not start at multiples of 16
+// bytes or an operand is transposed on the way. Held against the other tiles'
+// timing model and a pack in front of them (of transposed operands: rows are read
+// in place there, too). us, other route -> this: 512^3 12.8 -> 6.0; 512 tiles in place
+// x 512 13.2 -> 8.6, x 2048 23.9 -> 23.5; 1024 x 256 10.6 -> 8.8, x 1024 21.9 -> 23.7; 2112
+// (one 64x64 tile too many for two rounds) x 1024 60.5 -> 47.7; 256 tiles with one
+// side transposed x 1024 19.7 -> 9.2, both 21.8 -> 9.4; 1536 x 1024 43.4 -> 39.8, both
+// 47.6 -> 39.0.
 SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
   const int K = args.k_valid;
   const bool across = small_gemm::IsAcross(plan.source_a) || small_gemm::IsAcross(plan.source_b);
   plan.waves = 0;
-  if (K < 16 || tiles > 6 * num_cus) return plan;
+  if (K < 16 || tiles > 16 * num_cus) return plan;
   const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
-  const double here = 3.9 + 0.33 * (a_cu - 1) + (across ? 1.3 : 1.25) * a_cu * K / 1024.0;
+  const bool straddling = across || ((reinterpret_cast<uintptr_t>(args.a) | reinterpret_cast<uintptr_t>(args.b) |
+                                      static_cast<uint32_t>(args.lda) | static_cast<uint32_t>(args.ldb)) & 15) != 0;
+  const double here = 3.9 + 0.33 * (a_cu - 1) + (straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kF32);
   double other = 1e30;
   for (int i = 0; i < model.count; ++i)
@@ -80,7 +85,7 @@ SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan 
     plan.waves = K > 256 ? 8 : 4;
     if (across && K >= 1024) plan.step = 128;
     if (across && K >= 4096) plan.waves = 16;
-  } else if (across ? K >= 512 || a_cu == 2 : K >= 4096 && a_cu > 2) {
+  } else if (across && (K >= 512 || a_cu == 2)) {
     plan.step = 128;
   }
   return plan;

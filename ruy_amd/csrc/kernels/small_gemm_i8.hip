@@ -86,8 +86,8 @@ struct Int8Small {
 //   ... and at odd bytes: 256 x 8192 22.5 -> 21.5; 512 x 2048 13.4 -> 12.4, x 4096
 //     19.3 -> 20.8; 768 x 512 8.9 -> 8.1, x 1024 11.4 -> 11.5; 1024 x 128 7.4 -> 7.1.
 // More waves to a workgroup, or longer steps, where the grid leaves CUs room for
-// them: 256 tiles in place x 1024 4.8 with four waves, 4.4 with eight, packed x 8193
-// 20.3 with eight, 15.3 with sixteen.
+// them: 256 tiles in place x 1024 5.2 with four waves, 4.7 with eight; packed x 4097
+// 12.1 and 9.1; transposed x 8192 17.8 with eight, 16.8 with sixteen.
 SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
   const int K = args.k_valid;
@@ -109,19 +109,19 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
   if (K > deepest) return plan;
   plan.waves = 4;
   plan.step = 64;
-  if (a_cu == 1) {
-    plan.waves = K > 256 ? 8 : 4;
-    if (across || !bytes) plan.step = K >= 512 ? 128 : 64;
-    if (across ? K >= 4096 : bytes && K >= 2048) {
-      plan.waves = 16;
+  if (across) {
+    if (a_cu == 1) {
+      plan.waves = K >= 4096 ? 16 : K > 256 ? 8 : 4;
+      if (K >= 512) plan.step = 128;
+    } else if (a_cu == 2) {
       plan.step = 128;
     }
-  } else if (across) {
-    if (a_cu == 2) plan.step = 128;
+  } else if (a_cu == 1) {
+    if (K > 256) plan.waves = 8;
   } else if (bytes) {
-    if (a_cu == 2 && K > 128) plan.waves = 8;
+    if (a_cu == 2 && K > 128 && K < 2048) plan.waves = 8;
     if (a_cu == 3 && K >= 2048) plan.step = 128;
-  } else if (K >= 2048) {
+  } else if (K >= 1024) {
     plan.step = 128;
   }
   return plan;

@@ -397,7 +397,9 @@ bool SmallSourceOf(const PackSource& src, SmallGemmSource* source, int32_t* pitc
   const int64_t stride = (rows ? src.stride_c : src.stride_k) * element;
   const uint64_t extent =
       uint64_t((rows ? src.count : src.K) - 1) * uint64_t(stride) + uint64_t(rows ? src.K : src.count) * element;
-  if (extent >= (uint64_t(1) << 31)) return false;
+  // (A little room below 2^31: the offset of a row that does not exist is 2^31 less
+  // some bytes.)
+  if (extent >= (uint64_t(1) << 31) - 64) return false;
   const bool dwords = ((reinterpret_cast<uintptr_t>(src.data) | static_cast<uint64_t>(stride)) & 3) == 0;
   *source = rows ? (dwords ? kSmallRows : kSmallRowsBytes) : (dwords ? kSmallAcross : kSmallAcrossBytes);
   *pitch = static_cast<int32_t>(stride);
@@ -444,7 +446,8 @@ int RunInt8Small(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const 
   SmallGemmPlan plan;
   plan.source_a = swap ? source_b : source_a;
   plan.source_b = swap ? source_a : source_b;
-  plan = PlanSmallGemmI8(args, ctx->multiprocessor_count, plan, uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes);
+  const uint64_t packed_bytes = uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes;
+  plan = PlanSmallGemmI8(args, ctx->multiprocessor_count, plan, packed_bytes);
   if (plan.waves == 0) return RUYAMD_OK;
   for (const Operand8* op : {&a, &b}) {
     const bool sums = op->unpacked && op->sums_pending && PackFormsSums(op->src, op->ld);
@@ -802,7 +805,9 @@ int RunF32Small(ruyamd_ctx* ctx, const MulCall& call, const OperandF32& a, const
   SmallGemmPlan plan;
   plan.source_a = x.source;
   plan.source_b = y.source;
-  plan = PlanSmallGemmF32(args, ctx->multiprocessor_count, plan, uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes);
+  // (Rows are not packed for the other tiles either.)
+  const uint64_t packed_bytes = uint64_t(sides[0].source == kSmallAcross) * a.bytes + uint64_t(sides[1].source == kSmallAcross) * b.bytes;
+  plan = PlanSmallGemmF32(args, ctx->multiprocessor_count, plan, packed_bytes);
   if (plan.waves == 0) return RUYAMD_OK;
   for (const OperandF32* op : {&a, &b}) {
     if (!HasRoomToPack(ctx, op->unpacked, op->bytes, 0)) {
@@ -831,6 +836,26 @@ int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     bool done = false;
     if (int rc = RunF32Small(ctx, *call, a, b, &done, err)) return rc;
     if (done) return RUYAMD_OK;
+  }
+  // Rows at multiples of 4 bytes, of any depth: the tiled kernel reads them where
+  // they lie.
+  bool any_depth = false;
+  if (N > kSkinnyKernelWidth && M > kSkinnyKernelWidth && K >= 4) {
+    for (OperandF32* op : {&a, &b}) {
+      SmallGemmSource source;
+      int32_t pitch;
+      uint32_t bytes;
+      if (!op->unpacked || !SmallSourceOf(op->src, &source, &pitch, &bytes) || source != kSmallRows) continue;
+      if (!HasRoomToPack(ctx, true, op->bytes, 0)) {
+        *err = "workspace allocation failed";
+        return RUYAMD_E_HIP;
+      }
+      op->unpacked = false;
+      op->data = static_cast<const float*>(op->src.data);
+      op->ld = pitch / 4;
+      op->bytes = bytes;
+      any_depth = K % 4 != 0;
+    }
   }
   PendingPack pack_a, pack_b;
   if (int rc = PackOperandF32(ctx, &a, &pack_a, err)) return rc;
@@ -880,6 +905,7 @@ int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   args.M = swap ? N : M;
   args.N = swap ? M : N;
   args.n_logical = args.N;
+  if (any_depth) args.k_valid = K * 4;
   PlanDepthSplit(ctx, GemmKind::kF32, &args);
   const bool timed = ctx->TimingBegin();
   const hipError_t launched = LaunchGemmF32(ctx->LaunchStream(), args, ctx->multiprocessor_count);

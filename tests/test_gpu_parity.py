@@ -270,6 +270,32 @@ def test_products_on_tiles_of_32(device_ctx, tup, depth):
                 device_ctx.clear_prepacked_cache()
 
 
+@pytest.mark.parametrize("tile", [(64, 64), (128, 64), (64, 128), (128, 128), (256, 256)])
+@pytest.mark.parametrize("depth", [4, 5, 31, 33, 62, 95, 127, 129, 161, 190, 257, 515, 2051])
+def test_fp32_rows_of_any_depth_in_place(device_ctx, tile, depth):
+    """Every fp32 tile on rows that end in part of a granule: one step and many,
+    the end in the first and the last granule of a step, a depth in parts; what
+    lies between the rows must not be looked at (it is NaN here)."""
+    import torch
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(depth)
+    device_ctx.force_tile(*tile)
+    try:
+        for rows, cols, orders in [(65, 130, (1, 0, 0)), (300, 77, (1, 0, 1))]:
+            p = W.random_problem(rng, S.F32, S.F32, S.F32, S.F32, rows, depth, cols, *orders, strided=True,
+                                 name="any depth %dx%dx%d" % (rows, depth, cols))
+            for m in (p.lhs, p.rhs):
+                view = m.storage[:m.n_storage]
+                pad = np.ones(view.size, bool)
+                outer = m.rows if m.order == S.ORDER_ROW_MAJOR else m.cols
+                for v in range(outer):
+                    pad[v * m.stride:v * m.stride + depth] = False
+                view[pad] = np.nan
+            compare(p, D.device_mul(device_ctx, p, misalign=4), expected(p), exact_fp=False)
+    finally:
+        device_ctx.force_tile(0, 0)
+
+
 @pytest.mark.parametrize("shape", [
     (1, 16, 1),            # single bytes
     (128, 40, 128),        # a destination of exactly one workgroup's 16 KiB
