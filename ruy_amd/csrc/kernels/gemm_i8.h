@@ -197,6 +197,12 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
 SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes);
 hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan);
 hipError_t LaunchSmallGemmF32(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan);
+// int8 x int16, the int16 side (`int16_is_a`: the rows) as it lies: k_valid counts
+// depth positions, N destination columns, and the fused factor of the int8 side
+// is -128.
+SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes,
+                                 bool int16_is_a);
+hipError_t LaunchSmallGemmI8I16(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan, bool int16_is_a);
 // `count` <= kGemmBatchMax products of the shape and parameters of `args`, each
 // on its own buffers, in one launch. Only for arguments that run on the
 // smallest tile (GemmI8CanFuseSums), without sums arrays (zero points 0, or the

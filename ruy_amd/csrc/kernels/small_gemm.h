@@ -62,26 +62,39 @@ __device__ __forceinline__ int SlotOffset(int r, int g) {
 }
 
 // The kTile vectors of one operand that a tile needs, from vector `first` on.
+// kElement: bytes of a value. Values of two bytes become two planes of int8, high
+// and low byte (minus 128), which lie in the slot as 32 vectors each: v = 256 high
+// + low + 128. Across the vectors their bytes are what a piece transposes: byte 2 v
+// of a depth position belongs to the low plane of vector v, the next one to the
+// high plane.
 template <int S, int kSource, int kElement>
 struct Side {
   static constexpr bool kAcross = IsAcross(kSource);
   static constexpr bool kAnyByte = IsAnyByte(kSource);
+  static constexpr bool kPlanes = kElement == 2;
+  static constexpr int kSlotVectors = kPlanes ? 2 * kTile : kTile;
   static constexpr int kGranules = S / 16;
-  // Across the vectors: a piece is 16 bytes of vectors (16 or 4 of them) at
-  // four depth positions (4 or 16 bytes of depth).
-  static constexpr int kVectors = 16 / kElement;
-  static constexpr int kPieceDepth = 4 * kElement;
-  static constexpr int kGroups = kTile / kVectors;
+  // Bytes of depth that a position takes in a slot, and bytes of source for one
+  // of depth along a vector.
+  static constexpr int kPosition = kElement == 4 ? 4 : 1;
+  static constexpr int kScale = kPlanes ? 2 : 1;
+  // Across the vectors: a piece is 16 bytes of them (4 vectors, 16, or the bytes
+  // of 8) at four depth positions (4 or 16 bytes of depth).
+  static constexpr int kColumnBytes = kElement == 4 ? 4 : 1;  // what is transposed as one
+  static constexpr int kColumns = 16 / kColumnBytes;
+  static constexpr int kTileColumns = kTile * kScale;
+  static constexpr int kPieceDepth = 4 * kPosition;
+  static constexpr int kGroups = kTileColumns / kColumns;
   // What a step's work comes to a lane: granules, or pieces.
   static constexpr int kAll = kAcross ? kGroups * (S / kPieceDepth) : kTile * kGranules;
   static constexpr int kUnits = (kAll + 63) / 64;
-  static constexpr int kLoads = kAcross ? 4 : 1;  // of a unit
+  static constexpr int kLoads = kAcross ? 4 : kScale;  // of a unit
 
   const char* data;
-  int pitch, count, first, bytes;
+  int pitch, count, first, bytes;  // (bytes: of depth in a slot)
   uint32_t flip;
   int lane;
-  uint32_t offset[kUnits];  // of the unit's vector (first vector)
+  uint32_t offset[kUnits];  // of the unit's vector (first column)
 
   struct Held {
     v4i x[kUnits][kLoads];
@@ -89,11 +102,11 @@ struct Side {
   };
 
   __device__ __forceinline__ bool Exists(int u) const { return kAll % 64 == 0 || u * 64 + lane < kAll; }
-  // Vector (first vector) of unit u, counted inside the tile, and its first
+  // Vector (first column) of unit u, counted inside the tile, and its first
   // byte of depth, counted inside a step.
   __device__ __forceinline__ int VectorOf(int u) const {
     const int p = u * 64 + lane;
-    return kAcross ? p % kGroups * kVectors : p / kGranules;
+    return kAcross ? p % kGroups * kColumns : p / kGranules;
   }
   __device__ __forceinline__ int DepthOf(int u) const {
     const int p = u * 64 + lane;
@@ -113,27 +126,28 @@ struct Side {
     // in Store.)
 #pragma unroll
     for (int u = 0; u < kUnits; ++u)
-      offset[u] = kAcross ? uint32_t(min(first + VectorOf(u), count - kVectors) * kElement)
+      offset[u] = kAcross ? uint32_t(min(first * kScale + VectorOf(u), count * kScale - kColumns) * kColumnBytes)
                           : uint32_t(min(first + VectorOf(u), count - 1)) * uint32_t(pitch);
   }
 
   // Where load j of unit u of a step reads.
   __device__ __forceinline__ const char* From(int step, int u, int j) const {
     const int k = step * S + DepthOf(u);
-    // A granule that reaches past the end of its vector: the 16 bytes that end
-    // there, moved down in Store.
-    if constexpr (!kAcross) return data + (offset[u] + uint32_t(min(k, bytes - 16)));
+    // 16 bytes that reach past the end of their vector: those that end there,
+    // moved down in Store.
+    if constexpr (!kAcross) return data + (offset[u] + uint32_t(min(k * kScale + 16 * j, bytes * kScale - 16)));
     // Depth positions past the end read the last one and become zero in Store.
-    return data + (uint32_t(min(k / kElement + j, bytes / kElement - 1)) * uint32_t(pitch) + offset[u]);
+    return data + (uint32_t(min(k / kPosition + j, bytes / kPosition - 1)) * uint32_t(pitch) + offset[u]);
   }
-  // kAnyByte: whether the fifth dword of a lane's 16 bytes is loaded. Of a row it
-  // mostly is the first one of the next lane's, whose 16 bytes follow in memory:
-  // not at the end of a run of lanes, nor in the step that the depth ends in,
-  // whose last granule is read from elsewhere than its place. (512 tiles of 4097
-  // bytes of depth: 16.9 us with every lane's loaded, 15.3 so. Across the vectors
-  // a run is two lanes: 256 tiles 11.9 us, 15.1 so.)
+  // kAnyByte: whether the fifth dword of a lane's 16 bytes is loaded. Of an 8-bit
+  // row it mostly is the first one of the next lane's, whose 16 bytes follow in
+  // memory: not at the end of a run of lanes, nor in the step that the depth ends
+  // in, whose last granule is read from elsewhere than its place. (512 tiles of
+  // 4097 bytes of depth: 16.9 us with every lane's loaded, 15.3 so. Across the
+  // vectors a run is two lanes: 256 tiles 11.9 us, 15.1 so.)
+  static constexpr bool kFifthFromNextLane = !kAcross && !kPlanes;
   __device__ __forceinline__ bool LoadsFifth(int step, int u) const {
-    return kAcross || (step + 1) * S > bytes || DepthOf(u) == S - 16;
+    return !kFifthFromNextLane || (step + 1) * S > bytes || DepthOf(u) == S - 16;
   }
   __device__ __forceinline__ void Load(int step, Held& h) const {
 #pragma unroll
@@ -178,7 +192,7 @@ struct Side {
         if constexpr (kAnyByte) {
           const uint32_t shift = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(From(step, u, j)) & 3);
           int fifth = h.fifth[u][j];
-          if constexpr (!kAcross) {
+          if constexpr (kFifthFromNextLane) {
             // (row_shl:1: from the next lane of the 16.)
             const int next = __builtin_amdgcn_update_dpp(0, h.x[u][j][0], 0x101, 0xf, 0xf, false);
             if (!(partial || DepthOf(u) == S - 16)) fifth = next;
@@ -188,18 +202,29 @@ struct Side {
             x[j][d] = static_cast<int>(__builtin_amdgcn_alignbyte(d < 3 ? h.x[u][j][d + 1] : fifth, h.x[u][j][d], shift));
         }
         if constexpr (kAcross) {
-          if (first + kTile > count) x[j] = PlaceGranule(x[j], (first + VectorOf(u)) * kElement, count * kElement);
+          if (first + kTile > count)
+            x[j] = PlaceGranule(x[j], (first * kScale + VectorOf(u)) * kColumnBytes, count * kScale * kColumnBytes);
+        } else {
+          if (partial) x[j] = PlaceGranule(x[j], k * kScale + 16 * j, bytes * kScale);
         }
-        if constexpr (kElement == 1) x[j] ^= static_cast<int>(flip);
       }
       const int vector = VectorOf(u);
-      if constexpr (!kAcross) {
-        if (partial) {
-          // (The flip of the padding is taken back by the mask.)
-          if constexpr (kElement == 1) x[0] ^= static_cast<int>(flip);
-          x[0] = PlaceGranule(x[0], k, bytes);
+      if constexpr (!kAcross && kPlanes) {
+        // (Past the end: high 0, low -128, which meet zeros of the other operand.)
+        v4i high, low;
 #pragma unroll
-          for (int d = 0; d < 4; ++d) x[0][d] ^= static_cast<int>(flip & LowBytes(bytes - k - 4 * d));
+        for (int d = 0; d < 4; ++d) {
+          const v4i& y = x[d / 2];
+          high[d] = static_cast<int>(__builtin_amdgcn_perm(y[d % 2 * 2 + 1], y[d % 2 * 2], 0x07050301u));
+          low[d] = static_cast<int>(__builtin_amdgcn_perm(y[d % 2 * 2 + 1], y[d % 2 * 2], 0x06040200u) ^ 0x80808080u);
+        }
+        *reinterpret_cast<v4i*>(slot + SlotOffset<S>(vector, DepthOf(u) / 16)) = high;
+        *reinterpret_cast<v4i*>(slot + SlotOffset<S>(kTile + vector, DepthOf(u) / 16)) = low;
+      } else if constexpr (!kAcross) {
+        if constexpr (kElement == 1) {
+#pragma unroll
+          for (int d = 0; d < 4; ++d)  // (the padding stays zero)
+            x[0][d] ^= static_cast<int>(partial ? flip & LowBytes(bytes - k - 4 * d) : flip);
         }
         *reinterpret_cast<v4i*>(slot + SlotOffset<S>(vector, DepthOf(u) / 16)) = x[0];
       } else if constexpr (kElement == 4) {
@@ -216,7 +241,7 @@ struct Side {
         const uint32_t valid = partial ? LowBytes(bytes - k) : 0xffffffffu;
 #pragma unroll
         for (int quad = 0; quad < 4; ++quad) {
-          // 4 x 4 bytes: t[i] = four depth positions of vector 4 * quad + i.
+          // 4 x 4 bytes: t[i] = four depth positions of column 4 * quad + i.
           const uint32_t x0 = __builtin_amdgcn_perm(x[1][quad], x[0][quad], 0x05010400u);
           const uint32_t x1 = __builtin_amdgcn_perm(x[1][quad], x[0][quad], 0x07030602u);
           const uint32_t y0 = __builtin_amdgcn_perm(x[3][quad], x[2][quad], 0x05010400u);
@@ -224,9 +249,12 @@ struct Side {
           const uint32_t t[4] = {__builtin_amdgcn_perm(y0, x0, 0x05040100u), __builtin_amdgcn_perm(y0, x0, 0x07060302u),
                                  __builtin_amdgcn_perm(y1, x1, 0x05040100u), __builtin_amdgcn_perm(y1, x1, 0x07060302u)};
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<uint32_t*>(slot + SlotOffset<S>(vector + 4 * quad + i, DepthOf(u) / 16) + DepthOf(u) % 16) =
-                t[i] & valid;
+          for (int i = 0; i < 4; ++i) {
+            const int column = vector + 4 * quad + i;
+            const int to = kPlanes ? column / 2 + (i % 2 == 0 ? kTile : 0) : column;
+            const uint32_t value = kPlanes ? (i % 2 == 0 ? t[i] ^ 0x80808080u : t[i]) : (t[i] ^ flip) & valid;
+            *reinterpret_cast<uint32_t*>(slot + SlotOffset<S>(to, DepthOf(u) / 16) + DepthOf(u) % 16) = value;
+          }
         }
       }
     }
@@ -238,10 +266,10 @@ struct Side {
 // runs of 32 columns padded by one so that a column's pieces lie in different
 // banks); behind that the partial sums of the tile's vectors and the
 // write-back parameters of its rows and columns.
-template <int S, int kWaves>
+template <int S, int kWaves, int kSlotVectors>
 struct Memory {
   static constexpr int kVectors = 2 * kTile;
-  static constexpr int kSlot = kVectors * S;
+  static constexpr int kSlot = kSlotVectors * S;
   static constexpr int kPart = 8 * 33;  // granules of a wave's partial tile
   static constexpr int kSums = std::max(kWaves * kSlot, kWaves * kPart * 16);
   static constexpr int kParams = kSums + kWaves * kVectors * 4;
@@ -250,7 +278,9 @@ struct Memory {
 
 template <typename T, int S, int kWaves, int kSourceA, int kSourceB>
 __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void SmallGemmKernel(GemmArgs args) {
-  using Mem = Memory<S, kWaves>;
+  using SideA = Side<S, kSourceA, T::kElementA>;
+  using SideB = Side<S, kSourceB, T::kElementB>;
+  using Mem = Memory<S, kWaves, SideA::kSlotVectors + SideB::kSlotVectors>;
   constexpr int kSubSteps = S / 32;
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -277,8 +307,6 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
   const int steps = (K + S - 1) / S;
   const int my_steps = steps > wave ? (steps - wave + kWaves - 1) / kWaves : 0;
 
-  using SideA = Side<S, kSourceA, T::kElement>;
-  using SideB = Side<S, kSourceB, T::kElement>;
   SideA a;
   SideB b;
   a.Start(args.a, args.lda, args.M, m0, K, args.a_flip, lane);
@@ -307,15 +335,18 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
   // longer than where a depth is split over workgroups: four of eight waves, two
   // where there are more waves or the registers decide how many workgroups a CU
   // holds. Against 64 bits, 256 x 2048 x 256: split 2.1e-7, here 1.6e-7.)
-  constexpr int kChains = T::kElement == 1 ? 1 : kWaves == 8 ? 4 : 2;
+  // (Two planes: an accumulator each.)
+  constexpr bool kPlanes = SideA::kPlanes || SideB::kPlanes;
+  constexpr bool kInteger = T::kElementA != 4;
+  constexpr int kChains = kPlanes ? 2 : kInteger ? 1 : kWaves == 8 ? 4 : 2;
   typename T::Acc acc[kChains];
 #pragma unroll
   for (int c = 0; c < kChains; ++c)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[c][v] = 0;
   int sum_a = 0, sum_b = 0;
-  const bool sums_of_a = T::kElement == 1 && args.fused_a_factor != 0;
-  const bool sums_of_b = T::kElement == 1 && args.fused_b_factor != 0;
+  const bool sums_of_a = T::kElementA == 1 && args.fused_a_factor != 0;
+  const bool sums_of_b = T::kElementB == 1 && args.fused_b_factor != 0;
 
   char* const slot = lds + wave * Mem::kSlot;
   // `steady`: a step that lies inside the depth and whose place step i + kAhead
@@ -325,23 +356,33 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
     constexpr bool kSteady = decltype(steady)::value;
     const int step = wave + kWaves * i;
     a.template Store<kSteady>(step, held_a[decltype(at)::value], slot);
-    b.template Store<kSteady>(step, held_b[decltype(at)::value], slot + kTile * S);
+    b.template Store<kSteady>(step, held_b[decltype(at)::value], slot + SideA::kSlotVectors * S);
     if (kSteady || i + kAhead < my_steps) load(i + kAhead, at);
     // (Written and read by this wave only, whose LDS operations are performed
     // in order.)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    v4i fa[kSubSteps], fb[kSubSteps];
+    v4i fa[kSubSteps], fb[kSubSteps], low[kPlanes ? kSubSteps : 1];
 #pragma unroll
     for (int ks = 0; ks < kSubSteps; ++ks) {
+      // (32 vectors further on the swizzle is the same.)
       const int offset = SlotOffset<S>(lane & 31, ks * 2 + lane / 32);
       fa[ks] = *reinterpret_cast<const v4i*>(slot + offset);
-      fb[ks] = *reinterpret_cast<const v4i*>(slot + kTile * S + offset);
+      fb[ks] = *reinterpret_cast<const v4i*>(slot + SideA::kSlotVectors * S + offset);
+      if constexpr (kPlanes)
+        low[ks] = *reinterpret_cast<const v4i*>(slot + (SideA::kPlanes ? kTile : SideA::kSlotVectors + kTile) * S + offset);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < kSubSteps; ++ks) T::Mma(fa[ks], fb[ks], acc, ks);
+    for (int ks = 0; ks < kSubSteps; ++ks) {
+      if constexpr (kPlanes) {
+        T::Mma(fa[ks], fb[ks], acc[0]);
+        T::Mma(SideA::kPlanes ? low[ks] : fa[ks], SideB::kPlanes ? low[ks] : fb[ks], acc[1]);
+      } else {
+        T::Mma(fa[ks], fb[ks], acc, ks);
+      }
+    }
     if (sums_of_a) {
 #pragma unroll
       for (int ks = 0; ks < kSubSteps; ++ks)
@@ -386,7 +427,8 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         typename T::Value sum = acc[0][4 * q + e];
-        if constexpr (kChains == 2) sum += acc[1][4 * q + e];
+        if constexpr (kPlanes) sum = static_cast<int>(256u * static_cast<uint32_t>(sum) + static_cast<uint32_t>(acc[1][4 * q + e]));
+        if constexpr (kChains == 2 && !kPlanes) sum += acc[1][4 * q + e];
         if constexpr (kChains == 4) sum = (sum + acc[1][4 * q + e]) + (acc[2][4 * q + e] + acc[3][4 * q + e]);
         w[e] = T::Bits(sum);
       }
@@ -424,7 +466,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
       if (sums_of_b) of_column += static_cast<uint32_t>(sums[w * Mem::kVectors + kTile + col]);
     }
   }
-  if constexpr (T::kElement == 1) {
+  if constexpr (kInteger) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       value[e] = static_cast<int>(static_cast<uint32_t>(value[e]) - static_cast<uint32_t>(args.fused_a_factor) * of_row[e] -
@@ -465,7 +507,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
 
 template <typename T, int S, int kWaves, int kSourceA, int kSourceB>
 hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
-  using Mem = Memory<S, kWaves>;
+  using Mem = Memory<S, kWaves, Side<S, kSourceA, T::kElementA>::kSlotVectors + Side<S, kSourceB, T::kElementB>::kSlotVectors>;
   // (Rows: a granule must fit; across: 16 bytes of vectors.)
   if (args.k_valid < 16 || args.M < 16 || args.N < 16 || args.split_k != 1 || args.row_sums) return hipErrorInvalidValue;
   const int64_t total = int64_t((args.M + kTile - 1) / kTile) * ((args.N + kTile - 1) / kTile);
@@ -488,7 +530,7 @@ template <typename T, int S, int kWaves>
 hipError_t LaunchSources(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
   const bool across_a = IsAcross(plan.source_a), across_b = IsAcross(plan.source_b);
   const bool bytes = IsAnyByte(plan.source_a) || IsAnyByte(plan.source_b);
-  if constexpr (T::kElement == 1) {
+  if constexpr (T::kElementA != 4) {
     if (bytes) {
       if (across_a && across_b) return Launch<T, S, kWaves, kSmallAcrossBytes, kSmallAcrossBytes>(stream, args);
       if (across_a) return Launch<T, S, kWaves, kSmallAcrossBytes, kSmallRowsBytes>(stream, args);
@@ -506,9 +548,11 @@ template <typename T>
 hipError_t LaunchPlan(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
   if (plan.step == 64 && plan.waves == 4) return LaunchSources<T, 64, 4>(stream, args, plan);
   if (plan.step == 64 && plan.waves == 8) return LaunchSources<T, 64, 8>(stream, args, plan);
-  if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 128, 4>(stream, args, plan);
-  if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 128, 8>(stream, args, plan);
-  if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 128, 16>(stream, args, plan);
+  if constexpr (T::kElementA != 2 && T::kElementB != 2) {
+    if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 128, 4>(stream, args, plan);
+    if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 128, 8>(stream, args, plan);
+    if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 128, 16>(stream, args, plan);
+  }
   return hipErrorInvalidValue;
 }
 

@@ -14,7 +14,7 @@ using granule::v4i;
 struct F32Small {
   using Acc = mfma_gemm::v16f;
   using Value = float;
-  static constexpr int kElement = 4;
+  static constexpr int kElementA = 4, kElementB = 4;
   // A granule holds four consecutive depth values of a vector.
   template <int kChains>
   static __device__ __forceinline__ void Mma(const v4i& a, const v4i& b, Acc (&acc)[kChains], int sub_step) {

@@ -1,6 +1,8 @@
 // The GEMM on 32x32 tiles (small_gemm.h) for 8-bit operands.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "int8_traits.h"
 #include "small_gemm.h"
 
@@ -10,9 +12,12 @@ namespace {
 struct Int8Small {
   using Acc = mfma_gemm::v16i;
   using Value = int;
-  static constexpr int kElement = 1;
+  static constexpr int kElementA = 1, kElementB = 1;
   static __device__ __forceinline__ void Mma(const v4i& a, const v4i& b, Acc (&acc)[1], int) {
-    acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc[0], 0, 0, 0);
+    Mma(a, b, acc[0]);
+  }
+  static __device__ __forceinline__ void Mma(const v4i& a, const v4i& b, Acc& acc) {
+    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc, 0, 0, 0);
   }
   static __device__ __forceinline__ int Bits(int x) { return x; }
   static __device__ __forceinline__ int FromBits(int x) { return x; }
@@ -64,6 +69,17 @@ struct Int8Small {
       vals[e] = Median3(static_cast<int32_t>(static_cast<uint32_t>(vals[e]) + static_cast<uint32_t>(ep.dst_zero_point)),
                         ep.clamp_min_i, ep.clamp_max_i);
   }
+};
+
+// int8 x int16, the int16 operand's planes formed on the way to LDS: neither a
+// pack launch nor, whichever side it is, a destination to be reordered. What the
+// low plane lacks is 128 times the sum of the int8 vector (a zero point of -128,
+// which the dispatcher hands over as the fused factor).
+struct Int8Int16Small : Int8Small {
+  static constexpr int kElementA = 1, kElementB = 2;
+};
+struct Int16Int8Small : Int8Small {
+  static constexpr int kElementA = 2, kElementB = 1;
 };
 
 }  // namespace
@@ -129,6 +145,49 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
 
 hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
   return small_gemm::LaunchPlan<Int8Small>(stream, args, plan);
+}
+
+// Held against the other tiles' timing model as in fp32; what has to be packed,
+// split into planes or reordered for those costs them two to four launches.
+// This side is a fit to 16 to 4096 tiles and depths of 32 to 4096, where it takes
+// 3.9 us, 0.7 us (1.2) for every tile a CU has beyond the first, and to a KiB of
+// depth and tile 1.1 us on rows at whole dwords, more where operands are transposed
+// or lie at odd addresses. us per call, other route -> this: in place, 256 tiles x 512 6.5 -> 4.2,
+// x 4096 13.3 -> 8.9, 1024 (one round of 64x64) x 512 7.0 -> 8.3, 1152 x 512 11.7 -> 8.7, 2440 x
+// 1024 21.6 -> 18.9, 4096 x 1024 23.3 -> 31.2; rows of odd length, 256 x 1025 15.3 -> 7.2, 2440
+// x 1025 32.7 -> 29.9; int8 transposed 256 x 1024 10.6 -> 6.2; int16 transposed, its side
+// along the rows, 256 x 1024 14.4 -> 5.9, 2440 x 1024 33.4 -> 23.0; both transposed 256 x
+// 1024 16.9 -> 6.7.
+SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes,
+                                 bool int16_is_a) {
+  const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
+  const int K = args.k_valid;
+  plan.waves = 0;
+  if (K < 16 || tiles > 16 * num_cus) return plan;
+  const bool across8 = small_gemm::IsAcross(int16_is_a ? plan.source_b : plan.source_a);
+  const bool across16 = small_gemm::IsAcross(int16_is_a ? plan.source_a : plan.source_b);
+  const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b);
+  const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
+  const double to_a_kib = bytes ? (across8 || across16 ? 3.4 : 2.2) : across8 ? (across16 ? 2.2 : 1.7) : across16 ? 1.45 : 1.1;
+  const double here = 3.9 + (bytes && (across8 || across16) ? 1.2 : 0.7) * (a_cu - 1) + to_a_kib * a_cu * K / 1024.0;
+  // (The model counts plane vectors, 64 to 32 columns, with the int8 side along the rows.)
+  GemmArgs planes = args;
+  planes.M = int16_is_a ? args.N : args.M;
+  planes.N = ((int16_is_a ? args.M : args.N) + 31) / 32 * 64;
+  const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kInt8PlaneSplit);
+  double other = 1e30;
+  for (int i = 0; i < model.count; ++i)
+    other = std::min(other, mfma_gemm::ModelledMicroseconds(planes, num_cus, model, model.tiles[i]));
+  if (packed_bytes) other += 3.3 + 1.5e-6 * static_cast<double>(packed_bytes);
+  if (here >= other) return plan;
+  plan.waves = a_cu == 1 && K >= 256 ? 8 : 4;
+  plan.step = 64;
+  return plan;
+}
+
+hipError_t LaunchSmallGemmI8I16(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan, bool int16_is_a) {
+  return int16_is_a ? small_gemm::LaunchPlan<Int16Int8Small>(stream, args, plan)
+                    : small_gemm::LaunchPlan<Int8Int16Small>(stream, args, plan);
 }
 
 }  // namespace ruyamd

@@ -1077,6 +1077,88 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   return RUYAMD_OK;
 }
 
+// An int8 x int16 product on the small tiles, where the planner finds that better
+// (*done): with either type on either side and any storage order.
+int RunI8I16Small(ruyamd_ctx* ctx, MulCall* call, bool* done, std::string* err) {
+  const int M = call->lhs.rows, K = call->lhs.cols, N = call->rhs.cols;
+  const int side16 = call->lhs.dtype == RUYAMD_DTYPE_I16 ? 0 : 1;
+  const int side8 = 1 - side16;
+  const int policy16 = side16 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy;
+  if (ctx->forced_tile_rows || K < 16 || M <= kSkinnyKernelWidth || N <= kSkinnyKernelWidth ||
+      ShouldCache(policy16, side16 == 0 ? N : M))
+    return RUYAMD_OK;
+  GemmArgs args;
+  const bool swap = SetupDestination(*call, &args);
+  args.M = swap ? N : M;
+  args.N = swap ? M : N;
+  args.n_logical = args.N;
+  args.k_bytes = RoundUp(K, 16);
+  args.k_valid = K;
+  const bool int16_is_a = (side16 == 1) == swap;
+  auto view = [&](int side) {
+    const DevMat& m = side == 0 ? call->lhs : call->rhs;
+    return side == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
+                     : PackSource{m.data, m.cs, m.rs, m.cols, m.rows, m.dtype};
+  };
+  Operand8 a;
+  if (int rc = PrepareOperand8(ctx, call, side8, 0, /*need_sums=*/true,
+                               side8 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy,
+                               side8 == 0 ? call->lhs_src_key : call->rhs_src_key, side8 == 0 ? N : M,
+                               /*u8_depth_step=*/0, &a, err))
+    return rc;
+  if (int rc = EnsureOnDevice(ctx, call, side16, err)) return rc;
+  const PackSource src16 = view(side16);
+  Operand8 small;
+  SmallGemmSource source8, source16;
+  int32_t pitch16;
+  uint32_t bytes16;
+  if (!AsSmall(a, &small, &source8) || !SmallSourceOf(src16, &source16, &pitch16, &bytes16)) return RUYAMD_OK;
+  (int16_is_a ? args.b : args.a) = small.data;
+  (int16_is_a ? args.ldb : args.lda) = small.ld;
+  (int16_is_a ? args.b_bytes : args.a_bytes) = small.bytes;
+  (int16_is_a ? args.a : args.b) = src16.data;
+  (int16_is_a ? args.lda : args.ldb) = pitch16;
+  (int16_is_a ? args.a_bytes : args.b_bytes) = bytes16;
+  SmallGemmPlan plan;
+  plan.source_a = int16_is_a ? source16 : source8;
+  plan.source_b = int16_is_a ? source8 : source16;
+  // What the other tiles would need: planes of an int16 operand not in the
+  // kernels' layout, and a destination to reorder where it runs along the rows.
+  const uint64_t planes = uint64_t((src16.count + 31) / 32 * 64) * uint64_t(RoundUp(K, 16));
+  const bool in_place16 = source16 == kSmallRows && K % 16 == 0 && pitch16 % 16 == 0 && (reinterpret_cast<uintptr_t>(src16.data) & 15) == 0;
+  const uint64_t reordered = int16_is_a ? uint64_t(M) * uint64_t(N) * uint64_t(args.dst_elt) : 0;
+  if (planes >= (uint64_t(1) << 31) || reordered >= (uint64_t(1) << 31)) return RUYAMD_OK;
+  plan = PlanSmallGemmI8I16(args, ctx->multiprocessor_count, plan,
+                            uint64_t(a.unpacked) * a.bytes + (in_place16 ? 0 : planes) + reordered, int16_is_a);
+  if (plan.waves == 0) return RUYAMD_OK;
+  const bool sums_with_pack = a.unpacked && PackFormsSums(a.src, a.ld);
+  if (!HasRoomToPack(ctx, a.unpacked, a.bytes, sums_with_pack ? a.count : 0) ||
+      !HasRoomToPack(ctx, !in_place16, static_cast<uint32_t>(planes), 0) ||
+      !HasRoomToPack(ctx, reordered != 0, static_cast<uint32_t>(reordered), 0)) {
+    *err = "workspace allocation failed";
+    return RUYAMD_E_HIP;
+  }
+  // The low plane stores (v & 0xff) - 128.
+  args.ep.zp_product_depth = 0;
+  args.ep.lhs_zero_point = args.ep.rhs_zero_point = 0;
+  if (small.sums) {  // (from the cache)
+    (int16_is_a ? args.ep.lhs_zero_point : args.ep.rhs_zero_point) = -128;
+    (int16_is_a ? args.ep.rhs_sums : args.ep.lhs_sums) = small.sums;
+  } else {
+    (int16_is_a ? args.fused_b_factor : args.fused_a_factor) = -128;
+  }
+  const bool timed = ctx->TimingBegin();
+  const hipError_t launched = LaunchSmallGemmI8I16(ctx->LaunchStream(), args, plan, int16_is_a);
+  if (timed) ctx->TimingEnd();
+  if (launched != hipSuccess) {
+    *err = "int8 x int16 matrix-core kernel launch failed";
+    return RUYAMD_E_HIP;
+  }
+  ctx->last_kernel = RUYAMD_KERNEL_I8I16_MFMA;
+  *done = true;
+  return RUYAMD_OK;
+}
+
 }  // namespace
 
 int RunMulBatch(ruyamd_ctx* ctx, const MulCall& first, const BatchBuffers* items, int n, bool* handled,
@@ -1268,6 +1350,9 @@ int RunTuned(ruyamd_ctx* ctx, MulCall* call, TunedPath path, std::string* err) {
     case TunedPath::kF32:
       return RunF32(ctx, call, err);
     case TunedPath::kInt8Int16: {
+      bool done = false;
+      if (int rc = RunI8I16Small(ctx, call, &done, err)) return rc;
+      if (done) return RUYAMD_OK;
       // The kernel wants the int8 side along the destination's contiguous dimension.
       const bool dst_col_major = call->dst.rs == 1;
       const DevMat& contiguous_side = dst_col_major ? call->lhs : call->rhs;

@@ -250,6 +250,7 @@ def test_small_products_on_two_workgroups_a_cu(device_ctx):
 
 
 @pytest.mark.parametrize("tup", [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I16), (S.I8, S.U8, S.I32, S.I32),
+                                 (S.I8, S.I16, S.I32, S.I16), (S.I16, S.I8, S.I32, S.I32),
                                  (S.F32, S.F32, S.F32, S.F32)], ids=cases.tuple_name)
 @pytest.mark.parametrize("depth", [4, 16, 17, 31, 63, 64, 65, 127, 128, 131, 255, 257, 511, 513, 1029, 2049, 4095])
 def test_products_on_tiles_of_32(device_ctx, tup, depth):
@@ -265,7 +266,7 @@ def test_products_on_tiles_of_32(device_ctx, tup, depth):
             p = W.random_problem(rng, *tup, rows, depth, cols, *orders, strided=(depth + n) % 3 == 0,
                                  name="tiles of 32 %dx%dx%d %s" % (rows, depth, cols, orders))
             p.lhs.cache_policy = S.CACHE_ALWAYS if (depth + n) % 4 == 0 else S.CACHE_NEVER
-            for misalign in (0, 4 if tup[0] == S.F32 else 1):
+            for misalign in (0, 1):
                 compare(p, D.device_mul(device_ctx, p, misalign=misalign), expected(p), exact_fp=False)
                 device_ctx.clear_prepacked_cache()
 
@@ -291,7 +292,7 @@ def test_fp32_rows_of_any_depth_in_place(device_ctx, tile, depth):
                 for v in range(outer):
                     pad[v * m.stride:v * m.stride + depth] = False
                 view[pad] = np.nan
-            compare(p, D.device_mul(device_ctx, p, misalign=4), expected(p), exact_fp=False)
+            compare(p, D.device_mul(device_ctx, p, misalign=1), expected(p), exact_fp=False)
     finally:
         device_ctx.force_tile(0, 0)
 
