@@ -183,6 +183,7 @@ enum SmallGemmSource { kSmallRows, kSmallRowsBytes, kSmallAcross, kSmallAcrossBy
 struct SmallGemmPlan {
   int waves = 0;   // of a workgroup; 0: not for the small tiles
   int step = 128;  // bytes of depth
+  int tile = 32;   // rows and columns
   int source_a = kSmallRows, source_b = kSmallRows;
 };
 // Uses of GemmArgs: k_valid is the depth in bytes (at least 16), lda and ldb the
@@ -199,8 +200,8 @@ hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const Sma
 hipError_t LaunchSmallGemmF32(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan);
 // int8 x int16, the int16 side (`int16_is_a`: the rows) as it lies: k_valid counts
 // depth positions, N destination columns, and the fused factor of the int8 side
-// is -128.
-SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes,
+// is -128. `packs`: the launches that the other tiles would need besides theirs.
+SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, int packs, uint64_t packed_bytes,
                                  bool int16_is_a);
 hipError_t LaunchSmallGemmI8I16(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan, bool int16_is_a);
 // `count` <= kGemmBatchMax products of the shape and parameters of `args`, each

@@ -16,6 +16,7 @@ namespace ruyamd {
 // In rounds it loses to larger tiles on packed operands: 2048 x 251 x 2048
 // (1024 tiles of 64x64) 11.1 packed and 11.7 staged, 1500 x 1000 x 1500 (576)
 // 17.1 and 21.8.
+// (What the 32x32 tiles take, PlanSmallGemmI8, never gets here.)
 // Operands that can be used in place gain less, since nothing is packed (us per
 // call, direct -> staged). Up to 384 bytes of depth the direct loads are as good
 // on one workgroup a CU (256^3 4.8, staged 5.0), from 900 on the schedule that

@@ -1,7 +1,8 @@
 // Matrix-core GEMM for products whose run time is that of a launch, a trip to
 // memory and a write-back: 32x32 tiles, so that few destination values still
 // keep every CU busy, and operands of any layout and alignment read where they
-// lie, so that no pack launch stands in front.
+// lie, so that no pack launch stands in front. (8-bit operands also on tiles of
+// 64x64, for grids in between that would otherwise need one.)
 //
 // One workgroup per tile. The depth is dealt to its waves in steps of S bytes:
 // wave w takes steps w, w + kWaves, ..., computes the whole tile for them and
@@ -44,8 +45,6 @@ using granule::PlaceGranule;
 using granule::v4i;
 typedef v4i v4i_dwords __attribute__((aligned(4)));
 
-constexpr int kTile = 32;  // rows and columns
-
 RUYAMD_HOST_DEVICE constexpr bool IsAcross(int source) {
   return source == kSmallAcross || source == kSmallAcrossBytes;
 }
@@ -63,11 +62,11 @@ __device__ __forceinline__ int SlotOffset(int r, int g) {
 
 // The kTile vectors of one operand that a tile needs, from vector `first` on.
 // kElement: bytes of a value. Values of two bytes become two planes of int8, high
-// and low byte (minus 128), which lie in the slot as 32 vectors each: v = 256 high
+// and low byte (minus 128), which lie in the slot one behind the other: v = 256 high
 // + low + 128. Across the vectors their bytes are what a piece transposes: byte 2 v
 // of a depth position belongs to the low plane of vector v, the next one to the
 // high plane.
-template <int S, int kSource, int kElement>
+template <int kTile, int S, int kSource, int kElement>
 struct Side {
   static constexpr bool kAcross = IsAcross(kSource);
   static constexpr bool kAnyByte = IsAnyByte(kSource);
@@ -222,9 +221,14 @@ struct Side {
         *reinterpret_cast<v4i*>(slot + SlotOffset<S>(kTile + vector, DepthOf(u) / 16)) = low;
       } else if constexpr (!kAcross) {
         if constexpr (kElement == 1) {
+          if (partial) {
 #pragma unroll
-          for (int d = 0; d < 4; ++d)  // (the padding stays zero)
-            x[0][d] ^= static_cast<int>(partial ? flip & LowBytes(bytes - k - 4 * d) : flip);
+            for (int d = 0; d < 4; ++d)  // (the padding stays zero)
+              x[0][d] ^= static_cast<int>(flip & LowBytes(bytes - k - 4 * d));
+          } else {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) x[0][d] ^= static_cast<int>(flip);
+          }
         }
         *reinterpret_cast<v4i*>(slot + SlotOffset<S>(vector, DepthOf(u) / 16)) = x[0];
       } else if constexpr (kElement == 4) {
@@ -266,21 +270,23 @@ struct Side {
 // runs of 32 columns padded by one so that a column's pieces lie in different
 // banks); behind that the partial sums of the tile's vectors and the
 // write-back parameters of its rows and columns.
-template <int S, int kWaves, int kSlotVectors>
+template <int kTile, int S, int kWaves, int kSlotVectors>
 struct Memory {
   static constexpr int kVectors = 2 * kTile;
   static constexpr int kSlot = kSlotVectors * S;
-  static constexpr int kPart = 8 * 33;  // granules of a wave's partial tile
+  static constexpr int kBlocks = kTile / 32;              // 32 x 32 blocks each way
+  static constexpr int kPart = kBlocks * kBlocks * 8 * 33;  // granules of a wave's partial tile
   static constexpr int kSums = std::max(kWaves * kSlot, kWaves * kPart * 16);
   static constexpr int kParams = kSums + kWaves * kVectors * 4;
   static constexpr int kBytes = kParams + 3 * kVectors * 4;
 };
 
-template <typename T, int S, int kWaves, int kSourceA, int kSourceB>
+template <typename T, int kTile, int S, int kWaves, int kSourceA, int kSourceB>
 __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void SmallGemmKernel(GemmArgs args) {
-  using SideA = Side<S, kSourceA, T::kElementA>;
-  using SideB = Side<S, kSourceB, T::kElementB>;
-  using Mem = Memory<S, kWaves, SideA::kSlotVectors + SideB::kSlotVectors>;
+  using SideA = Side<kTile, S, kSourceA, T::kElementA>;
+  using SideB = Side<kTile, S, kSourceB, T::kElementB>;
+  using Mem = Memory<kTile, S, kWaves, SideA::kSlotVectors + SideB::kSlotVectors>;
+  constexpr int kBlocks = Mem::kBlocks;
   constexpr int kSubSteps = S / 32;
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -339,12 +345,19 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
   constexpr bool kPlanes = SideA::kPlanes || SideB::kPlanes;
   constexpr bool kInteger = T::kElementA != 4;
   constexpr int kChains = kPlanes ? 2 : kInteger ? 1 : kWaves == 8 ? 4 : 2;
-  typename T::Acc acc[kChains];
+  static_assert(kBlocks == 1 || kChains == 1, "the larger tile exists for 8-bit operands");
+  typename T::Acc acc[kBlocks][kBlocks][kChains];
+  int sum_a[kBlocks], sum_b[kBlocks];
 #pragma unroll
-  for (int c = 0; c < kChains; ++c)
+  for (int x = 0; x < kBlocks; ++x) {
+    sum_a[x] = sum_b[x] = 0;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[c][v] = 0;
-  int sum_a = 0, sum_b = 0;
+    for (int y = 0; y < kBlocks; ++y)
+#pragma unroll
+      for (int c = 0; c < kChains; ++c)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[x][y][c][v] = 0;
+  }
   const bool sums_of_a = T::kElementA == 1 && args.fused_a_factor != 0;
   const bool sums_of_b = T::kElementB == 1 && args.fused_b_factor != 0;
 
@@ -363,37 +376,46 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    v4i fa[kSubSteps], fb[kSubSteps], low[kPlanes ? kSubSteps : 1];
+    v4i fa[kSubSteps][kBlocks], fb[kSubSteps][kBlocks], low[kPlanes ? kSubSteps : 1];
 #pragma unroll
     for (int ks = 0; ks < kSubSteps; ++ks) {
       // (32 vectors further on the swizzle is the same.)
       const int offset = SlotOffset<S>(lane & 31, ks * 2 + lane / 32);
-      fa[ks] = *reinterpret_cast<const v4i*>(slot + offset);
-      fb[ks] = *reinterpret_cast<const v4i*>(slot + SideA::kSlotVectors * S + offset);
+#pragma unroll
+      for (int x = 0; x < kBlocks; ++x) {
+        fa[ks][x] = *reinterpret_cast<const v4i*>(slot + x * 32 * S + offset);
+        fb[ks][x] = *reinterpret_cast<const v4i*>(slot + (SideA::kSlotVectors + x * 32) * S + offset);
+      }
       if constexpr (kPlanes)
         low[ks] = *reinterpret_cast<const v4i*>(slot + (SideA::kPlanes ? kTile : SideA::kSlotVectors + kTile) * S + offset);
     }
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < kSubSteps; ++ks) {
       if constexpr (kPlanes) {
-        T::Mma(fa[ks], fb[ks], acc[0]);
-        T::Mma(SideA::kPlanes ? low[ks] : fa[ks], SideB::kPlanes ? low[ks] : fb[ks], acc[1]);
+        T::Mma(fa[ks][0], fb[ks][0], acc[0][0][0]);
+        T::Mma(SideA::kPlanes ? low[ks] : fa[ks][0], SideB::kPlanes ? low[ks] : fb[ks][0], acc[0][0][1]);
       } else {
-        T::Mma(fa[ks], fb[ks], acc, ks);
+#pragma unroll
+        for (int x = 0; x < kBlocks; ++x)
+#pragma unroll
+          for (int y = 0; y < kBlocks; ++y) T::Mma(fa[ks][x], fb[ks][y], acc[x][y], ks);
       }
     }
     if (sums_of_a) {
 #pragma unroll
       for (int ks = 0; ks < kSubSteps; ++ks)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) sum_a = __builtin_amdgcn_sdot4(fa[ks][d], 0x01010101, sum_a, false);
+        for (int x = 0; x < kBlocks; ++x)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) sum_a[x] = __builtin_amdgcn_sdot4(fa[ks][x][d], 0x01010101, sum_a[x], false);
     }
     if (sums_of_b) {
 #pragma unroll
       for (int ks = 0; ks < kSubSteps; ++ks)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) sum_b = __builtin_amdgcn_sdot4(fb[ks][d], 0x01010101, sum_b, false);
+        for (int x = 0; x < kBlocks; ++x)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) sum_b[x] = __builtin_amdgcn_sdot4(fb[ks][x][d], 0x01010101, sum_b[x], false);
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -422,100 +444,116 @@ __global__ __launch_bounds__(64 * kWaves, kWaves > 4 ? kWaves / 4 : 2) void Smal
   int* const area = reinterpret_cast<int*>(lds + Mem::kParams);
   if (my_steps > 0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      v4i w;
+    for (int x = 0; x < kBlocks; ++x)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        typename T::Value sum = acc[0][4 * q + e];
-        if constexpr (kPlanes) sum = static_cast<int>(256u * static_cast<uint32_t>(sum) + static_cast<uint32_t>(acc[1][4 * q + e]));
-        if constexpr (kChains == 2 && !kPlanes) sum += acc[1][4 * q + e];
-        if constexpr (kChains == 4) sum = (sum + acc[1][4 * q + e]) + (acc[2][4 * q + e] + acc[3][4 * q + e]);
-        w[e] = T::Bits(sum);
-      }
-      // Rows 8 q + 4 (lane / 32) .. + 3 of column lane % 32.
-      parts[wave * Mem::kPart + (2 * q + lane / 32) * 33 + (lane & 31)] = w;
-    }
+      for (int y = 0; y < kBlocks; ++y)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v4i w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const auto& of = acc[x][y];
+            typename T::Value sum = of[0][4 * q + e];
+            if constexpr (kPlanes)
+              sum = static_cast<int>(256u * static_cast<uint32_t>(sum) + static_cast<uint32_t>(of[1][4 * q + e]));
+            if constexpr (kChains == 2 && !kPlanes) sum += of[1][4 * q + e];
+            if constexpr (kChains == 4) sum = (sum + of[1][4 * q + e]) + (of[2][4 * q + e] + of[3][4 * q + e]);
+            w[e] = T::Bits(sum);
+          }
+          // Rows 8 q + 4 (lane / 32) .. + 3 of column lane % 32 of the block.
+          parts[wave * Mem::kPart + ((x * kBlocks + y) * 8 + 2 * q + lane / 32) * 33 + (lane & 31)] = w;
+        }
     // Lanes l and l + 32 hold the two halves of a vector's sum.
     auto put = [&](int value, int vector) {
       const auto halves = __builtin_amdgcn_permlane32_swap(value, value, false, false);
       if (lane < 32) sums[wave * Mem::kVectors + vector + lane] = halves[0] + halves[1];
     };
-    if (sums_of_a) put(sum_a, 0);
-    if (sums_of_b) put(sum_b, kTile);
+#pragma unroll
+    for (int x = 0; x < kBlocks; ++x) {
+      if (sums_of_a) put(sum_a[x], x * 32);
+      if (sums_of_b) put(sum_b[x], kTile + x * 32);
+    }
   }
   if (tid < Mem::kVectors) T::StageParams(args.ep, is_row, params, area + tid, Mem::kVectors);
   __syncthreads();
 
-  // A thread finishes four consecutive rows of a column.
-  if (tid >= kTile * kTile / 4) return;
-  const int row = tid % 8 * 4, col = tid / 8;
+  // A thread finishes four consecutive rows of a column. (A loop, not a lambda: in
+  // one, captured, the kernel's arguments lie in memory for the compiler, and what a
+  // lane chooses between two of them above becomes a load a lane from there, which
+  // waits for all operand loads. 1024 x 1024 x 196 per channel: 5.5 us so, 5.0 with the loop.)
   const int active = min(steps, kWaves);
-  typename T::Value value[4] = {0, 0, 0, 0};
-  uint32_t of_column = 0, of_row[4] = {0, 0, 0, 0};
+  constexpr int kQuads = kTile * kTile / 4;
+#pragma unroll 1
+  for (int quad = tid; quad < kQuads; quad += std::min(kQuads, 64 * kWaves)) {
+    const int row = quad % (kTile / 4) * 4, col = quad / (kTile / 4);
+    typename T::Value value[4] = {0, 0, 0, 0};
+    uint32_t of_column = 0, of_row[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    if (w < active) {
-      const v4i x = parts[w * Mem::kPart + row / 4 * 33 + col];
+    for (int w = 0; w < kWaves; ++w) {
+      if (w < active) {
+        const v4i x = parts[w * Mem::kPart + ((row / 32 * kBlocks + col / 32) * 8 + row % 32 / 4) * 33 + col % 32];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) value[e] += T::FromBits(x[e]);
-      if (sums_of_a) {
-        const v4i s = *reinterpret_cast<const v4i*>(sums + w * Mem::kVectors + row);
+        for (int e = 0; e < 4; ++e) value[e] += T::FromBits(x[e]);
+        if (sums_of_a) {
+          const v4i s = *reinterpret_cast<const v4i*>(sums + w * Mem::kVectors + row);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) of_row[e] += static_cast<uint32_t>(s[e]);
+          for (int e = 0; e < 4; ++e) of_row[e] += static_cast<uint32_t>(s[e]);
+        }
+        if (sums_of_b) of_column += static_cast<uint32_t>(sums[w * Mem::kVectors + kTile + col]);
       }
-      if (sums_of_b) of_column += static_cast<uint32_t>(sums[w * Mem::kVectors + kTile + col]);
     }
-  }
-  if constexpr (kInteger) {
+    if constexpr (kInteger) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      value[e] = static_cast<int>(static_cast<uint32_t>(value[e]) - static_cast<uint32_t>(args.fused_a_factor) * of_row[e] -
-                                  static_cast<uint32_t>(args.fused_b_factor) * of_column);
-  }
-  int vals[4];
-  T::Finish(value, area, Mem::kVectors, row, kTile + col, args.ep, vals);
-  const int i0 = m0 + row, j = n0 + col;
-  if (j >= args.N || i0 >= args.M) return;
-  char* const out = static_cast<char*>(args.dst.data) + (int64_t(j) * args.dst.cs + i0) * args.dst_elt;
-  // (Stores of any width take any address.)
-  if (i0 + 4 <= args.M) {
-    if (args.dst_elt == 1) {
-      const uint32_t w = uint32_t(vals[0] & 0xff) | uint32_t(vals[1] & 0xff) << 8 | uint32_t(vals[2] & 0xff) << 16 |
-                         uint32_t(vals[3]) << 24;
-      __builtin_memcpy(out, &w, sizeof(w));
-    } else if (args.dst_elt == 2) {
-      const uint32_t w[2] = {uint32_t(vals[0] & 0xffff) | uint32_t(vals[1]) << 16,
-                             uint32_t(vals[2] & 0xffff) | uint32_t(vals[3]) << 16};
-      __builtin_memcpy(out, w, sizeof(w));
+      for (int e = 0; e < 4; ++e)
+        value[e] = static_cast<int>(static_cast<uint32_t>(value[e]) - static_cast<uint32_t>(args.fused_a_factor) * of_row[e] -
+                                    static_cast<uint32_t>(args.fused_b_factor) * of_column);
+    }
+    int vals[4];
+    T::Finish(value, area, Mem::kVectors, row, kTile + col, args.ep, vals);
+    const int i0 = m0 + row, j = n0 + col;
+    if (j >= args.N || i0 >= args.M) continue;
+    char* const out = static_cast<char*>(args.dst.data) + (int64_t(j) * args.dst.cs + i0) * args.dst_elt;
+    // (Stores of any width take any address.)
+    if (i0 + 4 <= args.M) {
+      if (args.dst_elt == 1) {
+        const uint32_t w = uint32_t(vals[0] & 0xff) | uint32_t(vals[1] & 0xff) << 8 | uint32_t(vals[2] & 0xff) << 16 |
+                           uint32_t(vals[3]) << 24;
+        __builtin_memcpy(out, &w, sizeof(w));
+      } else if (args.dst_elt == 2) {
+        const uint32_t w[2] = {uint32_t(vals[0] & 0xffff) | uint32_t(vals[1]) << 16,
+                               uint32_t(vals[2] & 0xffff) | uint32_t(vals[3]) << 16};
+        __builtin_memcpy(out, w, sizeof(w));
+      } else {
+        __builtin_memcpy(out, vals, sizeof(vals));
+      }
     } else {
-      __builtin_memcpy(out, vals, sizeof(vals));
-    }
-  } else {
 #pragma unroll
-    for (int e = 0; e < 3; ++e) {
-      if (i0 + e < args.M) {
-        if (args.dst_elt == 1)
-          reinterpret_cast<int8_t*>(out)[e] = static_cast<int8_t>(vals[e]);
-        else if (args.dst_elt == 2)
-          reinterpret_cast<int16_t*>(out)[e] = static_cast<int16_t>(vals[e]);
-        else
-          reinterpret_cast<int32_t*>(out)[e] = vals[e];
+      for (int e = 0; e < 3; ++e) {
+        if (i0 + e < args.M) {
+          if (args.dst_elt == 1)
+            reinterpret_cast<int8_t*>(out)[e] = static_cast<int8_t>(vals[e]);
+          else if (args.dst_elt == 2)
+            reinterpret_cast<int16_t*>(out)[e] = static_cast<int16_t>(vals[e]);
+          else
+            reinterpret_cast<int32_t*>(out)[e] = vals[e];
+        }
       }
     }
   }
 }
 
-template <typename T, int S, int kWaves, int kSourceA, int kSourceB>
+template <typename T, int kTile, int S, int kWaves, int kSourceA, int kSourceB>
 hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
-  using Mem = Memory<S, kWaves, Side<S, kSourceA, T::kElementA>::kSlotVectors + Side<S, kSourceB, T::kElementB>::kSlotVectors>;
+  using Mem = Memory<kTile, S, kWaves,
+                     Side<kTile, S, kSourceA, T::kElementA>::kSlotVectors + Side<kTile, S, kSourceB, T::kElementB>::kSlotVectors>;
   // (Rows: a granule must fit; across: 16 bytes of vectors.)
   if (args.k_valid < 16 || args.M < 16 || args.N < 16 || args.split_k != 1 || args.row_sums) return hipErrorInvalidValue;
   const int64_t total = int64_t((args.M + kTile - 1) / kTile) * ((args.N + kTile - 1) / kTile);
   if (total > (1 << 24)) return hipErrorInvalidValue;
   const int grid = static_cast<int>((total + 7) / 8 * 8);
-  auto kernel = SmallGemmKernel<T, S, kWaves, kSourceA, kSourceB>;
+  auto kernel = SmallGemmKernel<T, kTile, S, kWaves, kSourceA, kSourceB>;
   if (Mem::kBytes > 48 * 1024) {
-    // Once per process; static initialisation is safe against concurrent callers.
+    // Once per process and kernel; static initialisation is safe against concurrent callers.
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, Mem::kBytes);
     if (attr != hipSuccess) return attr;
@@ -526,32 +564,39 @@ hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
 
 // The instantiation for a plan. Operands at any byte: both sides' byte forms
 // (which read aligned ones as well).
-template <typename T, int S, int kWaves>
+template <typename T, int kTile, int S, int kWaves>
 hipError_t LaunchSources(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
   const bool across_a = IsAcross(plan.source_a), across_b = IsAcross(plan.source_b);
   const bool bytes = IsAnyByte(plan.source_a) || IsAnyByte(plan.source_b);
   if constexpr (T::kElementA != 4) {
     if (bytes) {
-      if (across_a && across_b) return Launch<T, S, kWaves, kSmallAcrossBytes, kSmallAcrossBytes>(stream, args);
-      if (across_a) return Launch<T, S, kWaves, kSmallAcrossBytes, kSmallRowsBytes>(stream, args);
-      if (across_b) return Launch<T, S, kWaves, kSmallRowsBytes, kSmallAcrossBytes>(stream, args);
-      return Launch<T, S, kWaves, kSmallRowsBytes, kSmallRowsBytes>(stream, args);
+      if (across_a && across_b) return Launch<T, kTile, S, kWaves, kSmallAcrossBytes, kSmallAcrossBytes>(stream, args);
+      if (across_a) return Launch<T, kTile, S, kWaves, kSmallAcrossBytes, kSmallRowsBytes>(stream, args);
+      if (across_b) return Launch<T, kTile, S, kWaves, kSmallRowsBytes, kSmallAcrossBytes>(stream, args);
+      return Launch<T, kTile, S, kWaves, kSmallRowsBytes, kSmallRowsBytes>(stream, args);
     }
   }
   if (bytes) return hipErrorInvalidValue;
-  if (across_a && across_b) return Launch<T, S, kWaves, kSmallAcross, kSmallAcross>(stream, args);
-  if (across_a) return Launch<T, S, kWaves, kSmallAcross, kSmallRows>(stream, args);
-  if (across_b) return Launch<T, S, kWaves, kSmallRows, kSmallAcross>(stream, args);
-  return Launch<T, S, kWaves, kSmallRows, kSmallRows>(stream, args);
+  if (across_a && across_b) return Launch<T, kTile, S, kWaves, kSmallAcross, kSmallAcross>(stream, args);
+  if (across_a) return Launch<T, kTile, S, kWaves, kSmallAcross, kSmallRows>(stream, args);
+  if (across_b) return Launch<T, kTile, S, kWaves, kSmallRows, kSmallAcross>(stream, args);
+  return Launch<T, kTile, S, kWaves, kSmallRows, kSmallRows>(stream, args);
 }
 template <typename T>
 hipError_t LaunchPlan(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
-  if (plan.step == 64 && plan.waves == 4) return LaunchSources<T, 64, 4>(stream, args, plan);
-  if (plan.step == 64 && plan.waves == 8) return LaunchSources<T, 64, 8>(stream, args, plan);
+  if (plan.tile == 64) {
+    if constexpr (T::kElementA == 1 && T::kElementB == 1) {
+      if (plan.step == 64 && plan.waves == 4) return LaunchSources<T, 64, 64, 4>(stream, args, plan);
+      if (plan.step == 64 && plan.waves == 8) return LaunchSources<T, 64, 64, 8>(stream, args, plan);
+    }
+    return hipErrorInvalidValue;
+  }
+  if (plan.step == 64 && plan.waves == 4) return LaunchSources<T, 32, 64, 4>(stream, args, plan);
+  if (plan.step == 64 && plan.waves == 8) return LaunchSources<T, 32, 64, 8>(stream, args, plan);
   if constexpr (T::kElementA != 2 && T::kElementB != 2) {
-    if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 128, 4>(stream, args, plan);
-    if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 128, 8>(stream, args, plan);
-    if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 128, 16>(stream, args, plan);
+    if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 32, 128, 4>(stream, args, plan);
+    if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 32, 128, 8>(stream, args, plan);
+    if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 32, 128, 16>(stream, args, plan);
   }
   return hipErrorInvalidValue;
 }

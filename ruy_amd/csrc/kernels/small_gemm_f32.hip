@@ -78,7 +78,9 @@ SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan 
   for (int i = 0; i < model.count; ++i)
     other = std::min(other, mfma_gemm::ModelledMicroseconds(args, num_cus, model, model.tiles[i]));
   if (packed_bytes) other += 2.3 + 0.5e-6 * static_cast<double>(packed_bytes);
-  if (here >= other) return plan;
+  // (In place on both sides the models have to differ by more than they err: 1630
+  // tiles x 752 are 29.9 us on the larger tiles, 31.5 by their model, and 30.6 here.)
+  if (here >= (packed_bytes ? 1.0 : 0.95) * other) return plan;
   plan.waves = 4;
   plan.step = 64;
   if (a_cu == 1) {

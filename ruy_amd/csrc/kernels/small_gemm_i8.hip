@@ -82,63 +82,89 @@ struct Int16Int8Small : Int8Small {
   static constexpr int kElementA = 2, kElementB = 1;
 };
 
+// Whether an operand's runs do not all start at multiples of 16 bytes. Across the
+// vectors, 16-byte loads of such runs cost what those at odd addresses do (1000^3,
+// int8 transposed, int16 along the rows: 12.7 us expected, 21.2 measured).
+bool Straddling(const GemmArgs& args) {
+  return ((reinterpret_cast<uintptr_t>(args.a) | reinterpret_cast<uintptr_t>(args.b) | static_cast<uint32_t>(args.lda) |
+           static_cast<uint32_t>(args.ldb)) & 15) != 0;
+}
+
 }  // namespace
 
 // What the tiles of 32x32 win on is the time that does not depend on the work:
 // no pack launch (2.5 us and more), a quarter of the loads, of the adding up and
 // of the write-back of a 64x64 tile to a workgroup. What they lose is reuse: they
-// read an operand byte twice as often. So the lines run along tiles to a CU, with
-// a limit on the depth from where the two sides met on a grid of depths (64 to
-// 8192) and of 16 to 1536 tiles (us, other route -> this):
-//   used in place: 256 tiles x 512 5.2 -> 3.9, x 1024 6.8 -> 4.4, x 8192 11.8 -> 10.1;
-//     512 x 2048 8.0 -> 6.8, x 4096 10.3 -> 9.5, x 8192 14.3 -> 16.1; 768 x 1024
-//     6.9 -> 6.1, x 2048 7.9 -> 8.2; 1024 x 512 5.5 -> 5.5.
-//   packed by rows otherwise: 256 x 257 6.1 -> 4.5, x 2049 12.9 -> 7.8, x 8193 23.1 ->
-//     15.3; 512 x 1025 10.3 -> 7.5, x 4097 18.2 -> 15.3; 768 x 1025 10.7 -> 9.1, x
-//     4097 20.5 -> 19.6; 1024 x 65 5.0 -> 4.9, x 513 7.7 -> 8.0.
-//   one side transposed, at whole dwords: 256 x 512 8.2 -> 4.4, x 8192 19.0 -> 15.2; 512 x
-//     4096 16.4 -> 15.3; 768 x 1024 10.0 -> 9.4; 1024 x 512 8.5 -> 7.6, x 1024 10.1 ->
-//     11.4; 1536 x 256 9.0 -> 7.7, x 512 10.1 -> 10.5.
-//   ... and at odd bytes: 256 x 8192 22.5 -> 21.5; 512 x 2048 13.4 -> 12.4, x 4096
-//     19.3 -> 20.8; 768 x 512 8.9 -> 8.1, x 1024 11.4 -> 11.5; 1024 x 128 7.4 -> 7.1.
+// read an operand byte twice as often; the form with 64x64 tiles and the depth
+// dealt to eight waves lies in between where operands would have to be packed. So
+// the lines run along tiles to a CU (a_cu: of 32x32), with limits on the depth from
+// where the sides met on a grid of 64 to 2048 tiles and depths of 64 to 8192, three
+// sets of buffers in turn (us, other route -> this):
+//   used in place: 256 tiles x 512 5.3 -> 4.5, x 1024 6.9 -> 4.8, x 4096 10.8 -> 8.2;
+//     512 x 288 4.8 -> 5.0, x 1024 6.9 -> 5.7, x 2048 8.1 -> 7.8, x 4096 11.1 -> 11.3; 768 x
+//     1024 6.9 -> 6.8, x 1504 7.7 -> 9.2; 1024 x 512 5.5 -> 6.5.
+//   packed by rows otherwise: 256 x 289 6.2 -> 4.9, x 2049 13.6 -> 7.6, x 5697 17.2 ->
+//     12.3; 512 x 1025 11.4 -> 7.9, x 2049 13.9 -> 10.6, x 4097 15.8 -> 16.7; 768 x 1025
+//     11.6 -> 9.4, x 1505 12.5 -> 10.9, on 64x64 x 2049 13.3 -> 13.0; 1024 x 289 6.3 -> 6.6, x
+//     1025 11.7 -> 10.8, on 64x64 x 1505 12.5 -> 11.8, x 2049 13.1 -> 14.1.
+//   one side transposed, at whole dwords: 256 x 512 8.3 -> 4.6, x 5696 16.7 -> 14.1; 512 x
+//     1024 10.1 -> 7.8, x 2048 11.7 -> 10.6, x 4096 15.3 -> 17.7; 768 x 288 7.5 -> 6.4, on
+//     64x64 x 1024 10.2 -> 9.0, x 1504 11.8 -> 10.7, x 2048 11.5 -> 11.7; 1024 x 288 7.5 -> 6.8,
+//     x 1024 10.3 -> 9.4, x 1504 11.6 -> 11.4; with four waves 2048 x 256 9.0 -> 7.9.
+//   ... and at odd bytes: 256 x 1025 11.0 -> 8.5, x 4097 16.3 -> 16.1, x 5697 18.9 -> 19.0;
+//     512 x 513 9.0 -> 8.5, on 64x64 x 1025 11.9 -> 10.6, x 1505 12.7 -> 12.0, x 2049 14.0 ->
+//     14.9; 768 x 289 8.0 -> 7.2, x 1025 12.5 -> 10.9, x 1505 13.1 -> 13.1; 1024 x 1025 12.7 ->
+//     11.2, x 1505 13.0 -> 14.3; with four waves 2048 x 256 9.4 -> 8.8.
 // More waves to a workgroup, or longer steps, where the grid leaves CUs room for
-// them: 256 tiles in place x 1024 5.2 with four waves, 4.7 with eight; packed x 4097
-// 12.1 and 9.1; transposed x 8192 17.8 with eight, 16.8 with sixteen.
+// them: 256 tiles in place x 4096 8.8 with four waves, 8.2 with eight; packed x 4097
+// 12.9 and 10.4; transposed x 4096 11.3 with eight, 10.6 with sixteen.
 SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
+  const int64_t tiles64 = int64_t((args.M + 63) / 64) * ((args.N + 63) / 64);
   const int K = args.k_valid;
   const bool across = small_gemm::IsAcross(plan.source_a) || small_gemm::IsAcross(plan.source_b);
-  const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b);
-  const int a_cu = tiles <= num_cus ? 1 : tiles <= 2 * num_cus ? 2 : 4 * tiles <= 13 * num_cus ? 3 : tiles <= 4 * num_cus ? 4 : 6;
-  int deepest = 0;
-  if (tiles > 6 * num_cus || K < 16) {
-    deepest = 0;
-  } else if (across) {
-    deepest = a_cu == 1 ? 8192 : a_cu == 2 ? (bytes ? 2048 : 4096) : a_cu == 3 ? (bytes ? 512 : 1024)
-              : a_cu == 4 ? (bytes ? 128 : 512) : 256;
-  } else if (packed_bytes) {
-    deepest = a_cu == 1 ? 8192 : a_cu <= 3 ? 4100 : a_cu == 4 ? 128 : 0;
-  } else {
-    deepest = a_cu == 1 ? 8192 : a_cu == 2 ? 4096 : a_cu == 3 ? 1024 : 0;
-  }
+  const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b) ||
+                     (across && Straddling(args));
+  const int a_cu = tiles <= num_cus ? 1 : tiles <= 2 * num_cus ? 2 : 4 * tiles <= 13 * num_cus ? 3 : tiles <= 4 * num_cus ? 4 : 8;
   plan.waves = 0;
-  if (K > deepest) return plan;
+  if (tiles > 8 * num_cus || K < 16) return plan;
+  // Depths in [from32, to32] are for the 32x32 tiles, above that to to64 for the
+  // 64x64 ones.
+  int from32 = 16, to32 = 0, to64 = 0;
+  if (across) {
+    to32 = a_cu == 1 ? (bytes ? 4352 : 8192) : a_cu == 2 ? (bytes ? 700 : 2560) : a_cu == 3 ? (bytes ? 200 : 400) : a_cu == 4 ? 200 : 0;
+    to64 = a_cu == 1 ? 0 : a_cu == 2 ? (bytes ? 1600 : 0) : a_cu == 3 ? (bytes ? 1250 : 1800) : a_cu == 4 ? (bytes ? 1250 : 1400) : 300;
+  } else if (packed_bytes) {
+    from32 = a_cu == 4 && K > 128 ? 960 : 16;
+    to32 = a_cu == 1 ? 8192 : a_cu == 2 ? 2560 : a_cu == 3 ? 1536 : a_cu == 4 ? 1300 : 0;
+    to64 = a_cu == 4 ? 1700 : 0;
+  } else {
+    from32 = a_cu == 1 ? 16 : a_cu == 2 ? 448 : 700;
+    to32 = a_cu == 1 ? 8192 : a_cu == 2 ? 3072 : a_cu == 3 ? 1088 : 0;
+  }
+  if (K < from32) return plan;
+  if (K > to32) {
+    if (K > to64 || tiles64 > 2 * num_cus) return plan;
+    plan.tile = 64;
+    plan.waves = tiles64 <= num_cus ? 8 : 4;
+    plan.step = 64;
+    return plan;
+  }
   plan.waves = 4;
   plan.step = 64;
   if (across) {
     if (a_cu == 1) {
-      plan.waves = K >= 4096 ? 16 : K > 256 ? 8 : 4;
-      if (K >= 512) plan.step = 128;
+      plan.waves = K >= 4096 ? (bytes ? 4 : 16) : K > 256 ? 8 : 4;
+      if (K > 256) plan.step = 128;
     } else if (a_cu == 2) {
       plan.step = 128;
     }
   } else if (a_cu == 1) {
-    if (K > 256) plan.waves = 8;
-  } else if (bytes) {
-    if (a_cu == 2 && K > 128 && K < 2048) plan.waves = 8;
-    if (a_cu == 3 && K >= 2048) plan.step = 128;
-  } else if (K >= 1024) {
-    plan.step = 128;
+    // (In place, 256 tiles: x 512 4.64 with four waves, 4.54 with eight; x 1024 4.83
+    // and 5.17; x 1504 5.89 and 6.18; x 2048 6.21 and 5.97; x 4096 8.77 and 8.18.)
+    if (K > 256 && (packed_bytes || K <= 768 || K > 1792)) plan.waves = 8;
+  } else if (bytes && a_cu == 2 && K > 128 && K < 1024) {
+    plan.waves = 8;
   }
   return plan;
 }
@@ -151,24 +177,29 @@ hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const Sma
 // split into planes or reordered for those costs them two to four launches.
 // This side is a fit to 16 to 4096 tiles and depths of 32 to 4096, where it takes
 // 3.9 us, 0.7 us (1.2) for every tile a CU has beyond the first, and to a KiB of
-// depth and tile 1.1 us on rows at whole dwords, more where operands are transposed
+// depth and tile 1.4 us on aligned rows, more where operands are transposed
 // or lie at odd addresses. us per call, other route -> this: in place, 256 tiles x 512 6.5 -> 4.2,
 // x 4096 13.3 -> 8.9, 1024 (one round of 64x64) x 512 7.0 -> 8.3, 1152 x 512 11.7 -> 8.7, 2440 x
 // 1024 21.6 -> 18.9, 4096 x 1024 23.3 -> 31.2; rows of odd length, 256 x 1025 15.3 -> 7.2, 2440
 // x 1025 32.7 -> 29.9; int8 transposed 256 x 1024 10.6 -> 6.2; int16 transposed, its side
 // along the rows, 256 x 1024 14.4 -> 5.9, 2440 x 1024 33.4 -> 23.0; both transposed 256 x
 // 1024 16.9 -> 6.7.
-SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes,
+SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, int packs, uint64_t packed_bytes,
                                  bool int16_is_a) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
   const int K = args.k_valid;
   plan.waves = 0;
-  if (K < 16 || tiles > 16 * num_cus) return plan;
+  if (K < 16 || tiles > 10 * num_cus) return plan;
   const bool across8 = small_gemm::IsAcross(int16_is_a ? plan.source_b : plan.source_a);
   const bool across16 = small_gemm::IsAcross(int16_is_a ? plan.source_a : plan.source_b);
-  const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b);
+  const bool straddling = Straddling(args);
+  const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b) ||
+                     (straddling && (across8 || across16));
   const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
-  const double to_a_kib = bytes ? (across8 || across16 ? 3.4 : 2.2) : across8 ? (across16 ? 2.2 : 1.7) : across16 ? 1.45 : 1.1;
+  const double to_a_kib = bytes      ? (across8 || across16 ? 3.4 : 2.4)
+                          : across8  ? (across16 ? 2.2 : 1.7)
+                          : across16 ? 1.45
+                                     : straddling ? 1.8 : 1.4;
   const double here = 3.9 + (bytes && (across8 || across16) ? 1.2 : 0.7) * (a_cu - 1) + to_a_kib * a_cu * K / 1024.0;
   // (The model counts plane vectors, 64 to 32 columns, with the int8 side along the rows.)
   GemmArgs planes = args;
@@ -178,7 +209,7 @@ SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPla
   double other = 1e30;
   for (int i = 0; i < model.count; ++i)
     other = std::min(other, mfma_gemm::ModelledMicroseconds(planes, num_cus, model, model.tiles[i]));
-  if (packed_bytes) other += 3.3 + 1.5e-6 * static_cast<double>(packed_bytes);
+  if (packs) other += 0.5 + 2.0 * packs + 0.7e-6 * static_cast<double>(packed_bytes);
   if (here >= other) return plan;
   plan.waves = a_cu == 1 && K >= 256 ? 8 : 4;
   plan.step = 64;

@@ -1128,7 +1128,7 @@ int RunI8I16Small(ruyamd_ctx* ctx, MulCall* call, bool* done, std::string* err) 
   const bool in_place16 = source16 == kSmallRows && K % 16 == 0 && pitch16 % 16 == 0 && (reinterpret_cast<uintptr_t>(src16.data) & 15) == 0;
   const uint64_t reordered = int16_is_a ? uint64_t(M) * uint64_t(N) * uint64_t(args.dst_elt) : 0;
   if (planes >= (uint64_t(1) << 31) || reordered >= (uint64_t(1) << 31)) return RUYAMD_OK;
-  plan = PlanSmallGemmI8I16(args, ctx->multiprocessor_count, plan,
+  plan = PlanSmallGemmI8I16(args, ctx->multiprocessor_count, plan, int(a.unpacked) + !in_place16 + (reordered != 0),
                             uint64_t(a.unpacked) * a.bytes + (in_place16 ? 0 : planes) + reordered, int16_is_a);
   if (plan.waves == 0) return RUYAMD_OK;
   const bool sums_with_pack = a.unpacked && PackFormsSums(a.src, a.ld);

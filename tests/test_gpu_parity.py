@@ -271,6 +271,18 @@ def test_products_on_tiles_of_32(device_ctx, tup, depth):
                 device_ctx.clear_prepacked_cache()
 
 
+@pytest.mark.parametrize("tup", [(S.U8, S.I8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I32)], ids=cases.tuple_name)
+@pytest.mark.parametrize("shape", [(833, 1030, 770), (835, 270, 1003), (770, 1599, 517), (1600, 257, 1270), (1024, 1700, 1001)])
+def test_products_on_tiles_of_64_read_where_they_lie(device_ctx, tup, shape):
+    """Operands that would have to be packed, on grids of 64x64 tiles of one and of
+    two rounds, ragged on every side."""
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(shape[1])
+    for orders in [(0, 0, 0), (0, 0, 1), (1, 1, 0), (0, 1, 1), (1, 0, 0)]:
+        p = W.random_problem(rng, *tup, *shape, *orders, strided=True, name="tiles of 64 %s %s" % (shape, orders))
+        compare(p, D.device_mul(device_ctx, p, misalign=shape[0] % 2), expected(p))
+
+
 @pytest.mark.parametrize("tile", [(64, 64), (128, 64), (64, 128), (128, 128), (256, 256)])
 @pytest.mark.parametrize("depth", [4, 5, 31, 33, 62, 95, 127, 129, 161, 190, 257, 515, 2051])
 def test_fp32_rows_of_any_depth_in_place(device_ctx, tile, depth):
