@@ -161,8 +161,15 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
     }
   } else if (a_cu == 1) {
     // (In place, 256 tiles: x 512 4.64 with four waves, 4.54 with eight; x 1024 4.83
-    // and 5.17; x 1504 5.89 and 6.18; x 2048 6.21 and 5.97; x 4096 8.77 and 8.18.)
+    // and 5.17; x 1504 5.89 and 6.18; x 2048 6.21 and 5.97; x 4096 8.77 and 8.18. Deep rows that
+    // come from beyond L2 want more bytes in flight: eight waves, then sixteen on
+    // longer steps, 99 tiles x 4992 7.8 and 8.3, x 7312 12.9 and 11.6 (12.6 with the
+    // depth split on the larger tiles); 64 x 6144 10.4 and 9.5; 128 x 6016 9.6 and 9.4.)
     if (K > 256 && (packed_bytes || K <= 768 || K > 1792)) plan.waves = 8;
+    if (!packed_bytes && K > 5760) {
+      plan.waves = 16;
+      plan.step = 128;
+    }
   } else if (bytes && a_cu == 2 && K > 128 && K < 1024) {
     plan.waves = 8;
   }

@@ -272,6 +272,18 @@ def test_products_on_tiles_of_32(device_ctx, tup, depth):
 
 
 @pytest.mark.parametrize("tup", [(S.U8, S.I8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I32)], ids=cases.tuple_name)
+@pytest.mark.parametrize("depth", [5760, 5776, 6160, 8192])
+def test_deep_rows_on_tiles_of_32(device_ctx, tup, depth):
+    """Either side of the depth from which sixteen waves share it, up to the largest;
+    sums of either operand and a depth that ends inside a step."""
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(depth)
+    for rows, cols, orders in [(68, 131, (1, 0, 0)), (33, 100, (1, 0, 1))]:
+        p = W.random_problem(rng, *tup, rows, depth, cols, *orders, name="deep %dx%dx%d" % (rows, depth, cols))
+        compare(p, D.device_mul(device_ctx, p), expected(p))
+
+
+@pytest.mark.parametrize("tup", [(S.U8, S.I8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I32)], ids=cases.tuple_name)
 @pytest.mark.parametrize("shape", [(833, 1030, 770), (835, 270, 1003), (770, 1599, 517), (1600, 257, 1270), (1024, 1700, 1001)])
 def test_products_on_tiles_of_64_read_where_they_lie(device_ctx, tup, shape):
     """Operands that would have to be packed, on grids of 64x64 tiles of one and of
