@@ -420,9 +420,10 @@ bool AsSmall(const Operand8& op, Operand8* out, SmallGemmSource* source) {
 }
 
 // The small tiles need no packed copy of an operand. A call that is recorded or
-// may not allocate is refused all the same where there is no room for one, so
-// that it does not depend on the tiles whether it is; and so that one that has
-// run can be recorded, an ordinary call takes the room (if it can be had).
+// may not allocate is refused all the same where there is no room for one that
+// every other route needs, so that it does not depend on the tiles whether it is;
+// and so that one that has run can be recorded, an ordinary call takes the room
+// (if it can be had).
 bool HasRoomToPack(ruyamd_ctx* ctx, bool unpacked, uint32_t bytes, int32_t sums) {
   if (!unpacked) return true;
   bool room = true;
@@ -431,6 +432,23 @@ bool HasRoomToPack(ruyamd_ctx* ctx, bool unpacked, uint32_t bytes, int32_t sums)
     room = (ctx->capturing || ctx->no_alloc ? ctx->ws->Alloc(size) : ctx->ws->AllocOptional(size)) && room;
   }
   return room || !(ctx->capturing || ctx->no_alloc);
+}
+
+// Whether the staged form of the smallest tile is better for a product than the
+// tiles that need packed operands, and its arguments: it reads operands that
+// cannot be used in place as they are, without a pack launch in front, and forms
+// pending sums itself.
+bool StagedIsBetter(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
+                    GemmArgs* args) {
+  const int K = call.lhs.cols;
+  Operand8 sa, sb;
+  if (!AsStaged(a, K, &sa) || !AsStaged(b, K, &sb)) return false;
+  const bool swap = SetupInt8Gemm(ctx, call, sa, sb, lzp, rzp, /*staged=*/true, args);
+  if (!GemmI8StagedIsBetter(*args, ctx->multiprocessor_count, K, !a.unpacked && !b.unpacked)) return false;
+  args->k_valid = K;
+  args->ep.lhs_sums = (swap ? sb : sa).sums;
+  args->ep.rhs_sums = (swap ? sa : sb).sums;
+  return true;
 }
 
 // The product on the small tiles, where the planner finds that better (*done).
@@ -449,11 +467,15 @@ int RunInt8Small(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const 
   const uint64_t packed_bytes = uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes;
   plan = PlanSmallGemmI8(args, ctx->multiprocessor_count, plan, packed_bytes);
   if (plan.waves == 0) return RUYAMD_OK;
-  for (const Operand8* op : {&a, &b}) {
-    const bool sums = op->unpacked && op->sums_pending && PackFormsSums(op->src, op->ld);
-    if (!HasRoomToPack(ctx, op->unpacked, op->bytes, sums ? op->count : 0)) {
-      *err = "workspace allocation failed";
-      return RUYAMD_E_HIP;
+  // (What the staged form would take without a packed copy needs no room for one.)
+  GemmArgs staged;
+  if ((a.unpacked || b.unpacked) && !StagedIsBetter(ctx, call, a, b, lzp, rzp, &staged)) {
+    for (const Operand8* op : {&a, &b}) {
+      const bool sums = op->unpacked && op->sums_pending && PackFormsSums(op->src, op->ld);
+      if (!HasRoomToPack(ctx, op->unpacked, op->bytes, sums ? op->count : 0)) {
+        *err = "workspace allocation failed";
+        return RUYAMD_E_HIP;
+      }
     }
   }
   args.ep.lhs_sums = (swap ? sb : sa).sums;
@@ -470,20 +492,11 @@ int RunInt8Small(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const 
   return RUYAMD_OK;
 }
 
-// The product on the staged form of the smallest tile, where the planner finds
-// that better (*done): it reads operands that cannot be used in place as they
-// are, without a pack launch in front, and forms pending sums itself.
+// The product on the staged form of the smallest tile, where that is better (*done).
 int RunInt8Staged(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
                   bool* done, std::string* err) {
-  const int K = call.lhs.cols;
-  Operand8 sa, sb;
-  if (!AsStaged(a, K, &sa) || !AsStaged(b, K, &sb)) return RUYAMD_OK;
   GemmArgs args;
-  const bool swap = SetupInt8Gemm(ctx, call, sa, sb, lzp, rzp, /*staged=*/true, &args);
-  if (!GemmI8StagedIsBetter(args, ctx->multiprocessor_count, K, !a.unpacked && !b.unpacked)) return RUYAMD_OK;
-  args.k_valid = K;
-  args.ep.lhs_sums = (swap ? sb : sa).sums;
-  args.ep.rhs_sums = (swap ? sa : sb).sums;
+  if (!StagedIsBetter(ctx, call, a, b, lzp, rzp, &args)) return RUYAMD_OK;
   const bool timed = ctx->TimingBegin();
   const hipError_t launched = LaunchGemmI8Staged(ctx->LaunchStream(), args);
   if (timed) ctx->TimingEnd();

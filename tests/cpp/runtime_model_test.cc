@@ -9,7 +9,7 @@
 // wanted) for.
 //
 //   runtime_model_test failed_upload | page_locked_sources | page_locked_destinations | skinny_shapes |
-//       timing | capture | scratch_blocks | staged_rule
+//       timing | capture | raw_rows | scratch_blocks | staged_rule
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -590,6 +590,37 @@ void Capture() {
   }
 }
 
+// Rows of any length and alignment that a kernel reads where they lie, without a
+// packed copy: recorded on a context that has run nothing, taken without room in
+// the static area, and an ordinary call takes no scratch memory for them either.
+void RawRowsNeedNoScratch() {
+  struct {
+    int dtype, M, K, N;
+  } const cases[] = {
+      {RUYAMD_DTYPE_I8, 64, 100, 64},    {RUYAMD_DTYPE_I8, 300, 777, 300},    {RUYAMD_DTYPE_U8, 200, 333, 200},
+      {RUYAMD_DTYPE_U8, 64, 147, 12544}, {RUYAMD_DTYPE_I8, 1000, 1001, 900},  {RUYAMD_DTYPE_I8, 64, 1023, 16384},
+      {RUYAMD_DTYPE_I8, 1000, 511, 900}, {RUYAMD_DTYPE_U8, 1024, 1024, 1024},
+  };
+  for (const auto& k : cases) {
+    DeviceCall call(std::size_t(k.M) * k.K, std::size_t(k.K) * k.N, std::size_t(k.M) * k.N);
+    const ruyamd_mat l = Mat(k.dtype, call.lhs, k.M, k.K, RUYAMD_ORDER_ROW_MAJOR, 4);
+    const ruyamd_mat r = Mat(k.dtype, call.rhs, k.K, k.N, RUYAMD_ORDER_COL_MAJOR, 3);
+    const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
+    const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+    Context c;
+    R().capturing = true;
+    EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%d x %d x %d recorded first: %s", k.M, k.K, k.N,
+           ruyamd_ctx_last_error(c.ctx));
+    R().capturing = false;
+    EXPECT(ruyamd_mul_no_alloc(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%d x %d x %d without allocation: %s", k.M, k.K, k.N,
+           ruyamd_ctx_last_error(c.ctx));
+    R().allocations = 0;
+    EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+    EXPECT(R().allocations == 0, "%d x %d x %d: %d allocations", k.M, k.K, k.N, R().allocations);
+    EXPECT(R().log.size() == 3, "%d x %d x %d: %d launches", k.M, k.K, k.N, static_cast<int>(R().log.size()));
+  }
+}
+
 // Sums left to the product cost a call no scratch memory, although a recorded
 // call forms some of them in a launch of their own: a first call takes a block
 // for an operand that is packed and the sums the pack forms, nothing more.
@@ -665,6 +696,7 @@ int main(int argc, char** argv) {
   else if (which == "skinny_shapes") SkinnyShapes();
   else if (which == "timing") Timing();
   else if (which == "capture") Capture();
+  else if (which == "raw_rows") RawRowsNeedNoScratch();
   else if (which == "scratch_blocks") ScratchBlocks();
   else if (which == "staged_rule") StagedRule();
   else return 2;

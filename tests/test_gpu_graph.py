@@ -184,6 +184,49 @@ def test_large_operands_with_sums_are_recorded_after_one_call(size, lhs_order, r
         ctx.close()
 
 
+@pytest.mark.parametrize("tup,shape", [((S.U8, S.U8, S.I32, S.U8), (64, 147, 12544)),
+                                       ((S.I8, S.I8, S.I32, S.I8), (300, 777, 300)),
+                                       ((S.I8, S.I8, S.I32, S.I32), (64, 100, 64))])
+def test_rows_read_where_they_lie_are_recorded_first(tup, shape):
+    """Rows of odd depth that no kernel packs: a context that has run nothing
+    records them."""
+    import torch
+    from ruy_amd import device_problem as D
+    from ruy_amd import api
+    from test_gpu_parity import expected
+
+    rng = np.random.default_rng(shape[1])
+    p = W.random_problem(rng, *tup, *shape, S.ORDER_ROW_MAJOR, S.ORDER_COL_MAJOR, S.ORDER_COL_MAJOR,
+                         name="recorded first %s" % (shape,))
+    p.lhs.zero_point, p.rhs.zero_point = 4, 3
+    ctx = api.Context()
+    try:
+        stream = torch.cuda.Stream()
+        ctx.set_stream(stream.cuda_stream)
+        ctx.set_synchronous(False)
+        dp = D.DeviceProblem(p, dst_fill=0)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            dp.run(ctx)
+        for _ in range(3):
+            _refill_rhs(p, dp, rng)
+            dp.dst_all.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+            torch.cuda.synchronize()
+            want = expected(p, fill=0)
+            _check(p, dp.dst_t.cpu().numpy(), want)
+            with torch.cuda.stream(stream):  # ... and an eager call between the replays
+                dp.dst_all.zero_()
+                dp.run(ctx)
+            torch.cuda.synchronize()
+            _check(p, dp.dst_t.cpu().numpy(), want)
+        del graph
+    finally:
+        ctx.close()
+
+
 def test_captured_cache_entries_survive_ejection():
     """A cache entry that a recorded call reads stays put when newer entries
     overflow the budget; the replay after that still gives the right answer."""

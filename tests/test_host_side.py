@@ -190,6 +190,11 @@ def test_one_ordinary_call_is_enough_for_a_capture(runtime_model):
     runtime_model("capture")
 
 
+def test_rows_read_where_they_lie_need_no_scratch_memory(runtime_model):
+    """... under capture before any ordinary call, without allocation, and in ordinary calls."""
+    runtime_model("raw_rows")
+
+
 def test_sums_left_to_the_product_take_no_scratch_memory(runtime_model):
     runtime_model("scratch_blocks")
 
