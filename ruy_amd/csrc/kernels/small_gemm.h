@@ -156,7 +156,12 @@ struct Side {
       for (int j = 0; j < kLoads; ++j) {
         const char* from = From(step, u, j);
         if constexpr (!kAnyByte) {
-          h.x[u][j] = *reinterpret_cast<const v4i_dwords*>(from);
+          // (Runs start at multiples of 4 bytes, but the 16 bytes that end with one
+          // do not where its length is no multiple. fp32 has no such.)
+          if constexpr (kElement == 4)
+            h.x[u][j] = *reinterpret_cast<const v4i_dwords*>(from);
+          else
+            h.x[u][j] = *reinterpret_cast<const granule::v4i_unaligned*>(from);
         } else {
           const int shift = static_cast<int>(reinterpret_cast<uintptr_t>(from) & 3);
           h.x[u][j] = *reinterpret_cast<const v4i_dwords*>(from - shift);

@@ -124,6 +124,44 @@ def test_a_lane_of_a_row_pack_has_four_loads_in_flight(tmp_path):
         assert "LLLL" in steps and steps.count("L") == 4, (kernel, steps)
 
 
+def test_loads_of_the_small_tiles_claim_no_alignment_they_lack(tmp_path):
+    """Rows at multiples of 4 bytes whose length is none, and counts that are none:
+    the 16 bytes that end with them start anywhere, and the type of such a load has
+    to say so. (fp32 lies at multiples of 4 bytes throughout.) It is one load all
+    the same."""
+    from ruy_amd import build
+    source = tmp_path / "fetch.hip"
+    source.write_text("""
+#include "kernels/mfma_gemm.h"
+#include "kernels/small_gemm.h"
+namespace ruyamd {
+namespace small_gemm {
+template <int kSource, int kElement>
+__global__ void Fetch(const char* data, int pitch, int count, int bytes, int step, v4i* out) {
+  using S = Side<32, 64, kSource, kElement>;
+  S side;
+  side.Start(data, pitch, count, 0, bytes, 0, threadIdx.x);
+  typename S::Held held = {};
+  side.Load(step, held);
+  for (int u = 0; u < S::kUnits; ++u)
+    for (int j = 0; j < S::kLoads; ++j) out[(u * S::kLoads + j) * 64 + threadIdx.x] = held.x[u][j];
+}
+""" + "".join("template __global__ void Fetch<%d, %d>(const char*, int, int, int, int, v4i*);\n" % (form, element)
+              for form in (0, 2) for element in (1, 2, 4)) + "}\n}\n")
+    flags = [build.HIPCC] + build.COMMON + build.DEVICE + ["--offload-device-only", "-S", str(source), "-o"]
+    subprocess.check_call(flags + [str(tmp_path / "fetch.ll"), "-emit-llvm"])
+    claims, name = {}, None
+    for line in open(tmp_path / "fetch.ll"):
+        if line.startswith("define "):
+            name = re.search(r"FetchILi(\d)ELi(\d)E", line).groups()
+        if re.search(r" = load <4 x i32>, ptr addrspace\(1\)", line):
+            claims.setdefault(name, set()).add(int(re.search(r"align (\d+)", line).group(1)))
+    assert claims == {(source, element): {4 if element == "4" else 1} for source in "02" for element in "124"}, claims
+    subprocess.check_call(flags + [str(tmp_path / "fetch.s")])
+    loads = [line.split()[0] for line in open(tmp_path / "fetch.s") if line.strip().startswith(("global_load", "flat_load"))]
+    assert loads and set(loads) == {"global_load_dwordx4"}, loads
+
+
 def test_every_wave_of_a_download_awaits_its_stores(tmp_path):
     """The word that tells the host a workgroup's part of a download is there is
     stored by one wave (kernels/host_copy.hip). A workgroup barrier by itself
