@@ -567,25 +567,39 @@ hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
   return hipGetLastError();
 }
 
+// The forms on 32x32 tiles that the planners choose, and so the ones that are built.
+template <typename T>
+constexpr bool IsPlanned(int step, int waves, bool across, bool any_byte) {
+  constexpr bool kPlanes = T::kElementA == 2 || T::kElementB == 2;
+  constexpr bool kInt8 = T::kElementA == 1 && T::kElementB == 1;
+  if (T::kElementA == 4 && any_byte) return false;
+  if (step == 64) return waves == 4 || (waves == 8 && !(kInt8 && across));
+  if (kPlanes || step != 128) return false;
+  if (waves == 16) return !any_byte && (kInt8 || across);
+  return across;
+}
+
 // The instantiation for a plan. Operands at any byte: both sides' byte forms
 // (which read aligned ones as well).
+template <typename T, int kTile, int S, int kWaves, int kSourceA, int kSourceB>
+hipError_t LaunchPlanned(hipStream_t stream, const GemmArgs& args) {
+  if constexpr (kTile == 64 || IsPlanned<T>(S, kWaves, IsAcross(kSourceA) || IsAcross(kSourceB), IsAnyByte(kSourceA)))
+    return Launch<T, kTile, S, kWaves, kSourceA, kSourceB>(stream, args);
+  return hipErrorInvalidValue;
+}
 template <typename T, int kTile, int S, int kWaves>
 hipError_t LaunchSources(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
   const bool across_a = IsAcross(plan.source_a), across_b = IsAcross(plan.source_b);
-  const bool bytes = IsAnyByte(plan.source_a) || IsAnyByte(plan.source_b);
-  if constexpr (T::kElementA != 4) {
-    if (bytes) {
-      if (across_a && across_b) return Launch<T, kTile, S, kWaves, kSmallAcrossBytes, kSmallAcrossBytes>(stream, args);
-      if (across_a) return Launch<T, kTile, S, kWaves, kSmallAcrossBytes, kSmallRowsBytes>(stream, args);
-      if (across_b) return Launch<T, kTile, S, kWaves, kSmallRowsBytes, kSmallAcrossBytes>(stream, args);
-      return Launch<T, kTile, S, kWaves, kSmallRowsBytes, kSmallRowsBytes>(stream, args);
-    }
+  if (IsAnyByte(plan.source_a) || IsAnyByte(plan.source_b)) {
+    if (across_a && across_b) return LaunchPlanned<T, kTile, S, kWaves, kSmallAcrossBytes, kSmallAcrossBytes>(stream, args);
+    if (across_a) return LaunchPlanned<T, kTile, S, kWaves, kSmallAcrossBytes, kSmallRowsBytes>(stream, args);
+    if (across_b) return LaunchPlanned<T, kTile, S, kWaves, kSmallRowsBytes, kSmallAcrossBytes>(stream, args);
+    return LaunchPlanned<T, kTile, S, kWaves, kSmallRowsBytes, kSmallRowsBytes>(stream, args);
   }
-  if (bytes) return hipErrorInvalidValue;
-  if (across_a && across_b) return Launch<T, kTile, S, kWaves, kSmallAcross, kSmallAcross>(stream, args);
-  if (across_a) return Launch<T, kTile, S, kWaves, kSmallAcross, kSmallRows>(stream, args);
-  if (across_b) return Launch<T, kTile, S, kWaves, kSmallRows, kSmallAcross>(stream, args);
-  return Launch<T, kTile, S, kWaves, kSmallRows, kSmallRows>(stream, args);
+  if (across_a && across_b) return LaunchPlanned<T, kTile, S, kWaves, kSmallAcross, kSmallAcross>(stream, args);
+  if (across_a) return LaunchPlanned<T, kTile, S, kWaves, kSmallAcross, kSmallRows>(stream, args);
+  if (across_b) return LaunchPlanned<T, kTile, S, kWaves, kSmallRows, kSmallAcross>(stream, args);
+  return LaunchPlanned<T, kTile, S, kWaves, kSmallRows, kSmallRows>(stream, args);
 }
 template <typename T>
 hipError_t LaunchPlan(hipStream_t stream, const GemmArgs& args, const SmallGemmPlan& plan) {
@@ -598,11 +612,9 @@ hipError_t LaunchPlan(hipStream_t stream, const GemmArgs& args, const SmallGemmP
   }
   if (plan.step == 64 && plan.waves == 4) return LaunchSources<T, 32, 64, 4>(stream, args, plan);
   if (plan.step == 64 && plan.waves == 8) return LaunchSources<T, 32, 64, 8>(stream, args, plan);
-  if constexpr (T::kElementA != 2 && T::kElementB != 2) {
-    if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 32, 128, 4>(stream, args, plan);
-    if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 32, 128, 8>(stream, args, plan);
-    if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 32, 128, 16>(stream, args, plan);
-  }
+  if (plan.step == 128 && plan.waves == 4) return LaunchSources<T, 32, 128, 4>(stream, args, plan);
+  if (plan.step == 128 && plan.waves == 8) return LaunchSources<T, 32, 128, 8>(stream, args, plan);
+  if (plan.step == 128 && plan.waves == 16) return LaunchSources<T, 32, 128, 16>(stream, args, plan);
   return hipErrorInvalidValue;
 }
 

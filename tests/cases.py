@@ -51,3 +51,27 @@ SLOW_SHAPES = ([s for w in (1, 2, 3, 4, 5, 8) for s in ((w, 401, 601), (587, 443
 
 ALL_ORDERS = [(a, b, c) for a in (0, 1) for b in (0, 1) for c in (0, 1)]
 RCC = (S.ORDER_ROW_MAJOR, S.ORDER_COL_MAJOR, S.ORDER_COL_MAJOR)
+
+
+def small_tile_problems(types):
+    """(M, K, N, orders) of products that between them run on every form of the
+    kernel on 32x32 and 64x64 tiles (csrc/kernels/small_gemm.h) that the planner
+    chooses for these types on 256 CUs: test_host_side.py looks it up, and
+    test_gpu_parity.py runs them. Every number of tiles to a CU and of waves to a
+    tile, the depths at which those change, operands along the rows and across
+    them, with runs that start at multiples of 16 bytes, of 4 and at any byte."""
+    sizes = [(64, 32, 96), (64, 512, 96), (64, 4096, 96), (64, 6144, 96), (512, 512, 800), (512, 1200, 800),
+             (800, 1200, 1200), (800, 1504, 1200), (1040, 1200, 976), (1040, 1504, 976)]
+    if types[:2] == (S.F32, S.F32):
+        sizes = [(64, 32, 96), (64, 128, 96), (64, 512, 96), (64, 1280, 96), (512, 256, 800)]
+    elif S.I16 in types[:2]:
+        sizes = [(64, 32, 96), (64, 512, 96)]
+    for size in sizes:
+        for more in (0, 4, 1):
+            for lhs, rhs in [(1, 0), (1, 1), (0, 0), (0, 1)]:
+                for dst in ((0, 1) if size[0] * size[1] * size[2] <= 4000000 else (0,)):
+                    yield tuple(x + more for x in size) + ((lhs, rhs, dst),)
+
+
+SMALL_TILE_TYPES = [(S.U8, S.I8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I32), (S.I8, S.I16, S.I32, S.I16),
+                    (S.I16, S.I8, S.I32, S.I32), (S.F32, S.F32, S.F32, S.F32)]

@@ -9,7 +9,7 @@
 // wanted) for.
 //
 //   runtime_model_test failed_upload | page_locked_sources | page_locked_destinations | skinny_shapes |
-//       timing | capture | raw_rows | scratch_blocks | staged_rule
+//       timing | capture | raw_rows | scratch_blocks | staged_rule | routes | kernels
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 
@@ -53,6 +53,7 @@ struct Runtime {
   bool capturing = false;
   int capture_violations = 0;
   int allocations = 0;                                // of device memory
+  bool fill_allocations = true;
   dim3 grid, block;
   std::size_t shared = 0;
   hipStream_t stream = nullptr;
@@ -147,7 +148,7 @@ hipError_t hipLaunchKernel(const void* function, dim3, dim3, void** args, std::s
 
 static hipError_t Take(std::map<const char*, std::size_t>* ranges, void** p, std::size_t bytes) {
   *p = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096 + 4096);
-  std::memset(*p, 0xCD, bytes);
+  if (R().fill_allocations) std::memset(*p, 0xCD, bytes);
   (*ranges)[static_cast<char*>(*p)] = bytes;
   NotWhileCapturing();
   return hipSuccess;
@@ -686,10 +687,65 @@ void StagedRule() {
   }
 }
 
+// What calls read from the standard input run on: a line each of "ordinary",
+// "recorded" or "without_allocation", the types of LHS, RHS and destination, rows,
+// depth, columns, the three storage orders, what the three strides are longer
+// than the rows or columns, the operands' zero points, whether each is cached, the
+// address of their first element modulo 16 and the tile that is forced (0 0: none).
+// Answered by a line of the call's result, its allocations and what it launched.
+// Ordinary calls use one context, the others a new one each. (No operand is
+// touched.)
+int Routes() {
+  const std::size_t room = std::size_t(1) << 38;
+  char* const at = static_cast<char*>(mmap(nullptr, 3 * room, PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0));
+  if (at == MAP_FAILED) std::abort();
+  R().device[at] = 3 * room;
+  R().fill_allocations = false;
+  Context shared;
+  char how[32];
+  int types[3], m, k, n, order[3], pad[3], zero[2], cached[2], misaligned, tile[2];
+  while (std::scanf("%31s %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d", how, &types[0], &types[1], &types[2], &m,
+                    &k, &n, &order[0], &order[1], &order[2], &pad[0], &pad[1], &pad[2], &zero[0], &zero[1], &cached[0],
+                    &cached[1], &misaligned, &tile[0], &tile[1]) == 20) {
+    ruyamd_mat mats[3];
+    for (int i = 0; i < 3; ++i) {
+      mats[i] = Mat(types[i], at + i * room + misaligned, i == 1 ? k : m, i == 0 ? k : n, order[i], i < 2 ? zero[i] : 0,
+                    i < 2 && cached[i] ? RUYAMD_CACHE_ALWAYS : RUYAMD_CACHE_NEVER);
+      mats[i].stride += pad[i];
+    }
+    ruyamd_mul_params p = Params(types[2]);
+    if (types[2] == RUYAMD_DTYPE_I32) p.multiplier_fixedpoint = p.multiplier_exponent = 0;
+    const bool ordinary = std::strcmp(how, "ordinary") == 0;
+    Context* own = ordinary ? nullptr : new Context;
+    ruyamd_ctx* const ctx = ordinary ? shared.ctx : own->ctx;
+    (void)ruyamd_ctx_force_tile(ctx, tile[0], tile[1], 0);
+    R().log.clear();
+    R().allocations = 0;
+    R().capturing = std::strcmp(how, "recorded") == 0;
+    const int rc = (std::strcmp(how, "without_allocation") == 0 ? ruyamd_mul_no_alloc : ruyamd_mul)(ctx, &mats[0], &mats[1],
+                                                                                                  &p, &mats[2]);
+    R().capturing = false;
+    std::printf("%d %d", rc, R().allocations);
+    for (const std::string& kernel : R().log) std::printf(" %s", kernel.c_str());
+    std::printf("\n");
+    ruyamd_ctx_clear_prepacked_cache(ctx);
+    delete own;
+  }
+  return 0;
+}
+
+// The names of the library's kernels.
+int Kernels() {
+  for (const auto& k : R().kernels) std::printf("%s\n", k.second.c_str());
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
+  if (which == "routes") return Routes();
+  if (which == "kernels") return Kernels();
   if (which == "failed_upload") FailedUpload();
   else if (which == "page_locked_sources") PageLockedSources();
   else if (which == "page_locked_destinations") PageLockedDestinations();

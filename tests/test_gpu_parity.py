@@ -271,6 +271,18 @@ def test_products_on_tiles_of_32(device_ctx, tup, depth):
                 device_ctx.clear_prepacked_cache()
 
 
+@pytest.mark.parametrize("tup", cases.SMALL_TILE_TYPES, ids=cases.tuple_name)
+def test_every_small_tile_kernel(device_ctx, tup):
+    """The products that between them run on every form of the kernel there is
+    (which test_host_side.py looks up)."""
+    rng = np.random.default_rng(tup[1])
+    for M, K, N, orders in cases.small_tile_problems(tup):
+        p = W.random_problem(rng, *tup, M, K, N, *orders, name="small tiles %dx%dx%d %s" % (M, K, N, orders))
+        announce(p.name)
+        got, want = run_both(device_ctx, p)
+        compare(p, got, want, exact_fp=False)
+
+
 @pytest.mark.parametrize("tup", [(S.U8, S.I8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I32)], ids=cases.tuple_name)
 @pytest.mark.parametrize("depth", [5760, 5776, 6160, 8192])
 def test_deep_rows_on_tiles_of_32(device_ctx, tup, depth):

@@ -197,6 +197,21 @@ def runtime_model(tmp_path_factory):
     def run(what):
         result = subprocess.run([exe, what], capture_output=True, text=True)
         assert result.returncode == 0 and "all passed" in result.stdout, result.stdout + result.stderr
+
+    def kernels():
+        return subprocess.check_output([exe, "kernels"], text=True).split()
+
+    def routes(calls):
+        """What each of the calls (type tuple, M, K, N, orders) launches."""
+        eight_bit = (1, 2)
+        lines = ["ordinary %d %d %d %d %d %d %d %d %d 0 0 0 %s 0 0 0 0 0" % (
+            types[0], types[1], types[3], M, K, N, *orders,
+            "3 5" if types[0] in eight_bit and types[1] in eight_bit else "0 0") for types, M, K, N, orders in calls]
+        answers = subprocess.run([exe, "routes"], input="\n".join(lines) + "\n", capture_output=True, text=True,
+                                 check=True).stdout.splitlines()
+        assert len(answers) == len(calls) and all(a.startswith("0 ") for a in answers)
+        return [a.split()[2:] for a in answers]
+    run.kernels, run.routes = kernels, routes
     return run
 
 
@@ -239,6 +254,17 @@ def test_sums_left_to_the_product_take_no_scratch_memory(runtime_model):
 
 def test_products_the_staged_form_of_the_smallest_tile_takes(runtime_model):
     runtime_model("staged_rule")
+
+
+def test_every_small_tile_kernel_is_chosen_for_a_product_that_the_gpu_tests_run(runtime_model):
+    """... and the library holds no other."""
+    import cases
+    calls = []
+    for types in cases.SMALL_TILE_TYPES:
+        calls += [(types,) + p for p in cases.small_tile_problems(types)]
+    launched = {kernel for route in runtime_model.routes(calls) for kernel in route if "SmallGemmKernel" in kernel}
+    built = {kernel for kernel in runtime_model.kernels() if "SmallGemmKernel" in kernel}
+    assert built == launched, sorted(built ^ launched)
 
 
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
