@@ -75,3 +75,20 @@ def small_tile_problems(types):
 
 SMALL_TILE_TYPES = [(S.U8, S.I8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I32), (S.I8, S.I16, S.I32, S.I16),
                     (S.I16, S.I8, S.I32, S.I32), (S.F32, S.F32, S.F32, S.F32)]
+
+
+# Rows that the staged form of the 64x64 tile reads (csrc/kernels/gemm_i8_staged.hip):
+# depths either side of its ring of four and of eight stages and of a granule;
+# (rows, columns, padded, LHS from the cache).
+STAGED_DEPTHS = [16, 17, 31, 127, 128, 130, 383, 400, 511, 512, 513, 896, 1000, 1023, 1024, 1025]
+STAGED_SHAPES = [(64, 64, False, False), (65, 129, True, False), (17, 63, False, True)]
+STAGED_TYPES = [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I16), (S.I8, S.U8, S.I32, S.I32)]
+
+# Edges of the pack kernels: depths either side of a 16-byte granule, of what a
+# row's lanes hold and of a depth dealt to several workgroups.
+PACK_DEPTHS = [1, 3, 15, 17, 33, 65, 145, 257, 1023, 1025, 1041, 4099, 9001]
+PACK_SHAPES = [(65, 37), (19, 130)]
+PACK_ORDERS = [(1, 0, 0), (0, 0, 0), (1, 1, 1), (0, 1, 0)]
+
+# Grids of more fp32 tiles than CUs, which run on rings of two stages: (tile, rows, columns).
+F32_SHALLOW_RINGS = [((64, 128), 1100, 2100), ((128, 64), 2100, 1100), ((128, 128), 2100, 2100)]

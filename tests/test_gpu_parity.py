@@ -207,37 +207,49 @@ def test_large_host_pointer_operands_and_the_staging_advisory(device_ctx):
     compare(f, D.host_pointer_mul(device_ctx, f, dst_fill=0), O.oracle_mul(f, fill=0))
 
 
-@pytest.mark.parametrize("depth", [1, 3, 15, 17, 33, 65, 145, 257, 1023, 1025, 1041, 4099, 9001])
+@pytest.mark.parametrize("tile", [(0, 0), (128, 128)])
+@pytest.mark.parametrize("depth", cases.PACK_DEPTHS)
 @pytest.mark.parametrize("tup", [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.U8, S.I32, S.I32), (S.F32, S.F32, S.F32, S.F32)])
-def test_packed_operands_at_the_edges_of_granules_and_parts(device_ctx, tup, depth):
+def test_packed_operands_at_the_edges_of_granules_and_parts(device_ctx, tup, depth, tile):
     """Depths either side of a 16-byte granule, of what a row's lanes hold and
     of a depth dealt to several workgroups; counts that end inside a block; one
-    or both operands packed, by rows or transposed, in one launch."""
+    or both operands packed, by rows or transposed, in one launch. On the tiles the
+    planner chooses, some of which need no packed operands, and on one that does."""
     rng = np.random.default_rng(depth)
-    for rows, cols in [(65, 37), (19, 130)]:
-        for orders in [(1, 0, 0), (0, 0, 0), (1, 1, 1), (0, 1, 0)]:
-            p = W.random_problem(rng, *tup, rows, depth, cols, *orders, strided=bool(depth % 4 == 1),
-                                 name="pack %dx%dx%d %s" % (rows, depth, cols, orders))
-            got, want = run_both(device_ctx, p)
-            compare(p, got, want, exact_fp=False)
+    device_ctx.force_tile(*tile)
+    try:
+        for rows, cols in cases.PACK_SHAPES:
+            for orders in cases.PACK_ORDERS:
+                p = W.random_problem(rng, *tup, rows, depth, cols, *orders, strided=bool(depth % 4 == 1),
+                                     name="pack %dx%dx%d %s" % (rows, depth, cols, orders))
+                got, want = run_both(device_ctx, p)
+                compare(p, got, want, exact_fp=False)
+    finally:
+        device_ctx.force_tile(0, 0)
 
 
-@pytest.mark.parametrize("depth", [16, 17, 31, 127, 128, 130, 383, 400, 511, 512, 513, 896, 1000, 1023, 1024, 1025])
-@pytest.mark.parametrize("tup", [(S.U8, S.U8, S.I32, S.U8), (S.I8, S.I8, S.I32, S.I16), (S.I8, S.U8, S.I32, S.I32)])
-def test_small_products_read_through_registers(device_ctx, tup, depth):
-    """The 64x64 tile on rows of any length and alignment: depths either side of
+@pytest.mark.parametrize("tile", [(0, 0), (64, 64)])
+@pytest.mark.parametrize("depth", cases.STAGED_DEPTHS)
+@pytest.mark.parametrize("tup", cases.STAGED_TYPES)
+def test_small_products_read_through_registers(device_ctx, tup, depth, tile):
+    """The 64x64 tile (forced: products this small run on 32x32 tiles by themselves)
+    on rows of any length and alignment: depths either side of
     its ring of four and of eight stages and of a granule, counts either side of
     a tile, rows that start at whole dwords and at odd bytes, a packed operand
     from the cache beside a raw one."""
     rng = np.random.default_rng(depth)
-    for rows, cols, pad, cached in [(64, 64, False, False), (65, 129, True, False), (17, 63, False, True)]:
-        p = W.random_problem(rng, *tup, rows, depth, cols, 1, 0, depth % 2, strided=pad,
-                             name="staged %dx%dx%d" % (rows, depth, cols))
-        p.lhs.cache_policy = S.CACHE_ALWAYS if cached else S.CACHE_NEVER
-        for misalign in (0, 1):
-            from ruy_amd import device_problem as D
-            compare(p, D.device_mul(device_ctx, p, misalign=misalign), expected(p))
-        device_ctx.clear_prepacked_cache()
+    device_ctx.force_tile(*tile)
+    try:
+        for rows, cols, pad, cached in cases.STAGED_SHAPES:
+            p = W.random_problem(rng, *tup, rows, depth, cols, 1, 0, depth % 2, strided=pad,
+                                 name="staged %dx%dx%d" % (rows, depth, cols))
+            p.lhs.cache_policy = S.CACHE_ALWAYS if cached else S.CACHE_NEVER
+            for misalign in (0, 1):
+                from ruy_amd import device_problem as D
+                compare(p, D.device_mul(device_ctx, p, misalign=misalign), expected(p))
+            device_ctx.clear_prepacked_cache()
+    finally:
+        device_ctx.force_tile(0, 0)
 
 
 def test_small_products_on_two_workgroups_a_cu(device_ctx):
@@ -313,22 +325,41 @@ def test_fp32_rows_of_any_depth_in_place(device_ctx, tile, depth):
     """Every fp32 tile on rows that end in part of a granule: one step and many,
     the end in the first and the last granule of a step, a depth in parts; what
     lies between the rows must not be looked at (it is NaN here)."""
-    import torch
     from ruy_amd import device_problem as D
     rng = np.random.default_rng(depth)
     device_ctx.force_tile(*tile)
     try:
         for rows, cols, orders in [(65, 130, (1, 0, 0)), (300, 77, (1, 0, 1))]:
-            p = W.random_problem(rng, S.F32, S.F32, S.F32, S.F32, rows, depth, cols, *orders, strided=True,
-                                 name="any depth %dx%dx%d" % (rows, depth, cols))
-            for m in (p.lhs, p.rhs):
-                view = m.storage[:m.n_storage]
-                pad = np.ones(view.size, bool)
-                outer = m.rows if m.order == S.ORDER_ROW_MAJOR else m.cols
-                for v in range(outer):
-                    pad[v * m.stride:v * m.stride + depth] = False
-                view[pad] = np.nan
+            p = _rows_with_nan_between(rng, rows, depth, cols, orders)
             compare(p, D.device_mul(device_ctx, p, misalign=1), expected(p), exact_fp=False)
+    finally:
+        device_ctx.force_tile(0, 0)
+
+
+def _rows_with_nan_between(rng, rows, depth, cols, orders):
+    p = W.random_problem(rng, S.F32, S.F32, S.F32, S.F32, rows, depth, cols, *orders, strided=True,
+                         name="any depth %dx%dx%d" % (rows, depth, cols))
+    for m in (p.lhs, p.rhs):
+        view = m.storage[:m.n_storage]
+        pad = np.ones(view.size, bool)
+        outer = m.rows if m.order == S.ORDER_ROW_MAJOR else m.cols
+        for v in range(outer):
+            pad[v * m.stride:v * m.stride + depth] = False
+        view[pad] = np.nan
+    return p
+
+
+@pytest.mark.parametrize("tile,rows,cols", cases.F32_SHALLOW_RINGS)
+@pytest.mark.parametrize("depth", [1, 2, 3, 5, 31, 33, 63, 65, 98, 127, 163, 513, 1111])
+def test_fp32_rows_of_any_depth_on_rings_of_two_stages(device_ctx, tile, rows, cols, depth):
+    """The same on grids of more tiles than CUs, several workgroups to a CU: depths
+    of one step, of as many as the ring holds and of more, the last one partial."""
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(depth)
+    device_ctx.force_tile(*tile)
+    try:
+        p = _rows_with_nan_between(rng, rows, depth, cols, (1, 0, depth // 2 % 2))
+        compare(p, D.device_mul(device_ctx, p, misalign=1), expected(p), exact_fp=False)
     finally:
         device_ctx.force_tile(0, 0)
 

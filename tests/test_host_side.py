@@ -184,6 +184,7 @@ def test_every_wave_of_a_download_awaits_its_stores(tmp_path):
 @pytest.fixture(scope="module")
 def runtime_model(tmp_path_factory):
     """tests/cpp/runtime_model_test.cc: the library on a model of the HIP runtime."""
+    from ruy_amd import _structs as S
     from ruy_amd import build
     exe = str(tmp_path_factory.mktemp("runtime_model") / "runtime_model_test")
     here = os.path.join(ROOT, "ruy_amd")
@@ -202,11 +203,14 @@ def runtime_model(tmp_path_factory):
         return subprocess.check_output([exe, "kernels"], text=True).split()
 
     def routes(calls):
-        """What each of the calls (type tuple, M, K, N, orders) launches."""
-        eight_bit = (1, 2)
-        lines = ["ordinary %d %d %d %d %d %d %d %d %d 0 0 0 %s 0 0 0 0 0" % (
-            types[0], types[1], types[3], M, K, N, *orders,
-            "3 5" if types[0] in eight_bit and types[1] in eight_bit else "0 0") for types, M, K, N, orders in calls]
+        """What each call launches: (type tuple, M, K, N, orders) and options."""
+        lines = []
+        for types, M, K, N, orders, *rest in calls:
+            o = dict({"pad": 0, "zero_points": True, "cached": False, "misalign": 0, "tile": (0, 0)}, **(rest[0] if rest else {}))
+            zero = (3, 5) if o["zero_points"] and types[0] in (S.U8, S.I8) and types[1] in (S.U8, S.I8) else \
+                tuple(128 if t == S.U8 else 0 for t in types[:2])
+            lines.append("ordinary %d %d %d %d %d %d %d %d %d" % (types[0], types[1], types[3], M, K, N, *orders) +
+                         " %d" % o["pad"] * 3 + " %d %d %d 0 %d %d %d" % (*zero, o["cached"], o["misalign"], *o["tile"]))
         answers = subprocess.run([exe, "routes"], input="\n".join(lines) + "\n", capture_output=True, text=True,
                                  check=True).stdout.splitlines()
         assert len(answers) == len(calls) and all(a.startswith("0 ") for a in answers)
@@ -265,6 +269,45 @@ def test_every_small_tile_kernel_is_chosen_for_a_product_that_the_gpu_tests_run(
     launched = {kernel for route in runtime_model.routes(calls) for kernel in route if "SmallGemmKernel" in kernel}
     built = {kernel for kernel in runtime_model.kernels() if "SmallGemmKernel" in kernel}
     assert built == launched, sorted(built ^ launched)
+
+
+def test_products_of_the_staged_tests_run_on_every_staged_kernel(runtime_model):
+    """Both rings, both alignments, with sums and without, each beside rows of the
+    other operand that come from the cache."""
+    import cases
+    raw, cached = set(), set()
+    for depth in cases.STAGED_DEPTHS:
+        calls = [(types, rows, depth, cols, (1, 0, depth % 2),
+                  {"pad": pad, "cached": from_cache, "misalign": misalign, "zero_points": zero_points, "tile": (64, 64)})
+                 for types in cases.STAGED_TYPES for rows, cols, pad, from_cache in cases.STAGED_SHAPES
+                 for misalign in (0, 1) for zero_points in (False, True)]
+        for call, route in zip(calls, runtime_model.routes(calls)):
+            (cached if call[-1]["cached"] else raw).update(k for k in route if "GemmKernel" in k)
+    staged = re.compile(r"MfmaGemmKernel\w+Int8Traits\w*Lb0ELi[12]EEEv")
+    built = {k for k in runtime_model.kernels() if staged.search(k)}
+    assert len(built) == 8
+    assert built <= raw, sorted(built - raw)
+    assert built <= cached, sorted(built - cached)
+
+
+def test_products_of_the_pack_tests_are_packed(runtime_model):
+    import cases
+    from ruy_amd import _structs as S
+    for depth in cases.PACK_DEPTHS:
+        calls = [((S.U8, S.U8, S.I32, S.U8), rows, depth, cols, orders, {"pad": depth % 4 == 1, "tile": (128, 128)})
+                 for rows, cols in cases.PACK_SHAPES for orders in cases.PACK_ORDERS]
+        for call, route in zip(calls, runtime_model.routes(calls)):
+            assert "PackKernel" in route[0], (call, route)
+
+
+def test_fp32_grids_of_the_ring_tests_run_on_two_stages(runtime_model):
+    import cases
+    from ruy_amd import _structs as S
+    for tile, rows, cols in cases.F32_SHALLOW_RINGS:
+        for depth in (5, 1111):
+            calls = [((S.F32,) * 4, rows, depth, cols, (1, 0, 0), {"pad": 1, "misalign": 4, "tile": tile})]
+            form = "MfmaGemmKernelINS_12_GLOBAL__N_19F32TraitsELi%dELi%dELi128ELi2E" % (tile[0] // 64, tile[1] // 64)
+            assert [form in kernel for kernel in runtime_model.routes(calls)[0]] == [True]
 
 
 @pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "example")),
