@@ -1,8 +1,6 @@
 // The GEMM on 32x32 tiles (small_gemm.h) for fp32.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "mfma_gemm.h"
 #include "small_gemm.h"
 
@@ -74,13 +72,12 @@ SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan 
                                       static_cast<uint32_t>(args.lda) | static_cast<uint32_t>(args.ldb)) & 15) != 0;
   const double here = 3.9 + 0.33 * (a_cu - 1) + (straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kF32);
-  double other = 1e30;
-  for (int i = 0; i < model.count; ++i)
-    other = std::min(other, mfma_gemm::ModelledMicroseconds(args, num_cus, model, model.tiles[i]));
-  if (packed_bytes) other += 2.3 + 0.5e-6 * static_cast<double>(packed_bytes);
+  const double pack = packed_bytes ? 2.3 + 0.5e-6 * static_cast<double>(packed_bytes) : 0;
   // (In place on both sides the models have to differ by more than they err: 1630
   // tiles x 752 are 29.9 us on the larger tiles, 31.5 by their model, and 30.6 here.)
-  if (here >= (packed_bytes ? 1.0 : 0.95) * other) return plan;
+  const double margin = packed_bytes ? 1.0 : 0.95;
+  for (int i = 0; i < model.count; ++i)
+    if (here >= margin * (mfma_gemm::ModelledMicroseconds(args, num_cus, model, model.tiles[i]) + pack)) return plan;
   plan.waves = 4;
   plan.step = 64;
   if (a_cu == 1) {

@@ -1,8 +1,6 @@
 // The GEMM on 32x32 tiles (small_gemm.h) for 8-bit operands.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "int8_traits.h"
 #include "small_gemm.h"
 
@@ -213,11 +211,9 @@ SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPla
   planes.M = int16_is_a ? args.N : args.M;
   planes.N = ((int16_is_a ? args.M : args.N) + 31) / 32 * 64;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kInt8PlaneSplit);
-  double other = 1e30;
+  const double pack = packs ? 0.5 + 2.0 * packs + 0.7e-6 * static_cast<double>(packed_bytes) : 0;
   for (int i = 0; i < model.count; ++i)
-    other = std::min(other, mfma_gemm::ModelledMicroseconds(planes, num_cus, model, model.tiles[i]));
-  if (packs) other += 0.5 + 2.0 * packs + 0.7e-6 * static_cast<double>(packed_bytes);
-  if (here >= other) return plan;
+    if (here >= mfma_gemm::ModelledMicroseconds(planes, num_cus, model, model.tiles[i]) + pack) return plan;
   plan.waves = a_cu == 1 && K >= 256 ? 8 : 4;
   plan.step = 64;
   return plan;

@@ -434,42 +434,40 @@ bool HasRoomToPack(ruyamd_ctx* ctx, bool unpacked, uint32_t bytes, int32_t sums)
   return room || !(ctx->capturing || ctx->no_alloc);
 }
 
-// Whether the staged form of the smallest tile is better for a product than the
-// tiles that need packed operands, and its arguments: it reads operands that
-// cannot be used in place as they are, without a pack launch in front, and forms
-// pending sums itself.
-bool StagedIsBetter(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
-                    GemmArgs* args) {
+// The product without a pack launch in front, where the planner finds that better
+// (*done): on the small tiles, or on the staged form of the smallest of the others,
+// which reads rows that cannot be used in place as they are. Both form pending
+// sums themselves. (Arguments and operands are set up once for both: 45 ns less of
+// a call's host time than once for each, on a model of the runtime, of 280 to 400.)
+int RunInt8Unpacked(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
+                    bool* done, std::string* err) {
   const int K = call.lhs.cols;
-  Operand8 sa, sb;
-  if (!AsStaged(a, K, &sa) || !AsStaged(b, K, &sb)) return false;
-  const bool swap = SetupInt8Gemm(ctx, call, sa, sb, lzp, rzp, /*staged=*/true, args);
-  if (!GemmI8StagedIsBetter(*args, ctx->multiprocessor_count, K, !a.unpacked && !b.unpacked)) return false;
-  args->k_valid = K;
-  args->ep.lhs_sums = (swap ? sb : sa).sums;
-  args->ep.rhs_sums = (swap ? sa : sb).sums;
-  return true;
-}
-
-// The product on the small tiles, where the planner finds that better (*done).
-int RunInt8Small(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
-                 bool* done, std::string* err) {
-  const int K = call.lhs.cols;
+  if (K < 16) return RUYAMD_OK;
   Operand8 sa, sb;
   SmallGemmSource source_a, source_b;
-  if (ctx->forced_tile_rows || K < 16 || !AsSmall(a, &sa, &source_a) || !AsSmall(b, &sb, &source_b)) return RUYAMD_OK;
+  const bool small_can = AsSmall(a, &sa, &source_a) && AsSmall(b, &sb, &source_b);
+  // (Rows are the same operand for both. The staged form reaches a few bytes more.)
+  auto is_rows = [](SmallGemmSource s) { return s == kSmallRows || s == kSmallRowsBytes; };
+  const bool staged_can = small_can ? is_rows(source_a) && is_rows(source_b) : AsStaged(a, K, &sa) && AsStaged(b, K, &sb);
+  if (!small_can && !staged_can) return RUYAMD_OK;
   GemmArgs args;
   const bool swap = SetupInt8Gemm(ctx, call, sa, sb, lzp, rzp, /*staged=*/true, &args);
   args.k_valid = K;
+  args.ep.lhs_sums = (swap ? sb : sa).sums;
+  args.ep.rhs_sums = (swap ? sa : sb).sums;
   SmallGemmPlan plan;
-  plan.source_a = swap ? source_b : source_a;
-  plan.source_b = swap ? source_a : source_b;
-  const uint64_t packed_bytes = uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes;
-  plan = PlanSmallGemmI8(args, ctx->multiprocessor_count, plan, packed_bytes);
-  if (plan.waves == 0) return RUYAMD_OK;
-  // (What the staged form would take without a packed copy needs no room for one.)
-  GemmArgs staged;
-  if ((a.unpacked || b.unpacked) && !StagedIsBetter(ctx, call, a, b, lzp, rzp, &staged)) {
+  if (small_can && !ctx->forced_tile_rows) {
+    plan.source_a = swap ? source_b : source_a;
+    plan.source_b = swap ? source_a : source_b;
+    const uint64_t packed_bytes = uint64_t(a.unpacked) * a.bytes + uint64_t(b.unpacked) * b.bytes;
+    plan = PlanSmallGemmI8(args, ctx->multiprocessor_count, plan, packed_bytes);
+  }
+  const bool small = plan.waves != 0;
+  const bool staged =
+      staged_can && GemmI8StagedIsBetter(args, ctx->multiprocessor_count, K, !a.unpacked && !b.unpacked);
+  if (!small && !staged) return RUYAMD_OK;
+  // (What the staged form would take needs no room for a packed copy on either.)
+  if (!staged) {
     for (const Operand8* op : {&a, &b}) {
       const bool sums = op->unpacked && op->sums_pending && PackFormsSums(op->src, op->ld);
       if (!HasRoomToPack(ctx, op->unpacked, op->bytes, sums ? op->count : 0)) {
@@ -478,27 +476,9 @@ int RunInt8Small(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const 
       }
     }
   }
-  args.ep.lhs_sums = (swap ? sb : sa).sums;
-  args.ep.rhs_sums = (swap ? sa : sb).sums;
   const bool timed = ctx->TimingBegin();
-  const hipError_t launched = LaunchSmallGemmI8(ctx->LaunchStream(), args, plan);
-  if (timed) ctx->TimingEnd();
-  if (launched != hipSuccess) {
-    *err = "int8 MFMA kernel launch failed";
-    return RUYAMD_E_HIP;
-  }
-  ctx->last_kernel = RUYAMD_KERNEL_I8_MFMA;
-  *done = true;
-  return RUYAMD_OK;
-}
-
-// The product on the staged form of the smallest tile, where that is better (*done).
-int RunInt8Staged(ruyamd_ctx* ctx, const MulCall& call, const Operand8& a, const Operand8& b, int32_t lzp, int32_t rzp,
-                  bool* done, std::string* err) {
-  GemmArgs args;
-  if (!StagedIsBetter(ctx, call, a, b, lzp, rzp, &args)) return RUYAMD_OK;
-  const bool timed = ctx->TimingBegin();
-  const hipError_t launched = LaunchGemmI8Staged(ctx->LaunchStream(), args);
+  const hipError_t launched =
+      small ? LaunchSmallGemmI8(ctx->LaunchStream(), args, plan) : LaunchGemmI8Staged(ctx->LaunchStream(), args);
   if (timed) ctx->TimingEnd();
   if (launched != hipSuccess) {
     *err = "int8 MFMA kernel launch failed";
@@ -535,9 +515,7 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
     return rc;
   if (!skinny) {
     bool done = false;
-    if (int rc = RunInt8Small(ctx, *call, a, b, lzp, rzp, &done, err)) return rc;
-    if (done) return RUYAMD_OK;
-    if (int rc = RunInt8Staged(ctx, *call, a, b, lzp, rzp, &done, err)) return rc;
+    if (int rc = RunInt8Unpacked(ctx, *call, a, b, lzp, rzp, &done, err)) return rc;
     if (done) return RUYAMD_OK;
   }
   PendingPack pack_a, pack_b;
@@ -931,23 +909,17 @@ int RunF32(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
   return RUYAMD_OK;
 }
 
-// int8 x int16 (either side) when the int8 side runs along the destination's
-// contiguous dimension. All zero points are 0 here (ruy/validate.h:51-57).
-int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
+// int8 x int16 (either side) when the int8 side, prepared as `a`, runs along the
+// destination's contiguous dimension. All zero points are 0 here
+// (ruy/validate.h:51-57).
+int RunI8I16(ruyamd_ctx* ctx, MulCall* call, Operand8 a, std::string* err) {
   const int M = call->lhs.rows, K = call->lhs.cols, N = call->rhs.cols;
   GemmArgs args;
   args.forced_tile_rows = ctx->forced_tile_rows;
   args.forced_depth_parts = ctx->forced_depth_parts;
   args.forced_tile_cols = ctx->forced_tile_cols;
   const bool swap = SetupDestination(*call, &args);  // true: A side = rhs
-  const int side8 = swap ? 1 : 0;
-  const int side16 = 1 - side8;
-  Operand8 a;
-  if (int rc = PrepareOperand8(ctx, call, side8, 0, /*need_sums=*/true,
-                               side8 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy,
-                               side8 == 0 ? call->lhs_src_key : call->rhs_src_key,
-                               side8 == 0 ? N : M, /*u8_depth_step=*/0, &a, err))
-    return rc;
+  const int side16 = swap ? 0 : 1;
   PendingPack pack_a;
   if (int rc = PackOperand8(ctx, &a, &pack_a, err)) return rc;
   const DevMat& m16 = side16 == 0 ? call->lhs : call->rhs;  // shape only: its data may still be host memory
@@ -1091,11 +1063,11 @@ int RunI8I16(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
 }
 
 // An int8 x int16 product on the small tiles, where the planner finds that better
-// (*done): with either type on either side and any storage order.
-int RunI8I16Small(ruyamd_ctx* ctx, MulCall* call, bool* done, std::string* err) {
+// (*done): with either type on either side and any storage order. `a`: the int8
+// side, prepared.
+int RunI8I16Small(ruyamd_ctx* ctx, MulCall* call, const Operand8& a, bool* done, std::string* err) {
   const int M = call->lhs.rows, K = call->lhs.cols, N = call->rhs.cols;
   const int side16 = call->lhs.dtype == RUYAMD_DTYPE_I16 ? 0 : 1;
-  const int side8 = 1 - side16;
   const int policy16 = side16 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy;
   if (ctx->forced_tile_rows || K < 16 || M <= kSkinnyKernelWidth || N <= kSkinnyKernelWidth ||
       ShouldCache(policy16, side16 == 0 ? N : M))
@@ -1108,19 +1080,10 @@ int RunI8I16Small(ruyamd_ctx* ctx, MulCall* call, bool* done, std::string* err) 
   args.k_bytes = RoundUp(K, 16);
   args.k_valid = K;
   const bool int16_is_a = (side16 == 1) == swap;
-  auto view = [&](int side) {
-    const DevMat& m = side == 0 ? call->lhs : call->rhs;
-    return side == 0 ? PackSource{m.data, m.rs, m.cs, m.rows, m.cols, m.dtype}
-                     : PackSource{m.data, m.cs, m.rs, m.cols, m.rows, m.dtype};
-  };
-  Operand8 a;
-  if (int rc = PrepareOperand8(ctx, call, side8, 0, /*need_sums=*/true,
-                               side8 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy,
-                               side8 == 0 ? call->lhs_src_key : call->rhs_src_key, side8 == 0 ? N : M,
-                               /*u8_depth_step=*/0, &a, err))
-    return rc;
   if (int rc = EnsureOnDevice(ctx, call, side16, err)) return rc;
-  const PackSource src16 = view(side16);
+  const DevMat& m16 = side16 == 0 ? call->lhs : call->rhs;
+  const PackSource src16 = side16 == 0 ? PackSource{m16.data, m16.rs, m16.cs, m16.rows, m16.cols, m16.dtype}
+                                       : PackSource{m16.data, m16.cs, m16.rs, m16.cols, m16.rows, m16.dtype};
   Operand8 small;
   SmallGemmSource source8, source16;
   int32_t pitch16;
@@ -1363,17 +1326,25 @@ int RunTuned(ruyamd_ctx* ctx, MulCall* call, TunedPath path, std::string* err) {
     case TunedPath::kF32:
       return RunF32(ctx, call, err);
     case TunedPath::kInt8Int16: {
-      bool done = false;
-      if (int rc = RunI8I16Small(ctx, call, &done, err)) return rc;
-      if (done) return RUYAMD_OK;
-      // The kernel wants the int8 side along the destination's contiguous dimension.
+      // The tiled kernel wants the int8 side along the destination's contiguous dimension.
       const bool dst_col_major = call->dst.rs == 1;
       const DevMat& contiguous_side = dst_col_major ? call->lhs : call->rhs;
-      if (contiguous_side.dtype == RUYAMD_DTYPE_I8) return RunI8I16(ctx, call, err);
+      const bool contiguous_is_int8 = contiguous_side.dtype == RUYAMD_DTYPE_I8;
+      // (A single-column destination has no storage order to flip.)
+      if (!contiguous_is_int8 && dst_col_major && call->dst.cols == 1) return RunGeneric(ctx, call, err);
+      const int side8 = call->lhs.dtype == RUYAMD_DTYPE_I8 ? 0 : 1;
+      Operand8 a;
+      if (int rc = PrepareOperand8(ctx, call, side8, 0, /*need_sums=*/true,
+                                   side8 == 0 ? call->lhs_cache_policy : call->rhs_cache_policy,
+                                   side8 == 0 ? call->lhs_src_key : call->rhs_src_key,
+                                   side8 == 0 ? call->rhs.cols : call->lhs.rows, /*u8_depth_step=*/0, &a, err))
+        return rc;
+      bool done = false;
+      if (int rc = RunI8I16Small(ctx, call, a, &done, err)) return rc;
+      if (done) return RUYAMD_OK;
+      if (contiguous_is_int8) return RunI8I16(ctx, call, a, err);
       // The other way round: compute into a scratch destination of the
       // opposite storage order and reorder that into the caller's destination.
-      // (A single-column destination has no storage order to flip.)
-      if (dst_col_major && call->dst.cols == 1) return RunGeneric(ctx, call, err);
       MulCall flipped = *call;
       DevMat& t = flipped.dst;
       t.data = ctx->ws->Alloc(std::size_t(t.rows) * t.cols * DtypeSize(t.dtype));
@@ -1383,7 +1354,7 @@ int RunTuned(ruyamd_ctx* ctx, MulCall* call, TunedPath path, std::string* err) {
       }
       t.rs = dst_col_major ? t.cols : 1;
       t.cs = dst_col_major ? 1 : t.rows;
-      if (int rc = RunI8I16(ctx, &flipped, err)) return rc;
+      if (int rc = RunI8I16(ctx, &flipped, a, err)) return rc;
       call->staged_any = call->staged_any || flipped.staged_any;
       if (LaunchReorder(ctx->LaunchStream(), t, call->dst) != hipSuccess) {
         *err = "reorder kernel launch failed";
