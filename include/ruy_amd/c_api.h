@@ -271,7 +271,8 @@ RUYAMD_API void ruyamd_ctx_force_generic_kernel(ruyamd_ctx* ctx, int force);
 /* Makes the tiled matrix-core kernels run on the tile of tile_rows x
  * tile_cols destination elements (256x256, 128x128, 128x64, 64x128 or 64x64;
  * plane columns count for int8 x int16) instead of the one their timing model
- * picks, where the kernel has that tile; 0, 0 restores the model's choice.
+ * picks, where the kernel has that tile, also for products that would run on the
+ * kernel for small ones instead; 0, 0 restores the model's choice.
  * depth_parts, looked at with the 256x256 tile forced on int8 data: not 0 =
  * split the depth over that many workgroups per tile (2, 4 or 8; 1: over none;
  * rounded down to what leaves no part without a depth step) instead of what
@@ -340,16 +341,19 @@ RUYAMD_API int ruyamd_diag_mfma_ceiling(ruyamd_ctx* ctx, int instruction,
                                         double* tera_ops_per_second,
                                         double* ms_per_launch);
 
-/* Which tile of the tiled matrix-core kernels a product of `rows` x `depth` by
- * `depth` x `cols` would run on with `compute_units` CUs, and into how many
- * parts its depth would be split over workgroups: `kind` 0 = 8-bit operands,
+/* Which tile a product of `rows` x `depth` by `depth` x `cols` runs on with
+ * `compute_units` CUs if it runs on the tiled matrix-core kernels, and into how
+ * many parts its depth is split over workgroups there: `kind` 0 = 8-bit operands,
  * 1 = int8 x int16, 2 = fp32; `rows` and `cols` are those of the destination
  * as the kernel sees it (column-major; swap them for a row-major one). Host
  * arithmetic only, no device needed: the choice is made by a timing model of
  * each tile fitted to measurements on an MI355X, where the reference looks up
  * cache sizes and thread counts (MakeBlockMap, ruy/block_map.cc:339-496).
  * Shapes with a destination dimension of 16 or less run on the skinny kernels
- * instead. No counterpart in the reference. */
+ * instead, and products of up to some thousand tiles of 32x32 mostly on the kernel
+ * for small ones (on such tiles, or 64x64 ones), depending on depth, storage orders
+ * and alignment too; for these the answer is the tile that ruyamd_mul_batch and
+ * operands beyond that kernel's reach use. No counterpart in the reference. */
 RUYAMD_API int ruyamd_diag_tile_for(int kind, int rows, int depth, int cols,
                                     int compute_units, int* tile_rows,
                                     int* tile_cols, int* depth_parts);

@@ -356,7 +356,8 @@ class Context:
 def tile_for(kind, rows, depth, cols, compute_units=256):
     """(tile rows, tile columns, depth parts) of the tiled kernels for a product
     whose column-major destination is rows x cols; kind 0 = 8-bit, 1 = int8 x
-    int16, 2 = fp32. Host arithmetic, no device needed."""
+    int16, 2 = fp32. (Small and skinny products mostly run on kernels of their
+    own.) Host arithmetic, no device needed."""
     tr, tc, parts = C.c_int(0), C.c_int(0), C.c_int(0)
     rc = lib.ruyamd_diag_tile_for(kind, rows, depth, cols, compute_units, C.byref(tr), C.byref(tc), C.byref(parts))
     if rc != 0:

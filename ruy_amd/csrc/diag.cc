@@ -1,6 +1,6 @@
 // ruyamd_diag_mfma_ceiling: measures what the int8 matrix instructions sustain
 // on this card with nothing else running (see kernels/diag.hip).
-// ruyamd_diag_tile_for: which tile the tiled kernels would run a shape on.
+// ruyamd_diag_tile_for: which tile the tiled kernels run a shape on.
 #include <chrono>
 #include <cstdint>
 #include <vector>

@@ -393,8 +393,9 @@ def test_product_code_never_touches_the_checker():
 def test_tile_choice_of_the_timing_model():
     """The tile the tiled kernels run a shape on is host arithmetic (a timing
     model fitted to measurements, ruyamd_diag_tile_for): the benchmark
-    configurations that rely on the smallest tile (its fused sums, its batched
-    launch, the int16 operand read in place) get it, the 8192^3 product gets
+    configurations that rely on the smallest tile (the batched launch of the
+    small ones, which run on the small tiles one by one; the int16 operand read
+    in place) get it, the 8192^3 product gets
     the 256 x 256 tile, few tiles with a long depth split it over workgroups,
     and the choice splits the depth on no other tile but the 256 x 256 one of
     the int8 kernel. Arguments that make no sense are refused."""
