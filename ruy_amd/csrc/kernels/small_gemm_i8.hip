@@ -113,6 +113,15 @@ bool Straddling(const GemmArgs& args) {
 //     512 x 513 9.0 -> 8.5, on 64x64 x 1025 11.9 -> 10.6, x 1505 12.7 -> 12.0, x 2049 14.0 ->
 //     14.9; 768 x 289 8.0 -> 7.2, x 1025 12.5 -> 10.9, x 1505 13.1 -> 13.1; 1024 x 1025 12.7 ->
 //     11.2, x 1505 13.0 -> 14.3; with four waves 2048 x 256 9.4 -> 8.8.
+// The lines lie at whole numbers of tiles to a CU: a few tiles above one cost what
+// the next one costs (in place x 1024, where the others take 6.8 to 6.9: 768 tiles
+// 6.5, 784 7.2, 832 7.5, 1024 7.6). From 769 tiles to 1024, the others -> these:
+//   packed by rows: x 129 to 177 5.5 -> 5.0 to 5.1 (whole dwords 5.1 -> 4.7 to 4.8), where
+//     some of the four waves have no step; x 193 to 241 5.5 -> 5.4 to 5.6 (5.1 -> 5.0 to
+//     5.2); x 257 6.1 -> 6.2 to 6.3, x 513 7.4 -> 7.6, x 769 8.6 -> 8.6 to 8.8, x 961 9.2
+//     -> 9.1 to 9.4, x 1025 10.8 -> 9.9 to 10.7, x 1301 11.2 -> 12.5, on 64x64 10.9 to 11.3.
+//   one side transposed, whole dwords: x 200 7.3 -> 5.6 on either, x 288 7.5 -> 6.6, on 64x64
+//     6.3, x 1408 11.0 -> 10.4, x 1600 12.1 -> 10.8, x 1792 11.9 -> 11.1.
 // More waves to a workgroup, or longer steps, where the grid leaves CUs room for
 // them: 256 tiles in place x 4096 8.8 with four waves, 8.2 with eight; packed x 4097
 // 12.9 and 10.4; transposed x 4096 11.3 with eight, 10.6 with sixteen.
@@ -123,7 +132,7 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
   const bool across = small_gemm::IsAcross(plan.source_a) || small_gemm::IsAcross(plan.source_b);
   const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b) ||
                      (across && Straddling(args));
-  const int a_cu = tiles <= num_cus ? 1 : tiles <= 2 * num_cus ? 2 : 4 * tiles <= 13 * num_cus ? 3 : tiles <= 4 * num_cus ? 4 : 8;
+  const int a_cu = tiles <= num_cus ? 1 : tiles <= 2 * num_cus ? 2 : tiles <= 3 * num_cus ? 3 : tiles <= 4 * num_cus ? 4 : 8;
   plan.waves = 0;
   if (tiles > 8 * num_cus || K < 16) return plan;
   // Depths in [from32, to32] are for the 32x32 tiles, above that to to64 for the
@@ -131,9 +140,9 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
   int from32 = 16, to32 = 0, to64 = 0;
   if (across) {
     to32 = a_cu == 1 ? (bytes ? 4352 : 8192) : a_cu == 2 ? (bytes ? 700 : 2560) : a_cu == 3 ? (bytes ? 200 : 400) : a_cu == 4 ? 200 : 0;
-    to64 = a_cu == 1 ? 0 : a_cu == 2 ? (bytes ? 1600 : 0) : a_cu == 3 ? (bytes ? 1250 : 1800) : a_cu == 4 ? (bytes ? 1250 : 1400) : 300;
+    to64 = a_cu == 1 ? 0 : a_cu == 2 ? (bytes ? 1600 : 0) : a_cu <= 4 ? (bytes ? 1250 : 1800) : 300;
   } else if (packed_bytes) {
-    from32 = a_cu == 4 && K > 128 ? 960 : 16;
+    from32 = a_cu == 4 && K > 192 ? 960 : 16;
     to32 = a_cu == 1 ? 8192 : a_cu == 2 ? 2560 : a_cu == 3 ? 1536 : a_cu == 4 ? 1300 : 0;
     to64 = a_cu == 4 ? 1700 : 0;
   } else {

@@ -271,6 +271,23 @@ def test_every_small_tile_kernel_is_chosen_for_a_product_that_the_gpu_tests_run(
     assert built == launched, sorted(built ^ launched)
 
 
+def test_small_tiles_end_at_whole_numbers_of_tiles_to_a_cu(runtime_model):
+    """A grid of a few 32x32 tiles more than three to a CU takes as long as one of
+    four to a CU: 8-bit rows run where those do, from 769 tiles on."""
+    from ruy_amd import _structs as S
+    i8 = (S.I8, S.I8, S.I32, S.I8)
+    other, small, wide = "MfmaGemmKernel", "SmallGemmKernel.*Li32ELi64ELi4E", "SmallGemmKernel.*Li64ELi64ELi8E"
+    for rows, cols, ranges in [
+            (768, 1024, {1024: small, 1085: small, 129: small, 257: small, 1505: small}),
+            (769, 1000, {1024: other, 704: other, 1088: other, 191: small, 193: other, 257: other, 959: other, 961: small,
+                         1299: small, 1301: wide, 1505: wide, 1699: wide, 1701: other}),
+            (64, 12544, {1024: other, 147: small, 190: small, 250: other}),
+            (1024, 1024, {1024: other, 704: other, 147: small, 190: small, 250: other, 961: small, 1505: wide})]:
+        calls = [(i8, rows, depth, cols, (1, 0, 0)) for depth in ranges]
+        for (_, _, depth, _, _), route in zip(calls, runtime_model.routes(calls)):
+            assert re.search(ranges[depth], route[-1]), (rows, depth, cols, route)
+
+
 def test_products_of_the_staged_tests_run_on_every_staged_kernel(runtime_model):
     """Both rings, both alignments, with sums and without, each beside rows of the
     other operand that come from the cache."""
