@@ -61,6 +61,12 @@ struct F32Small {
 // (one 64x64 tile too many for two rounds) x 1024 60.5 -> 47.7; 256 tiles with one
 // side transposed x 1024 19.7 -> 9.2, both 21.8 -> 9.4; 1536 x 1024 43.4 -> 39.8, both
 // 47.6 -> 39.0.
+// More than six tiles to a CU: of more than 300 bytes of depth every further one costs
+// 0.5 us, with an operand transposed 0.75, and in place the models have to differ by
+// more. Of 460 products around the line, 16 to 4096 tiles, these tiles took 392 with
+// 0.33 us throughout, of which 31 were slower here (2176 x 288 x 1520 with one side
+// transposed 28.0 -> 33.1, 2232 x 1708 x 1352 106 -> 116); they take 354, 10 of them
+// slower, by 8 % at most.
 SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
   const int K = args.k_valid;
@@ -70,12 +76,13 @@ SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan 
   const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
   const bool straddling = across || ((reinterpret_cast<uintptr_t>(args.a) | reinterpret_cast<uintptr_t>(args.b) |
                                       static_cast<uint32_t>(args.lda) | static_cast<uint32_t>(args.ldb)) & 15) != 0;
-  const double here = 3.9 + 0.33 * (a_cu - 1) + (straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
+  const bool many = a_cu > 6 && K > 300;
+  const double here = 3.9 + (!many ? 0.33 : across ? 0.75 : 0.5) * (a_cu - 1) + (straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kF32);
   const double pack = packed_bytes ? 2.3 + 0.5e-6 * static_cast<double>(packed_bytes) : 0;
   // (In place on both sides the models have to differ by more than they err: 1630
   // tiles x 752 are 29.9 us on the larger tiles, 31.5 by their model, and 30.6 here.)
-  const double margin = packed_bytes ? 1.0 : 0.95;
+  const double margin = packed_bytes ? 1.0 : many ? 0.93 : 0.95;
   for (int i = 0; i < model.count; ++i)
     if (here >= margin * (mfma_gemm::ModelledMicroseconds(args, num_cus, model, model.tiles[i]) + pack)) return plan;
   plan.waves = 4;

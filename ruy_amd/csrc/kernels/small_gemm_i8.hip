@@ -197,7 +197,11 @@ hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const Sma
 // 1024 21.6 -> 18.9, 4096 x 1024 23.3 -> 31.2; rows of odd length, 256 x 1025 15.3 -> 7.2, 2440
 // x 1025 32.7 -> 29.9; int8 transposed 256 x 1024 10.6 -> 6.2; int16 transposed, its side
 // along the rows, 256 x 1024 14.4 -> 5.9, 2440 x 1024 33.4 -> 23.0; both transposed 256 x
-// 1024 16.9 -> 6.7.
+// 1024 16.9 -> 6.7. Of 700 products around the line 24 of 585 on these tiles were slower
+// there, by up to a third (448 x 3764 x 2816, rows of odd length, 38 -> 53; 1112 x 1888 x
+// 1536 with the int16 side transposed 24.6 -> 31.0), with 1.7 and 1.45 us for aligned
+// transposed operands and no margin against the 128x128 tile. Set as they are, 11 of
+// 558 are, by a sixth at most.
 SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, int packs, uint64_t packed_bytes,
                                  bool int16_is_a) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
@@ -211,8 +215,8 @@ SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPla
                      (straddling && (across8 || across16));
   const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
   const double to_a_kib = bytes      ? (across8 || across16 ? 3.4 : 2.4)
-                          : across8  ? (across16 ? 2.2 : 1.7)
-                          : across16 ? 1.45
+                          : across8  ? (across16 ? 2.3 : 1.9)
+                          : across16 ? 1.6
                                      : straddling ? 1.8 : 1.4;
   const double here = 3.9 + (bytes && (across8 || across16) ? 1.2 : 0.7) * (a_cu - 1) + to_a_kib * a_cu * K / 1024.0;
   // (The model counts plane vectors, 64 to 32 columns, with the int8 side along the rows.)
@@ -221,8 +225,13 @@ SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPla
   planes.N = ((int16_is_a ? args.M : args.N) + 31) / 32 * 64;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kInt8PlaneSplit);
   const double pack = packs ? 0.5 + 2.0 * packs + 0.7e-6 * static_cast<double>(packed_bytes) : 0;
-  for (int i = 0; i < model.count; ++i)
-    if (here >= mfma_gemm::ModelledMicroseconds(planes, num_cus, model, model.tiles[i]) + pack) return plan;
+  for (int i = 0; i < model.count; ++i) {
+    // (Deep products on the 128x128 tile with packs in front are over- and these tiles
+    // underestimated a little, other than those that transpose at odd addresses.)
+    const bool large = model.tiles[i].bm == 128 && model.tiles[i].bn == 128 && !(bytes && (across8 || across16));
+    const double other = mfma_gemm::ModelledMicroseconds(planes, num_cus, model, model.tiles[i]) + pack;
+    if (here >= (large ? 0.92 : 1.0) * other) return plan;
+  }
   plan.waves = a_cu == 1 && K >= 256 ? 8 : 4;
   plan.step = 64;
   return plan;

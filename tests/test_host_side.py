@@ -288,6 +288,22 @@ def test_small_tiles_end_at_whole_numbers_of_tiles_to_a_cu(runtime_model):
             assert re.search(ranges[depth], route[-1]), (rows, depth, cols, route)
 
 
+def test_products_that_the_larger_tiles_do_faster_stay_there(runtime_model):
+    """fp32 and int8 x int16 products measured on both: (types, M, K, N, orders, padding, small tiles)."""
+    from ruy_amd import _structs as S
+    f32, i8i16, i16i8 = (S.F32,) * 4, (S.I8, S.I16, S.I32, S.I16), (S.I16, S.I8, S.I32, S.I16)
+    measured = [
+        (f32, 2176, 288, 1520, (1, 1, 1), 0, False), (f32, 2174, 176, 1652, (1, 1, 0), 1, False),    # 28.0 33.1, 24.7 28.1 us
+        (f32, 2232, 1708, 1352, (1, 0, 0), 0, False), (f32, 2048, 176, 1424, (1, 1, 0), 0, False),   # 106 116, 22.5 24.4
+        (f32, 762, 28, 3856, (1, 1, 0), 0, True), (f32, 860, 2832, 1686, (1, 0, 0), 0, True),        # 15.6 11.5, 93.1 83.9
+        (i8i16, 448, 3764, 2816, (1, 0, 0), 1, False), (i16i8, 1112, 1888, 1536, (0, 0, 1), 0, False),  # 37.7 53.1, 24.6 31.0
+        (i8i16, 3312, 7112, 379, (0, 0, 0), 0, False), (i16i8, 3729, 3733, 390, (1, 0, 0), 1, False),   # 69.5 83.5, 50.5 59.7
+        (i8i16, 191, 2624, 5940, (1, 1, 1), 0, True), (i16i8, 351, 2016, 4218, (1, 0, 0), 0, True)]     # 1.49 and 1.18 times
+    calls = [(types, M, K, N, orders, {"pad": pad}) for types, M, K, N, orders, pad, _ in measured]
+    for (*call, small), route in zip(measured, runtime_model.routes(calls)):
+        assert ("SmallGemmKernel" in route[-1]) == small, (call, route)
+
+
 def test_products_of_the_staged_tests_run_on_every_staged_kernel(runtime_model):
     """Both rings, both alignments, with sums and without, each beside rows of the
     other operand that come from the cache."""
