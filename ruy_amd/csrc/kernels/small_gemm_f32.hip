@@ -66,7 +66,7 @@ struct F32Small {
 // more. Of 460 products around the line, 16 to 4096 tiles, these tiles took 392 with
 // 0.33 us throughout, of which 31 were slower here (2176 x 288 x 1520 with one side
 // transposed 28.0 -> 33.1, 2232 x 1708 x 1352 106 -> 116); they take 354, 10 of them
-// slower, by 8 % at most.
+// slower, by 9 % at most.
 SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
   const int K = args.k_valid;

@@ -201,7 +201,7 @@ hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const Sma
 // there, by up to a third (448 x 3764 x 2816, rows of odd length, 38 -> 53; 1112 x 1888 x
 // 1536 with the int16 side transposed 24.6 -> 31.0), with 1.7 and 1.45 us for aligned
 // transposed operands and no margin against the 128x128 tile. Set as they are, 11 of
-// 558 are, by a sixth at most.
+// 558 are, by a fifth at most.
 SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, int packs, uint64_t packed_bytes,
                                  bool int16_is_a) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
