@@ -1,6 +1,8 @@
 // The GEMM on 32x32 tiles (small_gemm.h) for fp32.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "mfma_gemm.h"
 #include "small_gemm.h"
 
@@ -67,6 +69,10 @@ struct F32Small {
 // 0.33 us throughout, of which 31 were slower here (2176 x 288 x 1520 with one side
 // transposed 28.0 -> 33.1, 2232 x 1708 x 1352 106 -> 116); they take 354, 10 of them
 // slower, by 9 % at most.
+// A side of up to three tiles has the other operand read once, and one of 48 MB and
+// more comes from beyond the 256 MB of cache that the card has (weights in turn): a
+// KiB of depth costs 1.75 us then. 4096 x 4096 x 32 27.4 -> 32.2, 8192 x 2048 x 64 27.7 ->
+// 31.0, 8192 x 4096 x 96 69.4 -> 77.1, but 8192 x 2048 x 32 26.7 -> 20.9.
 SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan plan, uint64_t packed_bytes) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
   const int K = args.k_valid;
@@ -77,7 +83,9 @@ SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan 
   const bool straddling = across || ((reinterpret_cast<uintptr_t>(args.a) | reinterpret_cast<uintptr_t>(args.b) |
                                       static_cast<uint32_t>(args.lda) | static_cast<uint32_t>(args.ldb)) & 15) != 0;
   const bool many = a_cu > 6 && K > 300;
-  const double here = 3.9 + (!many ? 0.33 : across ? 0.75 : 0.5) * (a_cu - 1) + (straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
+  const bool streamed = !across && std::min(args.M, args.N) <= 96 && int64_t(std::max(args.M, args.N)) * K >= 48000000;
+  const double here = 3.9 + (!many ? 0.33 : across ? 0.75 : 0.5) * (a_cu - 1) +
+                      (streamed ? 1.75 : straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kF32);
   const double pack = packed_bytes ? 2.3 + 0.5e-6 * static_cast<double>(packed_bytes) : 0;
   // (In place on both sides the models have to differ by more than they err: 1630

@@ -1,6 +1,8 @@
 // The GEMM on 32x32 tiles (small_gemm.h) for 8-bit operands.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "int8_traits.h"
 #include "small_gemm.h"
 
@@ -122,6 +124,10 @@ bool Straddling(const GemmArgs& args) {
 //     -> 9.1 to 9.4, x 1025 10.8 -> 9.9 to 10.7, x 1301 11.2 -> 12.5, on 64x64 10.9 to 11.3.
 //   one side transposed, whole dwords: x 200 7.3 -> 5.6 on either, x 288 7.5 -> 6.6, on 64x64
 //     6.3, x 1408 11.0 -> 10.4, x 1600 12.1 -> 10.8, x 1792 11.9 -> 11.1.
+// Operands that come from HBM (weights in turn, more than the caches hold) are slower
+// here at the largest depths unless most CUs have a tile: 2048 x 8192 x 32 (64 tiles) 11.5
+// -> 13.2, with one side transposed 14.3 -> 15.9, x 96 (192) 11.9 -> 12.9, 4096 x 8192 x 32
+// (128) 13.3 -> 14.0, x 48 (256) 13.7 -> 13.1, 8192 x 8192 x 32 (256) 18.6 -> 16.8.
 // More waves to a workgroup, or longer steps, where the grid leaves CUs room for
 // them: 256 tiles in place x 4096 8.8 with four waves, 8.2 with eight; packed x 4097
 // 12.9 and 10.4; transposed x 4096 11.3 with eight, 10.6 with sixteen.
@@ -138,8 +144,9 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
   // Depths in [from32, to32] are for the 32x32 tiles, above that to to64 for the
   // 64x64 ones.
   int from32 = 16, to32 = 0, to64 = 0;
+  const int deepest = 4 * tiles <= 3 * num_cus ? 7680 : 8192;
   if (across) {
-    to32 = a_cu == 1 ? (bytes ? 4352 : 8192) : a_cu == 2 ? (bytes ? 700 : 2560) : a_cu == 3 ? (bytes ? 200 : 400) : a_cu == 4 ? 200 : 0;
+    to32 = a_cu == 1 ? (bytes ? 4352 : deepest) : a_cu == 2 ? (bytes ? 700 : 2560) : a_cu == 3 ? (bytes ? 200 : 400) : a_cu == 4 ? 200 : 0;
     to64 = a_cu == 1 ? 0 : a_cu == 2 ? (bytes ? 1600 : 0) : a_cu <= 4 ? (bytes ? 1250 : 1800) : 300;
   } else if (packed_bytes) {
     from32 = a_cu == 4 && K > 192 ? 960 : 16;
@@ -147,7 +154,7 @@ SmallGemmPlan PlanSmallGemmI8(const GemmArgs& args, int num_cus, SmallGemmPlan p
     to64 = a_cu == 4 ? 1700 : 0;
   } else {
     from32 = a_cu == 1 ? 16 : a_cu == 2 ? 448 : 700;
-    to32 = a_cu == 1 ? 8192 : a_cu == 2 ? 3072 : a_cu == 3 ? 1088 : 0;
+    to32 = a_cu == 1 ? deepest : a_cu == 2 ? 3072 : a_cu == 3 ? 1088 : 0;
   }
   if (K < from32) return plan;
   if (K > to32) {
@@ -201,7 +208,10 @@ hipError_t LaunchSmallGemmI8(hipStream_t stream, const GemmArgs& args, const Sma
 // there, by up to a third (448 x 3764 x 2816, rows of odd length, 38 -> 53; 1112 x 1888 x
 // 1536 with the int16 side transposed 24.6 -> 31.0), with 1.7 and 1.45 us for aligned
 // transposed operands and no margin against the 128x128 tile. Set as they are, 11 of
-// 558 are, by a fifth at most.
+// 558 are, by a fifth at most. A side of up to three tiles has the other operand read
+// once, and one of 16 MB and more from HBM where weights take turns: 1.95 us to a KiB of
+// depth then (4096 x 8192 x 32 17.4 -> 20.3, 8192 x 4096 x 64 17.4 -> 19.2, 4096 x 4096 x 96
+// 15.2 -> 16.6, but 8192 x 4096 x 32 16.1 -> 13.9, 4096 x 4096 x 64 14.5 -> 12.2).
 SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPlan plan, int packs, uint64_t packed_bytes,
                                  bool int16_is_a) {
   const int64_t tiles = int64_t((args.M + 31) / 32) * ((args.N + 31) / 32);
@@ -214,9 +224,11 @@ SmallGemmPlan PlanSmallGemmI8I16(const GemmArgs& args, int num_cus, SmallGemmPla
   const bool bytes = small_gemm::IsAnyByte(plan.source_a) || small_gemm::IsAnyByte(plan.source_b) ||
                      (straddling && (across8 || across16));
   const int a_cu = static_cast<int>((tiles + num_cus - 1) / num_cus);
+  const bool streamed = std::min(args.M, args.N) <= 96 && int64_t(std::max(args.M, args.N)) * K >= 16000000;
   const double to_a_kib = bytes      ? (across8 || across16 ? 3.4 : 2.4)
                           : across8  ? (across16 ? 2.3 : 1.9)
                           : across16 ? 1.6
+                          : streamed ? 1.95
                                      : straddling ? 1.8 : 1.4;
   const double here = 3.9 + (bytes && (across8 || across16) ? 1.2 : 0.7) * (a_cu - 1) + to_a_kib * a_cu * K / 1024.0;
   // (The model counts plane vectors, 64 to 32 columns, with the int8 side along the rows.)

@@ -289,10 +289,19 @@ def test_small_tiles_end_at_whole_numbers_of_tiles_to_a_cu(runtime_model):
 
 
 def test_products_that_the_larger_tiles_do_faster_stay_there(runtime_model):
-    """fp32 and int8 x int16 products measured on both: (types, M, K, N, orders, padding, small tiles)."""
+    """Products measured on both: (types, M, K, N, orders, padding, small tiles)."""
     from ruy_amd import _structs as S
     f32, i8i16, i16i8 = (S.F32,) * 4, (S.I8, S.I16, S.I32, S.I16), (S.I16, S.I8, S.I32, S.I16)
+    i8 = (S.I8, S.I8, S.I32, S.I8)
     measured = [
+        # Weights that come from HBM.
+        (f32, 4096, 4096, 32, (1, 0, 0), 0, False), (f32, 8192, 2048, 64, (1, 0, 0), 0, False),      # 27.4 32.2, 27.7 31.0 us
+        (f32, 8192, 4096, 96, (1, 0, 0), 0, False), (f32, 8192, 2048, 32, (1, 0, 0), 0, True),       # 69.4 77.1, 26.7 20.9
+        (i8i16, 4096, 8192, 32, (1, 0, 0), 0, False), (i8i16, 8192, 4096, 64, (1, 0, 0), 0, False),  # 17.4 20.3, 17.4 19.2
+        (i8i16, 8192, 4096, 32, (1, 0, 0), 0, True), (i8i16, 4096, 4096, 64, (1, 0, 0), 0, True),    # 16.1 13.9, 14.5 12.2
+        (i8, 2048, 8192, 32, (1, 0, 0), 0, False), (i8, 2048, 8192, 64, (1, 1, 0), 0, False),        # 11.5 13.2, 15.1 16.7
+        (i8, 8192, 8192, 32, (1, 0, 0), 0, True), (i8, 4096, 8192, 48, (1, 0, 0), 0, True),          # 18.6 16.8, 13.7 13.1
+        # Operands that the caches hold.
         (f32, 2176, 288, 1520, (1, 1, 1), 0, False), (f32, 2174, 176, 1652, (1, 1, 0), 1, False),    # 28.0 33.1, 24.7 28.1 us
         (f32, 2232, 1708, 1352, (1, 0, 0), 0, False), (f32, 2048, 176, 1424, (1, 1, 0), 0, False),   # 106 116, 22.5 24.4
         (f32, 762, 28, 3856, (1, 1, 0), 0, True), (f32, 860, 2832, 1686, (1, 0, 0), 0, True),        # 15.6 11.5, 93.1 83.9
