@@ -1,0 +1,121 @@
+// fp32 products on the bf16 matrix instructions, without losing a bit of an
+// operand: a float is the sum of three bf16 values (24 bits of mantissa are
+// three times 8), and of the nine products of two such sums the six largest are
+// formed, high * high down to the 2^-16 terms. What is left out is at most
+// 2^-23 of a product, a fifth of 2^-24 of it in the mean, and has no sign of its
+// own. Every bf16 product is exact, sums are fp32 throughout, and an instruction
+// adds 16 depth positions with one rounding where the fp32 instruction adds two;
+// the five smaller products have accumulators of their own. Measured against 64
+// bits (values in [-1, 1], one accumulator chain): depth 256 7.8e-8 (fp32
+// instructions 2.9e-7), 1024 1.9e-7 (6.1e-7), 3072 3.1e-7 (9.8e-7).
+//
+// The fp32 matrix instruction does 256 operations a clock and CU, the bf16 one
+// 4096: six of them are 2.7 times as fast. The 5.5 vector instructions that
+// split an element cost half as much energy again as its matrix instructions
+// (random data, where the power limit sets the clock: 340 TFLOP/s of fp32
+// products without them, 225 with, fp32 instructions 150), so elements are
+// split as few times as possible.
+//
+// Not every float is such a sum: infinities and NaN are not, values that a
+// bf16 part rounds to infinity are not, and parts of values under 2^-110 are
+// lost. The first two leave an accumulator that is not finite, for the third
+// the bits of a vector's elements are collected (Magnitudes); in either case
+// the wave does its work again with fp32 instructions.
+#ifndef RUY_AMD_CSRC_KERNELS_FLOAT_PARTS_H_
+#define RUY_AMD_CSRC_KERNELS_FLOAT_PARTS_H_
+
+#include <hip/hip_runtime.h>
+
+#include "granule.h"
+
+namespace ruyamd {
+namespace float_parts {
+
+using granule::v4i;
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+// Two floats rounded to bf16 in one register, and its two halves as floats.
+__device__ __forceinline__ int RoundPair(float x, float y) {
+  const v2f both = {x, y};
+  return __builtin_bit_cast(int, __builtin_convertvector(both, v2bf));
+}
+__device__ __forceinline__ float LowHalf(int pair) { return __int_as_float(pair << 16); }
+__device__ __forceinline__ float HighHalf(int pair) { return __int_as_float(pair & static_cast<int>(0xffff0000u)); }
+
+// Eight depth values of a vector: two granules of floats, as the operands of one
+// matrix instruction a part. part[0] + part[1] + part[2] are the values.
+struct Parts {
+  v4i part[3];
+};
+
+// The splitting of one granule (four floats), an instruction or two at a time so
+// that a schedule can deal them out between matrix instructions (which leave a
+// wave five or six issue slots each). kSplitOps pieces: Op<0>() ... in order.
+constexpr int kSplitOps = 22;
+struct Splitter {
+  float rest[4];
+  int pair[2];
+  // (dot2 instructions, which would subtract a half without extracting it,
+  // wait for the matrix pipe: 22 cycles each behind a matrix instruction.)
+  template <int kOp>
+  __device__ __forceinline__ void Op(const v4i& x, int which, Parts& to, int& magnitudes) {
+    if constexpr (kOp < 20) {
+      constexpr int part = kOp / 10, op = kOp % 10;
+      if constexpr (op < 2) {
+        if constexpr (part == 0) {
+          rest[2 * op] = __int_as_float(x[2 * op]);
+          rest[2 * op + 1] = __int_as_float(x[2 * op + 1]);
+          magnitudes |= x[2 * op] | x[2 * op + 1];
+        }
+        pair[op] = RoundPair(rest[2 * op], rest[2 * op + 1]);
+        to.part[part][2 * which + op] = pair[op];
+      } else {
+        constexpr int e = (op - 2) % 4;
+        if constexpr (op < 6)
+          half[e] = e % 2 ? HighHalf(pair[e / 2]) : LowHalf(pair[e / 2]);
+        else
+          rest[e] -= half[e];
+      }
+    } else {
+      to.part[2][2 * which + kOp - 20] = RoundPair(rest[2 * (kOp - 20)], rest[2 * (kOp - 20) + 1]);
+    }
+  }
+  float half[4];
+};
+
+// Product number e (0 .. 5) of two vectors' parts, the smallest first; the last
+// one is high * high.
+constexpr int kProducts = 6;
+constexpr int kPartOfA[kProducts] = {2, 0, 1, 1, 0, 0};
+constexpr int kPartOfB[kProducts] = {0, 2, 1, 0, 1, 0};
+// (Given the builtin, the compiler moves the accumulators between the two
+// register files on every trip round a loop. What the assembler text keeps from
+// it: Drain() in front of the first ordinary read of the accumulators, which
+// it names so that no copy of one can be made ahead of it.)
+template <int kProduct>
+__device__ __forceinline__ void Mma(const Parts& a, const Parts& b, v16f& acc) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+               : "+a"(acc)
+               : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
+}
+template <int kA, int kB>
+__device__ __forceinline__ void Drain(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {
+  asm volatile("s_nop 15\n\ts_nop 7" : "+a"(x[0][0]), "+a"(y[0][0]));
+#pragma unroll
+  for (int b = 1; b < kA * kB; ++b) asm volatile("" : "+a"(x[b / kB][b % kB]), "+a"(y[b / kB][b % kB]));
+}
+
+// The OR of elements' bits: whether all of them are under 2^-95 and some are not
+// zero. (Then what their parts lack, up to 2^-134 each, could be seen beside the
+// largest of them; otherwise it is under 2^-38 of that one.)
+__device__ __forceinline__ bool AllTiny(int magnitudes) {
+  return (magnitudes & 0x70000000) == 0 && (magnitudes & 0x7fffffff) != 0;
+}
+
+}  // namespace float_parts
+}  // namespace ruyamd
+
+#endif  // RUY_AMD_CSRC_KERNELS_FLOAT_PARTS_H_

@@ -1,8 +1,10 @@
-// fp32 instantiation of the tiled matrix-core GEMM (true fp32 multiply and
-// accumulate, v_mfma_f32_32x32x2_f32), replacing the reference's float kernels
-// (ruy/kernel_avx512.cc:872-1236; generic ruy/kernel.h:174-241). A 16-byte
-// fragment holds four consecutive depth values of one row; they feed four
-// matrix instructions. The write-back is the float one of
+// fp32 instantiation of the tiled matrix-core GEMM, replacing the reference's
+// float kernels (ruy/kernel_avx512.cc:872-1236; generic ruy/kernel.h:174-241).
+// The 64x64 and 128x128 tiles multiply floats as sums of three bf16 parts
+// (float_parts.h), the others, and a tile whose values are no such sums, with
+// v_mfma_f32_32x32x2_f32: a 16-byte fragment holds four consecutive depth values
+// of one row, which feed four of these. Either way every product counts with the
+// 24 bits of both factors and sums are fp32. The write-back is the float one of
 // ruy/reference_mul.h:42-48: bias, then min with clamp_max, then max with
 // clamp_min. The summation order differs from the reference's ascending-k
 // loop, which is why fp32 parity is a tolerance, not bit equality.
@@ -16,6 +18,7 @@ namespace {
 using mfma_gemm::v16f;
 using mfma_gemm::v4i;
 
+struct F32EightWaves;
 struct F32Traits {
   using Acc = v16f;
   static __device__ __forceinline__ void Mma(const v4i& a, const v4i& b, Acc& acc) {
@@ -26,9 +29,12 @@ struct F32Traits {
   static __device__ __forceinline__ void DrainMma() {}
   static constexpr int kBlock = 32;
   static constexpr bool kAnyDepth = true;
+  static constexpr bool kParts = true;
+  static constexpr int kWavesN = 2;
+  using EightWaves = F32EightWaves;
   static constexpr bool kRawB = false;
   static constexpr bool kPaired = false;
-  using LargeTile = F32Traits;
+  using LargeTile = F32Traits;  // (there is none)
   static constexpr bool kSplitB = false;
   static constexpr mfma_gemm::Model kModel = mfma_gemm::Model::kF32;
   static __device__ __forceinline__ int Bits(float x, float) { return __float_as_int(x); }
@@ -89,6 +95,11 @@ struct F32Traits {
       vals[q] = __float_as_int(v);
     }
   }
+};
+
+// The 128x128 tile: its waves two by four.
+struct F32EightWaves : F32Traits {
+  static constexpr int kWavesN = 4;
 };
 
 }  // namespace

@@ -42,6 +42,8 @@ struct Int8Traits {
   static __device__ __forceinline__ void DrainMma() {}
   static constexpr int kBlock = 32;
   static constexpr bool kAnyDepth = false;
+  static constexpr bool kParts = false;
+  static constexpr int kWavesN = 2;
   static constexpr bool kRawB = false;
   static constexpr bool kPaired = false;
   // The 256x256 tile runs on 16x16 blocks (below).

@@ -9,9 +9,10 @@
 // the transposed LHS / of the RHS, ruy/pack.h:105-132). That is the operand
 // order of the matrix instructions: for v_mfma_i32_32x32x32_i8 lane l supplies
 // 16 consecutive depth bytes of row/column l%32, at depth offset 16*(l/32); for
-// fp32 the same 16 bytes are four floats fed to four v_mfma_f32_32x32x2_f32
-// (which depth positions meet in one instruction does not matter as long as
-// both operands agree).
+// fp32 the same 16 bytes are four floats fed to four v_mfma_f32_32x32x2_f32, or,
+// in three parts, half of what six v_mfma_f32_32x32x16_bf16 take (float_parts.h;
+// which depth positions meet in one instruction does not matter as long as both
+// operands agree).
 //
 // Work decomposition: one workgroup (4 waves, 2 x 2) per BM x BN destination
 // tile, each wave owning WM x WN blocks of 32x32. The depth is walked in steps
@@ -27,7 +28,9 @@
 // touches all 64 banks; since a direct-to-LDS load places lane l at
 // base + 16*l, the swizzle is applied to the global address each lane fetches.
 //
-// A Traits type supplies: kAnyDepth (below), kBlock (32: one matrix instruction per 32x32 block
+// A Traits type supplies: kAnyDepth (below), kParts (fp32: the 64x64 and 128x128
+// tiles run on float_parts.h), kWavesN (waves side by side along a tile's columns; two of
+// them along its rows), kBlock (32: one matrix instruction per 32x32 block
 // and 32 bytes of depth; 16: per 16x16 block and 64 bytes of depth), Acc (the
 // accumulator vector of one block: 16 or 4 elements), Mma(a, b, acc)
 // for one 16-byte fragment pair, DrainMma() (called once after the last Mma),
@@ -53,6 +56,7 @@
 #include "../epilogue.h"
 #include "../internal.h"
 #include "depth_split.h"
+#include "float_parts.h"
 #include "fused_sums.h"
 #include "gemm_i8.h"
 #include "granule.h"
@@ -183,20 +187,22 @@ __device__ __forceinline__ int LdsOffset(int r, int g) {
   return r * BK + ((g ^ Swizzle<BK>(r)) << 4);
 }
 
-template <int WM, int WN, int BK, int STAGES, bool SPLIT_B = false, int BLOCK = 32>
+// WAVES_N: waves side by side along the columns of a tile, two deep along its rows.
+template <int WM, int WN, int BK, int STAGES, bool SPLIT_B = false, int BLOCK = 32, int WAVES_N = 2>
 struct Cfg {
+  static constexpr int kWaves = 2 * WAVES_N;
   static constexpr int kBM = 2 * WM * 32;
-  static constexpr int kBN = 2 * WN * 32;
+  static constexpr int kBN = WAVES_N * WN * 32;
   static constexpr int kBK = BK;
-  static constexpr int kThreads = 256;
+  static constexpr int kThreads = 64 * kWaves;
   static constexpr int kStages = STAGES;
   // Matrix-instruction depth steps per stage: a 32x32 block instruction takes
   // 32 bytes of depth, a 16x16 block instruction 64.
   static constexpr int kKSteps = BK / (BLOCK == 16 ? 64 : 32);
   static constexpr int kGranulesPerRow = BK / kGranule;
   static constexpr int kRowsPerLoad = 64 / kGranulesPerRow;  // tile rows one wave-level load covers
-  static constexpr int kALoads = kBM / kRowsPerLoad / 4;     // per wave per stage
-  static constexpr int kBLoads = kBN / kRowsPerLoad / 4;
+  static constexpr int kALoads = kBM / kRowsPerLoad / kWaves;  // per wave per stage
+  static constexpr int kBLoads = kBN / kRowsPerLoad / kWaves;
   static constexpr int kLoadsPerStage = kALoads + kBLoads;
   static constexpr int kStageBytes = (kBM + kBN) * BK;
   // The write-back stages kEpilogueBlockCols columns of 32x32 blocks per wave
@@ -207,16 +213,20 @@ struct Cfg {
   static_assert(!SPLIT_B || WN % 2 == 0, "");
   static constexpr int kEpilogueBlockCols = kLogicalWN >= 2 ? kLogicalWN / 2 : 1;
   static constexpr int kEpiloguePitch = WM * 32 + 4;
-  static constexpr int kEpilogueBytes = 4 * kEpilogueBlockCols * 32 * kEpiloguePitch * 4;
+  static constexpr int kEpilogueBytes = kWaves * kEpilogueBlockCols * 32 * kEpiloguePitch * 4;
   // 3 KiB of write-back parameters per wave (those of its rows and columns,
   // fetched ahead of the main loop and handed round through LDS): behind the
   // ring for 16x16 blocks, whose write-back has no staging area (it transposes
   // between lanes); behind the staging area, inside the ring's memory where
   // that is large enough, for 32x32 blocks.
-  static constexpr int kParamBytes = 4 * 6 * 128 * 4;
+  static constexpr int kParamBytes = kWaves * 6 * 128 * 4;
+  // (Four waves side by side: the fp32 tile whose parts lie in LDS, two buffers of
+  // three parts of 256 rows of 64 bytes, in the ring's memory and past it.)
+  static constexpr int kPartsBytes = WAVES_N == 4 ? 2 * 3 * 256 * 64 : 0;
+  static constexpr int kRingBytes = kStages * kStageBytes > kPartsBytes ? kStages * kStageBytes : kPartsBytes;
   static constexpr int kLdsBytes = BLOCK == 16 ? kStages * kStageBytes + kParamBytes
-                                               : (kStages * kStageBytes > kEpilogueBytes + kParamBytes
-                                                      ? kStages * kStageBytes
+                                               : (kRingBytes > kEpilogueBytes + kParamBytes
+                                                      ? kRingBytes
                                                       : kEpilogueBytes + kParamBytes);
 };
 
@@ -299,6 +309,8 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   // block row and sub-step. That tile's steps wait for LDS, not for the matrix
   // pipe, as long as a CU holds one workgroup, which is when it is used.
   constexpr bool kRowSumsOfFourBlocks = kFusedSums && WM == 2 && WN == 2;
+  // Traits::kParts on the 128x128 tile: split on the way to LDS (below).
+  constexpr bool kPartsInLds = Traits::kParts && Traits::kWavesN == 4;
   static_assert(!kFusedSums || (WM == 1 && (WN == 1 || (Traits::kSplitB && WN == 2))) ||
                     (kRowSumsOfFourBlocks && Traits::kBlock == 32 && !kDepthWaves && !Traits::kSplitB),
                 "fused sums exist for the tiles with one block (one block per plane) per wave, and for the rows of "
@@ -320,7 +332,8 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   constexpr int kBB = WN * kNB;  // blocks of B rows (destination columns) per wave
   constexpr int kAccElems = kB * kB / 64;
   constexpr int kGranulesPerMma = 64 / kB;  // 16-byte depth granules of a row that one instruction consumes
-  using C = Cfg<WM, WN, BK, STAGES, Traits::kSplitB, kB>;
+  constexpr int kWavesN = Traits::kWavesN;
+  using C = Cfg<WM, WN, BK, STAGES, Traits::kSplitB, kB, kWavesN>;
   constexpr int kBK = BK;
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -445,8 +458,8 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave_m = wave >> 1;
-  const int wave_n = wave & 1;
+  const int wave_m = wave / kWavesN;
+  const int wave_n = wave % kWavesN;
 
   // The 32-bit LDS address of the dynamic shared array (what M0 wants).
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
@@ -815,6 +828,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     // Load n of a step fills rows 8n .. 8n+7 of the slot (A rows first).
     uint32_t goff[kLoads];
     int gk[kLoads];
+    auto set_offsets = [&]() {
 #pragma unroll
     for (int n = 0; n < kLoads; ++n) {
       const int r = (n % 8) * 8 + lane / 8;  // row inside its operand's tile
@@ -836,6 +850,8 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         goff[n] = col < args.n_logical ? uint32_t(col) * uint32_t(args.ldb) + gb * kGranule : kOutOfRange;
       }
     }
+    };
+    set_offsets();
     // Depth offset and limit of the b operand in bytes: twice those of `a`
     // when it is int16 data.
     constexpr int kBScale = kRawB ? 2 : 1;
@@ -931,10 +947,149 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     };
     // This wave's steps: depth_way, depth_way + kDepthWays, ... of the workgroup's k_tiles steps.
     const int my_steps = k_tiles > depth_way ? (k_tiles - depth_way + kDepthWays - 1) / kDepthWays : 0;
-    if (my_steps > 0) issue_step(depth_way, 0);
+    if (my_steps > 0 || Traits::kParts) issue_step(depth_way, 0);
     if (my_steps > 1) issue_step(depth_way + kDepthWays, 1);
     load_edge_params();
     if constexpr (kLeadSums) add_up_rows_of_share();
+    // Traits::kParts (fp32): the steps on bf16 matrix instructions
+    // (float_parts.h). A step is two phases of 24 of them, on 16 depth values
+    // each; between those of one phase the granules of the next are split, each
+    // granule's registers are read again from LDS for the one after as soon as
+    // they are free, and the loads of the step after the next are issued, so
+    // that nothing of a step is waited for that was not asked for a phase before.
+    // The matrix instructions of a step take 0.64 us at 2.4 GHz; with every CU at
+    // work a step takes 1.5 us, as the power limit has it (1.18 on 144 CUs; not
+    // waiting for the loads changes nothing; fp32 instructions 1.9). 1024^3 22.3 ->
+    // 18.0-19.1 us, 1024 x 4096 x 1024 67.5 -> 54.2.
+    // in_parts: the sums are what fp32 instructions would give.
+    bool in_parts = false;
+    if constexpr (Traits::kParts) {
+      using float_parts::Parts;
+      constexpr int kPhaseMmas = 4 * float_parts::kProducts;
+      constexpr int kGranules = 8;  // of a phase: two of each of the four blocks (a, a, b, b)
+      typename Traits::Acc small[2][2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) small[i / 2][i % 2][v] = 0;
+      int magnitudes[4] = {0, 0, 0, 0};
+      v4i raw[kGranules];
+      Parts parts[2][4];
+      int off[C::kKSteps];
+#pragma unroll
+      for (int ks = 0; ks < C::kKSteps; ++ks) off[ks] = LdsOffset<BK>(frag_row, ks * 2 + frag_half);
+      auto read_granule = [&](auto granule, auto phase, int slot) {
+        constexpr int g = decltype(granule)::value;
+        raw[g] = *reinterpret_cast<const v4i*>(ring + slot * kSlotBytes + (g / 2) * 32 * kBK +
+                                               off[2 * decltype(phase)::value + g % 2]);
+      };
+      // Waits for step i of this wave, of which nothing younger is in flight.
+      auto wait_for_step = [&](int i) {
+        WaitVmcnt<0>();
+        if (ends_in_part_of_granule && depth_way + kDepthWays * i == k_tiles - 1) {
+          place_row_ends(ring + (i & 1) * kSlotBytes, 0, 64);
+          place_row_ends(ring + (i & 1) * kSlotBytes + 64 * kBK, 0, 64);
+        }
+      };
+      // One phase on parts[from]: kSplit: the next phase's granules are split
+      // on the way; kRead: ... and read again for phase `from` of the step in
+      // `read_slot`; kRefill: the loads of a step go to `refill_slot`.
+      auto phase = [&](auto from_constant, auto split, auto read, auto refill, int read_slot, int refill_slot, int kbase) {
+        constexpr int from = decltype(from_constant)::value;
+        float_parts::Splitter splitter;
+        StaticFor<kPhaseMmas>([&](auto n_constant) {
+          constexpr int n = decltype(n_constant)::value;
+          constexpr int i = n / 12, j = n / 6 % 2, e = n % 6;
+          __builtin_amdgcn_sched_barrier(0);
+          float_parts::Mma<e>(parts[from][i], parts[from][2 + j], e < 5 ? small[i][j] : full[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (decltype(refill)::value && n < kLoads)
+            LoadToLds16(ring_base + refill_slot * kSlotBytes + n * 1024, goff[n], uint32_t(kbase), n < 8 ? a_rsrc : b_rsrc);
+          if constexpr (decltype(split)::value) {
+            constexpr int kOps = kGranules * float_parts::kSplitOps;
+            constexpr int first = n * kOps / kPhaseMmas;
+            StaticFor<(n + 1) * kOps / kPhaseMmas - first>([&](auto o) {
+              constexpr int op = first + decltype(o)::value;
+              constexpr int g = op / float_parts::kSplitOps;
+              splitter.template Op<op % float_parts::kSplitOps>(raw[g], g % 2, parts[1 - from][g / 2], magnitudes[g / 2]);
+              // (The first rounding's remainder has replaced the floats by then.)
+              if constexpr (decltype(read)::value && op % float_parts::kSplitOps == 10)
+                read_granule(std::integral_constant<int, g>(), from_constant, read_slot);
+            });
+          }
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      using First = std::integral_constant<int, 0>;
+      using Second = std::integral_constant<int, 1>;
+      constexpr std::true_type kYes;
+      constexpr std::false_type kNo;
+      // (A wave without a step has loaded zeros.)
+      const int steps = max(my_steps, 1);
+      const bool last_is_partial = phys(depth_way + kDepthWays * (steps - 1)) * kBK + kBK > K;
+      if (steps > 1)
+        WaitVmcnt<kLoads>();
+      else
+        wait_for_step(0);
+      StaticFor<kGranules>([&](auto g) { read_granule(g, First(), 0); });
+      float_parts::Splitter splitter;
+      StaticFor<kGranules>([&](auto granule) {
+        constexpr int g = decltype(granule)::value;
+        StaticFor<float_parts::kSplitOps>([&](auto op) {
+          splitter.template Op<decltype(op)::value>(raw[g], g % 2, parts[0][g / 2], magnitudes[g / 2]);
+        });
+        read_granule(granule, Second(), 0);
+      });
+      // Nothing in the loop stands behind a condition but these: a branch around
+      // matrix instructions has the compiler move the accumulators.
+      for (int i = 0; i + 1 < steps; ++i) {
+        const int refill = i + 2;  // the step that slot i & 1 is filled with
+        int kbase = __builtin_amdgcn_readfirstlane(phys_inside(depth_way + kDepthWays * refill) * kBK);
+        if (refill >= steps) {
+#pragma unroll
+          for (int n = 0; n < kLoads; ++n) goff[n] = kOutOfRange;
+        } else if (last_is_partial && refill + 1 == steps) {
+          // (With the step's offset in the lanes' own: a granule that ends with
+          // its row begins in front of the step.)
+#pragma unroll
+          for (int n = 0; n < kLoads; ++n)
+            goff[n] = kbase + gk[n] < K ? goff[n] + kbase - past_end(kbase + gk[n]) : kOutOfRange;
+          kbase = 0;
+        }
+        wait_for_step(i + 1);
+        // Slot i & 1 has been read as a whole (the granules of its second phase
+        // arrive before the first of them is split).
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        phase(First(), kYes, kYes, kYes, (i + 1) & 1, i & 1, kbase);
+        phase(Second(), kYes, kYes, kNo, (i + 1) & 1, 0, 0);
+      }
+      phase(First(), kYes, kNo, kNo, 0, 0, 0);
+      phase(Second(), kNo, kNo, kNo, 0, 0, 0);
+      float_parts::Drain(full, small);
+      float not_finite = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          full[b / 2][b % 2][v] += small[b / 2][b % 2][v];
+          not_finite = __builtin_fmaf(full[b / 2][b % 2][v], 0.f, not_finite);
+        }
+      bool tiny = false;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) tiny = tiny || float_parts::AllTiny(magnitudes[b]);
+      in_parts = !__any(not_finite != 0.f || tiny);
+      if (!in_parts) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) full[b / 2][b % 2][v] = 0;
+        WaitVmcnt<0>();  // (what the last steps asked for beyond the end)
+        set_offsets();
+        if (my_steps > 0) issue_step(depth_way, 0);
+        if (my_steps > 1) issue_step(depth_way + kDepthWays, 1);
+      }
+    }
+    if (!in_parts) {
     Frags4 fr[2];
     auto walk_slot = [&](int slot) {
       read4(slot, 0, fr[0]);
@@ -970,6 +1125,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       }
       walk_slot(i & 1);
       if (i + 2 < my_steps) issue_step(depth_way + kDepthWays * (i + 2), i & 1);
+    }
     }
     if constexpr (kFusedSums) {
       const uint32_t fa = static_cast<uint32_t>(args.fused_a_factor);
@@ -1318,6 +1474,178 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       between(kt + 1);
     }
   } else {
+    // ---- fp32 on the 128x128 tile: the steps on bf16 matrix instructions ----
+    // Eight waves, two to a SIMD, each 64 rows x 32 columns; all of them share
+    // every step, so a float is split (float_parts.h) on its way to LDS, once a
+    // workgroup, and what lies there are the three parts of a step's rows, in two
+    // buffers of 48 KiB. A step is two phases, on 16 depth values each. Between
+    // the matrix instructions of a phase: the reads of the next phase's parts;
+    // half of the granules that this thread holds of a later step split and
+    // written (those of b of the next step in a step's first phase, those of a of
+    // the step after it in its second); the load of the step after that into each
+    // granule's registers. A barrier stands between a step's phases: in front of
+    // it the buffer of the next step has been written as a whole, and that of
+    // this step read, so that it can be written again behind it.
+    // (Four waves of 64 x 64, one to a SIMD, had nothing to fill each other's
+    // waits: 1.30 us a step on 64 CUs, this 1.05, where the matrix instructions
+    // take 0.64. On all CUs the power limit leaves 1.3-1.4; 2048 x 4096 x 2048 is
+    // 178 TFLOP/s, on fp32 instructions 129. 1537 x 1111 x 2051 72.6 -> 52.7 us.)
+    bool in_parts = false;
+    if constexpr (kPartsInLds) {
+      using float_parts::Parts;
+      constexpr int kPhaseMmas = kAB * kBB * float_parts::kProducts;
+      constexpr int kHeldRows = C::kThreads / 8;
+      constexpr int kHeld = 256 / kHeldRows;  // granules of a step a thread loads: of every kHeldRows-th row, of a and then of b
+      constexpr int kReads = 3 * (kAB + kBB);
+      constexpr int kPartRow = 64, kPartBytes = 256 * kPartRow, kBufferBytes = 3 * kPartBytes;
+      static_assert(2 * kBufferBytes == C::kPartsBytes && C::kBM == 128 && C::kBN == 128, "");
+      using BufferRsrc = decltype(__builtin_amdgcn_make_buffer_rsrc(static_cast<void*>(nullptr), short(0), 0, 0));
+      const BufferRsrc a_buffer =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(args.a), 0, static_cast<int>(args.a_bytes), 0x00020000);
+      const BufferRsrc b_buffer =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(args.b), 0, static_cast<int>(args.b_bytes), 0x00020000);
+      const int held_row = tid / 8, held_granule = tid % 8;
+      uint32_t row_off[kHeld];
+#pragma unroll
+      for (int n = 0; n < kHeld; ++n) {
+        const int r = n % (kHeld / 2) * kHeldRows + held_row;
+        row_off[n] = n < kHeld / 2 ? (m0 + r < args.M ? MulLo(m0 + r, args.lda) : kOutOfRange)
+                           : (n0 + r < args.N ? MulLo(n0 + r, args.ldb) : kOutOfRange);
+      }
+      v4i raw[kHeld];
+      // Granule n of step kt; zeros past the end of the depth.
+      auto load = [&](auto n_constant, int kt) {
+        constexpr int n = decltype(n_constant)::value;
+        const int k = kt * kBK + held_granule * kGranule;
+        const uint32_t off = k < K && row_off[n] != kOutOfRange ? row_off[n] + uint32_t(k - past_end(k)) : kOutOfRange;
+        raw[n] = __builtin_bit_cast(
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(n < kHeld / 2 ? a_buffer : b_buffer, static_cast<int>(off), 0, 0));
+      };
+      // The granules that end with their row, moved into place (once loaded).
+      auto place = [&](int kt, int first, int end) {
+        const int k = kt * kBK + held_granule * kGranule;
+        if (bytes_in_last_granule != 0 && kt == k_tiles - 1) {
+          const bool here = k < K && k + kGranule > K;
+#pragma unroll
+          for (int n = 0; n < kHeld; ++n) {
+            if (n < first || n >= end) continue;
+            const v4i x = raw[n];
+            v4i y = {x[3], 0, 0, 0};
+            if (bytes_in_last_granule == 8) y = v4i{x[2], x[3], 0, 0};
+            if (bytes_in_last_granule == 12) y = v4i{x[1], x[2], x[3], 0};
+#pragma unroll
+            for (int d = 0; d < 4; ++d) raw[n][d] = here ? y[d] : x[d];
+          }
+        }
+      };
+      // Rows of 64 bytes to a part, granules swizzled as the ring's.
+      char* const write_at =
+          lds + held_row * kPartRow + (((held_granule / 2) ^ Swizzle<64>(held_row)) << 4) + held_granule % 2 * 8;
+      auto write_part = [&](int buffer, int n, int part, int low, int high) {
+        typedef int v2i __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<v2i*>(write_at + buffer * kBufferBytes + part * kPartBytes + n * kHeldRows * kPartRow) = v2i{low, high};
+      };
+      int read_off[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        read_off[q] = frag_row * kPartRow + (((2 * q + frag_half) ^ Swizzle<64>(frag_row)) << 4);
+      // Part `which % 3` of the rows of this wave's block which / 3 (those of a first).
+      auto read_part = [&](auto which_constant, int buffer, auto q_constant, Parts (&to)[kAB + kBB]) {
+        constexpr int block = decltype(which_constant)::value / 3, part = decltype(which_constant)::value % 3;
+        const int rows = block < kAB ? (wave_m * kAB + block) * 32 : 128 + (wave_n * kBB + block - kAB) * 32;
+        to[block].part[part] = *reinterpret_cast<const v4i*>(lds + buffer * kBufferBytes + part * kPartBytes +
+                                                             rows * kPartRow + read_off[decltype(q_constant)::value]);
+      };
+      typename Traits::Acc small[kAB][kBB];
+#pragma unroll
+      for (int b = 0; b < kAB * kBB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) small[b / kBB][b % kBB][v] = 0;
+      int magnitudes[kHeld] = {};
+      constexpr int kGranuleOps = float_parts::kSplitOps + 4;  // ... its three parts written, and the load behind it
+      float_parts::Splitter splitter;
+      Parts split_parts;
+      auto granule_op = [&](auto op_constant, auto n_constant, int buffer, int load_step) {
+        constexpr int op = decltype(op_constant)::value, n = decltype(n_constant)::value;
+        if constexpr (op < float_parts::kSplitOps)
+          splitter.template Op<op>(raw[n], 0, split_parts, magnitudes[n]);
+        else if constexpr (op < float_parts::kSplitOps + 3)
+          write_part(buffer, n, op - float_parts::kSplitOps, split_parts.part[op - float_parts::kSplitOps][0],
+                     split_parts.part[op - float_parts::kSplitOps][1]);
+        else
+          load(n_constant, load_step);
+      };
+      Parts parts[2][kAB + kBB];
+      // A phase on parts[q]; reads phase `1 - q` (of this step or the next) from
+      // `read_buffer`; splits the granules of a (q = 1) or b into `write_buffer` and loads
+      // them again of step `load_step`.
+      auto phase = [&](auto q_constant, int read_buffer, int write_buffer, int load_step) {
+        constexpr int q = decltype(q_constant)::value;
+        StaticFor<kPhaseMmas>([&](auto n_constant) {
+          constexpr int n = decltype(n_constant)::value;
+          constexpr int i = n / 6 / kBB, j = n / 6 % kBB, e = n % 6;
+          __builtin_amdgcn_sched_barrier(0);
+          float_parts::Mma<e>(parts[q][i], parts[q][kAB + j], e < 5 ? small[i][j] : acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (n < kReads)
+            read_part(n_constant, read_buffer, std::integral_constant<int, 1 - q>(), parts[1 - q]);
+          constexpr int kOps = kHeld / 2 * kGranuleOps;
+          constexpr int first = n * kOps / kPhaseMmas;
+          StaticFor<(n + 1) * kOps / kPhaseMmas - first>([&](auto o) {
+            constexpr int op = first + decltype(o)::value;
+            granule_op(std::integral_constant<int, op % kGranuleOps>(),
+                       std::integral_constant<int, kHeld / 2 * (1 - q) + op / kGranuleOps>(), write_buffer, load_step);
+          });
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+      using First = std::integral_constant<int, 0>;
+      using Second = std::integral_constant<int, 1>;
+      auto split_all = [&](auto first_constant, int buffer, int load_step) {
+        StaticFor<kHeld / 2>([&](auto g) {
+          StaticFor<kGranuleOps>([&](auto op) {
+            granule_op(op, std::integral_constant<int, decltype(first_constant)::value + decltype(g)::value>(), buffer,
+                       load_step);
+          });
+        });
+      };
+      StaticFor<kHeld>([&](auto n) { load(n, 0); });
+      load_edge_params();
+      place(0, 0, kHeld);
+      split_all(std::integral_constant<int, 0>(), 0, 1);
+      split_all(std::integral_constant<int, kHeld / 2>(), 0, 1);
+      place(1, 0, kHeld / 2);
+      split_all(std::integral_constant<int, 0>(), 1, 2);
+      barrier();
+      StaticFor<kReads>([&](auto which) { read_part(which, 0, First(), parts[0]); });
+      for (int kt = 0; kt < k_tiles; ++kt) {
+        const int buffer = kt & 1;
+        place(kt + 1, kHeld / 2, kHeld);
+        phase(First(), buffer, 1 - buffer, kt + 2);
+        barrier();
+        place(kt + 2, 0, kHeld / 2);
+        phase(Second(), 1 - buffer, buffer, kt + 3);
+      }
+      float_parts::Drain(acc, small);
+      float not_finite = 0;
+#pragma unroll
+      for (int b = 0; b < kAB * kBB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          acc[b / kBB][b % kBB][v] += small[b / kBB][b % kBB][v];
+          not_finite = __builtin_fmaf(acc[b / kBB][b % kBB][v], 0.f, not_finite);
+        }
+      bool tiny = false;
+#pragma unroll
+      for (int n = 0; n < kHeld; ++n) tiny = tiny || float_parts::AllTiny(magnitudes[n]);
+      in_parts = !__syncthreads_or(not_finite != 0.f || tiny);
+      if (!in_parts) {
+        clear_accumulators();
+        __syncthreads();
+      }
+    }
+    if (!in_parts) {
     Frags f[2];
     // The fragments of consecutive sub-steps alternate between f[0] and f[1].
     // `parity`: which of the two the step's first sub-step finds its fragments
@@ -1534,6 +1862,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         ring_step(kt + 1, std::false_type(), Odd(), std::true_type());
       }
       if (kt < k_tiles) ring_step(kt, std::false_type(), Even(), std::true_type());
+    }
     }
     }
   }
@@ -2213,10 +2542,25 @@ template <int WM, int WN, int STAGES, bool kDepthWaves>
 constexpr int WavesPerSimdWanted() {
   return (!kDepthWaves && STAGES == 2 && WM * WN == 2) ? 3 : 1;
 }
+// The form a kernel runs in: its own, or, on the 128x128 tile of fp32, eight waves
+// of 64x32 (Traits::EightWaves).
+template <typename Traits, int WM, int WN, bool kEight = Traits::kParts && WM == 2 && WN == 2>
+struct FormOf {
+  using T = Traits;
+  static constexpr int kWN = WN;
+};
+template <typename Traits, int WM, int WN>
+struct FormOf<Traits, WM, WN, true> {
+  using T = typename Traits::EightWaves;
+  static constexpr int kWN = 1;
+};
 template <typename Traits, int WM, int WN, int BK, int STAGES, bool kFusedSums = false, bool kFlip = false,
           bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false, int kStaged = kNotStaged>
-__global__ __launch_bounds__(256, (WavesPerSimdWanted<WM, WN, STAGES, kDepthWaves>())) void MfmaGemmKernel(GemmArgs args) {
-  MfmaGemmBody<Traits, WM, WN, BK, STAGES, kFusedSums, kFlip, kDepthWaves, kRowSums, kSplitLarge, kStaged>(args);
+__global__ __launch_bounds__((128 * FormOf<Traits, WM, WN>::T::kWavesN),
+                             (WavesPerSimdWanted<WM, WN, STAGES, kDepthWaves>())) void MfmaGemmKernel(GemmArgs args) {
+  using Form = FormOf<Traits, WM, WN>;
+  MfmaGemmBody<typename Form::T, WM, Form::kWN, BK, STAGES, kFusedSums, kFlip, kDepthWaves, kRowSums, kSplitLarge,
+               kStaged>(args);
 }
 
 // Several products of one shape in one launch: grid.z counts the products,
@@ -2239,7 +2583,7 @@ __global__ __launch_bounds__(256) void MfmaGemmBatchKernel(GemmArgs args, GemmBa
 template <typename Traits, int WM, int WN, int BK, int STAGES, bool kFusedSums = false, bool kFlip = false,
           bool kDepthWaves = false>
 hipError_t LaunchBatch(hipStream_t stream, const GemmArgs& args, const GemmBatch& batch, int count) {
-  using C = Cfg<WM, WN, BK, STAGES, Traits::kSplitB, Traits::kBlock>;
+  using C = Cfg<WM, WN, BK, STAGES, Traits::kSplitB, Traits::kBlock, Traits::kWavesN>;
   if (count < 1 || count > kGemmBatchMax || args.split_k != 1) return hipErrorInvalidValue;
   const int total = TileCount(args, C::kBM, C::kBN);
   const int grid = ((total + 7) / 8) * 8;
@@ -2257,7 +2601,8 @@ hipError_t LaunchBatch(hipStream_t stream, const GemmArgs& args, const GemmBatch
 template <typename Traits, int WM, int WN, int BK, int STAGES, bool kFusedSums = false, bool kFlip = false,
           bool kDepthWaves = false, bool kRowSums = false, bool kSplitLarge = false, int kStaged = kNotStaged>
 hipError_t Launch(hipStream_t stream, const GemmArgs& args) {
-  using C = Cfg<WM, WN, BK, STAGES, Traits::kSplitB, Traits::kBlock>;
+  using Form = FormOf<Traits, WM, WN>;
+  using C = Cfg<WM, Form::kWN, BK, STAGES, Traits::kSplitB, Traits::kBlock, Form::T::kWavesN>;
   const int tiles_m = (args.M + C::kBM - 1) / C::kBM;
   const int tiles_n = (args.N + C::kBN - 1) / C::kBN;
   const int total = tiles_m * tiles_n;
@@ -2344,9 +2689,11 @@ enum class Tile { k256x256, k128x128, k128x64, k64x128, k64x64 };
 // What the fit says about the kernels: on int8 the 256x256 tile's depth step
 // (1.16 us) is well under half of what the 64x64 tile needs for the same area
 // (16 x 0.195 us) and 54 % of the 128x128 tile's (4 x 1.07 us / 2 side by side), so it
-// wins whenever its tiles fill most of a round; fp32 is bound by its matrix
-// instructions at every tile size (7.85 us against 16 x 0.562 us) and the small
-// tiles, which fill the CUs more evenly, win up to destinations of 4096^2.
+// wins whenever its tiles fill most of a round. fp32 (fitted again to 110 shapes,
+// within 4-6 %; choosing by it costs 0.2 % over the fastest): the 128x128 tile's
+// step takes 1.27 us against 4 x 0.37 us, since it splits a float half as often and
+// asks L2 for half as much, and no larger one is needed. Step of the same area on
+// fp32 instructions: 2.15 and 0.56 us.
 // Tiles of 256x128 and 128x256 were built too, were the fastest at no shape
 // measured, and are not kept; neither is a second launch on a smaller tile for
 // the part of a 256x256 grid that does not fill its last round, which lost to
@@ -2374,12 +2721,14 @@ constexpr TileTiming kInt8Timings[] = {
     {Tile::k64x128, 64, 128, 4.55, 0.17, 0.334, 0.90, 3, {0.501, 0.742, 1.567}, 0.12},
     {Tile::k64x64, 64, 64, 1.47, 13.42, 0.195, 0.94, 1, {}, 0},
 };
+// (The 128x128 and 64x64 tiles of fp32 run on bf16 matrix instructions,
+// float_parts.h; those in between, whose waves hold too few blocks for that, on
+// fp32 ones, for grids of short depths.)
 constexpr TileTiming kF32Timings[] = {
-    {Tile::k256x256, 256, 256, 0.0, 2.21, 7.854, 0.88, 1, {}, 0},
-    {Tile::k128x128, 128, 128, 1.45, 3.02, 2.153, 0.85, 2, {1.751, 3.656}, 1.0},
+    {Tile::k128x128, 128, 128, 1.46, 6.93, 1.269, 0.78, 1, {}, 0},
     {Tile::k128x64, 128, 64, 2.74, 2.74, 1.190, 0.83, 3, {1.037, 1.980, 2.722}, 0.91},
     {Tile::k64x128, 64, 128, 3.03, 2.54, 1.152, 0.84, 3, {1.114, 1.977, 2.757}, 0.84},
-    {Tile::k64x64, 64, 64, 1.75, 6.46, 0.562, 0.86, 1, {}, 0},
+    {Tile::k64x64, 64, 64, 2.57, 13.39, 0.371, 0.74, 1, {}, 0},
 };
 // The plane-split form of the int16 kernel has the two square large tiles and
 // one of 64 rows x 128 plane columns (64 destination columns); `bn` counts
@@ -2393,7 +2742,7 @@ constexpr TileTiming kInt8PlaneSplitTimings[] = {
 inline TimingModel TimingModelOf(Model model) {
   switch (model) {
     case Model::kF32:
-      return {kF32Timings, 5, Tile::k64x64, 16, 3.1};
+      return {kF32Timings, 4, Tile::k64x64, 16, 2.6};
     case Model::kInt8PlaneSplit:
       return {kInt8PlaneSplitTimings, 3, Tile::k64x128, 8, 3.6};
     default:
@@ -2862,16 +3211,21 @@ hipError_t LaunchTile(hipStream_t stream, const GemmArgs& args, Tile tile, int n
         if (args.split_k > 1)
           return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, false, true>(stream, args);
       }
-      return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip>(stream, args);
+      if constexpr (!Traits::kParts) return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip>(stream, args);
+      break;
     case Tile::k128x128:
       if constexpr (Traits::kModel == Model::kInt8) {
         if (args.row_sums && ShallowRing(args, num_cus, 128, 128))
           return Launch<Traits, 2, 2, 128, 2, false, kFlip, false, true>(stream, args);
         if (args.row_sums) return Launch<Traits, 2, 2, 128, 4, false, kFlip, false, true>(stream, args);
       }
-      if (!Traits::kSplitB && ShallowRing(args, num_cus, 128, 128))
-        return Launch<Traits, 2, 2, 128, 2, false, kFlip>(stream, args);
-      return Launch<Traits, 2, 2, 128, 4, false, kFlip>(stream, args);
+      if constexpr (Traits::kParts) {
+        return Launch<Traits, 2, 2, 128, 2>(stream, args);
+      } else {
+        if (!Traits::kSplitB && ShallowRing(args, num_cus, 128, 128))
+          return Launch<Traits, 2, 2, 128, 2, false, kFlip>(stream, args);
+        return Launch<Traits, 2, 2, 128, 4, false, kFlip>(stream, args);
+      }
     case Tile::k64x128:
       if constexpr (Traits::kSplitB) return LaunchSmallestTile<Traits>(stream, args);
       if constexpr (Traits::kModel == Model::kInt8) {
@@ -2886,6 +3240,8 @@ hipError_t LaunchTile(hipStream_t stream, const GemmArgs& args, Tile tile, int n
   }
   if constexpr (!Traits::kSplitB) {
     switch (tile) {
+      case Tile::k256x256:
+        break;
       case Tile::k128x64:
         if constexpr (Traits::kModel == Model::kInt8) {
           if (args.row_sums && ShallowRing(args, num_cus, 128, 64))

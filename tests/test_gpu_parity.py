@@ -349,6 +349,65 @@ def _rows_with_nan_between(rng, rows, depth, cols, orders):
     return p
 
 
+@pytest.mark.parametrize("tile", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("values", ["ordinary", "mixed", "tiny", "infinite", "overflowing", "zeros"])
+def test_fp32_values_that_are_not_sums_of_bf16_parts(device_ctx, tile, values):
+    """The tiles that split a float into three bf16 parts, on values that the split
+    or the bf16 range loses: what comes out is what fp32 instructions give. Held
+    against 64-bit sums, element by element. An fp32 sum of K products errs by at
+    most K 2^-24 of the sum of their magnitudes; the parts leave 2^-23 of it out
+    besides, and errors have signs of their own, so a sixteenth of K + 2 such units
+    is allowed (measured: a fortieth of it at most)."""
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(7)
+    device_ctx.force_tile(*tile)
+    try:
+        for rows, depth, cols in [(130, 131, 70), (300, 1031, 140)]:
+            p = W.random_problem(rng, S.F32, S.F32, S.F32, S.F32, rows, depth, cols, 1, 0, 0, strided=False,
+                                 name="fp32 values %s %dx%dx%d" % (values, rows, depth, cols))
+            p.clamp_min, p.clamp_max = -np.inf, np.inf
+            if p.bias is not None:
+                p.bias[:] = 0
+            a = p.lhs.storage[:rows * depth].reshape(rows, depth)
+            b = p.rhs.storage[:cols * depth].reshape(cols, depth)
+            if values == "mixed":  # every product of order one, its factors over 2^+-100
+                powers = np.exp2(rng.integers(-100, 101, depth)).astype(np.float32)
+                a *= powers
+                b /= powers
+            elif values == "tiny":  # rows whose parts would be subnormal, and subnormal rows
+                a *= np.float32(2.0 ** -118)
+                a[::7] *= np.float32(2.0 ** -14)
+                b *= np.float32(2.0 ** 110)
+            elif values == "infinite":
+                a[rows // 2, depth // 3] = np.inf
+                a[rows // 3, depth - 1] = -np.inf
+                a[rows - 1, 0] = np.nan
+                b[cols // 2, depth // 3] = 0.0
+            elif values == "overflowing":  # rounds to infinity as bf16, and products beyond the range
+                a[1, 1] = np.float32(3.4028234e38)
+                b[:, 1] = np.float32(0.5)
+                a[2, 5] = np.float32(3e38)
+                b[3, 5] = np.float32(8.0)
+            elif values == "zeros":
+                a[:] = 0
+                a[5] = -0.0
+                b[2] = 0
+            got = O.dense_of(p, D.device_mul(device_ctx, p)).astype(np.float64).reshape(rows, cols)
+            with np.errstate(all="ignore"):
+                want = a.astype(np.float64) @ b.astype(np.float64).T
+                scale = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+                want = np.where(np.abs(want) > np.finfo(np.float32).max, np.sign(want) * np.inf, want)
+                finite = np.isfinite(want)
+                assert (np.isnan(got) == np.isnan(want)).all(), p.name
+                assert (got[~finite & ~np.isnan(want)] == want[~finite & ~np.isnan(want)]).all(), p.name
+                # (the smallest subnormal float is 2^-149)
+                bound = (depth / 16 + 2) * 2.0 ** -24 * scale[finite] + depth * 2.0 ** -149
+                worst = np.max(np.abs(got[finite] - want[finite]) / bound)
+            assert worst <= 1, (p.name, worst)
+    finally:
+        device_ctx.force_tile(0, 0)
+
+
 @pytest.mark.parametrize("tile,rows,cols", cases.F32_SHALLOW_RINGS)
 @pytest.mark.parametrize("depth", [1, 2, 3, 5, 31, 33, 63, 65, 98, 127, 163, 513, 1111])
 def test_fp32_rows_of_any_depth_on_rings_of_two_stages(device_ctx, tile, rows, cols, depth):

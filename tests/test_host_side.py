@@ -304,7 +304,7 @@ def test_products_that_the_larger_tiles_do_faster_stay_there(runtime_model):
         # Operands that the caches hold.
         (f32, 2176, 288, 1520, (1, 1, 1), 0, False), (f32, 2174, 176, 1652, (1, 1, 0), 1, False),    # 28.0 33.1, 24.7 28.1 us
         (f32, 2232, 1708, 1352, (1, 0, 0), 0, False), (f32, 2048, 176, 1424, (1, 1, 0), 0, False),   # 106 116, 22.5 24.4
-        (f32, 762, 28, 3856, (1, 1, 0), 0, True), (f32, 860, 2832, 1686, (1, 0, 0), 0, True),        # 15.6 11.5, 93.1 83.9
+        (f32, 762, 28, 3856, (1, 1, 0), 0, True), (f32, 860, 2832, 1686, (1, 0, 0), 0, False),       # 15.6 11.5, 71.1 80.4
         (i8i16, 448, 3764, 2816, (1, 0, 0), 1, False), (i16i8, 1112, 1888, 1536, (0, 0, 1), 0, False),  # 37.7 53.1, 24.6 31.0
         (i8i16, 3312, 7112, 379, (0, 0, 0), 0, False), (i16i8, 3729, 3733, 390, (1, 0, 0), 1, False),   # 69.5 83.5, 50.5 59.7
         (i8i16, 191, 2624, 5940, (1, 1, 1), 0, True), (i16i8, 351, 2016, 4218, (1, 0, 0), 0, True)]     # 1.49 and 1.18 times
