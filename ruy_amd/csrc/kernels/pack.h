@@ -24,7 +24,7 @@ struct PackSource {
 // of the reference's Pack (ruy/pack.h:105-132 with the uint8 -> int8 conversion
 // of ruy/pack_common.h:36-58): vector c goes to dst + c * ld (`ld` in bytes, a
 // multiple of 16; 8-bit values as int8), zero-filled from its K values up to
-// ld. With `sums`, sums[c] becomes the sum of the packed 8-bit values; only for
+// the end of their last 16 bytes. With `sums`, sums[c] becomes the sum of the packed 8-bit values; only for
 // operands of which PackFormsSums says so.
 struct PackJob {
   PackSource src;
@@ -37,7 +37,7 @@ hipError_t LaunchPack(hipStream_t stream, const PackJob* jobs, int count);
 // Whether the launch walks the whole depth of every vector in one place, so
 // that the sums come with it. Otherwise whoever reads the packed operand forms
 // them, like those of an operand used in place.
-bool PackFormsSums(const PackSource& src, int32_t ld);
+bool PackFormsSums(const PackSource& src);
 
 // int16 operand for the int8 matrix cores: each value v is split into
 // hi = v >> 8 (signed) and lo = (v & 0xff) - 128, both int8, so that

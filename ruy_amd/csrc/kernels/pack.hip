@@ -48,6 +48,12 @@ struct PackPlan {
   int32_t k_span = 0;          // depth bytes (fp32: positions) of a part
 };
 
+// Bytes of a packed vector, to the end of its last granule.
+__host__ __device__ inline int PackedDepth(const PackSource& src) {
+  const int bytes = src.K * (src.dtype == RUYAMD_DTYPE_F32 ? 4 : 1);
+  return bytes > 16 ? (bytes + 15) / 16 * 16 : 16;
+}
+
 // Depth-contiguous source of any alignment and depth (8-bit or fp32: bytes are
 // moved): kLanes lanes to a vector, four granules of a lane in flight. (Rows of
 // less than a granule are a case of their own, kShort: a fork in front of each
@@ -64,7 +70,7 @@ __device__ __forceinline__ void PackRowsOf(const PackJob& job, int k_span, int b
   const uint8_t* row =
       static_cast<const uint8_t*>(job.src.data) + int64_t(min(c, job.src.count - 1)) * job.src.stride_c * element;
   const uint32_t flip = job.src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
-  const int k_end = min(job.ld, (by + 1) * k_span);
+  const int k_end = min(PackedDepth(job.src), (by + 1) * k_span);
   const int end = min(k_end, bytes);
   char* out = static_cast<char*>(job.dst) + int64_t(c) * job.ld;
   constexpr int kInFlight = kShort ? 1 : 4;
@@ -116,9 +122,9 @@ __device__ __forceinline__ void PackTranspose8(const PackJob& job, int k_span, i
   const PackSource& src = job.src;
   const int tid = threadIdx.x;
   const int c0 = bx * kTileC;
-  const int ld = job.ld;
+  const int ld = job.ld, depth = PackedDepth(src);
   const int k_begin = by * k_span;
-  const int k_end = min(k_begin + k_span, ld);
+  const int k_end = min(k_begin + k_span, depth);
   const uint8_t* s = static_cast<const uint8_t*>(src.data);
   int8_t* dst = static_cast<int8_t*>(job.dst);
   const uint32_t flip = src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
@@ -160,7 +166,7 @@ __device__ __forceinline__ void PackTranspose8(const PackJob& job, int k_span, i
     __syncthreads();
     const int c = c0 + wc;
     const int k = k0 + wg * 16;
-    if (c < src.count && k < ld) {
+    if (c < src.count && k < depth) {
       const uint32_t* row = reinterpret_cast<const uint32_t*>(tile + wc * kPitch + wg * 16);
       v4i out;
 #pragma unroll
@@ -191,10 +197,10 @@ __device__ __forceinline__ void PackTranspose32(const PackJob& job, int k_span, 
   const int tx = threadIdx.x & 31;
   const int ty = threadIdx.x >> 5;  // 0..7
   const int c0 = bx * kTile32;
-  const int ld = job.ld / 4;
+  const int ld = job.ld / 4, depth = PackedDepth(src) / 4;
   const float* s = static_cast<const float*>(src.data);
   float* dst = static_cast<float*>(job.dst);
-  const int k_end = min(ld, (by + 1) * k_span);
+  const int k_end = min(depth, (by + 1) * k_span);
   for (int k0 = by * k_span; k0 < k_end; k0 += kTile32) {
 #pragma unroll
     for (int t = ty; t < kTile32; t += 8) {
@@ -209,7 +215,7 @@ __device__ __forceinline__ void PackTranspose32(const PackJob& job, int k_span, 
     for (int t = ty; t < kTile32; t += 8) {
       const int c = c0 + t;
       const int k = k0 + tx;
-      if (c < src.count && k < ld) dst[int64_t(c) * ld + k] = tile[t][tx];
+      if (c < src.count && k < depth) dst[int64_t(c) * ld + k] = tile[t][tx];
     }
     __syncthreads();
   }
@@ -296,8 +302,9 @@ int StepsPerPart(int steps, int blocks_c, int blocks_wanted, int* parts) {
   return per_part;
 }
 
-PackPlan PlanOf(const PackSource& src, int32_t ld) {
+PackPlan PlanOf(const PackSource& src) {
   PackPlan plan;
+  const int32_t ld = PackedDepth(src);
   if (src.stride_k == 1) {
     // 16 lanes to a row of up to 1 KiB (what they have in flight at a time).
     plan.kind = ld <= 1024 ? kRows16 : kRows64;
@@ -524,9 +531,9 @@ hipError_t LaunchPack(hipStream_t stream, const PackJob* jobs, int count) {
   for (int i = 0; i < count; ++i) {
     const PackJob& job = jobs[i];
     if (job.src.count == 0 || job.ld == 0) continue;
-    const PackPlan plan = PlanOf(job.src, job.ld);
+    const PackPlan plan = PlanOf(job.src);
     if (used == 2 || job.ld % 16 != 0 || (job.src.stride_k != 1 && job.src.stride_c != 1) ||
-        (job.sums && !PackFormsSums(job.src, job.ld)))
+        (job.sums && !PackFormsSums(job.src)))
       return hipErrorInvalidValue;
     launch.job[used] = job;
     launch.blocks_c[used] = plan.blocks_c;
@@ -543,8 +550,8 @@ hipError_t LaunchPack(hipStream_t stream, const PackJob* jobs, int count) {
   return hipGetLastError();
 }
 
-bool PackFormsSums(const PackSource& src, int32_t ld) {
-  return src.dtype != RUYAMD_DTYPE_F32 && (src.count == 0 || ld == 0 || PlanOf(src, ld).parts == 1);
+bool PackFormsSums(const PackSource& src) {
+  return src.dtype != RUYAMD_DTYPE_F32 && (src.count == 0 || PlanOf(src).parts == 1);
 }
 
 hipError_t LaunchSumsI8(hipStream_t stream, const int8_t* data, int32_t ld, int32_t count, int32_t K,
