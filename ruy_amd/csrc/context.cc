@@ -1,5 +1,7 @@
 #include "context.h"
 
+#include <algorithm>
+
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -34,8 +36,15 @@ void* Workspace::Alloc(std::size_t bytes) {
     if (b.size - b.used >= need) {
       void* p = b.base + b.used;
       b.used += need;
+      taken_ += need;
       return p;
     }
+  }
+  if (turn_ && turn_ * Piece() - wrapped_used_ >= need) {
+    void* p = blocks_[0].base + wrapped_used_;
+    wrapped_used_ += need;
+    taken_ += need;
+    return p;
   }
   if (!growth_allowed_ || fixed_) {
     exhausted_ = true;
@@ -49,6 +58,7 @@ void* Workspace::Alloc(std::size_t bytes) {
     return nullptr;
   }
   blocks_.push_back(Block{static_cast<char*>(p), size, need});
+  taken_ += need;
   return p;
 }
 
@@ -59,9 +69,18 @@ void* Workspace::AllocOptional(std::size_t bytes) {
   return p;
 }
 
+std::size_t Workspace::Piece() const { return blocks_[0].size / turns_ & ~std::size_t(255); }
+
 void Workspace::Reset() {
   exhausted_ = false;
-  if (blocks_.size() > 1 && !pinned_ && growth_allowed_ && !fixed_) {
+  const bool may_replace = !pinned_ && growth_allowed_ && !fixed_;
+  // Calls that go on needing scratch get room for several of them.
+  std::size_t wanted = 0;
+  if (may_replace && taken_ > 0 && taken_ <= kTurnsUpTo && (calls_ >= kTurnsFrom || ++calls_ >= kTurnsFrom)) {
+    wanted = TurnsFor(taken_) * (taken_ + 256);
+    if (capacity() >= wanted) wanted = 0;
+  }
+  if ((blocks_.size() > 1 && may_replace) || wanted) {
     // Coalesce: one block as large as everything the last call needed.
     std::size_t total = 0;
     for (auto& b : blocks_) {
@@ -69,15 +88,25 @@ void Workspace::Reset() {
       (void)hipFree(b.base);
     }
     blocks_.clear();
-    void* p = nullptr;
-    if (hipMalloc(&p, total) == hipSuccess) {
-      blocks_.push_back(Block{static_cast<char*>(p), total, 0});
-    } else {
+    for (std::size_t size : {std::max(total, wanted), total}) {
+      void* p = nullptr;
+      if (hipMalloc(&p, size) == hipSuccess) {
+        blocks_.push_back(Block{static_cast<char*>(p), size, 0});
+        break;
+      }
       (void)hipGetLastError();
     }
+    turn_ = 0;
+    taken_ = wrapped_used_ = 0;
     return;
   }
+  // (A call that may not add to the workspace has all of it in one piece.)
+  turns_ = TurnsFor(taken_);
+  const bool apart = growth_allowed_ && !fixed_ && blocks_.size() == 1 && taken_ > 0 && taken_ <= Piece();
+  turn_ = apart ? (turn_ + 1) % turns_ : 0;
+  taken_ = wrapped_used_ = 0;
   for (auto& b : blocks_) b.used = 0;
+  if (turn_) blocks_[0].used = turn_ * Piece();
 }
 
 HostStaging::~HostStaging() {

@@ -652,6 +652,68 @@ void ScratchBlocks() {
   }
 }
 
+// A workspace whose calls take turns with its pieces: made large enough once, from
+// the eighth call that needs scratch on, by no more than four times what a call
+// takes; a call that is recorded finds its room whoever's turn it is, also one that
+// takes more than a piece, and a growing one only adds what it needs.
+void ScratchInTurns() {
+  auto on_device = [] {
+    std::size_t sum = 0;
+    for (const auto& range : R().device) sum += range.second;
+    return sum;
+  };
+  struct {
+    int M, K, N;
+    bool turns;
+  } const cases[] = {{1000, 1501, 700, true}, {2000, 4099, 2100, true}, {6000, 15000, 1100, false}};
+  for (const auto& k : cases) {
+    DeviceCall call(std::size_t(k.M) * k.K, std::size_t(k.K) * k.N, std::size_t(k.M) * k.N);
+    const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, k.M, k.K, RUYAMD_ORDER_COL_MAJOR, 4);
+    const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, call.rhs, k.K, k.N, RUYAMD_ORDER_ROW_MAJOR, 3);
+    const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, k.M, k.N, RUYAMD_ORDER_COL_MAJOR);
+    ruyamd_mat small_l = l, small_d = d;
+    small_l.rows = small_d.rows = k.M / 3;
+    const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+    Context c;
+    const std::size_t before = on_device();
+    std::size_t once = 0;
+    for (int i = 1; i <= 20; ++i) {
+      R().allocations = 0;
+      EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+      if (i == 1) once = on_device() - before;
+      EXPECT(R().allocations == 0 || i <= 2 || (k.turns && i <= 10), "call %d: %d allocations", i, R().allocations);
+      EXPECT(on_device() - before <= (k.turns ? 4 : 1) * once + (1 << 20), "call %d: %zu bytes, one call %zu", i,
+             on_device() - before, once);
+      if (i >= 15) {
+        R().capturing = true;
+        EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "recorded behind call %d: %s", i, ruyamd_ctx_last_error(c.ctx));
+        R().capturing = false;
+        EXPECT(R().capture_violations == 0, "behind call %d", i);
+      }
+    }
+    Context fresh;
+    for (int i = 1; i <= 24; ++i) {
+      const bool small = i <= 12 || i % 3 == 0;
+      EXPECT(ruyamd_mul(fresh.ctx, small ? &small_l : &l, &r, &p, small ? &small_d : &d) == RUYAMD_OK, "%s",
+             ruyamd_ctx_last_error(fresh.ctx));
+    }
+    R().allocations = 0;
+    for (int i = 0; i < 9; ++i)
+      EXPECT(ruyamd_mul(fresh.ctx, i % 3 ? &l : &small_l, &r, &p, i % 3 ? &d : &small_d) == RUYAMD_OK, "%s",
+             ruyamd_ctx_last_error(fresh.ctx));
+    EXPECT(R().allocations == 0, "%d allocations", R().allocations);
+    for (const bool small : {false, true, false}) {
+      R().capturing = true;
+      EXPECT(ruyamd_mul(fresh.ctx, small ? &small_l : &l, &r, &p, small ? &small_d : &d) == RUYAMD_OK, "%s",
+             ruyamd_ctx_last_error(fresh.ctx));
+      R().capturing = false;
+      EXPECT(ruyamd_mul(fresh.ctx, small ? &l : &small_l, &r, &p, small ? &d : &small_d) == RUYAMD_OK, "%s",
+             ruyamd_ctx_last_error(fresh.ctx));
+    }
+    EXPECT(R().capture_violations == 0, "%d x %d x %d", k.M, k.K, k.N);
+  }
+}
+
 bool Staged(const std::string& kernel) {
   return kernel.find("MfmaGemmKernel") != std::string::npos &&
          (kernel.find("Lb0ELi1EEEv") != std::string::npos || kernel.find("Lb0ELi2EEEv") != std::string::npos);
@@ -754,6 +816,7 @@ int main(int argc, char** argv) {
   else if (which == "capture") Capture();
   else if (which == "raw_rows") RawRowsNeedNoScratch();
   else if (which == "scratch_blocks") ScratchBlocks();
+  else if (which == "scratch_in_turns") ScratchInTurns();
   else if (which == "staged_rule") StagedRule();
   else return 2;
   if (g_failures) {

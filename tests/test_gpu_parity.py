@@ -936,6 +936,35 @@ def test_first_and_last_ring_steps_of_every_tile(tup):
         ctx.close()
 
 
+def test_packed_operands_of_calls_in_a_row():
+    """Calls whose operands are packed, one behind the other on one context without a
+    wait, in more of them than its scratch memory has pieces, with larger and smaller
+    ones between: each is checked against the oracle when all have run."""
+    import torch
+    from ruy_amd import api
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(11)
+    types = (S.I8, S.I8, S.I32, S.I8)
+    small = [W.random_problem(rng, *types, 300, 1501, 260, 0, 1, 0, strided=True, name="in turns small") for _ in range(2)]
+    large = [W.random_problem(rng, *types, 900, 2051, 1030, 1, 0, 1, strided=False, name="in turns large")]
+    f32 = [W.random_problem(rng, S.F32, S.F32, S.F32, S.F32, 400, 515, 390, 0, 1, 0, strided=True, name="in turns fp32")]
+    order = (small * 6 + large + small + large * 3 + f32 * 2) * 2
+    ctx = api.Context()
+    try:
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        ctx.set_synchronous(False)
+        ctx.force_tile(128, 128)  # (tiles that need their operands packed)
+        problems = [D.DeviceProblem(p, dst_fill=0) for p in order]
+        for dp in problems:
+            dp.run(ctx)
+        torch.cuda.synchronize()
+        want = {p.name + str(id(p)): expected(p, fill=0) for p in order}
+        for p, dp in zip(order, problems):
+            compare(p, dp.result(), want[p.name + str(id(p))], exact_fp=False)
+    finally:
+        ctx.close()
+
+
 def test_two_contexts_on_two_threads():
     """The reference's rule (ruy/ruy.h:82-95): a Context serves one thread, and
     concurrent Mul calls need distinct Contexts. Two threads, each with its own

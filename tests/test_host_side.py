@@ -252,6 +252,10 @@ def test_rows_read_where_they_lie_need_no_scratch_memory(runtime_model):
     runtime_model("raw_rows")
 
 
+def test_calls_take_turns_with_the_pieces_of_their_scratch_memory(runtime_model):
+    runtime_model("scratch_in_turns")
+
+
 def test_sums_left_to_the_product_take_no_scratch_memory(runtime_model):
     runtime_model("scratch_blocks")
 
