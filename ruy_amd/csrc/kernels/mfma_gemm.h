@@ -305,9 +305,13 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   static_assert(!kLeadSums || (Traits::kBlock == 32 && !Traits::kSplitB && !kSplitLarge), "");
   static_assert(!kSplitLarge || Traits::kPaired, "kSplitLarge is the depth split of the paired schedule's tile");
   // kFusedSums on the 128x128 tile (two by two blocks per wave, waves sharing
-  // every step): the row sums of `a` only, one more matrix instruction per
-  // block row and sub-step. That tile's steps wait for LDS, not for the matrix
-  // pipe, as long as a CU holds one workgroup, which is when it is used.
+  // every step): the row sums of `a` only. Each of the two waves that hold the same
+  // 64 rows adds up 32 of them, one v_xor and one v_sad_u8 of its fragments behind
+  // every matrix instruction, which run while the matrix pipe is busy (v_dot4 would
+  // wait for it, 22 clocks behind a matrix instruction; a matrix instruction more
+  // per block row costs 0.10 us a step where these cost 0.03; with all 64 rows in
+  // both waves 0.06). 2048^3 13.9 us with the rows dealt out over the grid
+  // (kLeadSums), 13.4 so, 12.8 without sums; x 512 9.0, 8.1 and 7.9.
   constexpr bool kRowSumsOfFourBlocks = kFusedSums && WM == 2 && WN == 2;
   // Traits::kParts on the 128x128 tile: split on the way to LDS (below).
   constexpr bool kPartsInLds = Traits::kParts && Traits::kWavesN == 4;
@@ -637,6 +641,18 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     a_foff[ks] = LdsOffset<BK>(wave_m * WM * 32 + frag_row, ks * kGranulesPerMma + frag_half);
     b_foff[ks] = C::kBM * kBK + LdsOffset<BK>(wave_n * WN * 32 + frag_row, ks * kGranulesPerMma + frag_half);
   }
+  // (kRowSumsOfFourBlocks: the wave's first block row is the one it adds up; the
+  // two waves that hold the same rows have them in opposite order.)
+  const int first_block = kRowSumsOfFourBlocks ? wave_n : 0;
+  int a_second[C::kKSteps];
+  if constexpr (kRowSumsOfFourBlocks) {
+#pragma unroll
+    for (int ks = 0; ks < C::kKSteps; ++ks) {
+      a_second[ks] = a_foff[ks] + (1 - first_block) * kB * kBK;
+      a_foff[ks] += first_block * kB * kBK;
+    }
+  }
+  auto a_offset = [&](int ks, int i) { return kRowSumsOfFourBlocks && i == 1 ? a_second[ks] : a_foff[ks] + i * kB * kBK; };
   struct Frags {
     v4i a[kAB];
     v4i b[kBB];
@@ -645,7 +661,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     const char* stage = lds + (kt % C::kStages) * C::kStageBytes;
 #pragma unroll
     for (int i = 0; i < kAB; ++i)
-      f.a[i] = *reinterpret_cast<const v4i*>(stage + a_foff[ks] + i * kB * kBK);
+      f.a[i] = *reinterpret_cast<const v4i*>(stage + a_offset(ks, i));
 #pragma unroll
     for (int j = 0; j < kBB; ++j)
       f.b[j] = *reinterpret_cast<const v4i*>(stage + b_foff[ks] + j * kB * kBK);
@@ -659,7 +675,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     const bool is_a = kB == 32 ? r < kAB : r >= kBB;
     const int idx = kB == 32 ? (r < kAB ? r : r - kAB) : (r < kBB ? r : r - kBB);
     if (is_a)
-      f.a[idx] = *reinterpret_cast<const v4i*>(stage + a_foff[ks] + idx * kB * kBK);
+      f.a[idx] = *reinterpret_cast<const v4i*>(stage + a_offset(ks, idx));
     else
       f.b[idx] = *reinterpret_cast<const v4i*>(stage + b_foff[ks] + idx * kB * kBK);
   };
@@ -678,12 +694,13 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   if constexpr (!Traits::kPaired) clear_accumulators();
 
   typename Traits::Acc sum_a, sum_b;  // kFusedSums: row sums of a / column sums of b, in every column / row
-  typename Traits::Acc sum_a_second;  // kRowSumsOfFourBlocks: those of the wave's second block row
+  // kRowSumsOfFourBlocks: the lane's half of row l % 32 of the wave's first block
+  // row (v_sad_u8 takes every byte of the depth 128 too large).
+  uint32_t row_sum = 0u - static_cast<uint32_t>(kBK / 2 * 128) * static_cast<uint32_t>(k_tiles);
 #pragma unroll
   for (int v = 0; v < kAccElems; ++v) {
     sum_a[v] = 0;
     sum_b[v] = 0;
-    sum_a_second[v] = 0;
   }
   const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 
@@ -728,13 +745,16 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       constexpr int n = decltype(n_constant)::value;
       __builtin_amdgcn_sched_barrier(0);
       Traits::Mma(cur.a[n / kBB], cur.b[n % kBB], acc[n / kBB][n % kBB]);
-      if constexpr (kFusedSums && n == 0) {
+      if constexpr (kRowSumsOfFourBlocks) {
+        const uint32_t to_unsigned = 0x80808080u ^ (kFlip ? args.a_flip : 0u);
+        row_sum = __builtin_amdgcn_sad_u8(static_cast<uint32_t>(cur_raw.a[0][n]) ^ to_unsigned, 0u, row_sum);
+      }
+      if constexpr (kFusedSums && !kRowSumsOfFourBlocks && n == 0) {
         // Once per sub-step. The plane-split operand has zero point 0 by
         // definition, so its column sums are never needed.
         Traits::Mma(cur.a[0], ones, sum_a);
-        if constexpr (!Traits::kSplitB && !kRowSumsOfFourBlocks) Traits::Mma(ones, cur.b[0], sum_b);
+        if constexpr (!Traits::kSplitB) Traits::Mma(ones, cur.b[0], sum_b);
       }
-      if constexpr (kRowSumsOfFourBlocks && n == kBB) Traits::Mma(cur.a[1], ones, sum_a_second);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (!kReadsFirst && n < kReadSlots) {
         constexpr int kFirst = n * kFrags / kReadSlots;
@@ -1876,16 +1896,14 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     // (the write-back combines 256 * high + low).
     constexpr int kBlock = Traits::kSplitB ? 1 : 0;
     if constexpr (kRowSumsOfFourBlocks) {
-      // (A block of sums has the sum of its row in every column: it lines up
-      // with every accumulator block of that block row.)
-#pragma unroll
-      for (int j = 0; j < kBB; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          acc[0][j][v] = static_cast<int>(static_cast<uint32_t>(acc[0][j][v]) - fa * static_cast<uint32_t>(sum_a[v]));
-          acc[1][j][v] =
-              static_cast<int>(static_cast<uint32_t>(acc[1][j][v]) - fa * static_cast<uint32_t>(sum_a_second[v]));
-        }
+      // The two waves that hold the same 64 rows exchange their halves; lane l
+      // stages the parameters of row l.
+      static_assert(C::kEpilogueBytes + C::kParamBytes + C::kBM * 4 <= C::kLdsBytes, "");
+      int* const sums = reinterpret_cast<int*>(lds + C::kEpilogueBytes + C::kParamBytes) + wave_m * (WM * 32);
+      const auto halves = __builtin_amdgcn_permlane32_swap(row_sum, row_sum, false, false);
+      if (lane < 32) sums[first_block * 32 + lane] = static_cast<int>(halves[0] + halves[1]);
+      __syncthreads();
+      edge.bias[0] = static_cast<int>(static_cast<uint32_t>(edge.bias[0]) - fa * static_cast<uint32_t>(sums[lane]));
     } else {
 #pragma unroll
       for (int v = 0; v < 16; ++v)
@@ -2419,7 +2437,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
             w[1] = Traits::Bits(a[4 * q + 1], a2[4 * q + 1]);
             w[2] = Traits::Bits(a[4 * q + 2], a2[4 * q + 2]);
             w[3] = Traits::Bits(a[4 * q + 3], a2[4 * q + 3]);
-            const int r = bi * 32 + 8 * q + 4 * frag_half;
+            const int r = (bi ^ first_block) * 32 + 8 * q + 4 * frag_half;
             *reinterpret_cast<v4i*>(region + (bjj * 32 + frag_row) * kPitch + r) = w;
           }
         }
@@ -2779,13 +2797,16 @@ inline int DepthSplitParts(int tiles, int k_steps, int num_cus, int min_steps_pe
 // deals those of `a` out over its first workgroups where it may (a microsecond
 // and a half) and needs the kernel for those of `b`.
 inline double SumsKernelMicroseconds(double bytes) { return 1.5 + bytes / (1024.0 * 1024.0) * 0.134; }
-// The 128x128 tile can form the row sums of `a` itself (one matrix instruction
-// more per block row and sub-step) when only those are pending and the grid
-// leaves every CU at most one workgroup (with two, the matrix pipe is the
-// bound). Measured on 2048 x K x 2048 against the same launch without sums:
-// + 1.0 us at K = 512, + 2.3 us at 2048, + 7.2 us at 8192, where the sums
-// kernel in front costs 2.1, 2.3 and 3.8 us: it pays for short depths.
-inline double RowSumming128Microseconds(int k_steps) { return 0.6 + 0.103 * k_steps; }
+// The 128x128 tile can form the row sums of `a` itself, from the fragments that
+// its waves hold (two vector instructions behind every matrix instruction), when
+// only those are pending and the grid leaves every CU at most one workgroup.
+// 2048 x K x 2048 against the same launch without sums, us: K = 256 + 0.2, 512 + 0.2,
+// 1024 + 0.3, 2048 + 0.6; with the rows dealt out over the workgroups (below) + 1.1,
+// 1.2, 1.0 and 1.1. Where both forms may be used, the same call in us, dealt out ->
+// here: 2048 x 4096 x 2048 22.2 -> 22.0, x 6144 31.0 -> 30.9, x 8192 40.1 -> 39.7, but 1024 x
+// 8192 x 4096 39.0 -> 39.8 (x 4096 21.8 -> 21.9): up to 48 steps of the depth.
+constexpr int kRowSumming128Steps = 48;
+inline double RowSumming128Microseconds(int k_steps) { return 0.1 + 0.03 * k_steps; }
 // The tiles of 32x32 blocks whose waves share every step can have the rows of
 // `a` added up by the workgroups of their own grid, each taking a share of
 // the rows while its first loads are on their way (kLeadSums in the kernel),
@@ -2866,7 +2887,8 @@ inline double LeadColumnSumsMicroseconds(const GemmArgs& args, int num_cus, int 
 }
 inline bool RowSumming128Applies(const GemmArgs& args, int num_cus) {
   const int tiles = ((args.M + 127) / 128) * ((args.N + 127) / 128);
-  return (args.sums_wanted & 3) == 1 && tiles <= num_cus && !LeadSumsApply(args, num_cus, 128, 128) &&
+  return (args.sums_wanted & 3) == 1 && tiles <= num_cus &&
+         ((args.k_bytes + 127) / 128 <= kRowSumming128Steps || !LeadSumsApply(args, num_cus, 128, 128)) &&
          RowSumming128Microseconds((args.k_bytes + 127) / 128) < SumsKernelMicroseconds(double(args.M) * args.k_bytes);
 }
 inline double PendingSumsMicroseconds(const GemmArgs& args, int num_cus, const TimingModel& model,

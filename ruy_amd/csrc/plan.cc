@@ -1194,6 +1194,10 @@ int RunMulBatch(ruyamd_ctx* ctx, const MulCall& first, const BatchBuffers* items
   GemmArgs args;
   const bool swap = SetupInt8Gemm(ctx, first, a, b, lzp, rzp, /*staged=*/false, &args);
   if ((a.sums_pending || b.sums_pending) && !args.fuse_sums) return RUYAMD_OK;
+  // (With its sums in the launch the shape may be for the 128x128 tile, which has no batches.)
+  int tile_rows = 0, tile_cols = 0, parts = 0;
+  GemmTileFor(args, ctx->multiprocessor_count, GemmKind::kInt8, &tile_rows, &tile_cols, &parts);
+  if (tile_rows != 64 || tile_cols != 64) return RUYAMD_OK;
   const bool timed = ctx->TimingBegin();
   hipError_t launched = hipSuccess;
   for (int z0 = 0; z0 < n && launched == hipSuccess; z0 += kGemmBatchMax) {

@@ -1295,6 +1295,33 @@ def test_random_deep_and_weight_streaming_products_every_element(device_ctx):
     assert done == 14
 
 
+@pytest.mark.parametrize("depth", [16, 100, 128, 144, 512, 640, 1000, 6144, 6272])
+def test_sums_from_the_fragments_of_the_128x128_tile(depth):
+    """Grids of at most one 128x128 tile to a CU, operands in place: the zero
+    points' sums from the fragments that the waves hold, two waves to the same
+    rows. Depths that are no whole number of steps, that fit the ring as a whole,
+    and around the deepest that is done so; int8 and uint8 data, either
+    destination order, ragged tiles: the whole numbers of the oracle."""
+    from ruy_amd import api
+    from ruy_amd import device_problem as D
+    rng = np.random.default_rng(depth)
+    ctx = api.Context()
+    try:
+        ctx.force_tile(128, 128)
+        for tup, (M, N), orders, lzp, rzp in [((S.I8, S.I8, S.I32, S.I32), (129, 256), cases.RCC, 0, -3),
+                                              ((S.I8, S.I8, S.I32, S.I8), (200, 33), (1, 0, 1), 9, 0),
+                                              ((S.U8, S.U8, S.I32, S.U8), (97, 300), cases.RCC, 128, 121),
+                                              ((S.U8, S.I8, S.I32, S.I32), (260, 130), (1, 0, 1), 117, 0),
+                                              ((S.I8, S.U8, S.I32, S.I32), (140, 190), cases.RCC, 5, 130)]:
+            p = W.random_problem(rng, *tup, M, depth, N, *orders, strided=False, name="%s %dx%dx%d" % (tup, M, depth, N))
+            p.lhs.cache_policy = p.rhs.cache_policy = S.CACHE_NEVER
+            p.lhs.zero_point, p.rhs.zero_point = lzp, rzp
+            announce(p.name)
+            compare(p, D.device_mul(ctx, p, dst_fill=0), expected(p, fill=0))
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("mode", ["in launch", "own", "separate"])
 def test_row_sums_formed_by_the_workgroups_of_a_mid_tile_grid(mode):
     """Grids of 128x128, 128x64 or 64x128 tiles: the rows of the `a` operand
