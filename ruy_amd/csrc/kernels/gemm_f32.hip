@@ -30,6 +30,7 @@ struct F32Traits {
   static constexpr int kBlock = 32;
   static constexpr bool kAnyDepth = true;
   static constexpr bool kParts = true;
+  static constexpr bool kSumsOfBothSides = false;
   static constexpr int kWavesN = 2;
   using EightWaves = F32EightWaves;
   static constexpr bool kRawB = false;

@@ -148,6 +148,10 @@ hipError_t LaunchGemmI8(hipStream_t stream, const GemmArgs& args, int num_cus) {
   if (args.fuse_sums) {
     // Exists for the smallest tile only.
     if (!GemmI8CanFuseSums(args, num_cus)) return hipErrorInvalidValue;
+    if (mfma_gemm::PickTile(args, num_cus, mfma_gemm::Model::kInt8) == mfma_gemm::Tile::k128x128 &&
+        (args.sums_wanted & 2))
+      return flip ? mfma_gemm::LaunchRowSumming128<Int8BothSums, true>(stream, args, num_cus)
+                  : mfma_gemm::LaunchRowSumming128<Int8BothSums>(stream, args, num_cus);
     if (mfma_gemm::PickTile(args, num_cus, mfma_gemm::Model::kInt8) == mfma_gemm::Tile::k128x128)
       return flip ? mfma_gemm::LaunchRowSumming128<Int8Traits, true>(stream, args, num_cus)
                   : mfma_gemm::LaunchRowSumming128<Int8Traits>(stream, args, num_cus);

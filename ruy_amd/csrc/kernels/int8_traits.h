@@ -46,6 +46,7 @@ struct Int8Traits {
   static constexpr int kWavesN = 2;
   static constexpr bool kRawB = false;
   static constexpr bool kPaired = false;
+  static constexpr bool kSumsOfBothSides = false;
   // The 256x256 tile runs on 16x16 blocks (below).
   using LargeTile = Int8Traits16;
   using LargeTileStreamingA = Int8Traits16StreamingA;
@@ -191,6 +192,11 @@ struct Int8Traits {
       vals[q] = Median3(v, ep.clamp_min_i, ep.clamp_max_i);
     }
   }
+};
+
+// The same, for the form of the 128x128 tile that adds up the rows of both operands.
+struct Int8BothSums : Int8Traits {
+  static constexpr bool kSumsOfBothSides = true;
 };
 
 // The same arithmetic on v_mfma_i32_16x16x64_i8: a quarter of the accumulator

@@ -305,14 +305,15 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   static_assert(!kLeadSums || (Traits::kBlock == 32 && !Traits::kSplitB && !kSplitLarge), "");
   static_assert(!kSplitLarge || Traits::kPaired, "kSplitLarge is the depth split of the paired schedule's tile");
   // kFusedSums on the 128x128 tile (two by two blocks per wave, waves sharing
-  // every step): the row sums of `a` only. Each of the two waves that hold the same
-  // 64 rows adds up 32 of them, one v_xor and one v_sad_u8 of its fragments behind
+  // every step): the row sums of `a`, and of `b` where the traits ask for both. Each
+  // of the two waves that hold the same 64 rows adds up 32 of them, one v_xor and one v_sad_u8 of its fragments behind
   // every matrix instruction, which run while the matrix pipe is busy (v_dot4 would
   // wait for it, 22 clocks behind a matrix instruction; a matrix instruction more
   // per block row costs 0.10 us a step where these cost 0.03; with all 64 rows in
   // both waves 0.06). 2048^3 13.9 us with the rows dealt out over the grid
   // (kLeadSums), 13.4 so, 12.8 without sums; x 512 9.0, 8.1 and 7.9.
   constexpr bool kRowSumsOfFourBlocks = kFusedSums && WM == 2 && WN == 2;
+  constexpr bool kSumsOfBothSides = kRowSumsOfFourBlocks && Traits::kSumsOfBothSides;  // ... and the columns' of `b`
   // Traits::kParts on the 128x128 tile: split on the way to LDS (below).
   constexpr bool kPartsInLds = Traits::kParts && Traits::kWavesN == 4;
   static_assert(!kFusedSums || (WM == 1 && (WN == 1 || (Traits::kSplitB && WN == 2))) ||
@@ -642,17 +643,24 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     b_foff[ks] = C::kBM * kBK + LdsOffset<BK>(wave_n * WN * 32 + frag_row, ks * kGranulesPerMma + frag_half);
   }
   // (kRowSumsOfFourBlocks: the wave's first block row is the one it adds up; the
-  // two waves that hold the same rows have them in opposite order.)
+  // two waves that hold the same rows have them in opposite order. kSumsOfBothSides:
+  // its block columns likewise.)
   const int first_block = kRowSumsOfFourBlocks ? wave_n : 0;
-  int a_second[C::kKSteps];
-  if constexpr (kRowSumsOfFourBlocks) {
+  const int first_column_block = kSumsOfBothSides ? wave_m : 0;
+  int a_second[C::kKSteps], b_second[C::kKSteps];
 #pragma unroll
-    for (int ks = 0; ks < C::kKSteps; ++ks) {
+  for (int ks = 0; ks < C::kKSteps; ++ks) {
+    if constexpr (kRowSumsOfFourBlocks) {
       a_second[ks] = a_foff[ks] + (1 - first_block) * kB * kBK;
       a_foff[ks] += first_block * kB * kBK;
     }
+    if constexpr (kSumsOfBothSides) {
+      b_second[ks] = b_foff[ks] + (1 - first_column_block) * kB * kBK;
+      b_foff[ks] += first_column_block * kB * kBK;
+    }
   }
   auto a_offset = [&](int ks, int i) { return kRowSumsOfFourBlocks && i == 1 ? a_second[ks] : a_foff[ks] + i * kB * kBK; };
+  auto b_offset = [&](int ks, int j) { return kSumsOfBothSides && j == 1 ? b_second[ks] : b_foff[ks] + j * kB * kBK; };
   struct Frags {
     v4i a[kAB];
     v4i b[kBB];
@@ -664,7 +672,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       f.a[i] = *reinterpret_cast<const v4i*>(stage + a_offset(ks, i));
 #pragma unroll
     for (int j = 0; j < kBB; ++j)
-      f.b[j] = *reinterpret_cast<const v4i*>(stage + b_foff[ks] + j * kB * kBK);
+      f.b[j] = *reinterpret_cast<const v4i*>(stage + b_offset(ks, j));
   };
   // Fragment number r. 32x32 blocks: the A fragments, then the B fragments.
   // 16x16 blocks: the B fragments first, because the matrix instructions of a
@@ -677,7 +685,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     if (is_a)
       f.a[idx] = *reinterpret_cast<const v4i*>(stage + a_offset(ks, idx));
     else
-      f.b[idx] = *reinterpret_cast<const v4i*>(stage + b_foff[ks] + idx * kB * kBK);
+      f.b[idx] = *reinterpret_cast<const v4i*>(stage + b_offset(ks, idx));
   };
 
   typename Traits::Acc acc[kAB][kBB];
@@ -697,6 +705,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   // kRowSumsOfFourBlocks: the lane's half of row l % 32 of the wave's first block
   // row (v_sad_u8 takes every byte of the depth 128 too large).
   uint32_t row_sum = 0u - static_cast<uint32_t>(kBK / 2 * 128) * static_cast<uint32_t>(k_tiles);
+  uint32_t column_sum = row_sum;
 #pragma unroll
   for (int v = 0; v < kAccElems; ++v) {
     sum_a[v] = 0;
@@ -748,6 +757,9 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       if constexpr (kRowSumsOfFourBlocks) {
         const uint32_t to_unsigned = 0x80808080u ^ (kFlip ? args.a_flip : 0u);
         row_sum = __builtin_amdgcn_sad_u8(static_cast<uint32_t>(cur_raw.a[0][n]) ^ to_unsigned, 0u, row_sum);
+        if constexpr (kSumsOfBothSides)
+          column_sum = __builtin_amdgcn_sad_u8(
+              static_cast<uint32_t>(cur_raw.b[0][n]) ^ (0x80808080u ^ (kFlip ? args.b_flip : 0u)), 0u, column_sum);
       }
       if constexpr (kFusedSums && !kRowSumsOfFourBlocks && n == 0) {
         // Once per sub-step. The plane-split operand has zero point 0 by
@@ -1898,11 +1910,20 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     if constexpr (kRowSumsOfFourBlocks) {
       // The two waves that hold the same 64 rows exchange their halves; lane l
       // stages the parameters of row l.
-      static_assert(C::kEpilogueBytes + C::kParamBytes + C::kBM * 4 <= C::kLdsBytes, "");
+      static_assert(C::kEpilogueBytes + C::kParamBytes + (C::kBM + C::kBN) * 4 <= C::kLdsBytes, "");
       int* const sums = reinterpret_cast<int*>(lds + C::kEpilogueBytes + C::kParamBytes) + wave_m * (WM * 32);
       const auto halves = __builtin_amdgcn_permlane32_swap(row_sum, row_sum, false, false);
       if (lane < 32) sums[first_block * 32 + lane] = static_cast<int>(halves[0] + halves[1]);
+      int* const column_sums =
+          reinterpret_cast<int*>(lds + C::kEpilogueBytes + C::kParamBytes) + C::kBM + wave_n * (WN * 32);
+      if constexpr (kSumsOfBothSides) {
+        const auto column_halves = __builtin_amdgcn_permlane32_swap(column_sum, column_sum, false, false);
+        if (lane < 32)
+          column_sums[first_column_block * 32 + lane] = static_cast<int>(column_halves[0] + column_halves[1]);
+      }
       __syncthreads();
+      if constexpr (kSumsOfBothSides)
+        edge.bias[2] = static_cast<int>(static_cast<uint32_t>(edge.bias[2]) - fb * static_cast<uint32_t>(column_sums[lane]));
       edge.bias[0] = static_cast<int>(static_cast<uint32_t>(edge.bias[0]) - fa * static_cast<uint32_t>(sums[lane]));
     } else {
 #pragma unroll
@@ -2420,10 +2441,12 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
   // must be compile-time constants); everything after that is a compact loop,
   // which keeps the kernel's code well inside the instruction cache.
 #pragma unroll
-  for (int half = 0; half < C::kLogicalWN / C::kEpilogueBlockCols; ++half) {
+  for (int half_held = 0; half_held < C::kLogicalWN / C::kEpilogueBlockCols; ++half_held) {
+    static_assert(!kSumsOfBothSides || C::kEpilogueBlockCols == 1, "");
+    const int half = half_held ^ first_column_block;  // (which columns the blocks held are)
 #pragma unroll
     for (int bjj = 0; bjj < C::kEpilogueBlockCols; ++bjj) {
-      const int lb = half * C::kEpilogueBlockCols + bjj;  // logical block column (32 destination columns)
+      const int lb = half_held * C::kEpilogueBlockCols + bjj;  // logical block column (32 destination columns)
       if constexpr (kB == 32) {
 #pragma unroll
         for (int bi = 0; bi < WM; ++bi) {
@@ -2797,16 +2820,18 @@ inline int DepthSplitParts(int tiles, int k_steps, int num_cus, int min_steps_pe
 // deals those of `a` out over its first workgroups where it may (a microsecond
 // and a half) and needs the kernel for those of `b`.
 inline double SumsKernelMicroseconds(double bytes) { return 1.5 + bytes / (1024.0 * 1024.0) * 0.134; }
-// The 128x128 tile can form the row sums of `a` itself, from the fragments that
-// its waves hold (two vector instructions behind every matrix instruction), when
-// only those are pending and the grid leaves every CU at most one workgroup.
+// The 128x128 tile can form the row sums of `a`, or of both operands, itself,
+// from the fragments that its waves hold (two or four vector instructions behind
+// every matrix instruction), in grids that leave every CU at most one workgroup.
 // 2048 x K x 2048 against the same launch without sums, us: K = 256 + 0.2, 512 + 0.2,
 // 1024 + 0.3, 2048 + 0.6; with the rows dealt out over the workgroups (below) + 1.1,
 // 1.2, 1.0 and 1.1. Where both forms may be used, the same call in us, dealt out ->
 // here: 2048 x 4096 x 2048 22.2 -> 22.0, x 6144 31.0 -> 30.9, x 8192 40.1 -> 39.7, but 1024 x
-// 8192 x 4096 39.0 -> 39.8 (x 4096 21.8 -> 21.9): up to 48 steps of the depth.
-constexpr int kRowSumming128Steps = 48;
-inline double RowSumming128Microseconds(int k_steps) { return 0.1 + 0.03 * k_steps; }
+// 8192 x 4096 39.0 -> 39.8 (x 4096 21.8 -> 21.9): up to 48 steps of the depth. Both
+// operands: 2048 x 1024 x 2048 11.7 -> 10.2, x 2048 16.2 -> 15.0, x 4096 25.4 -> 24.5, x 6144
+// 34.7 -> 33.7, x 8192 44.1 -> 44.1: up to 64. Those of `b` alone, by the form for both:
+// x 1024 10.6 -> 10.2, x 2048 15.1 -> 14.9, x 4096 23.7 -> 24.2: up to 20.
+constexpr int kSumming128StepsOfA = 48, kSumming128StepsOfB = 20, kSumming128StepsBoth = 64;
 // The tiles of 32x32 blocks whose waves share every step can have the rows of
 // `a` added up by the workgroups of their own grid, each taking a share of
 // the rows while its first loads are on their way (kLeadSums in the kernel),
@@ -2885,11 +2910,21 @@ inline bool LeadColumnSumsApply(const GemmArgs& args) {
 inline double LeadColumnSumsMicroseconds(const GemmArgs& args, int num_cus, int bm, int bn) {
   return LeadShareMicroseconds(args.N, args.k_bytes, LeadSumsProducers(args, num_cus, bm, bn));
 }
+// Whether the 128x128 tile forms the sums itself, and what it costs it.
+inline double RowSumming128Microseconds(const GemmArgs& args) {
+  const int k_steps = (args.k_bytes + 127) / 128;
+  return (args.sums_wanted & 2) ? 0.1 + 0.06 * k_steps : 0.1 + 0.03 * k_steps;
+}
 inline bool RowSumming128Applies(const GemmArgs& args, int num_cus) {
   const int tiles = ((args.M + 127) / 128) * ((args.N + 127) / 128);
-  return (args.sums_wanted & 3) == 1 && tiles <= num_cus &&
-         ((args.k_bytes + 127) / 128 <= kRowSumming128Steps || !LeadSumsApply(args, num_cus, 128, 128)) &&
-         RowSumming128Microseconds((args.k_bytes + 127) / 128) < SumsKernelMicroseconds(double(args.M) * args.k_bytes);
+  const int k_steps = (args.k_bytes + 127) / 128;
+  const bool a = (args.sums_wanted & 1) != 0, b = (args.sums_wanted & 2) != 0;
+  if ((!a && !b) || tiles > num_cus) return false;
+  const bool dealt_out = (!a || LeadSumsApply(args, num_cus, 128, 128)) && (!b || LeadColumnSumsApply(args));
+  if (dealt_out) return k_steps <= (a && b ? kSumming128StepsBoth : b ? kSumming128StepsOfB : kSumming128StepsOfA);
+  return RowSumming128Microseconds(args) <
+         (a ? SumsKernelMicroseconds(double(args.M) * args.k_bytes) : 0.0) +
+             (b ? SumsKernelMicroseconds(double(args.N) * args.k_bytes) : 0.0);
 }
 inline double PendingSumsMicroseconds(const GemmArgs& args, int num_cus, const TimingModel& model,
                                       const TileTiming& t, double* factor) {
@@ -2903,7 +2938,7 @@ inline double PendingSumsMicroseconds(const GemmArgs& args, int num_cus, const T
     return 0.0;
   }
   if (t.tile == Tile::k128x128 && model.smallest == Tile::k64x64 && RowSumming128Applies(args, num_cus))
-    return RowSumming128Microseconds((args.k_bytes + 127) / 128);
+    return RowSumming128Microseconds(args);
   const double a_kernel = SumsKernelMicroseconds(double(args.M) * args.k_bytes);
   const double b_kernel = SumsKernelMicroseconds(double(args.N) * args.k_bytes);
   double extra = b ? b_kernel : 0.0;

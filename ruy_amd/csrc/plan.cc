@@ -647,6 +647,11 @@ int RunInt8(ruyamd_ctx* ctx, MulCall* call, std::string* err) {
         (sides & 2) ? args.col_sums_offset + args.N : RoundUp(args.M, fused_sums::kTileRows);
     ctx->row_sums_next = set ^ 1;
     ++ctx->row_sums_calls;
+  } else if (args.fuse_sums && (args.sums_wanted & 4)) {
+    // (The 128x128 tile adds up the fragments that it holds instead of shares of the rows.)
+    int tile_rows = 0, tile_cols = 0, parts = 0;
+    GemmTileFor(args, ctx->multiprocessor_count, GemmKind::kInt8, &tile_rows, &tile_cols, &parts);
+    if (tile_rows == 128 && tile_cols == 128) ++ctx->row_sums_calls;
   }
   ctx->last_kernel = RUYAMD_KERNEL_I8_MFMA;
   return RUYAMD_OK;
