@@ -243,14 +243,14 @@ RUYAMD_HOST_DEVICE inline int LeadShareLanesPerRow(int rows_in_share, int k_byte
 }
 
 // kFusedSums (64x64 tile of the int8 kernel; the 128x128 tile for the rows of
-// `a` only): the kernel also forms the
-// depth sums of its rows of `a` and columns of `b` - one more matrix
+// `a`, or for both): the kernel also forms the
+// depth sums of its rows of `a` and columns of `b` - by v_sad_u8 on the
+// fragments its waves hold; where the waves of the 64x64 tile share every step, by one more matrix
 // instruction each per depth sub-step, against a fragment of ones - and
 // subtracts args.fused_a_factor * rowsum + args.fused_b_factor * colsum from
 // every accumulator before the write-back. This is the zero-point correction
 // of ruy/kernel.h:219-232 without a separate pass over the operands, for
-// problems so small that a second kernel launch would cost more than the
-// extra matrix instructions.
+// problems so small that a second kernel launch would cost more.
 //
 // kFlip (int8 kernel): args.a_flip / args.b_flip are applied to every
 // fragment before use, which turns uint8 data used in place into the int8
@@ -944,18 +944,18 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         f.b[1] = low;
       }
     };
-    typename Traits::Acc full[2][2], rows_sum[2], cols_sum[2];
+    typename Traits::Acc full[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         full[i][0][v] = 0;
         full[i][1][v] = 0;
-        rows_sum[i][v] = 0;
-        cols_sum[i][v] = 0;
       }
     }
+    uint32_t rows_sum[2], cols_sum[2];  // kFusedSums: the lane's half of row (column) l % 32 of a block
     auto mma4 = [&](Frags4 f) {
+      const Frags4 raw = f;
       if constexpr (kFlip) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -968,17 +968,27 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) Traits::Mma(f.a[i], f.b[j], full[i][j]);
       if constexpr (kFusedSums) {
-        // The plane-split operand has zero point 0 by definition, so its
-        // column sums are never needed.
+        // (Beside the matrix instructions: v_sad_u8 does not wait for their pipe. The
+        // plane-split operand has zero point 0 by definition, so its column sums are
+        // never needed.)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          Traits::Mma(f.a[i], ones, rows_sum[i]);
-          if constexpr (!Traits::kSplitB) Traits::Mma(ones, f.b[i], cols_sum[i]);
-        }
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            rows_sum[i] = __builtin_amdgcn_sad_u8(
+                static_cast<uint32_t>(raw.a[i][d]) ^ (0x80808080u ^ (kFlip ? args.a_flip : 0u)), 0u, rows_sum[i]);
+            if constexpr (!Traits::kSplitB)
+              cols_sum[i] = __builtin_amdgcn_sad_u8(
+                  static_cast<uint32_t>(raw.b[i][d]) ^ (0x80808080u ^ (kFlip ? args.b_flip : 0u)), 0u, cols_sum[i]);
+          }
       }
     };
     // This wave's steps: depth_way, depth_way + kDepthWays, ... of the workgroup's k_tiles steps.
     const int my_steps = k_tiles > depth_way ? (k_tiles - depth_way + kDepthWays - 1) / kDepthWays : 0;
+    // (v_sad_u8 takes every byte 128 too large; a lane adds up half a row.)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      rows_sum[i] = cols_sum[i] = 0u - static_cast<uint32_t>(kBK / 2 * 128) * static_cast<uint32_t>(my_steps);
     if (my_steps > 0 || Traits::kParts) issue_step(depth_way, 0);
     if (my_steps > 1) issue_step(depth_way + kDepthWays, 1);
     load_edge_params();
@@ -1162,17 +1172,35 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     if constexpr (kFusedSums) {
       const uint32_t fa = static_cast<uint32_t>(args.fused_a_factor);
       const uint32_t fb = static_cast<uint32_t>(args.fused_b_factor);
+      // (An accumulator's lane has one column and 16 rows: the sums of the rows go
+      // through the wave's own ring, which it is done with.)
+      int* const handed = reinterpret_cast<int*>(ring);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const auto row_halves = __builtin_amdgcn_permlane32_swap(rows_sum[i], rows_sum[i], false, false);
+        const auto col_halves = __builtin_amdgcn_permlane32_swap(cols_sum[i], cols_sum[i], false, false);
+        rows_sum[i] = row_halves[0] + row_halves[1];
+        cols_sum[i] = col_halves[0] + col_halves[1];
+        if (lane < 32) handed[i * 32 + lane] = static_cast<int>(fa * rows_sum[i]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       // Plane-split operand: the correction belongs to the low plane's block
       // (the odd one of a pair; the write-back combines 256 * high + low).
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = Traits::kSplitB ? 1 : 0; j < 2; ++j)
+        for (int q = 0; q < 4; ++q) {
+          const v4i of_rows = *reinterpret_cast<const v4i*>(handed + i * 32 + 8 * q + 4 * (lane / 32));
 #pragma unroll
-          for (int v = 0; v < 16; ++v)
-            full[i][j][v] = static_cast<int>(static_cast<uint32_t>(full[i][j][v]) -
-                                             fa * static_cast<uint32_t>(rows_sum[i][v]) -
-                                             fb * static_cast<uint32_t>(cols_sum[j][v]));
+          for (int j = Traits::kSplitB ? 1 : 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              full[i][j][4 * q + v] =
+                  static_cast<int>(static_cast<uint32_t>(full[i][j][4 * q + v]) - static_cast<uint32_t>(of_rows[v]) -
+                                   (Traits::kSplitB ? 0u : fb * cols_sum[j]));
+        }
     }
     // Add the partial pieces: [wave][block][quarter][lane] in LDS.
     __syncthreads();  // every wave is done with its ring
@@ -2867,15 +2895,16 @@ inline double LeadShareMicroseconds(int rows, int k_bytes, int producers) {
 inline double LeadSumsMicroseconds(const GemmArgs& args, int num_cus, int bm, int bn) {
   return LeadShareMicroseconds(args.M, args.k_bytes, LeadSumsProducers(args, num_cus, bm, bn));
 }
-// The smallest int8 tile, which otherwise forms both operands' sums with two
-// more matrix instructions per four (measured on 256 tiles: + 1.1 us at a
-// depth of 8 steps, + 1.5 us at 32, + 3.2 us at 64, + 7.0 us at 128 - 15 to
-// 27 % of the launch): shared out where that is cheaper and the depth leaves
-// every wave a step (the depth-per-wave schedule). Measured on 256 tiles with
-// the rows of `a` shared out, against the matrix instructions: 7.8 us for 8.5
-// at 16 steps, 10.4 for 11.3 at 32, 16.5 for 18.3 at 64 - and 42.7 for 32.4
-// at 128 steps, where a workgroup's share took four batches of loads: two
-// batches a side at most (which whole waves to a row make of those four).
+// The smallest int8 tile, which otherwise forms both operands' sums from the
+// fragments that its waves hold (v_sad_u8 beside the matrix instructions): shared
+// out where that is cheaper and the depth leaves every wave a step (the
+// depth-per-wave schedule). 256 tiles, us from the fragments and shared out: a's
+// sums, 8 steps of the depth 7.1 and 7.1, 12 7.65 and 7.9, 16 8.7 and 8.5, 24 10.7 and
+// 10.0, 32 12.2 and 11.4, 64 18.8 and 17.5; both sides' 16 8.7 and 9.2, 24 10.65 and 10.75, 32
+// 12.2 and 12.3, 64 18.7 and 18.4. (With two more matrix instructions per four instead
+// of v_sad_u8: 16 steps 9.2, 4096 x 8192 x 256 20.3, 18.5 so.) At 128 steps 42.7 shared out for
+// 32.4 where a workgroup's share took four batches of loads: two batches a side at
+// most (which whole waves to a row make of those four).
 inline int SmallestTileParts(const GemmArgs& args, int num_cus) {
   const int tiles = ((args.M + 63) / 64) * ((args.N + 63) / 64);
   return DepthSplitParts(tiles, std::max(1, (args.k_bytes + 127) / 128), num_cus, 16);
@@ -2899,7 +2928,7 @@ inline bool SmallestTileSharesSumsOut(const GemmArgs& args, int num_cus) {
   const int producers = std::min((tiles + 7) / 8 * 8, num_cus);
   if ((args.sums_wanted & 1) && LeadShareBatches(args.M, args.k_bytes, producers) > 2) return false;
   if ((args.sums_wanted & 2) && LeadShareBatches(args.N, args.k_bytes, producers) > 2) return false;
-  return SmallestTileSharedSumsMicroseconds(args, num_cus) < 0.6 + 0.05 * steps_per_part;
+  return SmallestTileSharedSumsMicroseconds(args, num_cus) < 0.3 + 0.045 * steps_per_part;
 }
 // The same for the rows of `b` (the destination's columns), whose words stand
 // behind those of a's rows.

@@ -63,6 +63,9 @@ struct F32Small {
 // (one 64x64 tile too many for two rounds) x 1024 60.5 -> 47.7; 256 tiles with one
 // side transposed x 1024 19.7 -> 9.2, both 21.8 -> 9.4; 1536 x 1024 43.4 -> 39.8, both
 // 47.6 -> 39.0.
+// (Measured against the larger tiles on fp32 instructions. Since two of those run on
+// bf16 parts, their model gives them what they are faster at: 860 x 2832 x 1686 80.4 us
+// here, 71.1 there; 1024^3 23.7 and 18.3.)
 // More than six tiles to a CU: of more than 300 bytes of depth every further one costs
 // 0.5 us, with an operand transposed 0.75, and in place the models have to differ by
 // more. Of 460 products around the line, 16 to 4096 tiles, these tiles took 392 with
