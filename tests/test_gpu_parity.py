@@ -1331,7 +1331,7 @@ def test_row_sums_formed_by_the_workgroups_of_a_mid_tile_grid(mode):
     picks up the sums of its rows in front of its write-back. Modes: that; the
     sums never looked for, so that every wave forms those of its rows itself
     (what it does when the others' do not arrive); the separate kernel (and,
-    for a short depth on the 128x128 tile, the extra matrix instruction).
+    for a short depth on the 128x128 tile, the sums from its fragments).
     int8 and uint8 data, both destination orders, ragged edges, calls of
     different heights in a row on one context (each launch meets the words the
     launch before cleared for it): every element against the stock library."""
