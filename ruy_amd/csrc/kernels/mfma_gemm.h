@@ -1222,6 +1222,9 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         }
     }
     // Add the partial pieces: [wave][block][quarter][lane] in LDS.
+    // (In parts, the loads of a step past the end are still on their way to the ring,
+    // and the barrier does not wait for those.)
+    if constexpr (Traits::kParts) WaitVmcnt<0>();
     __syncthreads();  // every wave is done with its ring
     v4i* parts = reinterpret_cast<v4i*>(lds);
 #pragma unroll

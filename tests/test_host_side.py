@@ -181,6 +181,33 @@ def test_every_wave_of_a_download_awaits_its_stores(tmp_path):
     assert len(flag) == 1 and flag[0] > barrier, flag
 
 
+def test_no_load_is_on_its_way_to_lds_when_partial_sums_are_put_there(tmp_path):
+    """The 64x64 tile of fp32 gives every wave a ring of its own, whose memory the
+    waves' partial sums go to behind a workgroup barrier. The barrier does not wait for
+    loads that write to LDS, and on bf16 parts the last trip of the loop asks for a step
+    past the end (zeros): followed along the branches of the assembly, no path from
+    such a load to a barrier is without a wait for all of them."""
+    body = kernel_assembly(tmp_path, "gemm_f32.hip")("F32TraitsELi1ELi1ELi128ELi4ELb0ELb0ELb1E")
+    labels = {l[:-1]: i for i, l in enumerate(body) if l.endswith(":")}
+    loads = [i for i, l in enumerate(body) if l.startswith("buffer_load_dwordx4") and l.endswith(" lds")]
+    assert loads and any(l.startswith("v_mfma_f32_32x32x16_bf16") for l in body) and "s_barrier" in body
+    on_their_way, seen = [i + 1 for i in loads], set()
+    while on_their_way:
+        i = on_their_way.pop()
+        if i in seen or i >= len(body):
+            continue
+        seen.add(i)
+        l = body[i]
+        assert l != "s_barrier", body[max(0, i - 12):i + 1]
+        if l.startswith("s_endpgm") or l.startswith("s_waitcnt") and "vmcnt(0)" in l:
+            continue
+        branch = re.match(r"s_c?branch\w*\s+(\S+)", l)
+        if branch:
+            on_their_way.append(labels[branch.group(1)])
+        if not l.startswith("s_branch"):
+            on_their_way.append(i + 1)
+
+
 @pytest.fixture(scope="module")
 def runtime_model(tmp_path_factory):
     """tests/cpp/runtime_model_test.cc: the library on a model of the HIP runtime."""
