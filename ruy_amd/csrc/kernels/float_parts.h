@@ -94,12 +94,21 @@ constexpr int kPartOfB[kProducts] = {0, 2, 1, 0, 1, 0};
 // (Given the builtin, the compiler moves the accumulators between the two
 // register files on every trip round a loop. What the assembler text keeps from
 // it: Drain() in front of the first ordinary read of the accumulators, which
-// it names so that no copy of one can be made ahead of it.)
-template <int kProduct>
+// it names so that no copy of one can be made ahead of it. Nor does the compiler know
+// of the two wait states that a matrix instruction needs behind a vector instruction
+// that writes what it reads, and it may set or copy an accumulator right in front of
+// one: kBehindWrites, everywhere but in loops, which hold no such writes, brings them.
+// A test looks for either in the assembly of the whole kernel.)
+template <int kProduct, bool kBehindWrites = false>
 __device__ __forceinline__ void Mma(const Parts& a, const Parts& b, v16f& acc) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-               : "+a"(acc)
-               : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
+  if constexpr (kBehindWrites)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+                 : "+a"(acc)
+                 : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
+  else
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+                 : "+a"(acc)
+                 : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
 }
 template <int kA, int kB>
 __device__ __forceinline__ void Drain(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {

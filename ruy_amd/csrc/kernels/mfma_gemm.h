@@ -1054,7 +1054,8 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
           constexpr int n = decltype(n_constant)::value;
           constexpr int i = n / 12, j = n / 6 % 2, e = n % 6;
           __builtin_amdgcn_sched_barrier(0);
-          float_parts::Mma<e>(parts[from][i], parts[from][2 + j], e < 5 ? small[i][j] : full[i][j]);
+          // (What is read again belongs to the loop.)
+          float_parts::Mma<e, !decltype(read)::value>(parts[from][i], parts[from][2 + j], e < 5 ? small[i][j] : full[i][j]);
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (decltype(refill)::value && n < kLoads)
             LoadToLds16(ring_base + refill_slot * kSlotBytes + n * 1024, goff[n], uint32_t(kbase), n < 8 ? a_rsrc : b_rsrc);

@@ -208,6 +208,80 @@ def test_no_load_is_on_its_way_to_lds_when_partial_sums_are_put_there(tmp_path):
             on_their_way.append(i + 1)
 
 
+def test_matrix_instructions_written_as_text_keep_their_distances(tmp_path):
+    """v_mfma_f32_32x32x16_bf16 and v_mfma_i32_16x16x64_i8 stand in the larger kernels as
+    assembler text, which the compiler keeps no distances to: two wait states behind a
+    vector instruction that writes one of its operands, and 12 or 8 (eight and four
+    passes) in front of anything but a matrix instruction that touches its result. The
+    compiler is free to copy or clear an accumulator anywhere, so both are looked for
+    along the branches of these kernels as they were built."""
+    from ruy_amd import build
+    objdump = os.path.join(os.path.dirname(os.path.dirname(build.HIPCC)), "llvm", "bin", "llvm-objdump")
+    shutil.copy(LIB, tmp_path / "library.so")
+    subprocess.check_call([objdump, "--offloading", "library.so"], cwd=tmp_path, stdout=subprocess.DEVNULL)
+    wait_states = {"v_mfma_f32_32x32x16_bf16": 12, "v_mfma_i32_16x16x64_i8": 8}
+
+    def registers(operands):
+        found = set()
+        for kind, first, last, one in re.findall(r"\b([av])(?:\[(\d+):(\d+)\]|(\d+)\b)", operands):
+            found |= {kind + str(r) for r in range(int(first or one), int(last or one) + 1)}
+        return found
+
+    checked, faults = [], []
+    for code in sorted(tmp_path.glob("library.so.*gfx950")):
+        listing = subprocess.run([objdump, "-d", code], capture_output=True, text=True, check=True).stdout
+        for kernel in re.split(r"\n(?=[0-9a-f]+ <\S+>:\n)", listing)[1:]:
+            if not ("MfmaGemm" in kernel[:200] and any(name in kernel for name in wait_states)):
+                continue
+            base, name = re.match(r"([0-9a-f]+) <(\S+)>:", kernel).groups()
+            checked.append(name)
+            text, at, branches = [], {}, {}
+            for line in kernel.split("\n")[1:]:
+                instruction, _, rest = line.partition("//")
+                if not rest:
+                    continue
+                at[int(rest.split(":")[0], 16)] = len(text)
+                if re.match(r"\s*s_c?branch", instruction):
+                    branches[len(text)] = int(base, 16) + int(re.search(r"<\S+?(?:\+0x([0-9a-f]+))?>", rest).group(1) or "0", 16)
+                text.append(instruction.strip())
+            before = [[i - 1] if i and not text[i - 1].startswith(("s_branch", "s_endpgm")) else [] for i in range(len(text))]
+            for i, target in branches.items():
+                before[at[target]].append(i)
+            mnemonic = [t.split(" ")[0] for t in text]
+            operands = [t.partition(" ")[2].split(", ") for t in text]
+            touched = [registers(t.partition(" ")[2]) for t in text]
+            # (Comparisons and the like name a scalar register first; stores and loads to LDS write none.)
+            written = [registers(o[0]) | (registers(o[1]) if "swap" in m and len(o) > 1 else set())
+                       if m.startswith(("v_", "ds_read", "global_load", "buffer_load")) else set()
+                       for m, o in zip(mnemonic, operands)]
+
+            def close_in_front(i, states, hit):
+                """Instructions less than `states` wait states in front of the i-th that `hit` says yes to."""
+                ways, nearest = [(j, 0) for j in before[i]], {}
+                while ways:
+                    j, waited = ways.pop()
+                    if waited >= states or nearest.get(j, states) <= waited:
+                        continue
+                    nearest[j] = waited
+                    if hit(j, waited):
+                        yield j
+                        continue
+                    waited += int(operands[j][0], 0) + 1 if mnemonic[j] == "s_nop" else 1
+                    ways += [(k, waited) for k in before[j]]
+
+            for i in range(len(text)):
+                if mnemonic[i] in wait_states:
+                    read = set().union(*(registers(o) for o in operands[i][1:]))
+                    faults += [(name, text[j], text[i]) for j in close_in_front(
+                        i, 2, lambda j, _: mnemonic[j].startswith("v_") and not mnemonic[j].startswith("v_mfma") and
+                        written[j] & read)]
+                elif touched[i] and not mnemonic[i].startswith("v_mfma"):
+                    faults += [(name, text[j], text[i]) for j in close_in_front(
+                        i, 12, lambda j, waited: waited < wait_states.get(mnemonic[j], 0) and written[j] & touched[i])]
+    assert len(checked) >= 6 and any("F32Traits" in name for name in checked), checked
+    assert not faults, faults[:8]
+
+
 @pytest.fixture(scope="module")
 def runtime_model(tmp_path_factory):
     """tests/cpp/runtime_model_test.cc: the library on a model of the HIP runtime."""
