@@ -1,9 +1,13 @@
-// fp32 products on the bf16 matrix instructions, without losing a bit of an
-// operand: a float is the sum of three bf16 values (24 bits of mantissa are
-// three times 8), and of the nine products of two such sums the six largest are
-// formed, high * high down to the 2^-16 terms. What is left out is at most
-// 2^-23 of a product, a fifth of 2^-24 of it in the mean, and has no sign of its
-// own. Every bf16 product is exact, sums are fp32 throughout, and an instruction
+// fp32 products on the bf16 matrix instructions by the published method of
+// splitting a float into a sum of bf16 values (G. Henry, P. T. P. Tang, A. Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019: three parts, six products). A float is the sum of three
+// bf16 values, each the rest of the ones before it rounded to nearest (24 bits of
+// mantissa are three times 8), and of the nine products of two such sums the six
+// largest are formed, high * high down to the 2^-16 terms. What is left out is at most
+// 2^-24 of a product, a fifth of that in the mean, and has no sign of its
+// own: a product counts with the bits of both factors to about its own 24th, not
+// with all 48. Every bf16 product is exact, sums are fp32 throughout, and an instruction
 // adds 16 depth positions with one rounding where the fp32 instruction adds two;
 // the five smaller products have accumulators of their own. Measured against 64
 // bits (values in [-1, 1], one accumulator chain): depth 256 7.8e-8 (fp32
@@ -16,11 +20,21 @@
 // products without them, 225 with, fp32 instructions 150), so elements are
 // split as few times as possible.
 //
-// Not every float is such a sum: infinities and NaN are not, values that a
-// bf16 part rounds to infinity are not, and parts of values under 2^-110 are
-// lost. The first two leave an accumulator that is not finite, for the third
-// the bits of a vector's elements are collected (Magnitudes); in either case
-// the wave does its work again with fp32 instructions.
+// Not every float is such a sum: infinities and NaN are not, nor what a bf16 part
+// rounds to infinity, nor most of what lies under 2^-110, whose last bits are below
+// the smallest bf16 value (2^-133). The first two leave an accumulator that is not
+// finite. The last leaves a remainder that the third part does not hold as a whole:
+// one with bits in the lower half of its word, which are collected (Lost) and decide
+// exactly (6 million bit patterns, subnormal ones among them: no disagreement). In
+// either case the work is done again with fp32 instructions. How large the value lost
+// is beside its own vector's does not matter: what it meets in the other operand may
+// be large, and what its neighbours meet zero.
+//
+// What that costs, us, ordinary values / such a value in the first steps of every wave,
+// with which the loop ends / in the last / an infinity, which only the sums show (and
+// fp32 instructions throughout, as before there were parts): 1024^3 19.7 / 26.8 / 34.0 /
+// 33.9 (22.3), 1537 x 1111 x 2051 54.8 / 86.4 / 118.7 / 118.9 (72.5), 2048 x 3072 x 2048
+// 139.5 / 204 / 324 / 325 (186), 512 x 4096 x 512 22.1 / 29.5 / 36.0 / 36.1 (23.0).
 #ifndef RUY_AMD_CSRC_KERNELS_FLOAT_PARTS_H_
 #define RUY_AMD_CSRC_KERNELS_FLOAT_PARTS_H_
 
@@ -61,14 +75,13 @@ struct Splitter {
   // (dot2 instructions, which would subtract a half without extracting it,
   // wait for the matrix pipe: 22 cycles each behind a matrix instruction.)
   template <int kOp>
-  __device__ __forceinline__ void Op(const v4i& x, int which, Parts& to, int& magnitudes) {
+  __device__ __forceinline__ void Op(const v4i& x, int which, Parts& to, int& lost) {
     if constexpr (kOp < 20) {
       constexpr int part = kOp / 10, op = kOp % 10;
       if constexpr (op < 2) {
         if constexpr (part == 0) {
           rest[2 * op] = __int_as_float(x[2 * op]);
           rest[2 * op + 1] = __int_as_float(x[2 * op + 1]);
-          magnitudes |= x[2 * op] | x[2 * op + 1];
         }
         pair[op] = RoundPair(rest[2 * op], rest[2 * op + 1]);
         to.part[part][2 * which + op] = pair[op];
@@ -80,7 +93,10 @@ struct Splitter {
           rest[e] -= half[e];
       }
     } else {
-      to.part[2][2 * which + kOp - 20] = RoundPair(rest[2 * (kOp - 20)], rest[2 * (kOp - 20) + 1]);
+      constexpr int e = 2 * (kOp - 20);
+      to.part[2][2 * which + kOp - 20] = RoundPair(rest[e], rest[e + 1]);
+      // (As text, in place: the compiler collects the remainders in registers otherwise.)
+      asm volatile("v_or3_b32 %0, %1, %2, %0" : "+v"(lost) : "v"(rest[e]), "v"(rest[e + 1]));
     }
   }
   float half[4];
@@ -110,6 +126,14 @@ __device__ __forceinline__ void Mma(const Parts& a, const Parts& b, v16f& acc) {
                  : "+a"(acc)
                  : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
 }
+// Settle() behind the clearing of accumulators: from there on they are registers like
+// any other to the compiler, which otherwise clears others for the way past a loop and
+// copies all of them behind it (1024^3 0.4 us).
+template <int kA, int kB>
+__device__ __forceinline__ void Settle(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {
+#pragma unroll
+  for (int b = 0; b < kA * kB; ++b) asm volatile("" : "+a"(x[b / kB][b % kB]), "+a"(y[b / kB][b % kB]));
+}
 template <int kA, int kB>
 __device__ __forceinline__ void Drain(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {
   asm volatile("s_nop 15\n\ts_nop 7" : "+a"(x[0][0]), "+a"(y[0][0]));
@@ -117,12 +141,9 @@ __device__ __forceinline__ void Drain(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {
   for (int b = 1; b < kA * kB; ++b) asm volatile("" : "+a"(x[b / kB][b % kB]), "+a"(y[b / kB][b % kB]));
 }
 
-// The OR of elements' bits: whether all of them are under 2^-95 and some are not
-// zero. (Then what their parts lack, up to 2^-134 each, could be seen beside the
-// largest of them; otherwise it is under 2^-38 of that one.)
-__device__ __forceinline__ bool AllTiny(int magnitudes) {
-  return (magnitudes & 0x70000000) == 0 && (magnitudes & 0x7fffffff) != 0;
-}
+// The OR of elements' last remainders: whether one of the elements is not the sum of
+// its parts.
+__device__ __forceinline__ bool Lost(int lost) { return (lost & 0xffff) != 0; }
 
 }  // namespace float_parts
 }  // namespace ruyamd

@@ -3,8 +3,8 @@
 // The 64x64 and 128x128 tiles multiply floats as sums of three bf16 parts
 // (float_parts.h), the others, and a tile whose values are no such sums, with
 // v_mfma_f32_32x32x2_f32: a 16-byte fragment holds four consecutive depth values
-// of one row, which feed four of these. Either way every product counts with the
-// 24 bits of both factors and sums are fp32. The write-back is the float one of
+// of one row, which feed four of these. Sums are fp32 either way; of a product of
+// parts at most 2^-24 is left out. The write-back is the float one of
 // ruy/reference_mul.h:42-48: bias, then min with clamp_max, then max with
 // clamp_min. The summation order differs from the reference's ascending-k
 // loop, which is why fp32 parity is a tolerance, not bit equality.

@@ -223,7 +223,9 @@ struct Cfg {
   // (Four waves side by side: the fp32 tile whose parts lie in LDS, two buffers of
   // three parts of 256 rows of 64 bytes, in the ring's memory and past it.)
   static constexpr int kPartsBytes = WAVES_N == 4 ? 2 * 3 * 256 * 64 : 0;
-  static constexpr int kRingBytes = kStages * kStageBytes > kPartsBytes ? kStages * kStageBytes : kPartsBytes;
+  static constexpr int kToldBytes = WAVES_N == 4 ? 16 : 0;  // (and two words that its waves talk through)
+  static constexpr int kRingBytes =
+      kStages * kStageBytes > kPartsBytes + kToldBytes ? kStages * kStageBytes : kPartsBytes + kToldBytes;
   static constexpr int kLdsBytes = BLOCK == 16 ? kStages * kStageBytes + kParamBytes
                                                : (kRingBytes > kEpilogueBytes + kParamBytes
                                                       ? kRingBytes
@@ -1014,7 +1016,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     // work a step takes 1.5 us, as the power limit has it (1.18 on 144 CUs; not
     // waiting for the loads changes nothing; fp32 instructions 1.9). 1024^3 22.3 ->
     // 18.0-19.1 us, 1024 x 4096 x 1024 67.5 -> 54.2.
-    // in_parts: the sums are what fp32 instructions would give.
+    // in_parts: every operand value was the sum of its parts, and the sums are finite.
     bool in_parts = false;
     if constexpr (Traits::kParts) {
       using float_parts::Parts;
@@ -1025,7 +1027,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) small[i / 2][i % 2][v] = 0;
-      int magnitudes[4] = {0, 0, 0, 0};
+      int lost = 0;
       v4i raw[kGranules];
       Parts parts[2][4];
       int off[C::kKSteps];
@@ -1065,7 +1067,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
             StaticFor<(n + 1) * kOps / kPhaseMmas - first>([&](auto o) {
               constexpr int op = first + decltype(o)::value;
               constexpr int g = op / float_parts::kSplitOps;
-              splitter.template Op<op % float_parts::kSplitOps>(raw[g], g % 2, parts[1 - from][g / 2], magnitudes[g / 2]);
+              splitter.template Op<op % float_parts::kSplitOps>(raw[g], g % 2, parts[1 - from][g / 2], lost);
               // (The first rounding's remainder has replaced the floats by then.)
               if constexpr (decltype(read)::value && op % float_parts::kSplitOps == 10)
                 read_granule(std::integral_constant<int, g>(), from_constant, read_slot);
@@ -1078,6 +1080,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       using Second = std::integral_constant<int, 1>;
       constexpr std::true_type kYes;
       constexpr std::false_type kNo;
+      float_parts::Settle(full, small);
       // (A wave without a step has loaded zeros.)
       const int steps = max(my_steps, 1);
       const bool last_is_partial = phys(depth_way + kDepthWays * (steps - 1)) * kBK + kBK > K;
@@ -1090,13 +1093,15 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       StaticFor<kGranules>([&](auto granule) {
         constexpr int g = decltype(granule)::value;
         StaticFor<float_parts::kSplitOps>([&](auto op) {
-          splitter.template Op<decltype(op)::value>(raw[g], g % 2, parts[0][g / 2], magnitudes[g / 2]);
+          splitter.template Op<decltype(op)::value>(raw[g], g % 2, parts[0][g / 2], lost);
         });
         read_granule(granule, Second(), 0);
       });
       // Nothing in the loop stands behind a condition but these: a branch around
-      // matrix instructions has the compiler move the accumulators.
-      for (int i = 0; i + 1 < steps; ++i) {
+      // matrix instructions has the compiler move the accumulators. (`last`, in front
+      // of which the loop ends, is 0 once the sums are known to be no good.)
+      int last = steps - 1;
+      for (int i = 0; i < last; ++i) {
         const int refill = i + 2;  // the step that slot i & 1 is filled with
         int kbase = __builtin_amdgcn_readfirstlane(phys_inside(depth_way + kDepthWays * refill) * kBK);
         if (refill >= steps) {
@@ -1116,6 +1121,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         phase(First(), kYes, kYes, kYes, (i + 1) & 1, i & 1, kbase);
         phase(Second(), kYes, kYes, kNo, (i + 1) & 1, 0, 0);
+        last = __builtin_amdgcn_readfirstlane(__any(float_parts::Lost(lost)) ? 0 : last);
       }
       phase(First(), kYes, kNo, kNo, 0, 0, 0);
       phase(Second(), kNo, kNo, kNo, 0, 0, 0);
@@ -1128,16 +1134,13 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
           full[b / 2][b % 2][v] += small[b / 2][b % 2][v];
           not_finite = __builtin_fmaf(full[b / 2][b % 2][v], 0.f, not_finite);
         }
-      bool tiny = false;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) tiny = tiny || float_parts::AllTiny(magnitudes[b]);
-      in_parts = !__any(not_finite != 0.f || tiny);
+      in_parts = !__any(not_finite != 0.f || float_parts::Lost(lost));
       if (!in_parts) {
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
           for (int v = 0; v < 16; ++v) full[b / 2][b % 2][v] = 0;
-        WaitVmcnt<0>();  // (what the last steps asked for beyond the end)
+        WaitVmcnt<0>();  // (what the last trip of the loop asked for)
         set_offsets();
         if (my_steps > 0) issue_step(depth_way, 0);
         if (my_steps > 1) issue_step(depth_way + kDepthWays, 1);
@@ -1644,14 +1647,14 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       for (int b = 0; b < kAB * kBB; ++b)
 #pragma unroll
         for (int v = 0; v < 16; ++v) small[b / kBB][b % kBB][v] = 0;
-      int magnitudes[kHeld] = {};
+      int lost = 0;
       constexpr int kGranuleOps = float_parts::kSplitOps + 4;  // ... its three parts written, and the load behind it
       float_parts::Splitter splitter;
       Parts split_parts;
       auto granule_op = [&](auto op_constant, auto n_constant, int buffer, int load_step) {
         constexpr int op = decltype(op_constant)::value, n = decltype(n_constant)::value;
         if constexpr (op < float_parts::kSplitOps)
-          splitter.template Op<op>(raw[n], 0, split_parts, magnitudes[n]);
+          splitter.template Op<op>(raw[n], 0, split_parts, lost);
         else if constexpr (op < float_parts::kSplitOps + 3)
           write_part(buffer, n, op - float_parts::kSplitOps, split_parts.part[op - float_parts::kSplitOps][0],
                      split_parts.part[op - float_parts::kSplitOps][1]);
@@ -1700,15 +1703,26 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       split_all(std::integral_constant<int, kHeld / 2>(), 0, 1);
       place(1, 0, kHeld / 2);
       split_all(std::integral_constant<int, 0>(), 1, 2);
+      volatile int* const told = reinterpret_cast<int*>(lds + C::kPartsBytes);
+      if (tid < 2) told[tid] = 0;
       barrier();
       StaticFor<kReads>([&](auto which) { read_part(which, 0, First(), parts[0]); });
-      for (int kt = 0; kt < k_tiles; ++kt) {
+      // (In every eighth step a thread that knows that the sums are no good says so in
+      // front of the barrier, in one of two words in turn, and behind it every wave reads
+      // the same there. As a step of its own: asked in each, it costs 2 % of the time.)
+      auto step = [&](int kt, auto asks) {
         const int buffer = kt & 1;
         place(kt + 1, kHeld / 2, kHeld);
         phase(First(), buffer, 1 - buffer, kt + 2);
+        if (decltype(asks)::value && float_parts::Lost(lost)) told[kt / 8 % 2] = 1;
         barrier();
         place(kt + 2, 0, kHeld / 2);
         phase(Second(), 1 - buffer, buffer, kt + 3);
+        return decltype(asks)::value ? __builtin_amdgcn_readfirstlane(told[kt / 8 % 2]) : 0;
+      };
+      for (int kt = 0;; ++kt) {
+        for (const int end = min(kt + 7, k_tiles); kt < end; ++kt) step(kt, std::false_type());
+        if (kt >= k_tiles || step(kt, std::true_type())) break;
       }
       float_parts::Drain(acc, small);
       float not_finite = 0;
@@ -1719,10 +1733,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
           acc[b / kBB][b % kBB][v] += small[b / kBB][b % kBB][v];
           not_finite = __builtin_fmaf(acc[b / kBB][b % kBB][v], 0.f, not_finite);
         }
-      bool tiny = false;
-#pragma unroll
-      for (int n = 0; n < kHeld; ++n) tiny = tiny || float_parts::AllTiny(magnitudes[n]);
-      in_parts = !__syncthreads_or(not_finite != 0.f || tiny);
+      in_parts = !__syncthreads_or(not_finite != 0.f || float_parts::Lost(lost));
       if (!in_parts) {
         clear_accumulators();
         __syncthreads();

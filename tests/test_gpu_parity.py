@@ -350,7 +350,9 @@ def _rows_with_nan_between(rng, rows, depth, cols, orders):
 
 
 @pytest.mark.parametrize("tile", [(64, 64), (128, 128)])
-@pytest.mark.parametrize("values", ["ordinary", "mixed", "tiny", "infinite", "overflowing", "zeros"])
+@pytest.mark.parametrize("values", ["ordinary", "mixed", "mixed to 110", "mixed to 118", "mixed to 120", "mixed to 124",
+                                    "ones met by zeros", "one to a row", "first", "last", "tiny", "infinite",
+                                    "overflowing", "zeros"])
 def test_fp32_values_that_are_not_sums_of_bf16_parts(device_ctx, tile, values):
     """The tiles that split a float into three bf16 parts, on values that the split
     or the bf16 range loses: what comes out is what fp32 instructions give. Held
@@ -370,10 +372,27 @@ def test_fp32_values_that_are_not_sums_of_bf16_parts(device_ctx, tile, values):
                 p.bias[:] = 0
             a = p.lhs.storage[:rows * depth].reshape(rows, depth)
             b = p.rhs.storage[:cols * depth].reshape(cols, depth)
-            if values == "mixed":  # every product of order one, its factors over 2^+-100
-                powers = np.exp2(rng.integers(-100, 101, depth)).astype(np.float32)
+            if values.startswith("mixed"):  # every product of order one, its factors over 2^+-100 (or more)
+                most = int(values.split()[-1]) if " " in values else 100
+                powers = np.exp2(rng.integers(-most, most + 1, depth)).astype(np.float32)
                 a *= powers
                 b /= powers
+            elif values == "ones met by zeros":  # ... and what the parts lose by large values
+                a *= np.float32(2.0 ** -120)
+                a[:, ::4] = 1
+                b *= np.float32(2.0 ** 110)
+                b[:, ::4] = 0
+            elif values == "one to a row":
+                a *= np.float32(2.0 ** -120)
+                a[:, 0] = 1
+                b *= np.float32(2.0 ** 120)
+                b[:, 0] = 0
+            elif values in ("first", "last"):  # one value decides each result, and the parts lose it
+                k = 0 if values == "first" else depth - 1
+                others = np.arange(depth) != k
+                b[:, others] = 0
+                b[:, k] *= np.float32(2.0 ** 110)
+                a[:, k] *= np.float32(2.0 ** -122)
             elif values == "tiny":  # rows whose parts would be subnormal, and subnormal rows
                 a *= np.float32(2.0 ** -118)
                 a[::7] *= np.float32(2.0 ** -14)
