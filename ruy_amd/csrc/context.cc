@@ -1,7 +1,5 @@
 #include "context.h"
 
-#include <algorithm>
-
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -74,13 +72,24 @@ std::size_t Workspace::Piece() const { return blocks_[0].size / turns_ & ~std::s
 void Workspace::Reset() {
   exhausted_ = false;
   const bool may_replace = !pinned_ && growth_allowed_ && !fixed_;
-  // Calls that go on needing scratch get room for several of them.
-  std::size_t wanted = 0;
+  // Calls that go on needing scratch get room for several of them: a block beside
+  // those there are, which stay if it cannot be had.
   if (may_replace && taken_ > 0 && taken_ <= kTurnsUpTo && (calls_ >= kTurnsFrom || ++calls_ >= kTurnsFrom)) {
-    wanted = TurnsFor(taken_) * (taken_ + 256);
-    if (capacity() >= wanted) wanted = 0;
+    const std::size_t wanted = TurnsFor(taken_) * (taken_ + 256);
+    if (capacity() < wanted && wanted < refused_) {
+      void* p = nullptr;
+      if (hipMalloc(&p, wanted) == hipSuccess) {
+        for (auto& b : blocks_) (void)hipFree(b.base);
+        blocks_.assign(1, Block{static_cast<char*>(p), wanted, 0});
+        turn_ = 0;
+        taken_ = wrapped_used_ = 0;
+        return;
+      }
+      (void)hipGetLastError();
+      refused_ = wanted;
+    }
   }
-  if ((blocks_.size() > 1 && may_replace) || wanted) {
+  if (blocks_.size() > 1 && may_replace) {
     // Coalesce: one block as large as everything the last call needed.
     std::size_t total = 0;
     for (auto& b : blocks_) {
@@ -88,12 +97,10 @@ void Workspace::Reset() {
       (void)hipFree(b.base);
     }
     blocks_.clear();
-    for (std::size_t size : {std::max(total, wanted), total}) {
-      void* p = nullptr;
-      if (hipMalloc(&p, size) == hipSuccess) {
-        blocks_.push_back(Block{static_cast<char*>(p), size, 0});
-        break;
-      }
+    void* p = nullptr;
+    if (hipMalloc(&p, total) == hipSuccess) {
+      blocks_.push_back(Block{static_cast<char*>(p), total, 0});
+    } else {
       (void)hipGetLastError();
     }
     turn_ = 0;

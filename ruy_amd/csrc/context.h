@@ -62,7 +62,8 @@ class Workspace {
   // 31.1 -> 27.6.) Four pieces while a call takes no more than kFourTurnsUpTo, two (as good
   // there) up to kTurnsUpTo, none beyond. From its kTurnsFrom-th call that needs scratch
   // on, a workspace is made large enough for that, once: a program's first calls do not
-  // wait for it.
+  // wait for it. What the device has refused is not asked for again: an allocation and
+  // a free each call would cost more than the turns give.
   static constexpr std::size_t kFourTurnsUpTo = std::size_t(8) << 20;
   static constexpr std::size_t kTurnsUpTo = std::size_t(64) << 20;
   static constexpr int kTurnsFrom = 8;
@@ -70,9 +71,10 @@ class Workspace {
   std::vector<Block> blocks_;
   std::size_t taken_ = 0;       // by the call so far
   int calls_ = 0;               // that needed scratch, up to kTurnsFrom
-  std::size_t turns_ = 2;         // pieces,
-  std::size_t turn_ = 0;          // the one this call starts in,
-  std::size_t wrapped_used_ = 0;  // and what did not fit behind has taken in front of it
+  std::size_t refused_ = ~std::size_t(0);  // the smallest block for turns that could not be had
+  std::size_t turns_ = 2;                  // pieces,
+  std::size_t turn_ = 0;                   // the one this call starts in,
+  std::size_t wrapped_used_ = 0;           // and what did not fit behind has taken in front of it
   bool pinned_ = false;
   bool growth_allowed_ = true;
   bool fixed_ = false;

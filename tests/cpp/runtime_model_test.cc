@@ -52,7 +52,9 @@ struct Runtime {
   hipError_t last_error = hipSuccess;
   bool capturing = false;
   int capture_violations = 0;
-  int allocations = 0;                                // of device memory
+  int allocations = 0;                                // of device memory, refused ones too
+  int frees = 0;
+  std::size_t device_limit = ~std::size_t(0);         // bytes of device memory there are
   bool fill_allocations = true;
   dim3 grid, block;
   std::size_t shared = 0;
@@ -162,9 +164,15 @@ static hipError_t Give(std::map<const char*, std::size_t>* ranges, void* p) {
 }
 hipError_t hipMalloc(void** p, std::size_t bytes) {
   ++R().allocations;
+  std::size_t held = bytes;
+  for (const auto& range : R().device) held += range.second;
+  if (held > R().device_limit) return R().last_error = hipErrorOutOfMemory;
   return Take(&R().device, p, bytes);
 }
-hipError_t hipFree(void* p) { return Give(&R().device, p); }
+hipError_t hipFree(void* p) {
+  ++R().frees;
+  return Give(&R().device, p);
+}
 hipError_t hipHostMalloc(void** p, std::size_t bytes, unsigned) { return Take(&R().pinned, p, bytes); }
 hipError_t hipHostFree(void* p) { return Give(&R().pinned, p); }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
@@ -714,6 +722,45 @@ void ScratchInTurns() {
   }
 }
 
+// A device with no room for a workspace whose calls take turns: it is asked once (or
+// once more for a smaller size that calls come in), the block that there was stays, and calls go on in it
+// without a further allocation or free, which waits for the device.
+void ScratchInTurnsRefused() {
+  const int M = 2000, K = 2051, N = 1800;
+  DeviceCall call(std::size_t(M) * K, std::size_t(K) * N, std::size_t(M) * N);
+  const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, M, K, RUYAMD_ORDER_COL_MAJOR, 4);
+  const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, call.rhs, K, N, RUYAMD_ORDER_ROW_MAJOR, 3);
+  const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, M, N, RUYAMD_ORDER_COL_MAJOR);
+  ruyamd_mat small_l = l, small_d = d;
+  small_l.rows = small_d.rows = M / 3;
+  const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+  for (const bool two_sizes : {false, true}) {
+    Context c;
+    auto run = [&](int i) {
+      const bool small = two_sizes && i % 2;
+      EXPECT(ruyamd_mul(c.ctx, small ? &small_l : &l, &r, &p, small ? &small_d : &d) == RUYAMD_OK, "%s",
+             ruyamd_ctx_last_error(c.ctx));
+    };
+    for (int i = 0; i < 4; ++i) run(i);
+    const auto held = R().device;
+    std::size_t bytes = 0;
+    for (const auto& range : held) bytes += range.second;
+    R().device_limit = bytes + (std::size_t(1) << 20);
+    R().allocations = R().frees = 0;
+    for (int i = 0; i < 20; ++i) run(i);
+    // (What is larger than a size refused before is not asked for either.)
+    EXPECT(R().allocations >= 1 && R().allocations <= 1 + two_sizes && R().frees == 0, "%d allocations, %d frees",
+           R().allocations, R().frees);
+    EXPECT(R().device == held, "the block that there was is gone");
+    EXPECT(R().last_error == hipSuccess, "an error is left behind");
+    R().capturing = true;
+    run(0);
+    R().capturing = false;
+    EXPECT(R().capture_violations == 0, "while recording");
+    R().device_limit = ~std::size_t(0);
+  }
+}
+
 bool Staged(const std::string& kernel) {
   return kernel.find("MfmaGemmKernel") != std::string::npos &&
          (kernel.find("Lb0ELi1EEEv") != std::string::npos || kernel.find("Lb0ELi2EEEv") != std::string::npos);
@@ -817,6 +864,7 @@ int main(int argc, char** argv) {
   else if (which == "raw_rows") RawRowsNeedNoScratch();
   else if (which == "scratch_blocks") ScratchBlocks();
   else if (which == "scratch_in_turns") ScratchInTurns();
+  else if (which == "scratch_in_turns_refused") ScratchInTurnsRefused();
   else if (which == "staged_rule") StagedRule();
   else return 2;
   if (g_failures) {

@@ -357,6 +357,10 @@ def test_calls_take_turns_with_the_pieces_of_their_scratch_memory(runtime_model)
     runtime_model("scratch_in_turns")
 
 
+def test_scratch_memory_for_turns_that_cannot_be_had_is_not_asked_for_again(runtime_model):
+    runtime_model("scratch_in_turns_refused")
+
+
 def test_sums_left_to_the_product_take_no_scratch_memory(runtime_model):
     runtime_model("scratch_blocks")
 
