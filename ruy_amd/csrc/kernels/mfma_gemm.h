@@ -862,7 +862,6 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     // Load n of a step fills rows 8n .. 8n+7 of the slot (A rows first).
     uint32_t goff[kLoads];
     int gk[kLoads];
-    auto set_offsets = [&]() {
 #pragma unroll
     for (int n = 0; n < kLoads; ++n) {
       const int r = (n % 8) * 8 + lane / 8;  // row inside its operand's tile
@@ -884,8 +883,6 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         goff[n] = col < args.n_logical ? uint32_t(col) * uint32_t(args.ldb) + gb * kGranule : kOutOfRange;
       }
     }
-    };
-    set_offsets();
     // Depth offset and limit of the b operand in bytes: twice those of `a`
     // when it is int16 data.
     constexpr int kBScale = kRawB ? 2 : 1;
@@ -968,7 +965,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         for (int v = 0; v < 16; ++v) rows_sum_blocks[i][v] = 0;
     }
     auto mma4 = [&](Frags4 f) {
-      const Frags4 raw = f;
+      [[maybe_unused]] const Frags4 raw = f;
       if constexpr (kFlip) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -998,10 +995,12 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
     };
     // This wave's steps: depth_way, depth_way + kDepthWays, ... of the workgroup's k_tiles steps.
     const int my_steps = k_tiles > depth_way ? (k_tiles - depth_way + kDepthWays - 1) / kDepthWays : 0;
-    // (v_sad_u8 takes every byte 128 too large; a lane adds up half a row.)
+    if constexpr (kFusedSums && !Traits::kSplitB) {
+      // (v_sad_u8 takes every byte 128 too large; a lane adds up half a row.)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      rows_sum[i] = cols_sum[i] = 0u - static_cast<uint32_t>(kBK / 2 * 128) * static_cast<uint32_t>(my_steps);
+      for (int i = 0; i < 2; ++i)
+        rows_sum[i] = cols_sum[i] = 0u - static_cast<uint32_t>(kBK / 2 * 128) * static_cast<uint32_t>(my_steps);
+    }
     if (my_steps > 0 || Traits::kParts) issue_step(depth_way, 0);
     if (my_steps > 1) issue_step(depth_way + kDepthWays, 1);
     load_edge_params();
@@ -1049,6 +1048,9 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
       // One phase on parts[from]: kSplit: the next phase's granules are split
       // on the way; kRead: ... and read again for phase `from` of the step in
       // `read_slot`; kRefill: the loads of a step go to `refill_slot`.
+      uint32_t refill_off[kLoads];
+#pragma unroll
+      for (int n = 0; n < kLoads; ++n) refill_off[n] = goff[n];
       auto phase = [&](auto from_constant, auto split, auto read, auto refill, int read_slot, int refill_slot, int kbase) {
         constexpr int from = decltype(from_constant)::value;
         float_parts::Splitter splitter;
@@ -1060,7 +1062,8 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
           float_parts::Mma<e, !decltype(read)::value>(parts[from][i], parts[from][2 + j], e < 5 ? small[i][j] : full[i][j]);
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (decltype(refill)::value && n < kLoads)
-            LoadToLds16(ring_base + refill_slot * kSlotBytes + n * 1024, goff[n], uint32_t(kbase), n < 8 ? a_rsrc : b_rsrc);
+            LoadToLds16(ring_base + refill_slot * kSlotBytes + n * 1024, refill_off[n], uint32_t(kbase),
+                        n < 8 ? a_rsrc : b_rsrc);
           if constexpr (decltype(split)::value) {
             constexpr int kOps = kGranules * float_parts::kSplitOps;
             constexpr int first = n * kOps / kPhaseMmas;
@@ -1106,13 +1109,13 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         int kbase = __builtin_amdgcn_readfirstlane(phys_inside(depth_way + kDepthWays * refill) * kBK);
         if (refill >= steps) {
 #pragma unroll
-          for (int n = 0; n < kLoads; ++n) goff[n] = kOutOfRange;
+          for (int n = 0; n < kLoads; ++n) refill_off[n] = kOutOfRange;
         } else if (last_is_partial && refill + 1 == steps) {
           // (With the step's offset in the lanes' own: a granule that ends with
           // its row begins in front of the step.)
 #pragma unroll
           for (int n = 0; n < kLoads; ++n)
-            goff[n] = kbase + gk[n] < K ? goff[n] + kbase - past_end(kbase + gk[n]) : kOutOfRange;
+            refill_off[n] = kbase + gk[n] < K ? goff[n] + kbase - past_end(kbase + gk[n]) : kOutOfRange;
           kbase = 0;
         }
         wait_for_step(i + 1);
@@ -1141,7 +1144,6 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
 #pragma unroll
           for (int v = 0; v < 16; ++v) full[b / 2][b % 2][v] = 0;
         WaitVmcnt<0>();  // (what the last trip of the loop asked for)
-        set_offsets();
         if (my_steps > 0) issue_step(depth_way, 0);
         if (my_steps > 1) issue_step(depth_way + kDepthWays, 1);
       }
