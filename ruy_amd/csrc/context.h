@@ -60,12 +60,16 @@ class Workspace {
   // both sides packed, one place -> these: 2048 x 2051 x 2048 23.5 -> 17.7 us, 1024 x 4099 x
   // 1024 20.8 -> 15.6, 1000 x 1500 x 700 13.9 -> 12.8, in two places 14.0; 4000 x 4003 x 1008
   // 31.1 -> 27.6.) Four pieces while a call takes no more than kFourTurnsUpTo, two (as good
-  // there) up to kTurnsUpTo, none beyond. From its kTurnsFrom-th call that needs scratch
+  // there) up to kTurnsUpTo. None beyond: what the XCDs' caches (4 MiB each) hold of
+  // such a call is hardly in the way (160 x 4027 x 8000, 32 MiB packed, 24.1 -> 23.6 us; x 6260
+  // 34.2 -> 33.8), but two contexts' pieces and operands no longer fit the 256 MiB of the
+  // cache in front of memory: 160 x 6260 x 8768 36.2 -> 44.6, 160 x 8003 x 7500 40.5 -> 47.8.
+  // (24 MiB, 160 x 3011 x 8000: 21.3 -> 19.3, two contexts 19.3 and 19.3.) From its kTurnsFrom-th call that needs scratch
   // on, a workspace is made large enough for that, once: a program's first calls do not
   // wait for it. What the device has refused is not asked for again: an allocation and
   // a free each call would cost more than the turns give.
   static constexpr std::size_t kFourTurnsUpTo = std::size_t(8) << 20;
-  static constexpr std::size_t kTurnsUpTo = std::size_t(64) << 20;
+  static constexpr std::size_t kTurnsUpTo = std::size_t(24) << 20;
   static constexpr int kTurnsFrom = 8;
   static std::size_t TurnsFor(std::size_t taken) { return taken <= kFourTurnsUpTo ? 4 : 2; }
   std::vector<Block> blocks_;

@@ -663,7 +663,8 @@ void ScratchBlocks() {
 // A workspace whose calls take turns with its pieces: made large enough once, from
 // the eighth call that needs scratch on, by no more than four times what a call
 // takes; a call that is recorded finds its room whoever's turn it is, also one that
-// takes more than a piece, and a growing one only adds what it needs.
+// takes more than a piece, and a growing one only adds what it needs. Not where a call
+// takes so much that the pieces would crowd the operands out of the caches.
 void ScratchInTurns() {
   auto on_device = [] {
     std::size_t sum = 0;
@@ -673,7 +674,8 @@ void ScratchInTurns() {
   struct {
     int M, K, N;
     bool turns;
-  } const cases[] = {{1000, 1501, 700, true}, {2000, 4099, 2100, true}, {6000, 15000, 1100, false}};
+  } const cases[] = {{1000, 1501, 700, true}, {2000, 4099, 2100, true}, {160, 4027, 6300, false},
+                     {160, 6260, 8768, false}, {6000, 15000, 1100, false}};
   for (const auto& k : cases) {
     DeviceCall call(std::size_t(k.M) * k.K, std::size_t(k.K) * k.N, std::size_t(k.M) * k.N);
     const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, k.M, k.K, RUYAMD_ORDER_COL_MAJOR, 4);
