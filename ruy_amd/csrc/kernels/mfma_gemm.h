@@ -2794,9 +2794,9 @@ enum class Tile { k256x256, k128x128, k128x64, k64x128, k64x64 };
 // What the fit says about the kernels: on int8 the 256x256 tile's depth step
 // (1.16 us) is well under half of what the 64x64 tile needs for the same area
 // (16 x 0.195 us) and 54 % of the 128x128 tile's (4 x 1.07 us / 2 side by side), so it
-// wins whenever its tiles fill most of a round. fp32 (fitted again to 110 shapes,
-// within 4-6 %; choosing by it costs 0.2 % over the fastest): the 128x128 tile's
-// step takes 1.27 us against 4 x 0.37 us, since it splits a float half as often and
+// wins whenever its tiles fill most of a round. fp32 (fitted again to 110 shapes, the
+// 64x64 tile to 400, within 4-6 %; choosing by it costs 0.3 % over the fastest): the 128x128 tile's
+// step takes 1.27 us against 4 x 0.39 us, since it splits a float half as often and
 // asks L2 for half as much, and no larger one is needed. Step of the same area on
 // fp32 instructions: 2.15 and 0.56 us.
 // Tiles of 256x128 and 128x256 were built too, were the fastest at no shape
@@ -2833,7 +2833,7 @@ constexpr TileTiming kF32Timings[] = {
     {Tile::k128x128, 128, 128, 1.46, 6.93, 1.269, 0.78, 1, {}, 0},
     {Tile::k128x64, 128, 64, 2.74, 2.74, 1.190, 0.83, 3, {1.037, 1.980, 2.722}, 0.91},
     {Tile::k64x128, 64, 128, 3.03, 2.54, 1.152, 0.84, 3, {1.114, 1.977, 2.757}, 0.84},
-    {Tile::k64x64, 64, 64, 2.57, 13.39, 0.371, 0.74, 1, {}, 0},
+    {Tile::k64x64, 64, 64, 2.45, 13.0, 0.391, 0.75, 1, {}, 0},
 };
 // The plane-split form of the int16 kernel has the two square large tiles and
 // one of 64 rows x 128 plane columns (64 destination columns); `bn` counts
@@ -3029,8 +3029,16 @@ inline double ModelledMicroseconds(const GemmArgs& args, int num_cus, const Timi
     tiles *= parts;
     k_steps = depth_split::StepsPerPart(k_steps, parts);
   }
-  const int q = tiles / num_cus, r = tiles % num_cus;
-  const double fraction = double(r) / num_cus;
+  int at_once = num_cus;
+  if (parts > 1) {
+    // (The workgroups of a split: an eighth of the tiles, rounded up, with all their
+    // parts to each of the eight XCDs. 82 to 84 tiles in three parts are 33 for 32 CUs:
+    // 194 x 2208 x 1300 fp32 35.4 us, on 32x32 tiles 27.5.)
+    tiles = (tiles / parts + 7) / 8 * parts;
+    at_once = std::max(1, num_cus / 8);
+  }
+  const int q = tiles / at_once, r = tiles % at_once;
+  const double fraction = double(r) / at_once;
   double rounds;  // in units of one workgroup's (overhead + depth steps)
   if (t.occupancy == 1 || tiles <= num_cus) {
     rounds = (q + (r ? t.last_round + (1 - t.last_round) * fraction : 0.0)) * t.step;

@@ -65,7 +65,11 @@ struct F32Small {
 // 47.6 -> 39.0.
 // (Measured against the larger tiles on fp32 instructions. Since two of those run on
 // bf16 parts, their model gives them what they are faster at: 860 x 2832 x 1686 80.4 us
-// here, 71.1 there; 1024^3 23.7 and 18.3.)
+// here, 71.1 there; 1024^3 23.7 and 18.3. Held again against every tile for 840 products: by
+// these rules 2 % run 5 % or more slower than on the fastest, 4.5 % did by the rules for
+// fp32 instructions; 1 %, not 4 %, are over 4 % slower than on those. 205 x 2112 x 352 13.2 us
+// here, 15.4 on 64x64 tiles, 1035 x 2288 x 81 14.5 and 16.2, 488 x 1552 x 2336 41.7 and 45.6, 1088 x
+// 112 x 2145 with one side transposed 15.4 and 17.4.)
 // More than six tiles to a CU: of more than 300 bytes of depth every further one costs
 // 0.5 us, with an operand transposed 0.75, and in place the models have to differ by
 // more. Of 460 products around the line, 16 to 4096 tiles, these tiles took 392 with
@@ -87,13 +91,20 @@ SmallGemmPlan PlanSmallGemmF32(const GemmArgs& args, int num_cus, SmallGemmPlan 
                                       static_cast<uint32_t>(args.lda) | static_cast<uint32_t>(args.ldb)) & 15) != 0;
   const bool many = a_cu > 6 && K > 300;
   const bool streamed = !across && std::min(args.M, args.N) <= 96 && int64_t(std::max(args.M, args.N)) * K >= 48000000;
-  const double here = 3.9 + (!many ? 0.33 : across ? 0.75 : 0.5) * (a_cu - 1) +
-                      (streamed ? 1.75 : straddling ? 1.4 : 1.22) * a_cu * K / 1024.0;
+  // (In place in a single round, us to a KiB of depth: 1.13 on few CUs, on all of them 1.33 or, of
+  // straddling rows, 1.55.)
+  const double filled = static_cast<double>(tiles) / num_cus;
+  const double per_kib = streamed               ? 1.75
+                         : a_cu == 1 && !across ? 1.13 + (straddling ? 0.42 : 0.2) * filled
+                         : straddling           ? 1.4
+                                                : 1.22;
+  const double here = 3.9 + (!many ? 0.33 : across ? 0.75 : 0.5) * (a_cu - 1) + per_kib * a_cu * K / 1024.0;
   const mfma_gemm::TimingModel model = mfma_gemm::TimingModelOf(mfma_gemm::Model::kF32);
   const double pack = packed_bytes ? 2.3 + 0.5e-6 * static_cast<double>(packed_bytes) : 0;
-  // (In place on both sides the models have to differ by more than they err: 1630
-  // tiles x 752 are 29.9 us on the larger tiles, 31.5 by their model, and 30.6 here.)
-  const double margin = packed_bytes ? 1.0 : many ? 0.93 : 0.95;
+  // (Many tiles in place on both sides: where the models differ by more than they err. Shallow
+  // products of packed operands: the larger tiles err the other way, 1643 x 112 x 1502 16.8 us by
+  // their model and 18.8 measured, here 15.4.)
+  const double margin = packed_bytes ? (K < 512 ? 1.1 : 1.0) : many ? 0.96 : 1.0;
   for (int i = 0; i < model.count; ++i)
     if (here >= margin * (mfma_gemm::ModelledMicroseconds(args, num_cus, model, model.tiles[i]) + pack)) return plan;
   plan.waves = 4;

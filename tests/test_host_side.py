@@ -422,6 +422,20 @@ def test_products_that_the_larger_tiles_do_faster_stay_there(runtime_model):
         assert ("SmallGemmKernel" in route[-1]) == small, (call, route)
 
 
+def test_fp32_products_that_the_small_tiles_do_faster_run_there(runtime_model):
+    """Narrow and shallow products near the line to the tiles on bf16 parts, measured on
+    both, us: small tiles, larger ones."""
+    from ruy_amd import _structs as S
+    calls = [((S.F32,) * 4, M, K, N, orders) for M, K, N, orders in [
+        (205, 2112, 352, (1, 0, 0)), (190, 926, 5936, (1, 0, 0)),      # 13.2 15.4, 29.8 33.9
+        (124, 2067, 288, (1, 0, 0)), (212, 1902, 128, (1, 0, 0)),      # 13.0 15.1, 12.5 14.9
+        (1035, 2288, 81, (1, 0, 0)), (488, 1552, 2336, (1, 0, 0)),     # 14.5 16.2, 41.7 45.6
+        (194, 2208, 1300, (1, 1, 0)), (112, 2812, 1280, (0, 0, 1)),    # 27.5 35.4, 19.2 20.9
+        (1643, 112, 1502, (1, 1, 1)), (1088, 112, 2145, (0, 0, 1))]]   # 15.4 18.8, 15.4 17.4
+    for call, route in zip(calls, runtime_model.routes(calls)):
+        assert "SmallGemmKernel" in route[-1], (call, route)
+
+
 def test_products_of_the_staged_tests_run_on_every_staged_kernel(runtime_model):
     """Both rings, both alignments, with sums and without, each beside rows of the
     other operand that come from the cache."""
