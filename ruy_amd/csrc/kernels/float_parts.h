@@ -112,27 +112,23 @@ constexpr int kPartOfB[kProducts] = {0, 2, 1, 0, 1, 0};
 // it: Drain() in front of the first ordinary read of the accumulators, which
 // it names so that no copy of one can be made ahead of it. Nor does the compiler know
 // of the two wait states that a matrix instruction needs behind a vector instruction
-// that writes what it reads, and it may set or copy an accumulator right in front of
-// one: kBehindWrites, everywhere but in loops, which hold no such writes, brings them.
-// A test looks for either in the assembly of the whole kernel.)
-template <int kProduct, bool kBehindWrites = false>
+// that writes what it reads: Settle() brings them behind whatever clears or copies
+// accumulators, in front of a loop and behind it. Both are places where it would be
+// free to do either anyway; a test looks for it in the assembly of the whole kernel.)
+template <int kProduct>
 __device__ __forceinline__ void Mma(const Parts& a, const Parts& b, v16f& acc) {
-  if constexpr (kBehindWrites)
-    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-                 : "+a"(acc)
-                 : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
-  else
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-                 : "+a"(acc)
-                 : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+               : "+a"(acc)
+               : "v"(a.part[kPartOfA[kProduct]]), "v"(b.part[kPartOfB[kProduct]]));
 }
-// Settle() behind the clearing of accumulators: from there on they are registers like
-// any other to the compiler, which otherwise clears others for the way past a loop and
-// copies all of them behind it (1024^3 0.4 us).
+// (To the compiler the accumulators are registers like any other from there on.
+// Otherwise it clears others for the way past a loop and copies all of them behind
+// it: 1024^3 0.4 us.)
 template <int kA, int kB>
 __device__ __forceinline__ void Settle(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {
 #pragma unroll
   for (int b = 0; b < kA * kB; ++b) asm volatile("" : "+a"(x[b / kB][b % kB]), "+a"(y[b / kB][b % kB]));
+  asm volatile("s_nop 1" : "+a"(x[0][0]), "+a"(y[0][0]));
 }
 template <int kA, int kB>
 __device__ __forceinline__ void Drain(v16f (&x)[kA][kB], v16f (&y)[kA][kB]) {

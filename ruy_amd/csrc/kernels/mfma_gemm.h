@@ -1058,8 +1058,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
           constexpr int n = decltype(n_constant)::value;
           constexpr int i = n / 12, j = n / 6 % 2, e = n % 6;
           __builtin_amdgcn_sched_barrier(0);
-          // (What is read again belongs to the loop.)
-          float_parts::Mma<e, !decltype(read)::value>(parts[from][i], parts[from][2 + j], e < 5 ? small[i][j] : full[i][j]);
+          float_parts::Mma<e>(parts[from][i], parts[from][2 + j], e < 5 ? small[i][j] : full[i][j]);
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (decltype(refill)::value && n < kLoads)
             LoadToLds16(ring_base + refill_slot * kSlotBytes + n * 1024, refill_off[n], uint32_t(kbase),
@@ -1126,6 +1125,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         phase(Second(), kYes, kYes, kNo, (i + 1) & 1, 0, 0);
         last = __builtin_amdgcn_readfirstlane(__any(float_parts::Lost(lost)) ? 0 : last);
       }
+      float_parts::Settle(full, small);
       phase(First(), kYes, kNo, kNo, 0, 0, 0);
       phase(Second(), kNo, kNo, kNo, 0, 0, 0);
       float_parts::Drain(full, small);
@@ -1722,6 +1722,7 @@ __device__ __forceinline__ void MfmaGemmBody(const GemmArgs args) {
         phase(Second(), 1 - buffer, buffer, kt + 3);
         return decltype(asks)::value ? __builtin_amdgcn_readfirstlane(told[kt / 8 % 2]) : 0;
       };
+      float_parts::Settle(acc, small);
       for (int kt = 0;; ++kt) {
         for (const int end = min(kt + 7, k_tiles); kt < end; ++kt) step(kt, std::false_type());
         if (kt >= k_tiles || step(kt, std::true_type())) break;
