@@ -10,6 +10,22 @@
 #include "kernels/static_scratch.h"
 
 namespace ruyamd {
+namespace {
+
+// Lets this thread allocate and free device memory while a stream of another
+// thread records a graph in the mode that forbids it to all threads.
+class AllocationBesideCaptures {
+ public:
+  AllocationBesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  ~AllocationBesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  AllocationBesideCaptures(const AllocationBesideCaptures&) = delete;
+  AllocationBesideCaptures& operator=(const AllocationBesideCaptures&) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
+}  // namespace
 
 Workspace::~Workspace() {
   if (fixed_) return;
@@ -77,6 +93,9 @@ void Workspace::Reset() {
   if (may_replace && taken_ > 0 && taken_ <= kTurnsUpTo && (calls_ >= kTurnsFrom || ++calls_ >= kTurnsFrom)) {
     const std::size_t wanted = TurnsFor(taken_) * (taken_ + 256);
     if (capacity() < wanted && wanted < refused_) {
+      // (Another thread may record a graph meanwhile: a program's later calls allocate nothing
+      // else, and this must not end its recording.)
+      AllocationBesideCaptures scope;
       void* p = nullptr;
       if (hipMalloc(&p, wanted) == hipSuccess) {
         for (auto& b : blocks_) (void)hipFree(b.base);

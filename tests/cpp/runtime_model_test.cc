@@ -51,6 +51,8 @@ struct Runtime {
   int fail_at = 0;
   hipError_t last_error = hipSuccess;
   bool capturing = false;
+  bool captured_elsewhere = false;                    // by another thread, in the mode that binds all of them
+  hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;  // of this thread
   int capture_violations = 0;
   int allocations = 0;                                // of device memory, refused ones too
   int frees = 0;
@@ -148,18 +150,23 @@ hipError_t hipLaunchKernel(const void* function, dim3, dim3, void** args, std::s
   return hipSuccess;
 }
 
+// ... nor another thread meanwhile do.
+static void NotWhileAnyoneCaptures() {
+  NotWhileCapturing();
+  if (R().captured_elsewhere && R().mode != hipStreamCaptureModeRelaxed) ++R().capture_violations;
+}
 static hipError_t Take(std::map<const char*, std::size_t>* ranges, void** p, std::size_t bytes) {
   *p = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096 + 4096);
   if (R().fill_allocations) std::memset(*p, 0xCD, bytes);
   (*ranges)[static_cast<char*>(*p)] = bytes;
-  NotWhileCapturing();
+  NotWhileAnyoneCaptures();
   return hipSuccess;
 }
 static hipError_t Give(std::map<const char*, std::size_t>* ranges, void* p) {
   Drain();
   if (p) ranges->erase(static_cast<char*>(p));
   std::free(p);
-  NotWhileCapturing();
+  NotWhileAnyoneCaptures();
   return hipSuccess;
 }
 hipError_t hipMalloc(void** p, std::size_t bytes) {
@@ -172,6 +179,10 @@ hipError_t hipMalloc(void** p, std::size_t bytes) {
 hipError_t hipFree(void* p) {
   ++R().frees;
   return Give(&R().device, p);
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* mode) {
+  std::swap(*mode, R().mode);
+  return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, std::size_t bytes, unsigned) { return Take(&R().pinned, p, bytes); }
 hipError_t hipHostFree(void* p) { return Give(&R().pinned, p); }
@@ -763,6 +774,26 @@ void ScratchInTurnsRefused() {
   }
 }
 
+// The calls after a program's first ones while another thread records a graph: whatever
+// the workspace does for them does not end the recording.
+void ScratchInTurnsBesideACapture() {
+  const int M = 1000, K = 1501, N = 700;
+  DeviceCall call(std::size_t(M) * K, std::size_t(K) * N, std::size_t(M) * N);
+  const ruyamd_mat l = Mat(RUYAMD_DTYPE_I8, call.lhs, M, K, RUYAMD_ORDER_COL_MAJOR, 4);
+  const ruyamd_mat r = Mat(RUYAMD_DTYPE_I8, call.rhs, K, N, RUYAMD_ORDER_ROW_MAJOR, 3);
+  const ruyamd_mat d = Mat(RUYAMD_DTYPE_I8, call.dst, M, N, RUYAMD_ORDER_COL_MAJOR);
+  const ruyamd_mul_params p = Params(RUYAMD_DTYPE_I8);
+  Context c;
+  for (int i = 0; i < 20; ++i) {
+    R().captured_elsewhere = i >= 2;
+    EXPECT(ruyamd_mul(c.ctx, &l, &r, &p, &d) == RUYAMD_OK, "%s", ruyamd_ctx_last_error(c.ctx));
+  }
+  R().captured_elsewhere = false;
+  EXPECT(R().capture_violations == 0, "%d violations", R().capture_violations);
+  EXPECT(R().mode == hipStreamCaptureModeGlobal, "the thread's mode was not given back");
+  R().capture_violations = 0;
+}
+
 bool Staged(const std::string& kernel) {
   return kernel.find("MfmaGemmKernel") != std::string::npos &&
          (kernel.find("Lb0ELi1EEEv") != std::string::npos || kernel.find("Lb0ELi2EEEv") != std::string::npos);
@@ -867,6 +898,7 @@ int main(int argc, char** argv) {
   else if (which == "scratch_blocks") ScratchBlocks();
   else if (which == "scratch_in_turns") ScratchInTurns();
   else if (which == "scratch_in_turns_refused") ScratchInTurnsRefused();
+  else if (which == "scratch_in_turns_beside_a_capture") ScratchInTurnsBesideACapture();
   else if (which == "staged_rule") StagedRule();
   else return 2;
   if (g_failures) {

@@ -361,6 +361,10 @@ def test_scratch_memory_for_turns_that_cannot_be_had_is_not_asked_for_again(runt
     runtime_model("scratch_in_turns_refused")
 
 
+def test_scratch_memory_in_turns_does_not_end_another_threads_recording(runtime_model):
+    runtime_model("scratch_in_turns_beside_a_capture")
+
+
 def test_sums_left_to_the_product_take_no_scratch_memory(runtime_model):
     runtime_model("scratch_blocks")
 
