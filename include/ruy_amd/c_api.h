@@ -86,7 +86,9 @@ enum {
   RUYAMD_KERNEL_I8_MFMA = 2,   /* tiled 8-bit GEMM on the int8 matrix cores:
                                   v_mfma_i32_16x16x64_i8 (256x256 tile) or
                                   v_mfma_i32_32x32x32_i8 (smaller tiles) */
-  RUYAMD_KERNEL_F32_MFMA = 3,  /* tiled fp32 GEMM, v_mfma_f32_32x32x2_f32 */
+  RUYAMD_KERNEL_F32_MFMA = 3,  /* tiled fp32 GEMM: six v_mfma_f32_32x32x16_bf16 a
+                                  product (64x64 and 128x128 tiles) or
+                                  v_mfma_f32_32x32x2_f32 */
   RUYAMD_KERNEL_I8_GEMV = 4,   /* 8-bit skinny kernels, narrow side <= 16
                                   vectors: v_dot4 and a wavefront reduction for
                                   one, v_mfma_i32_16x16x64_i8 for 2..16 */

@@ -35,7 +35,6 @@ struct F32Traits {
   using EightWaves = F32EightWaves;
   static constexpr bool kRawB = false;
   static constexpr bool kPaired = false;
-  using LargeTile = F32Traits;  // (there is none)
   static constexpr bool kSplitB = false;
   static constexpr mfma_gemm::Model kModel = mfma_gemm::Model::kF32;
   static __device__ __forceinline__ int Bits(float x, float) { return __float_as_int(x); }

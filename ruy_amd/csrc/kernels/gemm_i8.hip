@@ -65,8 +65,8 @@ bool GemmI8CanFuseSums(const GemmArgs& args, int num_cus) {
   if (choice.large_parts != 1) return false;
   // (The smallest tile: unless sharing the rows out over its workgroups is cheaper.)
   if (choice.tile == mfma_gemm::Tile::k64x64) return !mfma_gemm::SmallestTileSharesSumsOut(args, num_cus);
-  // The 128x128 tile forms the row sums of `a`, and only those, in grids of
-  // at most one workgroup per CU.
+  // The 128x128 tile forms the row sums of `a`, of `b` or of both, in grids
+  // of at most one workgroup per CU.
   return choice.tile == mfma_gemm::Tile::k128x128 && mfma_gemm::RowSumming128Applies(args, num_cus);
 }
 
@@ -146,7 +146,7 @@ hipError_t LaunchGemmI8(hipStream_t stream, const GemmArgs& args, int num_cus) {
   // Flipped bytes need a whole number of depth steps: bytes past the depth read as zero, which would turn into -128.
   if (flip && args.k_bytes % 128 != 0) return hipErrorInvalidValue;
   if (args.fuse_sums) {
-    // Exists for the smallest tile only.
+    // Exists for the smallest tile and the 128x128 tile.
     if (!GemmI8CanFuseSums(args, num_cus)) return hipErrorInvalidValue;
     if (mfma_gemm::PickTile(args, num_cus, mfma_gemm::Model::kInt8) == mfma_gemm::Tile::k128x128 &&
         (args.sums_wanted & 2))

@@ -34,7 +34,7 @@
 // and 32 bytes of depth; 16: per 16x16 block and 64 bytes of depth), Acc (the
 // accumulator vector of one block: 16 or 4 elements), Mma(a, b, acc)
 // for one 16-byte fragment pair, DrainMma() (called once after the last Mma),
-// LargeTile (the Traits the 256x256 tile runs with), kSplitB (the B operand holds, for every 32
+// LargeTile (the Traits the 256x256 tile runs with; fp32 has no such tile), kSplitB (the B operand holds, for every 32
 // destination columns, 32 high-plane rows followed by 32 low-plane rows whose
 // accumulators are combined), Bits(x, x2) (accumulator element - or combined
 // pair - as raw 32 bits), RawBits(x) / FromRawBits(w) (one accumulator element
@@ -3309,8 +3309,9 @@ hipError_t LaunchSmallestTileBatch(hipStream_t stream, const GemmArgs& args, con
   return LaunchBatch<Traits, 1, kWN, 128, 4, kFusedSums, kFlip, true>(stream, args, batch, count);
 }
 
-// The 128x128 tile with the row sums of `a` formed in the kernel: for grids of
-// at most one workgroup per CU (see kRowSumsOfFourBlocks in the kernel).
+// The 128x128 tile with the row sums of `a`, or (Traits::kSumsOfBothSides) those of
+// both operands, formed in the kernel: for grids of at most one workgroup per CU (see
+// kRowSumsOfFourBlocks in the kernel).
 template <typename Traits, bool kFlip = false>
 hipError_t LaunchRowSumming128(hipStream_t stream, const GemmArgs& args, int num_cus) {
   if (ShallowRing(args, num_cus, 128, 128) || args.split_k > 1) return hipErrorInvalidValue;
@@ -3321,29 +3322,28 @@ template <typename Traits, bool kFlip = false>
 hipError_t LaunchTile(hipStream_t stream, const GemmArgs& args, Tile tile, int num_cus) {
   switch (tile) {
     case Tile::k256x256:
-      // One column of tiles over a large `a`: every byte of it is read once,
-      // with the cache policy for that (StreamsLargeA).
-      if constexpr (Traits::LargeTile::kPaired) {
-        if (args.split_k > 1 && StreamsLargeA(args)) {
+      if constexpr (Traits::kParts) {
+        return hipErrorInvalidValue;  // fp32 has no such tile
+      } else {
+        // One column of tiles over a large `a`: every byte of it is read once,
+        // with the cache policy for that (StreamsLargeA).
+        if constexpr (Traits::LargeTile::kPaired) {
+          if (args.split_k > 1 && StreamsLargeA(args)) {
+            if (args.row_sums)
+              return Launch<typename Traits::LargeTileStreamingA, 4, 4, 128, 2, false, kFlip, false, true, true>(stream,
+                                                                                                                args);
+            return Launch<typename Traits::LargeTileStreamingA, 4, 4, 128, 2, false, kFlip, false, false, true>(stream,
+                                                                                                               args);
+          }
+          if (args.row_sums && args.split_k > 1)
+            return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, true, true>(stream, args);
           if (args.row_sums)
-            return Launch<typename Traits::LargeTileStreamingA, 4, 4, 128, 2, false, kFlip, false, true, true>(stream,
-                                                                                                              args);
-          return Launch<typename Traits::LargeTileStreamingA, 4, 4, 128, 2, false, kFlip, false, false, true>(stream,
-                                                                                                             args);
+            return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, true>(stream, args);
+          if (args.split_k > 1)
+            return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, false, true>(stream, args);
         }
+        return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip>(stream, args);
       }
-      if constexpr (Traits::LargeTile::kPaired) {
-        if (args.row_sums && args.split_k > 1)
-          return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, true, true>(stream, args);
-        if (args.row_sums)
-          return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, true>(stream, args);
-      }
-      if constexpr (Traits::LargeTile::kPaired) {
-        if (args.split_k > 1)
-          return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip, false, false, true>(stream, args);
-      }
-      if constexpr (!Traits::kParts) return Launch<typename Traits::LargeTile, 4, 4, 128, 2, false, kFlip>(stream, args);
-      break;
     case Tile::k128x128:
       if constexpr (Traits::kModel == Model::kInt8) {
         if (args.row_sums && ShallowRing(args, num_cus, 128, 128))
@@ -3371,8 +3371,6 @@ hipError_t LaunchTile(hipStream_t stream, const GemmArgs& args, Tile tile, int n
   }
   if constexpr (!Traits::kSplitB) {
     switch (tile) {
-      case Tile::k256x256:
-        break;
       case Tile::k128x64:
         if constexpr (Traits::kModel == Model::kInt8) {
           if (args.row_sums && ShallowRing(args, num_cus, 128, 64))
