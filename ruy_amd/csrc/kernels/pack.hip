@@ -45,14 +45,9 @@ struct PackPlan {
   PackKind kind = kNone;
   int32_t blocks_c = 0;        // workgroups along the vectors ...
   int32_t parts = 1;           // ... and along the depth
+  int32_t depth = 0;           // bytes of a packed vector, to the end of its last granule
   int32_t k_span = 0;          // depth bytes (fp32: positions) of a part
 };
-
-// Bytes of a packed vector, to the end of its last granule.
-__host__ __device__ inline int PackedDepth(const PackSource& src) {
-  const int bytes = src.K * (src.dtype == RUYAMD_DTYPE_F32 ? 4 : 1);
-  return bytes > 16 ? (bytes + 15) / 16 * 16 : 16;
-}
 
 // Depth-contiguous source of any alignment and depth (8-bit or fp32: bytes are
 // moved): kLanes lanes to a vector, four granules of a lane in flight. (Rows of
@@ -60,7 +55,7 @@ __host__ __device__ inline int PackedDepth(const PackSource& src) {
 // load made the compiler await the first before it issued the next, and the
 // packing of 294 rows of 864 bytes took 4.1 us instead of 3.3.)
 template <int kLanes, bool kShort>
-__device__ __forceinline__ void PackRowsOf(const PackJob& job, int k_span, int bx, int by) {
+__device__ __forceinline__ void PackRowsOf(const PackJob& job, int depth, int k_span, int bx, int by) {
   constexpr int kStep = kLanes * 16;
   const int lane = threadIdx.x % kLanes;
   const int c = bx * (kThreads / kLanes) + static_cast<int>(threadIdx.x / kLanes);
@@ -70,7 +65,7 @@ __device__ __forceinline__ void PackRowsOf(const PackJob& job, int k_span, int b
   const uint8_t* row =
       static_cast<const uint8_t*>(job.src.data) + int64_t(min(c, job.src.count - 1)) * job.src.stride_c * element;
   const uint32_t flip = job.src.dtype == RUYAMD_DTYPE_U8 ? 0x80808080u : 0u;
-  const int k_end = min(PackedDepth(job.src), (by + 1) * k_span);
+  const int k_end = min(depth, (by + 1) * k_span);
   const int end = min(k_end, bytes);
   char* out = static_cast<char*>(job.dst) + int64_t(c) * job.ld;
   constexpr int kInFlight = kShort ? 1 : 4;
@@ -102,12 +97,12 @@ __device__ __forceinline__ void PackRowsOf(const PackJob& job, int k_span, int b
   }
 }
 template <int kLanes>
-__device__ __forceinline__ void PackRows(const PackJob& job, int k_span, int bx, int by) {
+__device__ __forceinline__ void PackRows(const PackJob& job, int depth, int k_span, int bx, int by) {
   const int bytes = job.src.K * (job.src.dtype == RUYAMD_DTYPE_F32 ? 4 : 1);
   if (kLanes == 64 || bytes >= 16)  // (64 lanes only take rows beyond 1 KiB: PlanOf)
-    PackRowsOf<kLanes, false>(job, k_span, bx, by);
+    PackRowsOf<kLanes, false>(job, depth, k_span, bx, by);
   else
-    PackRowsOf<kLanes, true>(job, k_span, bx, by);
+    PackRowsOf<kLanes, true>(job, depth, k_span, bx, by);
 }
 
 // 8-bit source contiguous along the vectors (the transposed case), base and
@@ -118,11 +113,11 @@ __device__ __forceinline__ void PackRows(const PackJob& job, int k_span, int bx,
 // transposes the 4x4 bytes in registers with v_perm_b32 and writes four
 // dwords to the LDS tile, from which the block writes depth-contiguous
 // 16-byte pieces.
-__device__ __forceinline__ void PackTranspose8(const PackJob& job, int k_span, int bx, int by, uint8_t* tile) {
+__device__ __forceinline__ void PackTranspose8(const PackJob& job, int depth, int k_span, int bx, int by, uint8_t* tile) {
   const PackSource& src = job.src;
   const int tid = threadIdx.x;
   const int c0 = bx * kTileC;
-  const int ld = job.ld, depth = PackedDepth(src);
+  const int ld = job.ld;
   const int k_begin = by * k_span;
   const int k_end = min(k_begin + k_span, depth);
   const uint8_t* s = static_cast<const uint8_t*>(src.data);
@@ -191,13 +186,13 @@ __device__ __forceinline__ void PackTranspose8(const PackJob& job, int k_span, i
 // The same for fp32: 32 vectors x 32 depth positions per step through LDS.
 // There are no sums and no conversion for floating point
 // (ruy/pack_common.h:100-133).
-__device__ __forceinline__ void PackTranspose32(const PackJob& job, int k_span, int bx, int by,
+__device__ __forceinline__ void PackTranspose32(const PackJob& job, int depth_bytes, int k_span, int bx, int by,
                                                 float (*tile)[kTile32 + 1]) {
   const PackSource& src = job.src;
   const int tx = threadIdx.x & 31;
   const int ty = threadIdx.x >> 5;  // 0..7
   const int c0 = bx * kTile32;
-  const int ld = job.ld / 4, depth = PackedDepth(src) / 4;
+  const int ld = job.ld / 4, depth = depth_bytes / 4;
   const float* s = static_cast<const float*>(src.data);
   float* dst = static_cast<float*>(job.dst);
   const int k_end = min(depth, (by + 1) * k_span);
@@ -232,18 +227,19 @@ __device__ __forceinline__ void PackTranspose32(const PackJob& job, int k_span, 
 struct PackLaunch {
   PackJob job[2];
   int32_t blocks_c[2];
+  int32_t depth[2];
   int32_t k_span[2];
   int32_t first;  // workgroups of the first operand
 };
 template <int kKind>
-__device__ __forceinline__ void PackOperand(const PackJob& job, int k_span, int blocks_c, int block, void* tile) {
+__device__ __forceinline__ void PackOperand(const PackJob& job, int depth, int k_span, int blocks_c, int block, void* tile) {
   const int by = block < blocks_c ? 0 : block / blocks_c;
   const int bx = block - by * blocks_c;
-  if constexpr (kKind == kRows16) PackRows<16>(job, k_span, bx, by);
-  if constexpr (kKind == kRows64) PackRows<64>(job, k_span, bx, by);
-  if constexpr (kKind == kTranspose8) PackTranspose8(job, k_span, bx, by, static_cast<uint8_t*>(tile));
+  if constexpr (kKind == kRows16) PackRows<16>(job, depth, k_span, bx, by);
+  if constexpr (kKind == kRows64) PackRows<64>(job, depth, k_span, bx, by);
+  if constexpr (kKind == kTranspose8) PackTranspose8(job, depth, k_span, bx, by, static_cast<uint8_t*>(tile));
   if constexpr (kKind == kTranspose32)
-    PackTranspose32(job, k_span, bx, by, static_cast<float(*)[kTile32 + 1]>(tile));
+    PackTranspose32(job, depth, k_span, bx, by, static_cast<float(*)[kTile32 + 1]>(tile));
 }
 constexpr int TileBytes(int kind) {
   return kind == kTranspose8 ? kTileC * kPitch : kind == kTranspose32 ? kTile32 * (kTile32 + 1) * 4 : 16;
@@ -254,9 +250,9 @@ __global__ __launch_bounds__(kThreads) void PackKernel(PackLaunch launch) {
   __shared__ __attribute__((aligned(16))) char tile[kBytes];
   const int block = blockIdx.x;
   if (kSecond == kNone || block < launch.first)
-    PackOperand<kFirst>(launch.job[0], launch.k_span[0], launch.blocks_c[0], block, tile);
+    PackOperand<kFirst>(launch.job[0], launch.depth[0], launch.k_span[0], launch.blocks_c[0], block, tile);
   else
-    PackOperand<kSecond>(launch.job[1], launch.k_span[1], launch.blocks_c[1], block - launch.first, tile);
+    PackOperand<kSecond>(launch.job[1], launch.depth[1], launch.k_span[1], launch.blocks_c[1], block - launch.first, tile);
 }
 
 // The kernel for two kinds (operands of one product have one element size).
@@ -304,10 +300,11 @@ int StepsPerPart(int steps, int blocks_c, int blocks_wanted, int* parts) {
 
 PackPlan PlanOf(const PackSource& src) {
   PackPlan plan;
-  const int32_t ld = PackedDepth(src);
+  const int32_t bytes = src.K * (src.dtype == RUYAMD_DTYPE_F32 ? 4 : 1);
+  const int32_t depth = plan.depth = bytes > 16 ? (bytes + 15) / 16 * 16 : 16;
   if (src.stride_k == 1) {
     // 16 lanes to a row of up to 1 KiB (what they have in flight at a time).
-    plan.kind = ld <= 1024 ? kRows16 : kRows64;
+    plan.kind = depth <= 1024 ? kRows16 : kRows64;
     const int lanes = plan.kind == kRows16 ? 16 : 64;
     const int rows_per_block = kThreads / lanes;
     plan.blocks_c = (src.count + rows_per_block - 1) / rows_per_block;
@@ -317,7 +314,7 @@ PackPlan PlanOf(const PackSource& src) {
     // least. So it is for a handful of vectors (the narrow side of a skinny
     // product: 10 x 7805 int8 4.3 us in 3 workgroups, 1.8 in 24).
     const int step = lanes * 16;
-    const int steps = (ld + step - 1) / step;
+    const int steps = (depth + step - 1) / step;
     int per_part = steps;
     if ((steps > 8 && plan.blocks_c < 256) || plan.blocks_c < 16)
       per_part = StepsPerPart(steps, plan.blocks_c, 512, &plan.parts);
@@ -325,7 +322,7 @@ PackPlan PlanOf(const PackSource& src) {
   } else if (src.dtype == RUYAMD_DTYPE_F32) {
     plan.kind = kTranspose32;
     plan.blocks_c = (src.count + kTile32 - 1) / kTile32;
-    plan.k_span = kTile32 * StepsPerPart((ld / 4 + kTile32 - 1) / kTile32, plan.blocks_c, 4096, &plan.parts);
+    plan.k_span = kTile32 * StepsPerPart((depth / 4 + kTile32 - 1) / kTile32, plan.blocks_c, 4096, &plan.parts);
   } else {
     plan.kind = kTranspose8;
     plan.blocks_c = (src.count + kTileC - 1) / kTileC;
@@ -333,7 +330,7 @@ PackPlan PlanOf(const PackSource& src) {
     // (about a microsecond each), so a block gets as few of them as some two
     // thousand blocks allow (a 2048 x 2048 operand: 7.2 -> 3.6 us); one or two
     // stay together, and the sums come with them.
-    const int steps = (ld + kTileK - 1) / kTileK;
+    const int steps = (depth + kTileK - 1) / kTileK;
     int per_part = steps;
     if (steps > 2) per_part = StepsPerPart(steps, plan.blocks_c, 2048, &plan.parts);
     plan.k_span = per_part * kTileK;
@@ -537,6 +534,7 @@ hipError_t LaunchPack(hipStream_t stream, const PackJob* jobs, int count) {
       return hipErrorInvalidValue;
     launch.job[used] = job;
     launch.blocks_c[used] = plan.blocks_c;
+    launch.depth[used] = plan.depth;
     launch.k_span[used] = plan.k_span;
     if (used == 0) launch.first = plan.blocks_c * plan.parts;
     kinds[used] = plan.kind;
